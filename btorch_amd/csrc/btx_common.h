@@ -72,6 +72,7 @@ struct Ctl {
     // the latest decided, that marked
     int lane_bits_mode[4];
     int lane_bits_run;
+    int bin_of_sub[64];  // delay bin by virtual-row offset, -1 = not read
 };
 
 // Slots per destination of the ordered mode are held in registers when the

@@ -292,9 +292,14 @@ __device__ __forceinline__ float prm(const float* p, int64_t stride, int64_t n) 
 
 // Neuron parameters requested at the start of the F role, so that their
 // loads overlap the reduction: the shared value of each (used when its
-// stride is 0).
+// stride is 0).  The gather step requests every parameter of its neuron; only
+// it fills the fields after the first six.
 struct PreParams {
     float vth, vr, cm, tref, tsyn, ksyn;
+    float vrest, kv;                                       // GLIF3
+    float asc_k[kMaxAsc], asc_kk[kMaxAsc], asc_amp[kMaxAsc];
+    float sg, tsyn2, ksyn2, sa;                            // alpha, dual exponential
+    float tc[BTX_TC_NPARAM];                               // two-compartment
 };
 
 __device__ __forceinline__ float prm_or(const float* p, int64_t stride, int64_t n, float shared) {
@@ -384,6 +389,17 @@ __device__ __forceinline__ uint32_t poisson_drive4(const StepArgs& a, const Driv
     return m;
 }
 
+// The same drive of one neuron.
+__device__ __forceinline__ bool poisson_drive1(const StepArgs& a, const DriveArgs& d,
+                                               int64_t nidx) {
+    if (a.in_prob == nullptr) return false;
+    const uint64_t step = (uint64_t)(d.t0 + a.t);
+    const uint64_t stream = mix64(d.seed ^ (step * 0x100000001b3ull));
+    const uint64_t h = mix64(stream + ((uint64_t)(nidx >> 1) + 1) * 0x9e3779b97f4a7c15ull);
+    const uint32_t bits = (uint32_t)(((nidx & 1) ? (h >> 16) : (h >> 40)) & 0xffffffull);
+    return (float)bits * (1.0f / 16777216.0f) < d.prob;
+}
+
 // Somatic input of a neuron: the stored psc (decayed current of the previous
 // step) plus the previous step's summed push `wz`, plus x and the drive.
 template <bool REC>
@@ -435,17 +451,17 @@ struct Syn2 {
 // (synapse.py:243-253, 307-317, 394-406): alpha kinds h = h + gain*(W z),
 // the dual exponential g_r + W z, g_d + W z and psc = a*(g_d - g_r).  psc
 // then holds the current the neuron receives.
-template <bool REC>
+template <bool REC, bool PRE>
 __device__ __forceinline__ float syn_x_input(const StepArgs& a, int64_t i, int64_t nidx,
                                             float& psc, Syn2& s2, float wz, float xin,
-                                            float drive) {
+                                            float drive, const PreParams& pq) {
     if (a.prev) {
         if (a.syn == BTX_SYN_DUAL_EXP) {
             s2.h1 = s2.h1 + wz;
             s2.h2 = s2.h2 + wz;
-            psc = prm(a.sa, a.sa_s, nidx) * (s2.h2 - s2.h1);
+            psc = (PRE ? pq.sa : prm(a.sa, a.sa_s, nidx)) * (s2.h2 - s2.h1);
         } else {
-            s2.h1 = s2.h1 + prm(a.sg, a.sg_s, nidx) * wz;
+            s2.h1 = s2.h1 + (PRE ? pq.sg : prm(a.sg, a.sg_s, nidx)) * wz;
         }
         if (REC) {
             if (a.rec_psc_prev) a.rec_psc_prev[i] = psc;
@@ -460,11 +476,12 @@ __device__ __forceinline__ float syn_x_input(const StepArgs& a, int64_t i, int64
 // The decay part of the next step's synapse update (conductance_charge,
 // synapse.py:239-241, 304-305, 390-392, through exp_euler_step, ode.py:50);
 // the push W z of this step completes it at the next step.
+template <bool PRE>
 __device__ __forceinline__ void syn_x_decay(const StepArgs& a, int64_t nidx, float& psc,
-                                           Syn2& s2) {
-    const float k = prm(a.ksyn, a.ksyn_s, nidx);
+                                           Syn2& s2, const PreParams& pq) {
+    const float k = PRE ? pq.ksyn : prm(a.ksyn, a.ksyn_s, nidx);
     if (a.syn == BTX_SYN_ALPHA) {
-        const float ts = prm(a.tsyn, a.tsyn_s, nidx);
+        const float ts = PRE ? pq.tsyn : prm(a.tsyn, a.tsyn_s, nidx);
         const float h = s2.h1;
         psc = psc + k * ((-psc) / ts + h / ts);
         s2.h1 = h + k * ((-h) / ts);
@@ -473,9 +490,9 @@ __device__ __forceinline__ void syn_x_decay(const StepArgs& a, int64_t nidx, flo
         psc = k * psc + k * h;
         s2.h1 = k * h;
     } else {
-        const float tr = prm(a.tsyn, a.tsyn_s, nidx);
-        const float td = prm(a.tsyn2, a.tsyn2_s, nidx);
-        const float kd = prm(a.ksyn2, a.ksyn2_s, nidx);
+        const float tr = PRE ? pq.tsyn : prm(a.tsyn, a.tsyn_s, nidx);
+        const float td = PRE ? pq.tsyn2 : prm(a.tsyn2, a.tsyn2_s, nidx);
+        const float kd = PRE ? pq.ksyn2 : prm(a.ksyn2, a.ksyn2_s, nidx);
         s2.h1 = s2.h1 + k * ((-s2.h1) / tr);
         s2.h2 = s2.h2 + kd * ((-s2.h2) / td);
     }
@@ -484,13 +501,14 @@ __device__ __forceinline__ void syn_x_decay(const StepArgs& a, int64_t nidx, flo
 // One LIF or GLIF3 neuron of the fused step.  `psc` enters as the stored psc
 // and leaves as this step's decayed current.  `ia` holds the neuron's
 // after-spike currents (GLIF3).  Returns the spike (0/1).
-template <int KIND, bool REC, bool SHR, bool SX = false>
+// SHR: the parameters other than tau are those of `q`; CM1: c_m is 1.
+template <int KIND, bool REC, bool SHR, bool SX = false, bool CM1 = SHR>
 __device__ __forceinline__ float lif_exp_neuron(const StepArgs& a, int64_t lane, int64_t nidx,
                                                 int64_t i, float& psc, float wz, float xin,
                                                 float drive, float& v, float& ref, float* ia,
                                                 const PreParams& q, float tau, Syn2* s2 = nullptr,
                                                 int hard = -1) {
-    const float I = SX ? syn_x_input<REC>(a, i, nidx, psc, *s2, wz, xin, drive)
+    const float I = SX ? syn_x_input<REC, SHR>(a, i, nidx, psc, *s2, wz, xin, drive, q)
                        : soma_input<REC>(a, i, psc, wz, xin, drive);
     const float vth = prm_sh<SHR>(a.vth, a.vth_s, nidx, q.vth);
     const float vr = prm_sh<SHR>(a.vr, a.vr_s, nidx, q.vr);
@@ -503,17 +521,19 @@ __device__ __forceinline__ float lif_exp_neuron(const StepArgs& a, int64_t lane,
 #pragma unroll
         for (int j = 0; j < kMaxAsc; ++j)
             if (j < a.n_asc) isum = isum + ia[j];
-        const float dv = (-(v - prm(a.vrest, a.vrest_s, nidx))) / tau +
+        const float dv = (-(v - (SHR ? q.vrest : prm(a.vrest, a.vrest_s, nidx)))) / tau +
                          (I + isum) / cm;
-        v1 = v + prm(a.kv, a.kv_s, nidx) * dv;
+        v1 = v + (SHR ? q.kv : prm(a.kv, a.kv_s, nidx)) * dv;
         // adaptation
         const int64_t qa = nidx * a.n_asc;
 #pragma unroll
         for (int j = 0; j < kMaxAsc; ++j)
-            if (j < a.n_asc) ia[j] = ia[j] + a.asc_kk[qa + j] * ((-a.asc_k[qa + j]) * ia[j]);
+            if (j < a.n_asc)
+                ia[j] = ia[j] + (SHR ? q.asc_kk[j] : a.asc_kk[qa + j]) *
+                                    ((-(SHR ? q.asc_k[j] : a.asc_k[qa + j])) * ia[j]);
     } else {
-        // SHR launches with c_m == 1 skip the division (x / 1 == x)
-        const float dv = (-(v - vr)) / tau + (SHR ? I : I / cm);
+        // launches with c_m == 1 skip the division (x / 1 == x)
+        const float dv = (-(v - vr)) / tau + (CM1 ? I : I / cm);
         v1 = v + a.dt * dv;
     }
     if (REC && a.rec_v_pre) a.rec_v_pre[i] = v1;
@@ -530,11 +550,11 @@ __device__ __forceinline__ float lif_exp_neuron(const StepArgs& a, int64_t lane,
         const int64_t qa = nidx * a.n_asc;
 #pragma unroll
         for (int j = 0; j < kMaxAsc; ++j)
-            if (j < a.n_asc) ia[j] = ia[j] + a.asc_amp[qa + j] * s;
+            if (j < a.n_asc) ia[j] = ia[j] + (SHR ? q.asc_amp[j] : a.asc_amp[qa + j]) * s;
     }
     if (SX) {
         step_records<REC>(a, lane, nidx, i, s, v);
-        syn_x_decay(a, nidx, psc, *s2);
+        syn_x_decay<SHR>(a, nidx, psc, *s2, q);
     } else {
         step_outputs<REC, SHR>(a, lane, nidx, i, s, v, psc, q);
     }
@@ -546,12 +566,12 @@ __device__ __forceinline__ float lif_exp_neuron(const StepArgs& a, int64_t lane,
 // exponential initiation term, Heaviside spike at the adaptive threshold,
 // hard reset, bAP current for the next step, threshold decay and increment.
 // `xa` is the apical input.  Returns the spike (0/1).
-template <bool REC>
+template <bool REC, bool PRE = false>
 __device__ __forceinline__ float two_comp_neuron(const StepArgs& a, int64_t lane, int64_t nidx,
                                                  int64_t i, float& psc, float wz, float xin,
                                                  float drive, float xa, float& v, float& ia,
                                                  float& ibap, float& th, const PreParams& q) {
-#define TCP(k) prm(a.tcp[k], a.tcs[k], nidx)
+#define TCP(k) (PRE ? q.tc[k] : prm(a.tcp[k], a.tcs[k], nidx))
     const float I = soma_input<REC>(a, i, psc, wz, xin, drive);
     if (REC && a.rec_v_prev) a.rec_v_prev[i] = v;
     // apical current: w_Ca * sigmoid(i_a - theta_Ca) is +-0 for w_Ca == 0
@@ -563,7 +583,7 @@ __device__ __forceinline__ float two_comp_neuron(const StepArgs& a, int64_t lane
                                                  : wca * (1.f / (1.f + expf(-z)));
     const float ia1 = (ia + TCP(BTX_TC_DA) * ((xa + plateau) + ibap)) / TCP(BTX_TC_DA1);
     // soma
-    const float thr = prm_or(a.vth, a.vth_s, nidx, q.vth) + th;
+    const float thr = prm_sh<PRE>(a.vth, a.vth_s, nidx, q.vth) + th;
     const float total = I + TCP(BTX_TC_W_AS) * ia1;
     const float dT = TCP(BTX_TC_DT);
     float ex = 0.f;
@@ -578,7 +598,7 @@ __device__ __forceinline__ float two_comp_neuron(const StepArgs& a, int64_t lane
     if (REC && a.rec_v_pre) a.rec_v_pre[i] = vp;
     const float s = (vp - thr) >= 0.f ? 1.f : 0.f;
     ia = ia1;
-    v = vp - (vp - prm_or(a.vr, a.vr_s, nidx, q.vr)) * s;
+    v = vp - (vp - prm_sh<PRE>(a.vr, a.vr_s, nidx, q.vr)) * s;
     ibap = TCP(BTX_TC_W_SA) * s;
     th = th / TCP(BTX_TC_DTH1) + TCP(BTX_TC_DELTA_TH) * s;
 #undef TCP
@@ -587,7 +607,7 @@ __device__ __forceinline__ float two_comp_neuron(const StepArgs& a, int64_t lane
         if (a.rec_ibap) a.rec_ibap[i] = ibap;
         if (a.rec_th) a.rec_th[i] = th;
     }
-    step_outputs<REC>(a, lane, nidx, i, s, v, psc, q);
+    step_outputs<REC, PRE>(a, lane, nidx, i, s, v, psc, q);
     return s;
 }
 
@@ -1204,7 +1224,7 @@ struct FastDiv {
     int l;
 };
 
-__device__ __forceinline__ FastDiv fast_div(int d) {
+__host__ __device__ __forceinline__ FastDiv fast_div(int d) {
     int l = 0;
     while ((1 << l) < d) ++l;
     const uint64_t m = ((uint64_t)1 << 32) * (((uint64_t)1 << l) - (uint64_t)d) / (uint64_t)d + 1;
@@ -1526,6 +1546,377 @@ __global__ __launch_bounds__(kThreads, KIND == kLif ? 7 : 1) void k_step(StepArg
     }
 }
 
+// The last push's sum wz added to the synapse of one neuron (and recorded:
+// psc in `rec`, the other synapse states in a.rec_sh1_prev / a.rec_sh2_prev).
+__device__ __forceinline__ void finish_neuron(const StepArgs& a, float* __restrict__ rec,
+                                              int64_t i, int64_t nidx, float wz) {
+    if (a.syn == BTX_SYN_EXP) {
+        const float q = a.psc[i] + wz;
+        a.psc[i] = q;
+        if (rec) rec[i] = q;
+    } else if (a.syn == BTX_SYN_DUAL_EXP) {
+        const float g1 = a.sh1[i] + wz;
+        const float g2 = a.sh2[i] + wz;
+        const float q = prm(a.sa, a.sa_s, nidx) * (g2 - g1);
+        a.sh1[i] = g1;
+        a.sh2[i] = g2;
+        a.psc[i] = q;
+        if (rec) rec[i] = q;
+        if (a.rec_sh1_prev) a.rec_sh1_prev[i] = g1;
+        if (a.rec_sh2_prev) a.rec_sh2_prev[i] = g2;
+    } else {
+        const float h = a.sh1[i] + prm(a.sg, a.sg_s, nidx) * wz;
+        a.sh1[i] = h;
+        if (rec) rec[i] = a.psc[i];
+        if (a.rec_sh1_prev) a.rec_sh1_prev[i] = h;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Gather step: nets whose edges are cheaper to read than a push is to bin
+// ---------------------------------------------------------------------------
+
+constexpr int kGatherNeurons = 32;             // neurons per workgroup = half a spike word
+constexpr int kGatherThreads = 512;            // 8 wavefronts, four neurons' edges each
+constexpr int kGatherLanes = 16;               // lanes per workgroup, at most
+constexpr int kGatherBits = 48 * 1024;         // bytes of spike words staged in LDS, at most
+constexpr int kGatherAhead = 8;                // 64-edge chunks a wavefront requests at a time
+
+struct GatherArgs {
+    const int64_t* csc_ptr;
+    const int32_t* csc_src;
+    const float* csc_w;
+    const uint64_t* ring_words;  // [R][lanes][nwords]
+    Ctl* ctl;                    // bin_delay, bin_of_sub
+    int64_t lanes;
+    const uint64_t* lane_bits;   // [R][n][lw]
+    uint16_t* lane_bits_out;     // this step's slot, 4*lw lane groups a neuron
+    int lw;
+    int nbins;
+    int csr_d;
+    FastDiv fd;                  // by csr_d
+    int R;
+    int slot0;                   // slot of the push being summed, (cursor + t - 1) mod R
+    int delay0;                  // the only bin's delay when nbins == 1
+    int fin;                     // 1 = add the run's last push, no step
+    float* rec_psc_last;         // fin: psc record or NULL
+};
+
+// One step of a net as one launch: every neuron sums its active incoming
+// edges of the previous step's push itself, in the coalesced order from +0.0f
+// (the terms and the order of the binned push, so the same bits), then
+// integrates.  No terms, bins, lists or sort, and no second launch for a net
+// whose synapses deliver without delay: the push of step t - 1 reads ring
+// slots up to its own, all written before this launch, which writes another.
+//
+// A workgroup owns 32 neurons of up to 16 lanes, a wavefront four of them,
+// whose edges are contiguous: 64 edges at a time, one per lane of the
+// wavefront, a chunk of one neuron.  ONE (a single lane): the spike words of
+// every delay bin's slot are staged in LDS and each edge tests its source's
+// bit there.  Otherwise each edge reads the lane bits of its source, and
+// thread b sums lane b.  Either way one ballot names the chunk's active edges
+// and a scalar loop adds their weights in order.  The first 512 edges and the
+// neurons' state are requested before anything is waited for.
+template <int KIND_SX, bool ONE>
+__global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, GatherArgs g) {
+    constexpr int KIND = KIND_SX & ~kSynX;
+    constexpr bool SX = (KIND_SX & kSynX) != 0;
+    constexpr bool MIX = KIND == kMixed;
+    constexpr bool GLIF = KIND == kGlif3 || MIX;
+    constexpr bool TC = KIND == kTwoComp || MIX;
+    // ONE: half words of every bin's slot, [nbins][2 * nwords], and a zero
+    extern __shared__ uint32_t __attribute__((aligned(16))) s_bits[];
+    __shared__ float s_sum[kGatherLanes * kGatherNeurons];
+    __shared__ uint32_t s_half[kGatherLanes];
+    // virtual-row offset -> first word of its bin (ONE) or its ring slot, or -1
+    __shared__ int s_row[BTX_MAX_BINS];
+    const int tid = threadIdx.x, ln = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform across the wavefront
+    const int64_t j0 = (int64_t)blockIdx.x * kGatherNeurons;
+    const int64_t lane0 = (int64_t)blockIdx.y * kGatherLanes;
+    const int lg = ONE ? 1 : (int)(g.lanes - lane0 < kGatherLanes ? g.lanes - lane0 : kGatherLanes);
+    const int nw32 = 2 * (int)a.nwords;
+
+    // this wavefront's edges: neurons d0 .. d0+3
+    const int64_t d0 = j0 + 4 * wv;
+    int64_t e0 = 0;
+    int bound[5] = {0, 0, 0, 0, 0};
+    if (a.prev) {
+        e0 = ld_const(g.csc_ptr + (d0 < a.n ? d0 : a.n));
+#pragma unroll
+        for (int k = 1; k < 5; ++k)
+            bound[k] = (int)(ld_const(g.csc_ptr + (d0 + k < a.n ? d0 + k : a.n)) - e0);
+    }
+    const int none = g.nbins * nw32;  // an LDS word that stays 0
+
+    // the neuron this thread integrates
+    const int my_lane = tid / kGatherNeurons, my_k = tid % kGatherNeurons;
+    const int64_t lane = lane0 + my_lane, nidx = j0 + my_k;
+    const int64_t i = lane * a.n + nidx;
+    const bool mine = my_lane < lg && nidx < a.n;
+    bool live = mine;
+    if (mine && a.lane_t_end != nullptr) live = a.in_t0[lane] + a.t < a.lane_t_end[lane];
+    float v = 0.f, p = 0.f, r = 0.f, x = 0.f, ta = 0.f, tb = 0.f, tt = 0.f, xa = 0.f, tau = 1.f;
+    Syn2 s2{0.f, 0.f};
+    float ia[GLIF ? kMaxAsc : 1] = {};
+    PreParams q{0.f, 0.f, 1.f, 0.f, 1.f, 0.f};  // the rest is read by its models only
+    uint32_t code = 0;
+    if (!g.fin && live) {
+        v = a.v[i];
+        p = a.psc[i];
+        if (SX) {
+            s2.h1 = a.sh1[i];
+            if (a.syn == BTX_SYN_DUAL_EXP) s2.h2 = a.sh2[i];
+        }
+        if (a.use_ref) r = a.ref[i];
+        if (a.x) x = a.x[i];
+        if (TC && (!MIX || a.tia != nullptr)) {
+            ta = a.tia[i];
+            tb = a.tibap[i];
+            tt = a.tth[i];
+            if (a.xa) xa = a.xa[i];
+        }
+        if (MIX) code = a.kinds[nidx];
+        if (!TC || MIX) tau = prm(a.tau, a.tau_s, nidx);
+        if (GLIF && a.iasc != nullptr) {
+#pragma unroll
+            for (int j = 0; j < kMaxAsc; ++j)
+                if (j < a.n_asc) ia[GLIF ? j : 0] = a.iasc[i * a.n_asc + j];
+        }
+        q.vth = prm(a.vth, a.vth_s, nidx);
+        q.vr = prm(a.vr, a.vr_s, nidx);
+        if (KIND != kTwoComp) q.cm = prm(a.cm, a.cm_s, nidx);
+        if (a.use_ref) q.tref = prm(a.tref, a.tref_s, nidx);
+        q.tsyn = prm(a.tsyn, a.tsyn_s, nidx);
+        q.ksyn = prm(a.ksyn, a.ksyn_s, nidx);
+        if (SX) {
+            if (a.syn == BTX_SYN_DUAL_EXP) {
+                q.tsyn2 = prm(a.tsyn2, a.tsyn2_s, nidx);
+                q.ksyn2 = prm(a.ksyn2, a.ksyn2_s, nidx);
+                q.sa = prm(a.sa, a.sa_s, nidx);
+            } else {
+                q.sg = prm(a.sg, a.sg_s, nidx);
+            }
+        }
+        if (GLIF && a.iasc != nullptr) {
+            q.vrest = prm(a.vrest, a.vrest_s, nidx);
+            q.kv = prm(a.kv, a.kv_s, nidx);
+#pragma unroll
+            for (int j = 0; j < kMaxAsc; ++j) {
+                if (j < a.n_asc) {
+                    q.asc_k[j] = a.asc_k[nidx * a.n_asc + j];
+                    q.asc_kk[j] = a.asc_kk[nidx * a.n_asc + j];
+                    q.asc_amp[j] = a.asc_amp[nidx * a.n_asc + j];
+                }
+            }
+        }
+        if (TC && (!MIX || a.tia != nullptr)) {
+#pragma unroll
+            for (int j = 0; j < BTX_TC_NPARAM; ++j) q.tc[j] = prm(a.tcp[j], a.tcs[j], nidx);
+        }
+    }
+
+    float wz = 0.f;
+    if (a.prev) {
+        const int32_t* es = g.csc_src + e0;
+        const float* ew = g.csc_w + e0;
+        // 64-edge chunks of one neuron each: `at` is the next edge, `ni` its
+        // neuron, `end` that neuron's last edge + 1
+        int at = 0, ni = 0, end = bound[1];
+        int er[kGatherAhead], own[kGatherAhead];
+        float wr[kGatherAhead];
+        auto request = [&]() {
+#pragma unroll
+            for (int u = 0; u < kGatherAhead; ++u) {
+                while (at == end && ni < 3) {
+                    ++ni;
+                    end = ni == 1 ? bound[2] : ni == 2 ? bound[3] : bound[4];
+                }
+                const int e = at + ln;
+                own[u] = at < end ? ni : 4;
+                er[u] = e < end ? es[e] : -1;
+                wr[u] = e < end ? ew[e] : 0.f;
+                at = at + 64 < end ? at + 64 : end;
+            }
+        };
+        request();
+        // the ring slot of a bin: its delay before the push being summed
+        auto slot_of = [&](int j) {
+            int slot = g.slot0 - (g.nbins == 1 ? g.delay0 : ld_const(&g.ctl->bin_delay[j]));
+            return slot + (slot < 0 ? g.R : 0);
+        };
+        if (ONE) {
+            // the spike words of every bin's slot, shared by the wavefronts
+            // when there are fewer bins than those
+            const int share = (kGatherThreads / 64) / g.nbins > 1 ? (kGatherThreads / 64) / g.nbins : 1;
+            const int part = (nw32 + share - 1) / share;
+            for (int row = wv; row < g.nbins * share; row += kGatherThreads / 64) {
+                const int j = share == 1 ? row : row / share;
+                const int w0 = (row - j * share) * part;
+                const int w1 = w0 + part < nw32 ? w0 + part : nw32;
+                const uint32_t* src = (const uint32_t*)(g.ring_words + slot_of(j) * a.nwords);
+                uint32_t* dst = s_bits + j * nw32;
+                // straight into LDS, a wavefront's 64 consecutive half words at a time
+                for (int w = w0; w < w1; w += 64)
+                    if (w + ln < w1)
+                        __builtin_amdgcn_global_load_lds(
+                            (const __attribute__((address_space(1))) uint32_t*)(src + w + ln),
+                            (__attribute__((address_space(3))) uint32_t*)(dst + w), 4, 0, 0);
+            }
+            if (tid == 0) s_bits[none] = 0u;
+        }
+        if (tid < g.csr_d) {
+            const int j = g.csr_d == 1 ? 0 : g.ctl->bin_of_sub[tid];
+            int dl = g.delay0;
+            if (g.nbins > 1 && j >= 0) dl = g.ctl->bin_delay[j];
+            const int slot = g.slot0 - dl + (g.slot0 < dl ? g.R : 0);
+            s_row[tid] = j < 0 ? -1 : ONE ? j * nw32 : slot;
+        }
+        if (ln < kGatherLanes * 4) s_sum[64 * wv + ln] = 0.f;
+        if (ONE) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the words are in LDS
+        __syncthreads();
+        // ONE: the running sum, the same in every thread; else thread b holds
+        // lane b's
+        float acc = 0.f;
+        int cur = 4;
+        for (;;) {
+            // four chunks at a time, to hold the register count
+#pragma unroll
+            for (int u0 = 0; u0 < kGatherAhead; u0 += 4) {
+                if (own[u0] == 4) break;
+                // what every edge's source pushed: its bit (ONE) or its lanes' bits
+                uint32_t wd[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int e = er[u0 + u];
+                    int src = e < 0 ? 0 : e, sub = 0;
+                    if (g.csr_d > 1) {
+                        const int vr = src;
+                        src = (int)div_u31(g.fd, (uint32_t)vr);
+                        sub = vr - src * g.csr_d;
+                    }
+                    const int first = s_row[sub];
+                    const bool in = e >= 0 && first >= 0;
+                    if (ONE) {
+                        wd[u] = (s_bits[in ? first + (src >> 5) : none] >> (src & 31)) & 1u;
+                    } else {
+                        const uint16_t* q = (const uint16_t*)(g.lane_bits +
+                                                              ((int64_t)first * a.n + src) * g.lw);
+                        wd[u] = in ? q[blockIdx.y] : 0u;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (own[u0 + u] != cur) {
+                        if (cur < 4 && ln < lg) s_sum[ln * kGatherNeurons + 4 * wv + cur] = acc;
+                        cur = own[u0 + u];
+                        acc = 0.f;
+                    }
+                    uint64_t on = __ballot(wd[u] != 0u);
+                    while (on) {
+                        const int k = __ffsll((unsigned long long)on) - 1;
+                        const float w = __int_as_float(
+                            __builtin_amdgcn_readlane(__float_as_int(wr[u0 + u]), k));
+                        if (ONE) {
+                            acc = acc + w;
+                        } else {
+                            // a lane without the bit adds +0.0f: its sum, never
+                            // -0.0f, keeps its bits
+                            const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)wd[u], k);
+                            acc = acc + (((m >> (ln & 15)) & 1u) ? w : 0.f);
+                        }
+                        on &= on - 1ull;
+                    }
+                }
+            }
+            if (at == bound[4]) break;
+            request();
+        }
+        if (cur < 4 && ln < lg) s_sum[ln * kGatherNeurons + 4 * wv + cur] = acc;
+        __syncthreads();
+        if (mine) wz = s_sum[tid];
+    }
+
+    if (g.fin) {
+        // every step was pulled and every slot's lane bits are current; a run
+        // of the other route that follows marks them anew before it pulls
+        // again (its slots are not zeroed ahead)
+        if (blockIdx.x == 0 && blockIdx.y == 0 && tid < 4) {
+            g.ctl->push_mode[tid] = 1;
+            if (tid == 0) g.ctl->lane_bits_run = 0;
+        }
+        // a lane past its trial end at the last step pushed nothing
+        if (mine) finish_neuron(a, g.rec_psc_last, i, nidx, live ? wz : 0.f);
+        return;
+    }
+    float s = 0.f;
+    if (live) {
+        const DriveArgs dargs = drive_args(a, lane);
+        const float drv = poisson_drive1(a, dargs, nidx) ? a.in_kick : 0.f;
+        const bool ref_live = __float_as_uint(r) != 0u, bap_live = __float_as_uint(tb) != 0u;
+        if (MIX) {
+            const uint32_t model = code & BTX_MIXED_MODEL_MASK;
+            const int hard = (code & BTX_MIXED_HARD_RESET) ? 1 : 0;
+            if (model == BTX_NEURON_TWO_COMPARTMENT)
+                s = two_comp_neuron<true, true>(a, lane, nidx, i, p, wz, x, drv, xa, v, ta, tb, tt, q);
+            else if (model == BTX_NEURON_GLIF3)
+                s = lif_exp_neuron<kGlif3, true, true, false, false>(a, lane, nidx, i, p, wz, x, drv,
+                                                                     v, r, ia, q, tau, nullptr,
+                                                                     hard);
+            else
+                s = lif_exp_neuron<kLif, true, true, false, false>(a, lane, nidx, i, p, wz, x, drv,
+                                                                   v, r, ia, q, tau, nullptr, hard);
+        } else if (TC) {
+            s = two_comp_neuron<true, true>(a, lane, nidx, i, p, wz, x, drv, xa, v, ta, tb, tt, q);
+        } else {
+            s = lif_exp_neuron<(KIND == kGlif3 ? kGlif3 : kLif), true, true, SX, false>(
+                a, lane, nidx, i, p, wz, x, drv, v, r, ia, q, tau, &s2);
+        }
+        if (GLIF && a.iasc != nullptr) {
+#pragma unroll
+            for (int j = 0; j < kMaxAsc; ++j)
+                if (j < a.n_asc) a.iasc[i * a.n_asc + j] = ia[GLIF ? j : 0];
+        }
+        a.v[i] = v;
+        if (a.use_ref && (ref_live || __float_as_uint(r) != 0u)) a.ref[i] = r;
+        a.psc[i] = p;
+        if (SX) {
+            a.sh1[i] = s2.h1;
+            if (a.syn == BTX_SYN_DUAL_EXP) a.sh2[i] = s2.h2;
+        }
+        if (TC && (!MIX || a.tia != nullptr)) {
+            a.tia[i] = ta;
+            if (bap_live || __float_as_uint(tb) != 0u) a.tibap[i] = tb;
+            a.tth[i] = tt;
+        }
+    }
+    // half a spike word per lane: a wavefront holds two lanes' 32 neurons
+    const uint64_t on = __ballot(s != 0.f);
+    if (my_k == 0 && my_lane < lg) {
+        const uint32_t half = (uint32_t)(on >> (32 * (my_lane & 1)));
+        const int64_t h = lane * nw32 + blockIdx.x;
+        // a lane without a trial pushes nothing and leaves its raster
+        const bool run = a.lane_t_end == nullptr || a.in_t0[lane] + a.t < a.lane_t_end[lane];
+        if (run) ((uint32_t*)a.raster)[h] = half;
+        uint32_t push = half;
+        if (a.teacher != nullptr) {
+            push = ((const uint32_t*)a.teacher)[h];
+            const int64_t room = a.n - j0;  // bits past n never count
+            if (room < 32) push &= room > 0 ? (1u << room) - 1u : 0u;
+        }
+        push = run ? push : 0u;
+        ((uint32_t*)a.ring_words)[h] = push;
+        s_half[my_lane] = push;
+    }
+    __syncthreads();
+    // the lane bits of neuron j0 + tid in this group of 16 lanes
+    if (tid < kGatherNeurons && j0 + tid < a.n) {
+        uint32_t m = 0u;
+        for (int b = 0; b < lg; ++b) m |= ((s_half[b] >> tid) & 1u) << b;
+        g.lane_bits_out[(j0 + tid) * 4 * g.lw + blockIdx.y] = (uint16_t)m;
+    }
+}
+
 // The dense pull of a step as a launch of its own, after the step's launch
 // (batches of more than 32 lanes): one wavefront per destination and 64-lane
 // group, four destinations per workgroup.  Ends at once unless the previous
@@ -1536,8 +1927,7 @@ __global__ __launch_bounds__(kThreads) void k_pull(PushStep p) {
     pull_role<true>(p, L, (int64_t)blockIdx.x, (int64_t)gridDim.x);
 }
 
-// FIN: the last push reduced into the synapse (and recorded: psc in `rec`,
-// the other synapse states in a.rec_sh1_prev / a.rec_sh2_prev).
+// FIN: the last push reduced into the synapse.
 __global__ __launch_bounds__(kThreads) void k_finish(StepArgs a, float* __restrict__ rec) {
     __shared__ StepLds lds;
     const int64_t lane = blockIdx.y, seg = blockIdx.x;
@@ -1545,32 +1935,8 @@ __global__ __launch_bounds__(kThreads) void k_finish(StepArgs a, float* __restri
     reduce_segment(a.red, lds.red, a.n, a.nchunks, lane, seg, wz);
     const int64_t n0 = seg * kChunk + threadIdx.x * 4;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (n0 + k < a.n) {
-            const int64_t nidx = n0 + k;
-            const int64_t i = lane * a.n + nidx;
-            if (a.syn == BTX_SYN_EXP) {
-                const float q = a.psc[i] + wz[k];
-                a.psc[i] = q;
-                if (rec) rec[i] = q;
-            } else if (a.syn == BTX_SYN_DUAL_EXP) {
-                const float g1 = a.sh1[i] + wz[k];
-                const float g2 = a.sh2[i] + wz[k];
-                const float q = prm(a.sa, a.sa_s, nidx) * (g2 - g1);
-                a.sh1[i] = g1;
-                a.sh2[i] = g2;
-                a.psc[i] = q;
-                if (rec) rec[i] = q;
-                if (a.rec_sh1_prev) a.rec_sh1_prev[i] = g1;
-                if (a.rec_sh2_prev) a.rec_sh2_prev[i] = g2;
-            } else {
-                const float h = a.sh1[i] + prm(a.sg, a.sg_s, nidx) * wz[k];
-                a.sh1[i] = h;
-                if (rec) rec[i] = a.psc[i];
-                if (a.rec_sh1_prev) a.rec_sh1_prev[i] = h;
-            }
-        }
-    }
+    for (int k = 0; k < 4; ++k)
+        if (n0 + k < a.n) finish_neuron(a, rec, lane * a.n + n0 + k, n0 + k, wz[k]);
 }
 
 // Ring lists of all ring slots from spike words [R][lanes][nwords]
@@ -1645,7 +2011,7 @@ __global__ __launch_bounds__(256) void k_syn_decay(StepArgs a, int64_t m) {
     const bool dual = a.syn == BTX_SYN_DUAL_EXP;
     float psc = a.psc[i];
     Syn2 s2{a.sh1[i], dual ? a.sh2[i] : 0.f};
-    syn_x_decay(a, nidx, psc, s2);
+    syn_x_decay<false>(a, nidx, psc, s2, PreParams{});
     a.sh1[i] = s2.h1;
     if (dual) a.sh2[i] = s2.h2;
     else a.psc[i] = psc;
@@ -1682,17 +2048,19 @@ struct RunTables {
     int age_of_sub[BTX_MAX_BINS];
     int bin_delay[BTX_MAX_BINS];
     int bin_sub[BTX_MAX_BINS];
+    int bin_of_sub[BTX_MAX_BINS];
 };
 
 __global__ __launch_bounds__(64) void k_set_tables(RunTables t, Ctl* __restrict__ ctl) {
-#pragma unroll
-    for (int k = 0; k < BTX_MAX_BINS; ++k) {
-        if ((int)threadIdx.x == k) {
-            ctl->age_of_sub[k] = t.age_of_sub[k];
-            ctl->bin_delay[k] = t.bin_delay[k];
-            ctl->bin_sub[k] = t.bin_sub[k];
-        }
-    }
+    // the tables are the first bytes of the argument segment, read by a
+    // per-lane load (a select over 64 values each took 55 us, cold)
+    const auto* arg = (const __attribute__((address_space(4))) RunTables*)
+        __builtin_amdgcn_kernarg_segment_ptr();
+    const int k = threadIdx.x;
+    ctl->age_of_sub[k] = arg->age_of_sub[k];
+    ctl->bin_delay[k] = arg->bin_delay[k];
+    ctl->bin_sub[k] = arg->bin_sub[k];
+    ctl->bin_of_sub[k] = arg->bin_of_sub[k];
 }
 
 static inline int64_t mod(int64_t a, int64_t b) {
@@ -2046,6 +2414,55 @@ static void launch_step(int ordered, const StepArgs& a, const PushStep& ps,
     else launch_step_k<false>(a, ps, ca, np, nc, group, grid, s);
 }
 
+template <int KIND>
+static void launch_gather(const StepArgs& a, const GatherArgs& g, hipStream_t s) {
+    const dim3 grid((unsigned)(2 * a.nwords), (unsigned)((g.lanes + kGatherLanes - 1) / kGatherLanes));
+    if (g.lanes == 1)
+        hipLaunchKernelGGL((k_gather_step<KIND, true>), grid, dim3(kGatherThreads),
+                           (size_t)g.nbins * 8 * a.nwords + 16, s, a, g);
+    else
+        hipLaunchKernelGGL((k_gather_step<KIND, false>), grid, dim3(kGatherThreads), 0, s, a, g);
+}
+
+static void launch_gather_k(const StepArgs& a, const GatherArgs& g, hipStream_t s) {
+    const bool sx = a.syn != BTX_SYN_EXP;
+    if (a.kind == kGlif3) sx ? launch_gather<kGlif3 | kSynX>(a, g, s) : launch_gather<kGlif3>(a, g, s);
+    else if (a.kind == kTwoComp) launch_gather<kTwoComp>(a, g, s);
+    else if (a.kind == kMixed) launch_gather<kMixed>(a, g, s);
+    else sx ? launch_gather<kLif | kSynX>(a, g, s) : launch_gather<kLif>(a, g, s);
+}
+
+// Whether a run's steps gather (k_gather_step) instead of pushing: when the
+// gather's time, which its edges set whatever the activity, is under what a
+// push step takes even in a quiet net.  Both as fitted to steps measured on
+// MI355X (us per step of a 100-step call at 0.02 % activity, push / gather):
+//   LIF, no delays, 4096 neurons, 0.33M edges, 1 lane     13.8 / 6.8
+//   LIF, no delays, 20000 neurons, 7.1M edges, 1 lane     20.4 / 16.5
+//   LIF, no delays, 10000 neurons, 3.0M edges, 8 lanes    18.8 / 15.0
+//   LIF, no delays, 20000 neurons, 7.1M edges, 8 lanes    24.1 / 37.0
+//   LIF, 8 delays, 10000 neurons, 1.2M edges, 1 lane      9.7 / 9.1
+//   LIF, 8 delays, 10000 neurons, 1.2M edges, 8 lanes     9.9 / 12.4
+//   GLIF3 + alpha, 8 delays, 1.2M edges, 8 lanes          17.6 / 14.8
+//   two-compartment, 8 delays, 1.2M edges, 8 lanes        13.0 / 13.8
+// An active net widens the gap (0.33M edges at 0.9 %: 26.9 / 7.5; 3.6M at
+// 1 %: 50 / 11.8).
+static bool gather_route(const btx_rsnn_plan* p, bool fused) {
+    if (!p->ordered || p->ring_lane_bits == nullptr || p->lanes > 65535) return false;
+    for (int j = 0; j < p->nbins; ++j)
+        for (int k = 0; k < j; ++k)
+            if (p->bin_sub[j] == p->bin_sub[k]) return false;
+    if (p->lanes == 1 && (int64_t)p->nbins * 8 * ((p->n + 63) / 64) > kGatherBits) return false;
+    const double edges = 1e-6 * (double)p->nnz;
+    const double groups = (double)((p->lanes + kGatherLanes - 1) / kGatherLanes);
+    const double gather = 7.5 + edges * (p->lanes == 1 ? 1.2 : (p->csr_d > 1 ? 4.6 : 2.6) * groups);
+    const double kind = p->neuron_model == BTX_NEURON_LIF                ? 0.0
+                        : p->neuron_model == BTX_NEURON_TWO_COMPARTMENT ? 3.4
+                                                                         : 4.5;
+    const double push = (fused ? 9.6 : 14.5 + 0.45 * edges) + kind +
+                        (p->syn_kind == BTX_SYN_EXP ? 0.0 : 2.5);
+    return gather < push;
+}
+
 }  // namespace btx
 
 BTX_API int btx_rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, void* stream) {
@@ -2133,18 +2550,25 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         tb.age_of_sub[k] = -1;
         tb.bin_delay[k] = 0;
         tb.bin_sub[k] = 0;
+        tb.bin_of_sub[k] = -1;
     }
     for (int j = 0; j < p->nbins; ++j) {
         tb.age_of_sub[p->bin_sub[j]] = p->bin_delay[j];
         tb.bin_delay[j] = p->bin_delay[j];
         tb.bin_sub[j] = p->bin_sub[j];
+        tb.bin_of_sub[p->bin_sub[j]] = j;
     }
-    if (!p->tables_ready) hipLaunchKernelGGL(k_set_tables, dim3(1), dim3(64), 0, s, tb, ctl);
+    const bool gather = gather_route(p, min_delay >= 1);
+    if (!p->tables_ready)
+        hipLaunchKernelGGL(k_set_tables, dim3(1), dim3(64), 0, s, tb, ctl);
     // lane-bit ring of the dense pull (ordered mode with the plan's ring of
     // lane bits); 64-lane words per neuron
     uint64_t* lane_bits = p->ordered ? p->ring_lane_bits : nullptr;
     const int lw = (int)((lanes + 63) / 64);
-    if (p->ring_rebuild) {
+    if (gather && (p->ring_rebuild || !p->tables_ready)) {
+        hipLaunchKernelGGL(k_ring_lane_bits, dim3((unsigned)nwords, (unsigned)lw, (unsigned)R),
+                           dim3(64), 0, s, p->ring_words, lane_bits, lanes, nwords, n, lw);
+    } else if (p->ring_rebuild) {
         hipLaunchKernelGGL(k_ring_from_words,
                            dim3((unsigned)nchunks, (unsigned)lanes, (unsigned)R),
                            dim3(kThreads), 0, s, p->ring_words, n, nwords, lanes, nchunks,
@@ -2281,6 +2705,23 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
     const int above = (lanes * nchunks < 256 && kBinCap < cap / 2) ? kBinCap : cap / 2;
     ca.above = (float)above * (float)(lanes * nchunks);
 
+    GatherArgs ga{};
+    if (gather) {
+        ga.csc_ptr = p->csc_ptr;
+        ga.csc_src = p->csc_src;
+        ga.csc_w = p->csc_w;
+        ga.ring_words = p->ring_words;
+        ga.ctl = ctl;
+        ga.lanes = lanes;
+        ga.lane_bits = lane_bits;
+        ga.lw = lw;
+        ga.nbins = p->nbins;
+        ga.csr_d = p->csr_d;
+        ga.fd = fast_div(p->csr_d);
+        ga.R = R;
+        ga.delay0 = p->bin_delay[0];
+    }
+
     const int64_t rec_step = m;
     for (int64_t t = 0; t < n_steps; ++t) {
         a.prev = t > 0;
@@ -2329,7 +2770,13 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         ps.ev_d = (uint16_t*)cur.ev_d;
         ps.acc = cur.acc;
         ps.pull_acc = cur.pull_acc ? (float*)cur.pull_acc : nullptr;
-        if (fused) {
+        if (gather) {
+            ga.slot0 = (int)mod(p->ring_cursor + t - 1, R);
+            ga.lane_bits_out = (uint16_t*)a.lane_bits;
+            kt.begin(0);
+            launch_gather_k(a, ga, s);
+            kt.end(0);
+        } else if (fused) {
             kt.begin(0);
             const dim3 grid((unsigned)lanes, (unsigned)(nc + npb + ps.nh + nf));
             launch_step(p->ordered, a, ps, ca, npb, nc, group, grid, s);
@@ -2358,9 +2805,27 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
     a.rec_sh2_prev = p->rec_syn_h2 ? p->rec_syn_h2 + (n_steps - 1) * rec_step : nullptr;
     a.red.pull.clock = p->ring_cursor + n_steps - 1;
     a.red.pull.slot0 = (int)mod(a.red.pull.clock, R);
+    float* const rec_last = p->rec_psc ? p->rec_psc + (n_steps - 1) * rec_step : nullptr;
     kt.begin(3);
-    hipLaunchKernelGGL(k_finish, dim3((unsigned)nchunks, (unsigned)lanes), dim3(kThreads), 0, s,
-                       a, p->rec_psc ? p->rec_psc + (n_steps - 1) * rec_step : nullptr);
+    if (gather) {
+        a.prev = 1;
+        ga.fin = 1;
+        ga.slot0 = (int)mod(p->ring_cursor + n_steps - 1, R);
+        ga.rec_psc_last = rec_last;
+        launch_gather_k(a, ga, s);
+    } else {
+        hipLaunchKernelGGL(k_finish, dim3((unsigned)nchunks, (unsigned)lanes), dim3(kThreads), 0,
+                           s, a, rec_last);
+    }
     kt.end(3);
+    if (gather && (p->ring_d > 1 || min_delay > 0)) {
+        // the lists follow the words the steps kept, so that a later run of
+        // any route continues from this ring (a net without delays reads no
+        // earlier step's slot)
+        hipLaunchKernelGGL(k_ring_from_words,
+                           dim3((unsigned)nchunks, (unsigned)lanes, (unsigned)R), dim3(kThreads),
+                           0, s, p->ring_words, n, nwords, lanes, nchunks, p->ring_idx,
+                           p->ring_cnt);
+    }
     return check_launch("btx_rsnn_run");
 }

@@ -683,7 +683,7 @@ class Engine:
         ws = self._workspace(lanes, n, p.slots, p.ordered, dev)
         p.workspace = ws.data_ptr()
         p.workspace_bytes = ws.numel()
-        tables = (ws.data_ptr(), tuple(sp.bins))
+        tables = (ws.data_ptr(), tuple(sp.bins), self.dense_pull())
         p.tables_ready = 1 if tables in self._tables_ok else 0
         stream = _lib.stream_ptr()
         if timings is None:
@@ -698,7 +698,7 @@ class Engine:
             for k, name in enumerate(("step", "reduce", "push", "finish")):
                 timings[name] = (float(ms[k]), int(calls[k]))
                 timings[name + "_each"] = [per[k * cap + i] for i in range(min(calls[k], cap))]
-        self._tables_ok.add(tables)
+        self._tables_ok = {tables}
         if want_z:
             from .._kernels import unpack_rows
             z = torch.empty((T, lanes, n), dtype=torch.float32, device=dev)

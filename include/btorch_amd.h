@@ -418,8 +418,9 @@ typedef struct btx_rsnn_plan {
     /* workspace from btx_rsnn_workspace_bytes(), zero-filled once */
     void* workspace;      size_t workspace_bytes;
     /* 1 = the workspace already holds this plan's delay-bin tables (an
-     * earlier run with the same workspace, nbins, bin_delay and bin_sub
-     * wrote them), so the run skips writing them; 0 = write them first */
+     * earlier run with the same workspace, n, lanes, nnz, ordered, nbins,
+     * bin_delay, bin_sub and the same ring_lane_bits being NULL or not wrote
+     * them), so the run skips writing them; 0 = write them first */
     int tables_ready;
     /* BTX_NEURON_MIXED (MixedNeuronPopulation.single_step_forward,
      * mixed.py:113-141: each group's own step on its range of the axis):
@@ -448,7 +449,11 @@ typedef struct btx_rsnn_plan {
      * lanes of the ring clears their bits too.  The decision is made one
      * step ahead from the ring's spike totals (the newest slot estimated by
      * the one before).  Batches of more than 32 lanes pull in a launch of
-     * their own queued after each step's (it ends at once on a push step). */
+     * their own queued after each step's (it ends at once on a push step).
+     * Nets of few edges per step of work run every step as a pull fused with
+     * the neuron update instead (the rule is at gather_route in
+     * btx_step.hip); such a run needs distinct bin_sub, keeps the words and
+     * these lane bits current each step, and the lists at its end. */
     uint64_t* ring_lane_bits;
 } btx_rsnn_plan;
 

@@ -418,3 +418,59 @@ def test_engine_high_activity_large_bins_and_dense_pull(bin_cap, lanes, expect):
     assert bits_equal(z, ref["z"])
     assert bits_equal(st["neuron.v"], ref["v"]) and bits_equal(st["synapse.psc"], ref["psc"])
     assert bits_equal(model.synapse.history.history.reshape(lanes, D, n), ref["final"]["history"])
+
+
+@pytest.mark.parametrize("n,lanes,D", [(31, 1, 1), (1000, 1, 7), (1025, 1, 1), (97, 2, 1),
+                                       (2081, 16, 5), (640, 17, 1), (300, 70, 3)])
+def test_engine_gather_steps_match_pushed_steps_and_oracle(n, lanes, D):
+    # nets small enough that every step sums its incoming edges itself
+    # (dense_pull on) against the same net pushed into term bins (off): runs
+    # that switch between the two and back continue from the same ring, and
+    # every record, memory and the delay ring stay bit-exact.  Sizes around
+    # the 32 neurons and 16 lanes of a workgroup, rows of no edges included
+    c = workloads.powerlaw_net_fast(n=n, k_min=1, k_max=min(n // 2, 200), delay_lo=1,
+                                    delay_hi=max(1, D - 1), seed=51)
+    keep = c.post % 13 != 3   # neurons without incoming edges
+    import scipy.sparse
+    rows = c.pre[keep] * D + (c.delay[keep] if D > 1 else 0)
+    mat = scipy.sparse.coo_array((c.w[keep], (rows, c.post[keep])), shape=(n * D, n))
+    T = 24
+    x = torch.from_numpy(workloads.poisson_input(4 * T, lanes, n, 300.0, 0.1, seed=51) * 25.0)
+
+    def build():
+        conn = SparseConn(mat)
+        syn = (HeterSynapsePSC(n, 1, None, conn, base_psc=ExponentialPSC, max_delay_steps=D,
+                               use_circular_buffer=True, tau_syn=5.0)
+               if D > 1 else ExponentialPSC(n, 5.0, conn))
+        m = RecurrentNN(LIF(n, tau_ref=2.0), syn, step_mode="m",
+                        update_state_names=["neuron.v", "synapse.psc"]).to(DEV)
+        functional.init_net_state(m, batch_size=lanes, device=DEV, dtype=torch.float32)
+        return m, conn
+
+    def run(order):
+        m, conn = build()
+        out, pulled = [], []
+        with environ.context(dt=0.1), torch.no_grad():
+            for k, pull in enumerate(order):
+                conn.sparse_config.dense_pull = pull
+                z, st = m(x[k * T:(k + 1) * T].to(DEV))
+                out.append((z.cpu(), st["neuron.v"].cpu(), st["synapse.psc"].cpu()))
+                ws = next(iter(m.fused_engine()._ws.values())).view(torch.int32)
+                pulled.append(ws[256:260].cpu().tolist())
+        hist = (m.synapse.history.history.reshape(lanes, D, n).cpu() if D > 1
+                else torch.zeros(0))
+        return [torch.cat(t) for t in zip(*out)], hist, pulled
+
+    pushed, h0, _ = run([False] * 4)
+    gathered, h1, flags = run([True] * 4)
+    mixed, h2, _ = run([True, False, True, False])
+    assert all(f == [1, 1, 1, 1] for f in flags)  # every step pulled
+    net = rsnn.Net(n, mat, rsnn.LIFParams.make(n, tau_ref=2.0), torch.tensor(5.0), 0.1,
+                   **(dict(delay_mode="hetero", max_delay_steps=D, circular=True) if D > 1
+                      else {}))
+    ref = rsnn.simulate(net, x)
+    assert float(ref["z"].sum()) > 20
+    for got in (pushed, gathered, mixed):
+        assert bits_equal(got[0], ref["z"])
+        assert bits_equal(got[1], ref["v"]) and bits_equal(got[2], ref["psc"])
+    assert torch.equal(h0, h1) and torch.equal(h0, h2)
