@@ -43,6 +43,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -57,6 +58,8 @@ constexpr int kThreads = 256;           // 4 neurons per thread in the F role
 constexpr int kBinCap = 1024;           // terms per bin sorted in LDS
 constexpr int kBinCapMax = 8192;        // terms per bin in the workspace (larger bins are
                                         // sorted through a global order array)
+constexpr int kBinHead = 64;            // ints ahead of a buffer's bin counts; the last one is
+                                        // its overflow flag
 constexpr int kSortMax = 32;            // most terms a neuron sorts in LDS
 constexpr int kMaxChunks = 1024;        // n <= 1,048,576 (push reservation table)
 constexpr int kStage = 1024;            // terms a push workgroup stages in LDS
@@ -1243,13 +1246,6 @@ __device__ __forceinline__ uint32_t div_u31(const FastDiv& f, uint32_t x) {
 // slot that sub's age points at is set (every slot the step reads was marked
 // when it was written: the pull is only taken then).  Groups of Gp threads
 // (one per lane of a 64-lane group) walk one destination's edges together.
-// WAVE (k_pull only): a 64-lane group takes 64 of a destination's edges at a
-// time, lane k reading edge c + k and its source's lane-bit word, and the
-// wavefront walks them in order out of register lanes (three requests per
-// 64 edges instead of three per edge).  Inside k_step this form put the
-// kernel at 300-400 B of scratch per lane next to the other, so the step
-// keeps the 12-edge rounds.
-template <bool WAVE>
 __device__ void pull_role(const PushStep& a, PushLds& L, int64_t wid, int64_t nwg) {
     const int tid = threadIdx.x;
     const FastDiv fd = fast_div(a.csr_d);
@@ -1272,38 +1268,6 @@ __device__ void pull_role(const PushStep& a, PushLds& L, int64_t wid, int64_t nw
             float acc = 0.f;
             int64_t e = a.csc_ptr[d];
             const int64_t e1 = a.csc_ptr[d + 1];
-            if (WAVE && Gp == 64) {
-                // one destination per wavefront: e and e1 are uniform.  The
-                // next 64 edges and their lane-bit words are requested before
-                // the current ones are summed
-                const int sh = gl & 31;
-                auto edges = [&](int64_t c, int& wi) -> uint64_t {
-                    const int m = (int)(e1 - c < 64 ? e1 - c : 64);
-                    const bool in = c < e1 && gl < m;
-                    const int r = in ? a.csc_src[c + gl] : 0;
-                    wi = in ? __float_as_int(a.csc_w[c + gl]) : 0;
-                    const int src = (int)div_u31(fd, (uint32_t)r);
-                    const int slot = L.slot[r - src * a.csr_d];
-                    return (in && slot >= 0) ? bits[((int64_t)slot * a.n + src) * a.lw] : 0ull;
-                };
-                int wi_next = 0;
-                uint64_t wb_next = e < e1 ? edges(e, wi_next) : 0ull;
-                for (int64_t c = e; c < e1; c += 64) {
-                    const int m =
-                        __builtin_amdgcn_readfirstlane((int)(e1 - c < 64 ? e1 - c : 64));
-                    const int wi = wi_next;
-                    const uint64_t wb = wb_next;
-                    if (c + 64 < e1) wb_next = edges(c + 64, wi_next);
-                    const int lo = (int)(uint32_t)wb, hi = (int)(uint32_t)(wb >> 32);
-                    for (int k = 0; k < m; ++k) {
-                        const uint32_t wl = (uint32_t)__builtin_amdgcn_readlane(lo, k);
-                        const uint32_t wh = (uint32_t)__builtin_amdgcn_readlane(hi, k);
-                        if (((gl < 32 ? wl : wh) >> sh) & 1u)
-                            acc = acc + __int_as_float(__builtin_amdgcn_readlane(wi, k));
-                    }
-                }
-                e = e1;
-            }
             // 12 edges in flight per round of dependent loads (edges, then
             // lane bits): the most that keeps the step within its registers
             constexpr int U = 12;
@@ -1358,8 +1322,9 @@ __device__ void p_role(const PushStep& a, PushLds& L, int64_t px, int64_t lane) 
         // unzeroed, which no pull reads: the pull needs R marking launches
         // in a row, by when that slot is written again.
         pull = ld_const(&a.ctl->push_mode[a.clock & 3]);
-        const int64_t zn =
-            !helper && ld_const(&a.ctl->lane_bits_mode[a.clock & 3]) ? a.n * a.lw : 0;
+        // (a batch that pulls in k_pull marks in k_mark)
+        const int64_t zn = !helper && !a.pull_sep && ld_const(&a.ctl->lane_bits_mode[a.clock & 3])
+                               ? a.n * a.lw : 0;
         uint64_t* nb = a.lane_bits + (int64_t)ring_slot(a.clock + 1, 0, a.R) * a.n * a.lw;
         for (int64_t i = wid * kThreads + threadIdx.x; i < zn; i += nwg * kThreads) nb[i] = 0ull;
     }
@@ -1395,7 +1360,7 @@ __device__ void p_role(const PushStep& a, PushLds& L, int64_t px, int64_t lane) 
     if (ORDERED && pull) {
         if (!a.pull_sep) {
             const int64_t npp = np + a.nh;
-            pull_role<false>(a, L, lane * npp + px, npp * a.lanes);
+            pull_role(a, L, lane * npp + px, npp * a.lanes);
         }
         return;
     }
@@ -1457,6 +1422,7 @@ __device__ void p_role(const PushStep& a, PushLds& L, int64_t px, int64_t lane) 
                 const int ct = L.tile[t];
                 if (ct) {
                     const int b = atomicAdd(&a.bin_cnt[lane * a.nchunks + t], ct);
+                    if (b + ct > a.cap) a.bin_cnt[-1] = 1;  // the buffer's overflow flag
                     L.base[t] = (uint16_t)(b < a.cap ? b : a.cap);
                     L.tile[t] = 0;
                 }
@@ -1578,9 +1544,66 @@ __device__ __forceinline__ void finish_neuron(const StepArgs& a, float* __restri
 
 constexpr int kGatherNeurons = 32;             // neurons per workgroup = half a spike word
 constexpr int kGatherThreads = 512;            // 8 wavefronts, four neurons' edges each
-constexpr int kGatherLanes = 16;               // lanes per workgroup, at most
 constexpr int kGatherBits = 48 * 1024;         // bytes of spike words staged in LDS, at most
 constexpr int kGatherAhead = 8;                // 64-edge chunks a wavefront requests at a time
+
+// Which lanes a workgroup of k_gather_step takes: the only one, a group of 16
+// lanes, or (nets of more than 16 lanes) one of 64, a lane per thread of the
+// wavefront that sums them.
+enum GatherMode { kGatherOne, kGatherFew, kGatherWide };
+constexpr int gather_lanes(int mode) { return mode == kGatherOne ? 1 : mode == kGatherFew ? 16 : 64; }
+
+// acc += the weights of a chunk's active edges (thread k of the wavefront
+// holds edge k's weight w and its source's lane bits), in edge order, in the
+// threads whose lane has the edge's bit.  `on`: the edges with any bit.  Up
+// to eight such edges are taken one by one, more in blocks of eight with
+// fixed lane numbers (a third of the instructions per edge).  The lane bits
+// become the execution mask of the add.  Every thread of the wavefront is
+// active when it is called, and on return.
+__device__ __forceinline__ void add_lanes(float& acc, float w, uint64_t word, uint64_t on) {
+    const int wi = __float_as_int(w), lo = (int)(uint32_t)word, hi = (int)(uint32_t)(word >> 32);
+    if (__popcll((unsigned long long)on) <= 8) {
+        while (on) {
+            const int k = __ffsll((unsigned long long)on) - 1;
+            const uint32_t ml = (uint32_t)__builtin_amdgcn_readlane(lo, k);
+            const uint32_t mh = (uint32_t)__builtin_amdgcn_readlane(hi, k);
+            const int wk = __builtin_amdgcn_readlane(wi, k);
+            const uint64_t m = ((uint64_t)mh << 32) | ml;
+            asm("s_mov_b64 exec, %1\n\t"
+                "v_add_f32 %0, %2, %0\n\t"
+                "s_mov_b64 exec, -1"
+                : "+v"(acc)
+                : "s"(m), "s"(wk));
+            on &= on - 1ull;
+        }
+        return;
+    }
+#pragma unroll
+    for (int k0 = 0; k0 < 64; k0 += 4) {
+        if (((on >> k0) & 0xfull) == 0ull) continue;
+        uint64_t m[4];
+        int wk[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t ml = (uint32_t)__builtin_amdgcn_readlane(lo, k0 + k);
+            const uint32_t mh = (uint32_t)__builtin_amdgcn_readlane(hi, k0 + k);
+            m[k] = ((uint64_t)mh << 32) | ml;
+            wk[k] = __builtin_amdgcn_readlane(wi, k0 + k);
+        }
+        asm("s_mov_b64 exec, %1\n\t"
+            "v_add_f32 %0, %5, %0\n\t"
+            "s_mov_b64 exec, %2\n\t"
+            "v_add_f32 %0, %6, %0\n\t"
+            "s_mov_b64 exec, %3\n\t"
+            "v_add_f32 %0, %7, %0\n\t"
+            "s_mov_b64 exec, %4\n\t"
+            "v_add_f32 %0, %8, %0\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(acc)
+            : "s"(m[0]), "s"(m[1]), "s"(m[2]), "s"(m[3]), "s"(wk[0]), "s"(wk[1]), "s"(wk[2]),
+              "s"(wk[3]));
+    }
+}
 
 struct GatherArgs {
     const int64_t* csc_ptr;
@@ -1590,7 +1613,7 @@ struct GatherArgs {
     Ctl* ctl;                    // bin_delay, bin_of_sub
     int64_t lanes;
     const uint64_t* lane_bits;   // [R][n][lw]
-    uint16_t* lane_bits_out;     // this step's slot, 4*lw lane groups a neuron
+    uint64_t* lane_bits_out;     // this step's slot, [n][lw]
     int lw;
     int nbins;
     int csr_d;
@@ -1617,24 +1640,26 @@ struct GatherArgs {
 // thread b sums lane b.  Either way one ballot names the chunk's active edges
 // and a scalar loop adds their weights in order.  The first 512 edges and the
 // neurons' state are requested before anything is waited for.
-template <int KIND_SX, bool ONE>
+template <int KIND_SX, int MODE>
 __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, GatherArgs g) {
     constexpr int KIND = KIND_SX & ~kSynX;
     constexpr bool SX = (KIND_SX & kSynX) != 0;
     constexpr bool MIX = KIND == kMixed;
     constexpr bool GLIF = KIND == kGlif3 || MIX;
     constexpr bool TC = KIND == kTwoComp || MIX;
+    constexpr bool ONE = MODE == kGatherOne, WIDE = MODE == kGatherWide;
+    constexpr int LG = gather_lanes(MODE);  // lanes of a workgroup, at most
     // ONE: half words of every bin's slot, [nbins][2 * nwords], and a zero
     extern __shared__ uint32_t __attribute__((aligned(16))) s_bits[];
-    __shared__ float s_sum[kGatherLanes * kGatherNeurons];
-    __shared__ uint32_t s_half[kGatherLanes];
+    __shared__ float s_sum[LG * kGatherNeurons];
+    __shared__ uint32_t s_half[LG];
     // virtual-row offset -> first word of its bin (ONE) or its ring slot, or -1
     __shared__ int s_row[BTX_MAX_BINS];
     const int tid = threadIdx.x, ln = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform across the wavefront
     const int64_t j0 = (int64_t)blockIdx.x * kGatherNeurons;
-    const int64_t lane0 = (int64_t)blockIdx.y * kGatherLanes;
-    const int lg = ONE ? 1 : (int)(g.lanes - lane0 < kGatherLanes ? g.lanes - lane0 : kGatherLanes);
+    const int64_t lane0 = (int64_t)blockIdx.y * LG;
+    const int lg = ONE ? 1 : (int)(g.lanes - lane0 < LG ? g.lanes - lane0 : LG);
     const int nw32 = 2 * (int)a.nwords;
 
     // this wavefront's edges: neurons d0 .. d0+3
@@ -1649,19 +1674,25 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
     }
     const int none = g.nbins * nw32;  // an LDS word that stays 0
 
-    // the neuron this thread integrates
+    // the neurons this thread integrates: neuron my_k of lanes my_lane, + 16, ...
+    constexpr int kRound = kGatherThreads / kGatherNeurons;  // lanes integrated at a time
     const int my_lane = tid / kGatherNeurons, my_k = tid % kGatherNeurons;
-    const int64_t lane = lane0 + my_lane, nidx = j0 + my_k;
-    const int64_t i = lane * a.n + nidx;
-    const bool mine = my_lane < lg && nidx < a.n;
-    bool live = mine;
-    if (mine && a.lane_t_end != nullptr) live = a.in_t0[lane] + a.t < a.lane_t_end[lane];
+    const int64_t nidx = j0 + my_k;
+    int64_t lane = 0, i = 0;
+    bool mine = false, live = false;
     float v = 0.f, p = 0.f, r = 0.f, x = 0.f, ta = 0.f, tb = 0.f, tt = 0.f, xa = 0.f, tau = 1.f;
     Syn2 s2{0.f, 0.f};
     float ia[GLIF ? kMaxAsc : 1] = {};
     PreParams q{0.f, 0.f, 1.f, 0.f, 1.f, 0.f};  // the rest is read by its models only
     uint32_t code = 0;
-    if (!g.fin && live) {
+    auto request_state = [&](int round) {
+        const int b = my_lane + kRound * round;
+        lane = lane0 + b;
+        i = lane * a.n + nidx;
+        mine = b < lg && nidx < a.n;
+        live = mine;
+        if (mine && a.lane_t_end != nullptr) live = a.in_t0[lane] + a.t < a.lane_t_end[lane];
+        if (g.fin || !live) return;
         v = a.v[i];
         p = a.psc[i];
         if (SX) {
@@ -1676,13 +1707,14 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
             tt = a.tth[i];
             if (a.xa) xa = a.xa[i];
         }
-        if (MIX) code = a.kinds[nidx];
-        if (!TC || MIX) tau = prm(a.tau, a.tau_s, nidx);
         if (GLIF && a.iasc != nullptr) {
 #pragma unroll
             for (int j = 0; j < kMaxAsc; ++j)
                 if (j < a.n_asc) ia[GLIF ? j : 0] = a.iasc[i * a.n_asc + j];
         }
+        if (round > 0) return;  // the parameters are the neuron's, whatever the lane
+        if (MIX) code = a.kinds[nidx];
+        if (!TC || MIX) tau = prm(a.tau, a.tau_s, nidx);
         q.vth = prm(a.vth, a.vth_s, nidx);
         q.vr = prm(a.vr, a.vr_s, nidx);
         if (KIND != kTwoComp) q.cm = prm(a.cm, a.cm_s, nidx);
@@ -1714,9 +1746,9 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
 #pragma unroll
             for (int j = 0; j < BTX_TC_NPARAM; ++j) q.tc[j] = prm(a.tcp[j], a.tcs[j], nidx);
         }
-    }
+    };
+    request_state(0);
 
-    float wz = 0.f;
     if (a.prev) {
         const int32_t* es = g.csc_src + e0;
         const float* ew = g.csc_w + e0;
@@ -1772,7 +1804,7 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
             const int slot = g.slot0 - dl + (g.slot0 < dl ? g.R : 0);
             s_row[tid] = j < 0 ? -1 : ONE ? j * nw32 : slot;
         }
-        if (ln < kGatherLanes * 4) s_sum[64 * wv + ln] = 0.f;
+        for (int w = tid; w < LG * kGatherNeurons; w += kGatherThreads) s_sum[w] = 0.f;
         if (ONE) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the words are in LDS
         __syncthreads();
         // ONE: the running sum, the same in every thread; else thread b holds
@@ -1785,7 +1817,7 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
             for (int u0 = 0; u0 < kGatherAhead; u0 += 4) {
                 if (own[u0] == 4) break;
                 // what every edge's source pushed: its bit (ONE) or its lanes' bits
-                uint32_t wd[4];
+                typename std::conditional<WIDE, uint64_t, uint32_t>::type wd[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     const int e = er[u0 + u];
@@ -1800,9 +1832,9 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
                     if (ONE) {
                         wd[u] = (s_bits[in ? first + (src >> 5) : none] >> (src & 31)) & 1u;
                     } else {
-                        const uint16_t* q = (const uint16_t*)(g.lane_bits +
-                                                              ((int64_t)first * a.n + src) * g.lw);
-                        wd[u] = in ? q[blockIdx.y] : 0u;
+                        const uint64_t* words = g.lane_bits + ((int64_t)first * a.n + src) * g.lw;
+                        if (WIDE) wd[u] = in ? words[blockIdx.y] : 0u;
+                        else wd[u] = in ? ((const uint16_t*)words)[blockIdx.y] : 0u;
                     }
                 }
 #pragma unroll
@@ -1813,6 +1845,10 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
                         acc = 0.f;
                     }
                     uint64_t on = __ballot(wd[u] != 0u);
+                    if (WIDE) {
+                        add_lanes(acc, wr[u0 + u], (uint64_t)wd[u], on);
+                        continue;
+                    }
                     while (on) {
                         const int k = __ffsll((unsigned long long)on) - 1;
                         const float w = __int_as_float(
@@ -1834,97 +1870,190 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
         }
         if (cur < 4 && ln < lg) s_sum[ln * kGatherNeurons + 4 * wv + cur] = acc;
         __syncthreads();
-        if (mine) wz = s_sum[tid];
     }
 
-    if (g.fin) {
+    if (g.fin && blockIdx.x == 0 && blockIdx.y == 0 && tid < 4) {
         // every step was pulled and every slot's lane bits are current; a run
         // of the other route that follows marks them anew before it pulls
         // again (its slots are not zeroed ahead)
-        if (blockIdx.x == 0 && blockIdx.y == 0 && tid < 4) {
-            g.ctl->push_mode[tid] = 1;
-            if (tid == 0) g.ctl->lane_bits_run = 0;
-        }
-        // a lane past its trial end at the last step pushed nothing
-        if (mine) finish_neuron(a, g.rec_psc_last, i, nidx, live ? wz : 0.f);
-        return;
+        g.ctl->push_mode[tid] = 1;
+        if (tid == 0) g.ctl->lane_bits_run = 0;
     }
-    float s = 0.f;
-    if (live) {
-        const DriveArgs dargs = drive_args(a, lane);
-        const float drv = poisson_drive1(a, dargs, nidx) ? a.in_kick : 0.f;
-        const bool ref_live = __float_as_uint(r) != 0u, bap_live = __float_as_uint(tb) != 0u;
-        if (MIX) {
-            const uint32_t model = code & BTX_MIXED_MODEL_MASK;
-            const int hard = (code & BTX_MIXED_HARD_RESET) ? 1 : 0;
-            if (model == BTX_NEURON_TWO_COMPARTMENT)
+    for (int round = 0; round * kRound < lg; ++round) {
+        if (round > 0) request_state(round);
+        const int b = my_lane + kRound * round;
+        const float wz = mine && a.prev ? s_sum[b * kGatherNeurons + my_k] : 0.f;
+        if (g.fin) {
+            // a lane past its trial end at the last step pushed nothing
+            if (mine) finish_neuron(a, g.rec_psc_last, i, nidx, live ? wz : 0.f);
+            continue;
+        }
+        float s = 0.f;
+        if (live) {
+            const DriveArgs dargs = drive_args(a, lane);
+            const float drv = poisson_drive1(a, dargs, nidx) ? a.in_kick : 0.f;
+            const bool ref_live = __float_as_uint(r) != 0u, bap_live = __float_as_uint(tb) != 0u;
+            if (MIX) {
+                const uint32_t model = code & BTX_MIXED_MODEL_MASK;
+                const int hard = (code & BTX_MIXED_HARD_RESET) ? 1 : 0;
+                if (model == BTX_NEURON_TWO_COMPARTMENT)
+                    s = two_comp_neuron<true, true>(a, lane, nidx, i, p, wz, x, drv, xa, v, ta, tb, tt, q);
+                else if (model == BTX_NEURON_GLIF3)
+                    s = lif_exp_neuron<kGlif3, true, true, false, false>(a, lane, nidx, i, p, wz, x, drv,
+                                                                         v, r, ia, q, tau, nullptr,
+                                                                         hard);
+                else
+                    s = lif_exp_neuron<kLif, true, true, false, false>(a, lane, nidx, i, p, wz, x, drv,
+                                                                       v, r, ia, q, tau, nullptr, hard);
+            } else if (TC) {
                 s = two_comp_neuron<true, true>(a, lane, nidx, i, p, wz, x, drv, xa, v, ta, tb, tt, q);
-            else if (model == BTX_NEURON_GLIF3)
-                s = lif_exp_neuron<kGlif3, true, true, false, false>(a, lane, nidx, i, p, wz, x, drv,
-                                                                     v, r, ia, q, tau, nullptr,
-                                                                     hard);
-            else
-                s = lif_exp_neuron<kLif, true, true, false, false>(a, lane, nidx, i, p, wz, x, drv,
-                                                                   v, r, ia, q, tau, nullptr, hard);
-        } else if (TC) {
-            s = two_comp_neuron<true, true>(a, lane, nidx, i, p, wz, x, drv, xa, v, ta, tb, tt, q);
-        } else {
-            s = lif_exp_neuron<(KIND == kGlif3 ? kGlif3 : kLif), true, true, SX, false>(
-                a, lane, nidx, i, p, wz, x, drv, v, r, ia, q, tau, &s2);
+            } else {
+                s = lif_exp_neuron<(KIND == kGlif3 ? kGlif3 : kLif), true, true, SX, false>(
+                    a, lane, nidx, i, p, wz, x, drv, v, r, ia, q, tau, &s2);
+            }
+            if (GLIF && a.iasc != nullptr) {
+    #pragma unroll
+                for (int j = 0; j < kMaxAsc; ++j)
+                    if (j < a.n_asc) a.iasc[i * a.n_asc + j] = ia[GLIF ? j : 0];
+            }
+            a.v[i] = v;
+            if (a.use_ref && (ref_live || __float_as_uint(r) != 0u)) a.ref[i] = r;
+            a.psc[i] = p;
+            if (SX) {
+                a.sh1[i] = s2.h1;
+                if (a.syn == BTX_SYN_DUAL_EXP) a.sh2[i] = s2.h2;
+            }
+            if (TC && (!MIX || a.tia != nullptr)) {
+                a.tia[i] = ta;
+                if (bap_live || __float_as_uint(tb) != 0u) a.tibap[i] = tb;
+                a.tth[i] = tt;
+            }
         }
-        if (GLIF && a.iasc != nullptr) {
-#pragma unroll
-            for (int j = 0; j < kMaxAsc; ++j)
-                if (j < a.n_asc) a.iasc[i * a.n_asc + j] = ia[GLIF ? j : 0];
-        }
-        a.v[i] = v;
-        if (a.use_ref && (ref_live || __float_as_uint(r) != 0u)) a.ref[i] = r;
-        a.psc[i] = p;
-        if (SX) {
-            a.sh1[i] = s2.h1;
-            if (a.syn == BTX_SYN_DUAL_EXP) a.sh2[i] = s2.h2;
-        }
-        if (TC && (!MIX || a.tia != nullptr)) {
-            a.tia[i] = ta;
-            if (bap_live || __float_as_uint(tb) != 0u) a.tibap[i] = tb;
-            a.tth[i] = tt;
+        // half a spike word per lane: a wavefront holds two lanes' 32 neurons
+        const uint64_t on = __ballot(s != 0.f);
+        if (my_k == 0 && b < lg) {
+            const uint32_t half = (uint32_t)(on >> (32 * (my_lane & 1)));
+            const int64_t h = lane * nw32 + blockIdx.x;
+            // a lane without a trial pushes nothing and leaves its raster
+            const bool run = a.lane_t_end == nullptr || a.in_t0[lane] + a.t < a.lane_t_end[lane];
+            if (run) ((uint32_t*)a.raster)[h] = half;
+            uint32_t push = half;
+            if (a.teacher != nullptr) {
+                push = ((const uint32_t*)a.teacher)[h];
+                const int64_t room = a.n - j0;  // bits past n never count
+                if (room < 32) push &= room > 0 ? (1u << room) - 1u : 0u;
+            }
+            push = run ? push : 0u;
+            ((uint32_t*)a.ring_words)[h] = push;
+            s_half[b] = push;
         }
     }
-    // half a spike word per lane: a wavefront holds two lanes' 32 neurons
-    const uint64_t on = __ballot(s != 0.f);
-    if (my_k == 0 && my_lane < lg) {
-        const uint32_t half = (uint32_t)(on >> (32 * (my_lane & 1)));
-        const int64_t h = lane * nw32 + blockIdx.x;
-        // a lane without a trial pushes nothing and leaves its raster
-        const bool run = a.lane_t_end == nullptr || a.in_t0[lane] + a.t < a.lane_t_end[lane];
-        if (run) ((uint32_t*)a.raster)[h] = half;
-        uint32_t push = half;
-        if (a.teacher != nullptr) {
-            push = ((const uint32_t*)a.teacher)[h];
-            const int64_t room = a.n - j0;  // bits past n never count
-            if (room < 32) push &= room > 0 ? (1u << room) - 1u : 0u;
-        }
-        push = run ? push : 0u;
-        ((uint32_t*)a.ring_words)[h] = push;
-        s_half[my_lane] = push;
-    }
+    if (g.fin) return;
     __syncthreads();
-    // the lane bits of neuron j0 + tid in this group of 16 lanes
+    // the lane bits of neuron j0 + tid in this group of lanes
     if (tid < kGatherNeurons && j0 + tid < a.n) {
-        uint32_t m = 0u;
-        for (int b = 0; b < lg; ++b) m |= ((s_half[b] >> tid) & 1u) << b;
-        g.lane_bits_out[(j0 + tid) * 4 * g.lw + blockIdx.y] = (uint16_t)m;
+        uint64_t m = 0u;
+        for (int b = 0; b < lg; ++b) m |= (uint64_t)((s_half[b] >> tid) & 1u) << b;
+        uint64_t* words = g.lane_bits_out + (j0 + tid) * g.lw;
+        if (WIDE) words[blockIdx.y] = m;
+        else ((uint16_t*)words)[blockIdx.y] = (uint16_t)m;
+    }
+}
+
+// Before k_pull: the lane bits of the ring slot that the last complete step
+// wrote (a wavefront per word and 64-lane group), when the launch marks or a
+// bin of this step's push overflowed; then every slot, unless each was marked
+// already, and the step becomes a pull.  (An atomic per spike in the F role
+// instead held a 64-lane step at 19 % activity to 46 us; without it, 18.  A
+// step whose bins overflowed, each neuron pulling for itself, took 3 - 6 ms.)
+__global__ __launch_bounds__(kThreads) void k_mark(const uint64_t* __restrict__ words, int64_t n,
+                                                   int64_t lanes, int lw,
+                                                   uint64_t* __restrict__ bits, int R,
+                                                   int64_t clock, int age, Ctl* __restrict__ ctl,
+                                                   const int* __restrict__ overflow,
+                                                   int* __restrict__ other_overflow) {
+    const int c = (int)(clock & 3);
+    const int over = *overflow, pull = ctl->push_mode[c];
+    // the other buffer's flag was last read by the previous step's k_pull
+    if (blockIdx.x == 0 && threadIdx.x == 0) *other_overflow = 0;
+    if (!over && !ctl->lane_bits_mode[c]) return;
+    const int64_t nwords = (n + 63) >> 6;
+    const bool all = over && !pull;
+    if (all && blockIdx.x == 0 && threadIdx.x == 0) ctl->lane_bits_run = 1 << 20;
+    const int64_t per = nwords * lw;
+    for (int64_t u = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+         u < per * (all ? R : 1); u += (int64_t)gridDim.x * (kThreads / 64)) {
+        const int64_t slot = all ? u / per : ring_slot(clock, age, R);
+        const int64_t v = all ? u % per : u;
+        transpose_lane_bits(words + slot * lanes * nwords, bits + slot * n * lw, lanes, nwords, n,
+                            lw, v / lw, (int)(v % lw));
     }
 }
 
 // The dense pull of a step as a launch of its own, after the step's launch
 // (batches of more than 32 lanes): one wavefront per destination and 64-lane
-// group, four destinations per workgroup.  Ends at once unless the previous
-// launch chose the pull for this step.
-__global__ __launch_bounds__(kThreads) void k_pull(PushStep p) {
-    __shared__ PushLds L;
-    if (ld_const(&p.ctl->push_mode[p.clock & 3]) == 0) return;
-    pull_role<true>(p, L, (int64_t)blockIdx.x, (int64_t)gridDim.x);
+// group, four destinations per workgroup.  A destination's edges are taken
+// 64 at a time, thread k reading edge c + k and its source's lane bits, and
+// added in order, a batch lane per thread; four such chunks are requested
+// together.  Ends at once unless the previous launch chose the pull for this
+// step or the step's bins overflowed (they are emptied then).
+__global__ __launch_bounds__(kThreads) void k_pull(PushStep a) {
+    __shared__ int s_slot[BTX_MAX_BINS];
+    const int over = ld_const(a.bin_cnt - 1);
+    if (ld_const(&a.ctl->push_mode[a.clock & 3]) == 0 && over == 0) return;
+    if (over) {
+        const int64_t m = a.lanes * a.nchunks;
+        for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < m;
+             k += (int64_t)gridDim.x * kThreads)
+            a.bin_cnt[k] = 0;
+        // the next launch takes the sums (its workgroups and this launch's
+        // others read the same answer from either word)
+        if (blockIdx.x == 0 && threadIdx.x == 0) const_cast<Ctl*>(a.ctl)->push_mode[a.clock & 3] = 1;
+    }
+    const int tid = threadIdx.x, ln = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const FastDiv fd = fast_div(a.csr_d);
+    if (tid < a.csr_d) {
+        const int age = a.ctl->age_of_sub[tid];
+        s_slot[tid] = age < 0 ? -1 : ring_slot(a.clock, age, a.R);
+    }
+    __syncthreads();
+    constexpr int U = 4;
+    for (int64_t d = (int64_t)blockIdx.x * (kThreads / 64) + wv; d < a.n;
+         d += (int64_t)gridDim.x * (kThreads / 64)) {
+        const int64_t e0 = ld_const(a.csc_ptr + d);
+        const int len = (int)(ld_const(a.csc_ptr + d + 1) - e0);
+        for (int g = 0; g < a.lw; ++g) {
+            const int64_t lane = 64 * (int64_t)g + ln;
+            float acc = 0.f;
+            for (int c = 0; c < len; c += 64 * U) {
+                float w[U];
+                uint64_t word[U];
+                int r[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int e = c + 64 * u + ln;
+                    r[u] = e < len ? a.csc_src[e0 + e] : -1;
+                    w[u] = e < len ? a.csc_w[e0 + e] : 0.f;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int vr = r[u] < 0 ? 0 : r[u];
+                    const int src = (int)div_u31(fd, (uint32_t)vr);
+                    const int slot = s_slot[vr - src * a.csr_d];
+                    word[u] = r[u] >= 0 && slot >= 0
+                                  ? a.lane_bits[((int64_t)slot * a.n + src) * a.lw + g] : 0ull;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) add_lanes(acc, w[u], word[u], __ballot(word[u] != 0ull));
+            }
+            if (lane < a.lanes) {
+                const bool live = a.lane_t_end == nullptr ||
+                                  a.in_t0[lane] + a.t < a.lane_t_end[lane];
+                a.pull_acc[lane * a.n + d] = live ? acc : 0.f;
+            }
+        }
+    }
 }
 
 // FIN: the last push reduced into the synapse.
@@ -2083,7 +2212,7 @@ static EngineWs engine_ws(int64_t lanes, int64_t n, int ordered) {
     if (ordered) {
         L.bins = lanes * nchunks;
         L.bin_cnt = off;
-        off = align256(off + sizeof(int) * 2 * L.bins);
+        off = align256(off + sizeof(int) * 2 * (kBinHead + L.bins));
         L.ev_r = off;
         off = align256(off + sizeof(int32_t) * 2 * L.bins * kBinCapMax);
         L.ev_w = off;
@@ -2416,12 +2545,19 @@ static void launch_step(int ordered, const StepArgs& a, const PushStep& ps,
 
 template <int KIND>
 static void launch_gather(const StepArgs& a, const GatherArgs& g, hipStream_t s) {
-    const dim3 grid((unsigned)(2 * a.nwords), (unsigned)((g.lanes + kGatherLanes - 1) / kGatherLanes));
+    auto grid = [&](int mode) {
+        const int64_t lg = gather_lanes(mode);
+        return dim3((unsigned)(2 * a.nwords), (unsigned)((g.lanes + lg - 1) / lg));
+    };
     if (g.lanes == 1)
-        hipLaunchKernelGGL((k_gather_step<KIND, true>), grid, dim3(kGatherThreads),
-                           (size_t)g.nbins * 8 * a.nwords + 16, s, a, g);
+        hipLaunchKernelGGL((k_gather_step<KIND, kGatherOne>), grid(kGatherOne),
+                           dim3(kGatherThreads), (size_t)g.nbins * 8 * a.nwords + 16, s, a, g);
+    else if (g.lanes <= gather_lanes(kGatherFew))
+        hipLaunchKernelGGL((k_gather_step<KIND, kGatherFew>), grid(kGatherFew),
+                           dim3(kGatherThreads), 0, s, a, g);
     else
-        hipLaunchKernelGGL((k_gather_step<KIND, false>), grid, dim3(kGatherThreads), 0, s, a, g);
+        hipLaunchKernelGGL((k_gather_step<KIND, kGatherWide>), grid(kGatherWide),
+                           dim3(kGatherThreads), 0, s, a, g);
 }
 
 static void launch_gather_k(const StepArgs& a, const GatherArgs& g, hipStream_t s) {
@@ -2453,7 +2589,8 @@ static bool gather_route(const btx_rsnn_plan* p, bool fused) {
             if (p->bin_sub[j] == p->bin_sub[k]) return false;
     if (p->lanes == 1 && (int64_t)p->nbins * 8 * ((p->n + 63) / 64) > kGatherBits) return false;
     const double edges = 1e-6 * (double)p->nnz;
-    const double groups = (double)((p->lanes + kGatherLanes - 1) / kGatherLanes);
+    const int lg = gather_lanes(p->lanes <= 16 ? kGatherFew : kGatherWide);
+    const double groups = (double)((p->lanes + lg - 1) / lg);
     const double gather = 7.5 + edges * (p->lanes == 1 ? 1.2 : (p->csr_d > 1 ? 4.6 : 2.6) * groups);
     const double kind = p->neuron_model == BTX_NEURON_LIF                ? 0.0
                         : p->neuron_model == BTX_NEURON_TWO_COMPARTMENT ? 3.4
@@ -2589,7 +2726,7 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         r.cap = cap;
         r.sort_max = p->slots;
         if (p->ordered) {
-            r.bin_cnt = (int*)(ws + L.bin_cnt) + b * L.bins;
+            r.bin_cnt = (int*)(ws + L.bin_cnt) + b * (kBinHead + L.bins) + kBinHead;
             r.ev_r = (const int32_t*)(ws + L.ev_r) + b * L.bins * kBinCapMax;
             r.ev_w = (const float*)(ws + L.ev_w) + b * L.bins * kBinCapMax;
             r.ev_d = (const uint16_t*)(ws + L.ev_d) + b * L.bins * kBinCapMax;
@@ -2704,6 +2841,12 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
     // push of 71k terms.
     const int above = (lanes * nchunks < 256 && kBinCap < cap / 2) ? kBinCap : cap / 2;
     ca.above = (float)above * (float)(lanes * nchunks);
+    // k_pull reads every edge for 64 lanes at ~7.6 us per million (102 us for
+    // 13.4M); a push costs ~58 us per million terms (4.3M terms in 1024 bins,
+    // 16k neurons, 64 lanes: 283 us a step): pull from 0.2 terms per edge on,
+    // where the push takes half as long again
+    if (ps.pull_sep && ca.above > 0.2f * (float)p->nnz * (float)lw)
+        ca.above = 0.2f * (float)p->nnz * (float)lw;
 
     GatherArgs ga{};
     if (gather) {
@@ -2722,6 +2865,13 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         ga.delay0 = p->bin_delay[0];
     }
 
+    int* other_bins = nullptr;
+    // the launches of a batch whose dense pull is one of its own
+    auto pull_step = [&]() {
+        hipLaunchKernelGGL(k_mark, dim3(256), dim3(kThreads), 0, s, p->ring_words, n, lanes, lw,
+                           lane_bits, R, ps.clock, fused ? 1 : 0, ctl, ps.bin_cnt - 1, other_bins - 1);
+        hipLaunchKernelGGL(k_pull, pull_grid, dim3(kThreads), 0, s, ps);
+    };
     const int64_t rec_step = m;
     for (int64_t t = 0; t < n_steps; ++t) {
         a.prev = t > 0;
@@ -2742,7 +2892,8 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         a.ring_idx = p->ring_idx + slot * lanes * n;
         a.ring_cnt = p->ring_cnt + slot * lanes * nchunks;
         a.ring_words = p->ring_words + slot * lanes * nwords;
-        a.lane_bits = lane_bits ? lane_bits + slot * n * lw : nullptr;
+        // batches that pull in a launch of their own mark in k_mark
+        a.lane_bits = lane_bits && !ps.pull_sep ? lane_bits + slot * n * lw : nullptr;
         a.lw = lw;
         a.lane_bits_on = lane_bits ? &ctl->lane_bits_mode[(p->ring_cursor + t) & 3] : nullptr;
         a.rec_z = p->rec_z ? p->rec_z + t * rec_step : nullptr;
@@ -2765,6 +2916,9 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         ReduceIn cur{};
         bins_of((int)(t & 1), p->ring_cursor + t, cur);
         ps.bin_cnt = cur.bin_cnt;
+        ReduceIn other{};
+        bins_of((int)((t + 1) & 1), 0, other);
+        other_bins = other.bin_cnt;
         ps.ev_r = (int32_t*)cur.ev_r;
         ps.ev_w = (float*)cur.ev_w;
         ps.ev_d = (uint16_t*)cur.ev_d;
@@ -2772,7 +2926,7 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         ps.pull_acc = cur.pull_acc ? (float*)cur.pull_acc : nullptr;
         if (gather) {
             ga.slot0 = (int)mod(p->ring_cursor + t - 1, R);
-            ga.lane_bits_out = (uint16_t*)a.lane_bits;
+            ga.lane_bits_out = lane_bits + slot * n * lw;
             kt.begin(0);
             launch_gather_k(a, ga, s);
             kt.end(0);
@@ -2783,7 +2937,7 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
             kt.end(0);
             if (ps.pull_sep) {
                 kt.begin(2);
-                hipLaunchKernelGGL(k_pull, pull_grid, dim3(kThreads), 0, s, ps);
+                pull_step();
                 kt.end(2);
             }
         } else {
@@ -2796,7 +2950,7 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
             kt.begin(2);
             const dim3 pgrid((unsigned)lanes, (unsigned)(nc + npb + ps.nh));
             launch_step(p->ordered, a, ps, ca, npb, nc, group, pgrid, s);
-            if (ps.pull_sep) hipLaunchKernelGGL(k_pull, pull_grid, dim3(kThreads), 0, s, ps);
+            if (ps.pull_sep) pull_step();
             kt.end(2);
         }
     }
