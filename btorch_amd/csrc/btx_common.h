@@ -72,6 +72,8 @@ struct Ctl {
     // the latest decided, that marked
     int lane_bits_mode[4];
     int lane_bits_run;
+    int next_idx;        // batches that pull in a launch of their own: 1 + the index of the
+                         // latest decision in push_mode (0 = none)
     int bin_of_sub[64];  // delay bin by virtual-row offset, -1 = not read
 };
 

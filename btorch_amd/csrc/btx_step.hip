@@ -1960,34 +1960,34 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
     }
 }
 
-// Before k_pull: the lane bits of the ring slot that the last complete step
-// wrote (a wavefront per word and 64-lane group), when the launch marks or a
-// bin of this step's push overflowed; then every slot, unless each was marked
-// already, and the step becomes a pull.  (An atomic per spike in the F role
-// instead held a 64-lane step at 19 % activity to 46 us; without it, 18.  A
+// The lane bits of ring slot `slot`, or of every slot (slot < 0), a wavefront
+// per word and 64-lane group.
+__device__ __forceinline__ void mark_slots(const PushStep& a, const uint64_t* ring_words,
+                                           int64_t slot) {
+    const int64_t nwords = (a.n + 63) >> 6, per = nwords * a.lw;
+    for (int64_t u = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+         u < per * (slot < 0 ? a.R : 1); u += (int64_t)gridDim.x * (kThreads / 64)) {
+        const int64_t q = slot < 0 ? u / per : slot, v = slot < 0 ? u % per : u;
+        transpose_lane_bits(ring_words + q * a.lanes * nwords, a.lane_bits + q * a.n * a.lw,
+                            a.lanes, nwords, a.n, a.lw, v / a.lw, (int)(v % a.lw));
+    }
+}
+
+// Between the push and k_pull of a net with synapses of no delay, whose pull
+// reads the slot of its own step: that slot's lane bits (every slot's, unless
+// the step before pulled too), when the step pulls or a bin of its push
+// overflowed; k_pull then pulls that step.  (With an atomic per spike in the
+// F role instead, a 64-lane step at 19 % activity took 46 us; without, 19.  A
 // step whose bins overflowed, each neuron pulling for itself, took 3 - 6 ms.)
-__global__ __launch_bounds__(kThreads) void k_mark(const uint64_t* __restrict__ words, int64_t n,
-                                                   int64_t lanes, int lw,
-                                                   uint64_t* __restrict__ bits, int R,
-                                                   int64_t clock, int age, Ctl* __restrict__ ctl,
-                                                   const int* __restrict__ overflow,
+__global__ __launch_bounds__(kThreads) void k_mark(PushStep a,
+                                                   const uint64_t* __restrict__ ring_words,
                                                    int* __restrict__ other_overflow) {
-    const int c = (int)(clock & 3);
-    const int over = *overflow, pull = ctl->push_mode[c];
+    const int over = a.bin_cnt[-1];
     // the other buffer's flag was last read by the previous step's k_pull
     if (blockIdx.x == 0 && threadIdx.x == 0) *other_overflow = 0;
-    if (!over && !ctl->lane_bits_mode[c]) return;
-    const int64_t nwords = (n + 63) >> 6;
-    const bool all = over && !pull;
-    if (all && blockIdx.x == 0 && threadIdx.x == 0) ctl->lane_bits_run = 1 << 20;
-    const int64_t per = nwords * lw;
-    for (int64_t u = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-         u < per * (all ? R : 1); u += (int64_t)gridDim.x * (kThreads / 64)) {
-        const int64_t slot = all ? u / per : ring_slot(clock, age, R);
-        const int64_t v = all ? u % per : u;
-        transpose_lane_bits(words + slot * lanes * nwords, bits + slot * n * lw, lanes, nwords, n,
-                            lw, v / lw, (int)(v % lw));
-    }
+    if (!over && !a.ctl->push_mode[a.clock & 3]) return;
+    const bool newest = a.R == 2 || a.ctl->push_mode[(a.clock - 1) & 3] != 0;
+    mark_slots(a, ring_words, newest ? ring_slot(a.clock, 0, a.R) : -1);
 }
 
 // The dense pull of a step as a launch of its own, after the step's launch
@@ -1995,12 +1995,29 @@ __global__ __launch_bounds__(kThreads) void k_mark(const uint64_t* __restrict__ 
 // group, four destinations per workgroup.  A destination's edges are taken
 // 64 at a time, thread k reading edge c + k and its source's lane bits, and
 // added in order, a batch lane per thread; four such chunks are requested
-// together.  Ends at once unless the previous launch chose the pull for this
-// step or the step's bins overflowed (they are emptied then).
-__global__ __launch_bounds__(kThreads) void k_pull(PushStep a) {
+// together (13.4M edges, 64 lanes, 19 % activity: 241 us with a select and an
+// add per edge out of register lanes, 112 with the lane bits as the add's
+// execution mask).  Ends at once unless the previous launch chose the pull
+// for this step or the step's bins overflowed (they are emptied then; nets
+// with synapses of no delay).  Where every synapse delays, the launch before
+// a pull has marked the slots it reads: the newest alone if that one pulled.
+__global__ __launch_bounds__(kThreads) void k_pull(PushStep a,
+                                                   const uint64_t* __restrict__ ring_words,
+                                                   int fused) {
     __shared__ int s_slot[BTX_MAX_BINS];
-    const int over = ld_const(a.bin_cnt - 1);
-    if (ld_const(&a.ctl->push_mode[a.clock & 3]) == 0 && over == 0) return;
+    const int over = fused ? 0 : ld_const(a.bin_cnt - 1);
+    const int pull = ld_const(&a.ctl->push_mode[a.clock & 3]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        // the slots a pull reads are marked when it is known: the step
+        // control need not have marked ahead
+        Ctl* ctl = const_cast<Ctl*>(a.ctl);
+        ctl->lane_bits_mode[(a.clock + 1) & 3] = 1;
+        ctl->lane_bits_run = 1 << 20;
+        ctl->next_idx = 1 + (int)((a.clock + 1) & 3);
+    }
+    if (fused && ld_const(&a.ctl->push_mode[(a.clock + 1) & 3]))
+        mark_slots(a, ring_words, pull ? ring_slot(a.clock, 0, a.R) : -1);
+    if (!pull && !over) return;
     if (over) {
         const int64_t m = a.lanes * a.nchunks;
         for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < m;
@@ -2008,7 +2025,8 @@ __global__ __launch_bounds__(kThreads) void k_pull(PushStep a) {
             a.bin_cnt[k] = 0;
         // the next launch takes the sums (its workgroups and this launch's
         // others read the same answer from either word)
-        if (blockIdx.x == 0 && threadIdx.x == 0) const_cast<Ctl*>(a.ctl)->push_mode[a.clock & 3] = 1;
+        if (blockIdx.x == 0 && threadIdx.x == 0)
+            const_cast<Ctl*>(a.ctl)->push_mode[a.clock & 3] = 1;
     }
     const int tid = threadIdx.x, ln = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2190,6 +2208,13 @@ __global__ __launch_bounds__(64) void k_set_tables(RunTables t, Ctl* __restrict_
     ctl->bin_delay[k] = arg->bin_delay[k];
     ctl->bin_sub[k] = arg->bin_sub[k];
     ctl->bin_of_sub[k] = arg->bin_of_sub[k];
+    // the last run's decision about the step after it, at whichever index
+    // this run's clock reads it
+    const int next = ctl->next_idx;
+    if (next > 0) {
+        const int push = ctl->push_mode[(next - 1) & 3];
+        if (k < 4) ctl->push_mode[k] = push;
+    }
 }
 
 static inline int64_t mod(int64_t a, int64_t b) {
@@ -2868,9 +2893,11 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
     int* other_bins = nullptr;
     // the launches of a batch whose dense pull is one of its own
     auto pull_step = [&]() {
-        hipLaunchKernelGGL(k_mark, dim3(256), dim3(kThreads), 0, s, p->ring_words, n, lanes, lw,
-                           lane_bits, R, ps.clock, fused ? 1 : 0, ctl, ps.bin_cnt - 1, other_bins - 1);
-        hipLaunchKernelGGL(k_pull, pull_grid, dim3(kThreads), 0, s, ps);
+        if (!fused)
+            hipLaunchKernelGGL(k_mark, dim3(256), dim3(kThreads), 0, s, ps, p->ring_words,
+                               other_bins - 1);
+        hipLaunchKernelGGL(k_pull, pull_grid, dim3(kThreads), 0, s, ps, p->ring_words,
+                           fused ? 1 : 0);
     };
     const int64_t rec_step = m;
     for (int64_t t = 0; t < n_steps; ++t) {

@@ -275,7 +275,7 @@ class _RingState:
         self.idx, self.cnt, self.words, self.lane_bits = Engine._ring_buffers(ring_d, lanes, n,
                                                                               dev)
         self.R = ring_d + 1
-        self.cursor = ring_d          # device slot of the next run's first step
+        self.cursor = ring_d          # clock of the next run's first step (its slot: mod R)
         self.token = None             # module history the ring holds (Engine._hist_token), or None
         self.fresh = True             # lists not built yet
 
@@ -706,7 +706,9 @@ class Engine:
             recs["z"] = z
         if mixed:
             sp.neuron.scatter()
-        ring.cursor = (ring.cursor + T) % ring.R
+        # the clock of the next run: its slot is that modulo R, and the step
+        # control's decisions are indexed by it modulo 4
+        ring.cursor = (ring.cursor + T) % (4 * ring.R)
         self._defer_history(ring, lanes, n, T)
         return raster, recs
 

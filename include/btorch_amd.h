@@ -311,7 +311,10 @@ typedef struct btx_rsnn_plan {
     int ring_d;
     int32_t* ring_idx;    /* [ring_d][lanes][n] */
     int32_t* ring_cnt;    /* [ring_d][lanes][ceil(n/BTX_RING_CHUNK)] */
-    int ring_cursor;      /* ring slot that receives z of the first step */
+    int ring_cursor;      /* clock of the first step: its z goes to ring slot ring_cursor
+                           * mod (ring_d + 1); a run that continues another with
+                           * tables_ready = 1 passes that run's clock plus its steps
+                           * (reduced, if at all, by a multiple of 4*(ring_d + 1)) */
     int nbins;            /* delay bins read each step */
     int bin_delay[BTX_MAX_BINS];  /* ring age of bin j (0 = this step) */
     int bin_sub[BTX_MAX_BINS];    /* virtual-row offset of bin j */

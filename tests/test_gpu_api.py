@@ -474,3 +474,37 @@ def test_engine_gather_steps_match_pushed_steps_and_oracle(n, lanes, D):
         assert bits_equal(got[0], ref["z"])
         assert bits_equal(got[1], ref["v"]) and bits_equal(got[2], ref["psc"])
     assert torch.equal(h0, h1) and torch.equal(h0, h2)
+
+
+@pytest.mark.parametrize("lanes,bin_cap", [(33, 256), (40, 0), (70, 512)])
+def test_engine_undelayed_bursts_pull_in_their_own_launch(lanes, bin_cap):
+    # nets whose synapses deliver without delay, too many edges to gather
+    # every step, more than 32 lanes: a burst overflows the term bins of a
+    # quiet net (the step is pulled once that is seen), then steps pull as
+    # decided one ahead, then the net falls quiet and pushes again; two calls,
+    # so that the second continues from the first's last decision
+    n, T = 6000, 14
+    c = workloads.er_net_fast(n=n, p=0.1, seed=61, w_mu=-7.0)
+    assert c.nnz > 3_400_000
+    conn = SparseConn(c.matrix(), sparse_config={"bin_cap": bin_cap})
+    model = RecurrentNN(LIF(n, tau_ref=0.3), ExponentialPSC(n, 5.0, conn), step_mode="m",
+                        update_state_names=["neuron.v", "synapse.psc"]).to(DEV)
+    functional.init_net_state(model, batch_size=lanes, device=DEV, dtype=torch.float32)
+    g = torch.Generator().manual_seed(61)
+    rate = torch.zeros(2 * T)
+    rate[2:] = 1e-3
+    rate[5:9] = 0.4     # the burst
+    rate[12:16] = 0.3   # another, across the two calls
+    x = (torch.rand((2 * T, lanes, n), generator=g) < rate[:, None, None]).float() * 14.0
+    out = []
+    with environ.context(dt=0.1), torch.no_grad():
+        for k in range(2):
+            z, st = model(x[k * T:(k + 1) * T].to(DEV))
+            out.append((z.cpu(), st["neuron.v"].cpu(), st["synapse.psc"].cpu()))
+    z, v, psc = (torch.cat(t) for t in zip(*out))
+    net = rsnn.Net(n, c.matrix(), rsnn.LIFParams.make(n, tau_ref=0.3), torch.tensor(5.0), 0.1)
+    ref = rsnn.simulate(net, x)
+    per_step = ref["z"].sum((1, 2)) / (lanes * n)
+    assert per_step[5:8].max() > 0.2 and per_step[:5].max() < 0.01
+    assert bits_equal(z, ref["z"])
+    assert bits_equal(v, ref["v"]) and bits_equal(psc, ref["psc"])
