@@ -185,6 +185,19 @@ def pack_rows(x: torch.Tensor) -> torch.Tensor:
     return words
 
 
+def lane_masks(words: torch.Tensor, n: int) -> torch.Tensor:
+    """(K, B, ceil(n/64)) int64 spike words -> (K, n) int64 lane masks (bit b
+    of mask (t, j) = lane b spiked at neuron j; B <= 64)."""
+    _lib.require_hip(words)
+    K, B, nw = words.shape
+    if nw != (n + 63) // 64 or not words.is_contiguous() or not 1 <= B <= 64:
+        raise ValueError("words must be contiguous (K, B <= 64, ceil(n/64))")
+    masks = torch.empty((K, n), dtype=torch.int64, device=words.device)
+    _lib.check(_lib.load().btx_lane_masks(words.data_ptr(), K, B, n, masks.data_ptr(),
+                                          _lib.stream_ptr()), "btx_lane_masks")
+    return masks
+
+
 def unpack_rows(words: torch.Tensor, n: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """(rows, ceil(n/64)) int64 words -> (rows, n) float32 0/1 (into ``out`` rows if given)."""
     _lib.require_hip(words)

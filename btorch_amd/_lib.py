@@ -164,6 +164,8 @@ class AdjLifArgs(ctypes.Structure):
         ("gpsc", _vp),
         ("gx", _vp),
         ("gtau", _vp),
+        ("gpsc_out", _vp),
+        ("lane_major", _c_int),
     ]
 
 
@@ -210,6 +212,9 @@ _SIGNATURES = {
     "btx_adj_lif_step": (_c_int, [ctypes.POINTER(AdjLifArgs), _vp]),
     "btx_adj_lif_chunk": (_c_int, [ctypes.POINTER(AdjLifArgs), _c_i64, _vp, _vp, _vp, _vp, _vp,
                                    _vp]),
+    "btx_adj_lif_sweep": (_c_int, [ctypes.POINTER(AdjLifArgs), _c_i64, _c_i64, _vp, _vp, _vp, _vp,
+                                   _c_int, _vp, _vp, _vp, _vp, _vp]),
+    "btx_lane_masks": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp, _vp]),
     "btx_adj_transpose": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i64, _vp, _vp, _vp]),
     "btx_adj_wgrad": (_c_int, [_vp, _vp, _c_i64, _c_i64, _vp, _vp, _vp, _vp]),
     "btx_adj_transpose_delayed": (_c_int, [_vp, _vp, _vp, _c_i64, _c_int, _c_i64, _vp, _c_i64,

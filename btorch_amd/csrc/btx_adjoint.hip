@@ -51,6 +51,7 @@ struct AdjArgs {
     float* gpsc;
     float* gx;
     float* gtau;
+    float* gpsc_out;
 };
 
 __device__ __forceinline__ float surrogate_grad(int kind, float u, float alpha, float damping) {
@@ -99,11 +100,92 @@ __global__ __launch_bounds__(256) void k_adj_lif(AdjArgs a) {
     a.gx[i] = gI;
     const float k = a.ksyn[a.ksyn_s * j];
     const float ts = a.tsyn[a.tsyn_s * j];
-    a.gpsc[i] = gI + gpn * (1.f - k / ts);
+    a.gpsc_out[i] = gI + gpn * (1.f - k / ts);
     if (a.gtau) {
         const float gt = gv1 * a.dt * (v - vr) / (tau * tau);
         atomicAdd(&a.gtau[a.tau_s * j], gt);
     }
+}
+
+// The reverse step where everything but gsyn and gpsc, which the products
+// read and write, is lane-major (lanes, n), as the forward run left it: no
+// array is transposed ahead of the sweep.  A workgroup takes 32 neurons of all
+// lanes; gsyn and gpsc pass through LDS.  Bound by its eleven arrays (46 MB a
+// step at 16k neurons x 64 lanes).  dL/dtau is summed over the lanes in the
+// workgroup (an atomic per element, 64 to one address, took 140 us a step).
+constexpr int kAdjTile = 32;
+
+__global__ __launch_bounds__(256) void k_adj_lif_lanes(AdjArgs a) {
+    __shared__ float s_syn[kAdjTile * 65], s_psc[kAdjTile * 65], s_tau[256];
+    const int tid = threadIdx.x, lanes = (int)a.lanes;
+    const int pad = lanes | 1;
+    const int64_t j0 = (int64_t)blockIdx.x * kAdjTile;
+    const int rows = (int)(a.n - j0 < kAdjTile ? a.n - j0 : kAdjTile);
+    const int64_t base = j0 * lanes;
+    for (int k = tid; k < rows * lanes; k += 256) {
+        const int j = k / lanes, b = k - j * lanes;
+        s_syn[j * pad + b] = a.gsyn[base + k];
+        s_psc[j * pad + b] = a.gpsc[base + k];
+    }
+    __syncthreads();
+    const int j = tid & (kAdjTile - 1);
+    float gt = 0.f;
+    if (j < rows) {
+        const int64_t jn = j0 + j;
+        const float tau = a.tau[a.tau_s * jn], vth = a.vth[a.vth_s * jn];
+        const float vr = a.vr[a.vr_s * jn], cm = a.cm[a.cm_s * jn];
+        const float dpsc = 1.f - a.ksyn[a.ksyn_s * jn] / a.tsyn[a.tsyn_s * jn];
+        for (int b = tid / kAdjTile; b < lanes; b += 256 / kAdjTile) {
+            const int64_t i = (int64_t)b * a.n + jn;
+            const float v = a.v_prev[i], v1 = a.v_pre[i], s = a.z[i];
+            const float mask = a.ref_prev ? (a.ref_prev[i] == 0.f ? 1.f : 0.f) : 1.f;
+            const float gvn = a.gv[i], gpn = s_psc[j * pad + b];
+            float gs = (a.gz ? a.gz[i] : 0.f) + s_syn[j * pad + b];
+            float dvdv1 = 1.f;
+            if (a.hard_reset) {
+                dvdv1 = 1.f - s;
+                if (!a.detach_reset) gs += gvn * (-(v1 - vr));
+            } else if (!a.detach_reset) {
+                gs += gvn * (-(vth - vr));
+            }
+            const float u = (v1 - vth) / (vth - vr);
+            const float gu = gs * mask * surrogate_grad(a.surrogate, u, a.alpha, a.damping);
+            const float gv1 = gvn * dvdv1 + gu / (vth - vr);
+            a.gv[i] = gv1 * (1.f - a.dt / tau);
+            const float gI = gv1 * (a.dt / cm);
+            a.gx[i] = gI;
+            s_psc[j * pad + b] = gI + gpn * dpsc;
+            gt += gv1 * a.dt * (v - vr) / (tau * tau);
+        }
+    }
+    s_tau[tid] = gt;
+    __syncthreads();
+    for (int k = tid; k < rows * lanes; k += 256) {
+        const int jj = k / lanes;
+        a.gpsc_out[base + k] = s_psc[jj * pad + (k - jj * lanes)];
+    }
+    if (a.gtau && tid < kAdjTile) {
+        float t = 0.f;
+#pragma unroll
+        for (int k = 0; k < 256 / kAdjTile; ++k) t += s_tau[k * kAdjTile + tid];
+        if (a.tau_s) {
+            if (tid < rows) a.gtau[j0 + tid] += t;  // this workgroup's neuron alone
+        } else {
+#pragma unroll
+            for (int o = kAdjTile / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+            if (tid == 0) atomicAdd(a.gtau, t);
+        }
+    }
+}
+
+// Lane masks of K steps from their spike words [K][lanes][nwords] (lanes <=
+// 64): masks[K][n], one wavefront per word.
+__global__ __launch_bounds__(64) void k_lane_masks(const uint64_t* __restrict__ words,
+                                                   int64_t lanes, int64_t n,
+                                                   uint64_t* __restrict__ masks) {
+    const int64_t t = blockIdx.y, nwords = (n + 63) >> 6;
+    transpose_lane_bits(words + t * lanes * nwords, masks + t * n, lanes, nwords, n, 1,
+                        blockIdx.x, 0);
 }
 
 // g_src[j, b] = sum over edges e of row j of w[e] * g_dst[col[e], b]; one
@@ -250,85 +332,100 @@ __global__ __launch_bounds__(256) void k_adj_wgrad(const int64_t* __restrict__ r
     }
 }
 
-// k_adj_transpose and k_adj_wgrad of one reverse step in one pass (lanes <=
-// 64): each destination row of g_dst is loaded once per edge, feeds the
+// k_adj_transpose and k_adj_wgrad of one reverse step in one pass (33 to 64
+// lanes): each destination row of g_dst is loaded once per edge, feeds the
 // transposed sum of its lane and, when the neuron spiked in some lane, the
-// wavefront's LDS tile for the weight gradient.  Same sums in the same order
-// as the two kernels.
+// wavefront's LDS tile for the weight gradient.  Bound by the latency of the
+// gathered rows (4 MB of g_dst at 16k neurons x 64 lanes, from L2): the 32
+// rows of a tile are requested together, those of the next tile before the
+// current one is summed, and gw's old values before either (eight rows at a
+// time, gw last: 512 us a step at 13.4M edges; so: 392).
 __global__ __launch_bounds__(256) void k_adj_transpose_wgrad(
     const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
     const float* __restrict__ w, int64_t n_rows, int64_t lanes,
     const uint64_t* __restrict__ masks, const float* __restrict__ g_dst,
     float* __restrict__ g_src, float* __restrict__ gw) {
     __shared__ float tile[4][kWgradTile * 65];
-    const int wv = threadIdx.x >> 6;
-    const int64_t row = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4u + (unsigned)wv));
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t row = (int64_t)blockIdx.x * 4 + wv;
     const int ln = threadIdx.x & 63;
     if (row >= n_rows) return;
     const uint64_t mk = masks[row];
-    const int64_t e0 = rp[row], e1 = rp[row + 1];
+    const int64_t e0 = rp[row];
+    const int len = (int)(rp[row + 1] - e0);
     const bool on = ln < lanes;
     // lanes past `lanes` read column 0 (never stored, never summed)
     const float* gb = g_dst + (on ? ln : 0);
+    const int32_t* cs = col + e0;
+    const float* ws = w + e0;
+    float* gws = gw + e0;
     float* t = tile[wv];
     float acc0 = 0.f, acc1 = 0.f;
-    for (int64_t c = e0; c < e1; c += kWgradTile) {
-        const int m = (int)(e1 - c < kWgradTile ? e1 - c : kWgradTile);
-        const int my_d = ln < m ? col[c + ln] : 0;
-        const int my_w = ln < m ? __float_as_int(w[c + ln]) : 0;
-        int k = 0;
-        for (; k + 8 <= m; k += 8) {
-            float g8[8], w8[8];
+    float g[kWgradTile];
+    if (ln < kWgradTile) t[ln * 65 + 64] = 0.f;  // the column an odd set bit is missing from
+    int my_d = ln < len ? cs[ln] : 0;
+    auto request = [&](int m) {
+        if (m >= kWgradTile) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int64_t d = __builtin_amdgcn_readlane(my_d, k + j);
-                w8[j] = __int_as_float(__builtin_amdgcn_readlane(my_w, k + j));
-                g8[j] = gb[d * lanes];
-            }
+            for (int k = 0; k < kWgradTile; ++k)
+                g[k] = gb[(int64_t)__builtin_amdgcn_readlane(my_d, k) * lanes];
+        } else {
 #pragma unroll
-            for (int j = 0; j < 8; j += 2) {
-                acc0 += w8[j] * g8[j];
-                acc1 += w8[j + 1] * g8[j + 1];
-            }
-            if (mk) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) t[(k + j) * 65 + ln] = g8[j];
-            }
+            for (int k = 0; k < kWgradTile; ++k)
+                g[k] = k < m ? gb[(int64_t)__builtin_amdgcn_readlane(my_d, k) * lanes] : 0.f;
         }
-        for (; k + 2 <= m; k += 2) {
-            const int64_t d0 = __builtin_amdgcn_readlane(my_d, k);
-            const int64_t d1 = __builtin_amdgcn_readlane(my_d, k + 1);
-            const float w0 = __int_as_float(__builtin_amdgcn_readlane(my_w, k));
-            const float w1 = __int_as_float(__builtin_amdgcn_readlane(my_w, k + 1));
-            const float g0 = gb[d0 * lanes], g1 = gb[d1 * lanes];
-            acc0 += w0 * g0;
-            acc1 += w1 * g1;
-            if (mk) {
-                t[k * 65 + ln] = g0;
-                t[(k + 1) * 65 + ln] = g1;
+    };
+    if (len > 0) request(len);
+    for (int c = 0; c < len; c += kWgradTile) {
+        const int m = len - c < kWgradTile ? len - c : kWgradTile;
+        const bool mine = ln < m;
+        const int my_w = mine ? __float_as_int(ws[c + ln]) : 0;
+        const float old = mk && mine ? gws[c + ln] : 0.f;
+        // the next tile's destinations
+        const int nc = c + kWgradTile + ln;
+        my_d = ln < kWgradTile && nc < len ? cs[nc] : 0;
+        if (m == kWgradTile) {
+#pragma unroll
+            for (int k = 0; k < kWgradTile; k += 2) {
+                acc0 = fmaf(__int_as_float(__builtin_amdgcn_readlane(my_w, k)), g[k], acc0);
+                acc1 = fmaf(__int_as_float(__builtin_amdgcn_readlane(my_w, k + 1)), g[k + 1], acc1);
             }
-        }
-        if (k < m) {
-            const int64_t d0 = __builtin_amdgcn_readlane(my_d, k);
-            const float w0 = __int_as_float(__builtin_amdgcn_readlane(my_w, k));
-            const float g0 = gb[d0 * lanes];
-            acc0 += w0 * g0;
-            if (mk) t[k * 65 + ln] = g0;
+        } else {
+#pragma unroll
+            for (int k = 0; k < kWgradTile; ++k) {
+                if (k < m) {
+                    const float wk = __int_as_float(__builtin_amdgcn_readlane(my_w, k));
+                    if (k & 1) acc1 = fmaf(wk, g[k], acc1);
+                    else acc0 = fmaf(wk, g[k], acc0);
+                }
+            }
         }
         if (mk) {
+            // rows past m hold zeros or stale values nobody sums
+#pragma unroll
+            for (int k = 0; k < kWgradTile; ++k) t[k * 65 + ln] = g[k];
+        }
+        if (c + kWgradTile < len) request(len - c - kWgradTile);
+        if (mk) {
+            // the tile is the wavefront's own: its LDS writes land before its
+            // reads, the fences keep the compiler from moving them across
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (ln < m) {
-                float acc = 0.f;
-                uint64_t q = mk;
-                while (q) {
-                    const int b = __ffsll((unsigned long long)q) - 1;
-                    acc += t[ln * 65 + b];
-                    q &= q - 1;
-                }
-                gw[c + ln] += acc;
+            // thread ln sums row ln & 31 over half the set lanes: threads
+            // below 32 the even ones of mk, in order, the others the odd ones
+            const float* tr = t + (ln & (kWgradTile - 1)) * 65;
+            float acc = 0.f;
+            uint64_t q = mk;
+            while (q) {
+                const int b0 = __ffsll((unsigned long long)q) - 1;
+                q &= q - 1;
+                const int b1 = q ? __ffsll((unsigned long long)q) - 1 : 64;  // 64: a zero column
+                q &= q - 1;
+                acc += tr[ln < kWgradTile ? b0 : b1];
             }
+            acc += __shfl_xor(acc, 32, 64);
+            if (mine) gws[c + ln] = old + acc;
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -343,32 +440,88 @@ __global__ __launch_bounds__(256) void k_adj_transpose_wgrad(
 // -- the reverse delay ring.  G holds dL/dpsc of the K steps of a window,
 // [K][n][lanes]; step tau of the window reads G[tau + age] when that index
 // lies in [0, K) (later steps belong to another window).
-__global__ __launch_bounds__(256) void k_adj_transpose_delayed(
+//
+// One wavefront per neuron, 64 of whose edges are read at a time, a lane each
+// with the step its virtual row reads; PER = 64 / (lanes rounded up to a
+// power of two) edges are then summed side by side, eight of each in flight,
+// and the PER partial sums added at the end (an edge at a time, one wavefront
+// for 16 lanes: 36 us a step at 4096 neurons, 0.41M edges).  Also the
+// undelayed product of at most 32 lanes (csr_d = 1, age 0, K = 1).
+template <int PER>
+__global__ __launch_bounds__(256) void k_adj_transpose_rows(
     const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
     const float* __restrict__ w, int64_t n, int csr_d, int64_t lanes,
     const float* __restrict__ G, int64_t K, int64_t tau, const int* __restrict__ ages,
     float* __restrict__ g_src, int accumulate) {
-    const int64_t j = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t j = (int64_t)blockIdx.x * 4 + wv;
     const int ln = threadIdx.x & 63;
     if (j >= n) return;
-    for (int64_t b0 = 0; b0 < lanes; b0 += 64) {
-        const int64_t b = b0 + ln;
+    constexpr int W = 64 / PER;  // threads per edge
+    const int grp = ln / W;
+    const int64_t e0 = rp[j * csr_d];
+    const int len = (int)(rp[(j + 1) * csr_d] - e0);
+    // thread s: where virtual row s ends, and the step it reads (-1 = none)
+    int ends = 0x7fffffff, step = -1;
+    if (ln < csr_d) {
+        ends = (int)(rp[j * csr_d + ln + 1] - e0);
+        const int age = ages ? ages[ln] : 0;
+        const int64_t st = tau + age;
+        step = age >= 0 && st >= 0 && st < K ? (int)st : -1;
+    }
+    for (int64_t b0 = 0; b0 < lanes; b0 += W) {
+        const int64_t b = b0 + ln % W;
         const bool on = b < lanes;
+        const float* gb = G + (on ? b : 0);
         float acc = 0.f;
-        for (int sub = 0; sub < csr_d; ++sub) {
-            const int age = ages[sub];
-            const int64_t st = tau + age;
-            if (age < 0 || st < 0 || st >= K) continue;
-            const float* g = G + st * n * lanes;
-            const int64_t r = j * csr_d + sub;
-            for (int64_t e = rp[r]; e < rp[r + 1]; ++e) {
-                const int64_t d = col[e];
-                const float wv = w[e];
-                if (on) acc += wv * g[d * lanes + b];
+        for (int c = 0; c < len; c += 64) {
+            const int e = c + ln;
+            int sub = 0;
+            for (int s = 0; s + 1 < csr_d; ++s) sub += e >= __builtin_amdgcn_readlane(ends, s);
+            const int st = __shfl(step, sub, 64);
+            const bool in = e < len && st >= 0;
+            // row of G the edge reads, -1 = none
+            const int my_r = in ? (int)(st * n) + col[e0 + e] : -1;
+            const float my_w = in ? w[e0 + e] : 0.f;
+            if (__ballot(in) == 0ull) continue;
+            const int m = len - c < 64 ? len - c : 64;
+            for (int k = 0; k < m; k += 8 * PER) {
+                float g8[8], w8[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int src = k + u * PER + grp;
+                    const int r = __shfl(my_r, src & 63, 64);
+                    w8[u] = __shfl(my_w, src & 63, 64);
+                    const bool use = src < m && r >= 0;
+                    g8[u] = use ? gb[(int64_t)r * lanes] : 0.f;
+                    w8[u] = use ? w8[u] : 0.f;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) acc = fmaf(w8[u], g8[u], acc);
             }
         }
-        if (on) g_src[j * lanes + b] = accumulate ? g_src[j * lanes + b] + acc : acc;
+#pragma unroll
+        for (int o = W; o < 64; o <<= 1) acc += __shfl_xor(acc, o, 64);
+        if (on && grp == 0) g_src[j * lanes + b] = accumulate ? g_src[j * lanes + b] + acc : acc;
     }
+}
+
+static void launch_transpose_rows(const int64_t* rp, const int32_t* col, const float* w, int64_t n,
+                                  int csr_d, int64_t lanes, const float* G, int64_t K, int64_t tau,
+                                  const int* ages, float* g_src, int accumulate, hipStream_t s) {
+    const dim3 grid((unsigned)((n + 3) / 4)), block(256);
+    if (lanes > 32)
+        hipLaunchKernelGGL(k_adj_transpose_rows<1>, grid, block, 0, s, rp, col, w, n, csr_d, lanes,
+                           G, K, tau, ages, g_src, accumulate);
+    else if (lanes > 16)
+        hipLaunchKernelGGL(k_adj_transpose_rows<2>, grid, block, 0, s, rp, col, w, n, csr_d, lanes,
+                           G, K, tau, ages, g_src, accumulate);
+    else if (lanes > 8)
+        hipLaunchKernelGGL(k_adj_transpose_rows<4>, grid, block, 0, s, rp, col, w, n, csr_d, lanes,
+                           G, K, tau, ages, g_src, accumulate);
+    else
+        hipLaunchKernelGGL(k_adj_transpose_rows<8>, grid, block, 0, s, rp, col, w, n, csr_d, lanes,
+                           G, K, tau, ages, g_src, accumulate);
 }
 
 // gw[e] += sum over lanes b spiking at neuron j (mask bit b) of
@@ -438,6 +591,14 @@ BTX_API int btx_adj_lif_step(const btx_adj_lif_args* p, void* stream) {
     a.gpsc = p->gpsc;
     a.gx = p->gx;
     a.gtau = p->gtau;
+    a.gpsc_out = p->gpsc_out ? p->gpsc_out : p->gpsc;
+    if (p->lane_major) {
+        if (p->lanes > 64) return fail("btx_adj_lif_step: at most 64 lanes lane-major");
+        hipLaunchKernelGGL(k_adj_lif_lanes, dim3((unsigned)((p->n + kAdjTile - 1) / kAdjTile)),
+                           dim3(256), 0, (hipStream_t)stream, a);
+        return check_launch("btx_adj_lif_step");
+    }
+    if (p->gz == nullptr) return fail("btx_adj_lif_step: gz is required neuron-major");
     hipLaunchKernelGGL(k_adj_lif, dim3((unsigned)((m + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream, a);
     return check_launch("btx_adj_lif_step");
@@ -466,29 +627,76 @@ BTX_API int btx_adj_lif_chunk(const btx_adj_lif_args* p, int64_t K, const int64_
                               const int32_t* col, const float* w, const uint64_t* masks,
                               float* gw, void* stream) {
     if (p == nullptr) return fail("btx_adj_lif_chunk: null args");
+    return btx_adj_lif_sweep(p, K, p->n * p->lanes, nullptr, row_ptr, col, w, 1, nullptr, nullptr,
+                             masks, gw, stream);
+}
+
+BTX_API int btx_adj_lif_sweep(const btx_adj_lif_args* p, int64_t K, int64_t gz_stride,
+                              const float* ref_entry, const int64_t* row_ptr, const int32_t* col,
+                              const float* w, int csr_d, const int* ages, float* G,
+                              const uint64_t* masks, float* gw, void* stream) {
+    if (p == nullptr) return fail("btx_adj_lif_sweep: null args");
     if (K <= 0 || p->n <= 0 || p->lanes <= 0) return 0;
-    if (p->lanes > 64) return fail("btx_adj_lif_chunk: at most 64 lanes per mask word");
+    if (p->lanes > 64) return fail("btx_adj_lif_sweep: at most 64 lanes per mask word");
     if (p->gsyn == nullptr || p->gpsc == nullptr || masks == nullptr || gw == nullptr)
-        return fail("btx_adj_lif_chunk: gsyn, gpsc, masks and gw are required");
+        return fail("btx_adj_lif_sweep: gsyn, gpsc, masks and gw are required");
+    const bool delayed = ages != nullptr;
+    if (delayed && (G == nullptr || csr_d < 1 || csr_d > BTX_MAX_BINS))
+        return fail("btx_adj_lif_sweep: delays need G and 1 <= csr_d <= 64");
+    if (delayed && K * p->n >= (int64_t)1 << 31)
+        return fail("btx_adj_lif_sweep: K*n exceeds int32");
     const int64_t m = p->n * p->lanes;
+    const hipStream_t st = (hipStream_t)stream;
+    const dim3 rows((unsigned)((p->n + 3) / 4));
     btx_adj_lif_args s = *p;
     for (int64_t t = K - 1; t >= 0; --t) {
         // dL/dpsc after step t through the transposed product and the weight
-        // gradient of step t's spikes (one pass), then the elementwise
-        // reverse step
-        hipLaunchKernelGGL(k_adj_transpose_wgrad, dim3((unsigned)((p->n + 3) / 4)), dim3(256), 0,
-                           (hipStream_t)stream, row_ptr, col, w, p->n, p->lanes,
-                           masks + t * p->n, p->gpsc, (float*)p->gsyn, gw);
-        if (int rc = check_launch("btx_adj_lif_chunk")) return rc;
+        // gradient of step t's spikes (33 to 64 lanes without delays: one
+        // pass), then the elementwise reverse step
+        const uint64_t* mk = masks + t * p->n;
+        float* gsyn = (float*)p->gsyn;
+        if (delayed) {
+            launch_transpose_rows(row_ptr, col, w, p->n, csr_d, p->lanes, G, K, t, ages, gsyn, 0, st);
+            hipLaunchKernelGGL(k_adj_wgrad_delayed, rows, dim3(256), 0, st, row_ptr, col, p->n,
+                               csr_d, p->lanes, mk, G, K, t, ages, gw);
+            s.gpsc = G + t * m;
+            s.gpsc_out = t > 0 ? G + (t - 1) * m : p->gpsc;
+        } else if (p->lanes > 32) {
+            hipLaunchKernelGGL(k_adj_transpose_wgrad, rows, dim3(256), 0, st, row_ptr, col, w, p->n,
+                               p->lanes, mk, p->gpsc, gsyn, gw);
+        } else {
+            launch_transpose_rows(row_ptr, col, w, p->n, 1, p->lanes, p->gpsc, 1, 0, nullptr, gsyn,
+                                  0, st);
+            hipLaunchKernelGGL(k_adj_wgrad, rows, dim3(256), 0, st, row_ptr, col, p->n, p->lanes,
+                               mk, p->gpsc, gw);
+        }
+        if (int rc = check_launch("btx_adj_lif_sweep")) return rc;
         s.v_prev = p->v_prev + t * m;
         s.v_pre = p->v_pre + t * m;
         s.z = p->z + t * m;
-        s.ref_prev = p->ref_prev ? p->ref_prev + t * m : nullptr;
-        s.gz = p->gz + t * m;
+        if (p->ref_prev)
+            s.ref_prev = ref_entry == nullptr ? p->ref_prev + t * m
+                         : t == 0             ? ref_entry
+                                              : p->ref_prev + (t - 1) * m;
+        s.gz = p->gz ? p->gz + t * gz_stride : nullptr;
         s.gx = p->gx + t * m;
         if (int rc = btx_adj_lif_step(&s, stream)) return rc;
     }
     return 0;
+}
+
+BTX_API int btx_lane_masks(const uint64_t* words, int64_t steps, int64_t lanes, int64_t n,
+                           uint64_t* masks, void* stream) {
+    if (steps <= 0 || lanes <= 0 || n <= 0) return 0;
+    if (lanes > 64) return fail("btx_lane_masks: at most 64 lanes per mask word");
+    const int64_t nwords = (n + 63) / 64;
+    for (int64_t t0 = 0; t0 < steps; t0 += 65535) {
+        const int64_t t = steps - t0 < 65535 ? steps - t0 : 65535;
+        hipLaunchKernelGGL(k_lane_masks, dim3((unsigned)nwords, (unsigned)t), dim3(64), 0,
+                           (hipStream_t)stream, words + t0 * lanes * nwords, lanes, n,
+                           masks + t0 * n);
+    }
+    return check_launch("btx_lane_masks");
 }
 
 BTX_API int btx_adj_transpose_delayed(const int64_t* row_ptr, const int32_t* col, const float* w,
@@ -497,9 +705,9 @@ BTX_API int btx_adj_transpose_delayed(const int64_t* row_ptr, const int32_t* col
                                       int accumulate, void* stream) {
     if (n <= 0 || lanes <= 0) return 0;
     if (csr_d < 1 || csr_d > BTX_MAX_BINS) return fail("btx_adj_transpose_delayed: bad csr_d");
-    hipLaunchKernelGGL(k_adj_transpose_delayed, dim3((unsigned)((n + 3) / 4)), dim3(256), 0,
-                       (hipStream_t)stream, row_ptr, col, w, n, csr_d, lanes, G, K, tau, ages,
-                       g_src, accumulate);
+    if (K * n >= (int64_t)1 << 31) return fail("btx_adj_transpose_delayed: K*n exceeds int32");
+    launch_transpose_rows(row_ptr, col, w, n, csr_d, lanes, G, K, tau, ages, g_src, accumulate,
+                          (hipStream_t)stream);
     return check_launch("btx_adj_transpose_delayed");
 }
 

@@ -52,6 +52,27 @@ __device__ __forceinline__ int block_excl_scan(int v, int& total) {
     return r;
 }
 
+// Lane words from spike words without atomics: one wavefront turns word `wi`
+// of the 64 lanes of group g (one load per lane) into the 64 neurons' lane
+// words, bit b of neuron 64*wi + k = bit k of lane 64*g + b, one ballot per
+// neuron.  Every lane of the wavefront calls it with the same (wi, g).
+__device__ __forceinline__ void transpose_lane_bits(const uint64_t* __restrict__ slot_words,
+                                                    uint64_t* __restrict__ slot_bits,
+                                                    int64_t lanes, int64_t nwords, int64_t n,
+                                                    int lw, int64_t wi, int g) {
+    const int l = (int)(threadIdx.x & 63);
+    const int64_t lane = 64 * (int64_t)g + l;
+    const uint64_t word = lane < lanes ? slot_words[lane * nwords + wi] : 0ull;
+    uint64_t mine = 0ull;
+#pragma unroll 8
+    for (int k = 0; k < 64; ++k) {
+        const uint64_t m = __ballot((word >> k) & 1ull);
+        if (l == k) mine = m;
+    }
+    const int64_t j = 64 * wi + l;
+    if (j < n) slot_bits[j * lw + g] = mine;
+}
+
 // Control block at the head of every workspace: per-run tables that kernels
 // index with a run-time value.  (Indexing an array held in the kernel
 // argument block with a run-time index makes the compiler copy the whole

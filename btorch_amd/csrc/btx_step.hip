@@ -901,28 +901,6 @@ __device__ __forceinline__ void mark_lane_bits(uint64_t* __restrict__ slot_bits,
     }
 }
 
-// The lane-bit ring of the dense pull, transposed from the ring's spike
-// words without atomics (when the ring is rebuilt): one wavefront turns word `wi` of the 64 lanes of
-// group g (one load per lane) into the 64 neurons' lane words, bit b of
-// neuron 64*wi + k = bit k of lane 64*g + b, one ballot per neuron.  Every
-// lane of the wavefront calls it with the same (wi, g).
-__device__ __forceinline__ void transpose_lane_bits(const uint64_t* __restrict__ slot_words,
-                                                    uint64_t* __restrict__ slot_bits,
-                                                    int64_t lanes, int64_t nwords, int64_t n,
-                                                    int lw, int64_t wi, int g) {
-    const int l = (int)(threadIdx.x & 63);
-    const int64_t lane = 64 * (int64_t)g + l;
-    const uint64_t word = lane < lanes ? slot_words[lane * nwords + wi] : 0ull;
-    uint64_t mine = 0ull;
-#pragma unroll 8
-    for (int k = 0; k < 64; ++k) {
-        const uint64_t m = __ballot((word >> k) & 1ull);
-        if (l == k) mine = m;
-    }
-    const int64_t j = 64 * wi + l;
-    if (j < n) slot_bits[j * lw + g] = mine;
-}
-
 // State of neurons n0 .. n0+3 of a lane (`room` of them exist): one 16-byte
 // access when `vec` (uniform), else one per neuron.  Neurons past n read the
 // lane's first element `safe` instead (their values are never used), so no

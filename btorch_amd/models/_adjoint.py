@@ -1,13 +1,13 @@
 """Training path of the fused engine: BPTT through the hand-written adjoint.
 
 The forward of a chunk of K steps runs the fused engine; its backward walks
-the chunk in reverse with ``btx_adj_transpose`` (W dL/dpsc),
-``btx_adj_wgrad`` (event-driven dL/dW over the step's spiking neurons) and
-``btx_adj_lif_step`` (surrogate derivative, reset and synapse-decay adjoint,
-dL/dtau).  With delayed synapses the spike of step t reaches psc at steps
-t + age, so the transposed product and the weight gradient read dL/dpsc of
-those later steps (``btx_adj_transpose_delayed`` / ``btx_adj_wgrad_delayed``,
-the reverse delay ring); the spikes of the ring_d steps before a chunk enter
+the chunk in reverse in one call, ``btx_adj_lif_sweep``: per step the
+transposed product W dL/dpsc, the event-driven dL/dW over the step's spiking
+neurons, and the elementwise adjoint (surrogate derivative, reset and
+synapse decay, dL/dtau), on the forward's (K, B, N) arrays as they are.  With
+delayed synapses the spike of step t reaches psc at steps t + age, so the
+transposed product and the weight gradient read dL/dpsc of those later steps
+(the reverse delay ring); the spikes of the ring_d steps before a chunk enter
 it as a differentiable input and receive their gradient from it.  With ``grad_checkpoint`` a chunk keeps only its entry state and
 recomputes its forward in the backward (checkpoint every ``chunk_size``
 steps, rnn.py:177-240); otherwise the forward records are kept.
@@ -103,7 +103,9 @@ def adjoint_chunk(spec, traj: dict, grads: dict, w_csr: torch.Tensor, dt: float,
     """Reverse a chunk.
 
     traj: (K, B, N) ``v_prev``, ``v_pre``, ``z`` and ``ref_prev`` (or None),
-        the forward values of every step.
+        the forward values of every step; in place of ``ref_prev`` the
+        counters after each step, ``ref``, and those entering the chunk,
+        ``ref_entry``.
     grads: ``gz`` (K, B, N) or None, ``gv``/``gpsc`` (B, N) or None -- the
         gradients of the outputs and of the state after the chunk.
     valued_weights: z holds real values (relaxed forward) -- the weight
@@ -124,18 +126,12 @@ def adjoint_chunk(spec, traj: dict, grads: dict, w_csr: torch.Tensor, dt: float,
     def nb(t):  # (B, N) -> (N, B)
         return t.transpose(-1, -2).contiguous()
 
-    v_prev, v_pre, zz = nb(traj["v_prev"]), nb(traj["v_pre"]), nb(z)
-    ref_prev = nb(traj["ref_prev"]) if traj.get("ref_prev") is not None else None
-    gz = nb(grads["gz"]) if grads.get("gz") is not None else torch.zeros_like(zz)
-    gv = nb(grads["gv"]) if grads.get("gv") is not None else torch.zeros(n, B, device=dev)
-    gpsc = nb(grads["gpsc"]) if grads.get("gpsc") is not None else torch.zeros(n, B,
-                                                                              device=dev)
+    gpsc_in = nb(grads["gpsc"]) if grads.get("gpsc") is not None else torch.zeros(n, B, device=dev)
     gsyn = torch.empty(n, B, device=dev)
-    gx = torch.empty(K, n, B, device=dev)
     gw = torch.zeros(conn.nnz, device=dev)
     keep: list = []
     plan = _plan.lif_plan(neuron, B, dev, keep)
-    tau_vec, tau_s = keep[0], plan.tau_stride
+    tau_vec = keep[0]
     gtau = torch.zeros(tau_vec.numel(), device=dev)
     ts, tss, k, ks = syn.decay_coefficients(dev)
     kind, alpha, damping = _surrogate_code(neuron.surrogate_function, require_spiking=False)
@@ -151,42 +147,90 @@ def adjoint_chunk(spec, traj: dict, grads: dict, w_csr: torch.Tensor, dt: float,
     a.tau_syn, a.tau_syn_stride = ts.data_ptr(), tss
     a.k_syn, a.k_syn_stride = k.data_ptr(), ks
     a.gsyn = gsyn.data_ptr()
-    a.gv = gv.data_ptr()
-    a.gpsc = gpsc.data_ptr()
     a.gtau = gtau.data_ptr()
     layout = conn._layout
     w = w_csr.detach().to(torch.float32).contiguous()
-    shifts = torch.arange(B, device=dev, dtype=torch.int64)
-    if not valued_weights:
-        masks = ((zz != 0).to(torch.int64) << shifts).sum(-1).contiguous()  # (K, N)
-    if _delayed(spec):
-        if valued_weights:
+    delayed = _delayed(spec)
+    if valued_weights:
+        if delayed:
             raise NotImplementedError("the relaxed weight gradient covers undelayed synapses")
-        return _adjoint_delayed(spec, a, lib, stream, layout, w, masks, zz, v_prev, v_pre,
-                                ref_prev, gz, gv, gpsc, gsyn, gx, gw, gtau, past, shifts)
-    if not valued_weights:
-        # the whole reverse sweep in one call
-        a.v_prev, a.v_pre, a.z = v_prev.data_ptr(), v_pre.data_ptr(), zz.data_ptr()
-        a.ref_prev = ref_prev.data_ptr() if ref_prev is not None else None
-        a.gz, a.gx = gz.data_ptr(), gx.data_ptr()
-        _lib.check(lib.btx_adj_lif_chunk(a, K, layout.row_ptr.data_ptr(),
-                                         layout.col.data_ptr(), w.data_ptr(), masks.data_ptr(),
-                                         gw.data_ptr(), stream), "btx_adj_lif_chunk")
-        return {"gx": gx.permute(0, 2, 1).contiguous(), "gw": gw, "gtau": gtau,
-                "gv": gv.t().contiguous(), "gpsc": gpsc.t().contiguous()}
+        return _adjoint_relaxed(a, lib, stream, layout, w, traj, grads, gpsc_in, gsyn, gw, gtau, nb)
+    # the forward's arrays as they are, (K, B, N); a gradient that is the
+    # same every step (a mean over time) is read with step stride 0
+    v_prev, v_pre, zz = (traj[key].contiguous() for key in ("v_prev", "v_pre", "z"))
+    ref, ref_entry = traj.get("ref"), traj.get("ref_entry")
+    if ref is None and traj.get("ref_prev") is not None:
+        ref = traj["ref_prev"]
+    ref = ref.contiguous() if ref is not None else None
+    ref_entry = ref_entry.reshape(B, n).contiguous() if ref_entry is not None else None
+    gz, gz_stride = grads.get("gz"), 0
+    if gz is not None:
+        if gz.stride(0) == 0:
+            gz = gz[0].contiguous()
+        else:
+            gz, gz_stride = gz.contiguous(), B * n
+    gv = (grads["gv"].reshape(B, n).clone(memory_format=torch.contiguous_format)
+          if grads.get("gv") is not None else torch.zeros(B, n, device=dev))
+    gx = torch.empty(K, B, n, device=dev)
+    a.lane_major = 1
+    a.v_prev, a.v_pre, a.z = v_prev.data_ptr(), v_pre.data_ptr(), zz.data_ptr()
+    a.ref_prev = ref.data_ptr() if ref is not None else None
+    a.gz = gz.data_ptr() if gz is not None else None
+    a.gv, a.gx = gv.data_ptr(), gx.data_ptr()
+    from .._kernels import lane_masks, pack_rows
+    masks = lane_masks(pack_rows(zz.view(K * B, n)).view(K, B, -1), n)  # (K, N)
+    rp, col = layout.row_ptr.data_ptr(), layout.col.data_ptr()
+    ages, G, gpsc = None, None, gpsc_in
+    if delayed:
+        ages = _ages(spec, dev)
+        G = torch.empty(K, n, B, device=dev)  # dL/dpsc of every step of the chunk
+        G[K - 1].copy_(gpsc_in)
+        gpsc = torch.empty(n, B, device=dev)
+    a.gpsc = gpsc.data_ptr()
+    _lib.check(lib.btx_adj_lif_sweep(a, K, gz_stride,
+                                     None if ref_entry is None else ref_entry.data_ptr(), rp, col,
+                                     w.data_ptr(), spec.csr_d,
+                                     None if ages is None else ages.data_ptr(),
+                                     None if G is None else G.data_ptr(), masks.data_ptr(),
+                                     gw.data_ptr(), stream), "btx_adj_lif_sweep")
+    out = {"gx": gx, "gw": gw, "gtau": gtau, "gv": gv, "gpsc": gpsc.t().contiguous()}
+    if delayed:
+        # the spikes before the chunk: their share of this chunk's psc
+        D = past.shape[0]
+        pmasks = lane_masks(pack_rows(past.detach().contiguous().view(D * B, n)).view(D, B, -1), n)
+        gpast = torch.empty(D, n, B, device=dev)
+        for p in range(D):
+            _lib.check(lib.btx_adj_transpose_delayed(rp, col, w.data_ptr(), n, spec.csr_d, B,
+                                                     G.data_ptr(), K, p - D, ages.data_ptr(),
+                                                     gpast[p].data_ptr(), 0, stream),
+                       "btx_adj_transpose_delayed")
+            _lib.check(lib.btx_adj_wgrad_delayed(rp, col, n, spec.csr_d, B, pmasks[p].data_ptr(),
+                                                 G.data_ptr(), K, p - D, ages.data_ptr(),
+                                                 gw.data_ptr(), stream), "btx_adj_wgrad_delayed")
+        out["gpast"] = gpast.permute(0, 2, 1).contiguous()
+    return out
+
+
+def _adjoint_relaxed(a, lib, stream, layout, w, traj, grads, gpsc, gsyn, gw, gtau, nb):
+    """Reverse sweep of a chunk whose spikes hold real values (see
+    adjoint_chunk): neuron-major steps, the valued product for dL/dW."""
+    z = traj["z"]
+    K, B, n = z.shape
+    dev = z.device
+    v_prev, v_pre, zz = nb(traj["v_prev"]), nb(traj["v_pre"]), nb(z)
+    ref_prev = nb(traj["ref_prev"]) if traj.get("ref_prev") is not None else None
+    gz = nb(grads["gz"]) if grads.get("gz") is not None else torch.zeros_like(zz)
+    gv = nb(grads["gv"]) if grads.get("gv") is not None else torch.zeros(n, B, device=dev)
+    gx = torch.empty(K, n, B, device=dev)
+    a.gv, a.gpsc = gv.data_ptr(), gpsc.data_ptr()
+    from .._kernels import compact_dense, spmv_weight_grad
     for t in range(K - 1, -1, -1):
         _lib.check(lib.btx_adj_transpose(layout.row_ptr.data_ptr(), layout.col.data_ptr(),
                                          w.data_ptr(), n, B, gpsc.data_ptr(),
                                          gsyn.data_ptr(), stream), "btx_adj_transpose")
-        if valued_weights:
-            zt = traj["z"][t].contiguous()
-            from .._kernels import compact_dense, spmv_weight_grad
-            act, cnt = compact_dense(zt)
-            spmv_weight_grad(layout, zt, act, cnt, gpsc.t().contiguous(), gw)
-        else:
-            _lib.check(lib.btx_adj_wgrad(layout.row_ptr.data_ptr(), layout.col.data_ptr(), n,
-                                         B, masks[t].data_ptr(), gpsc.data_ptr(),
-                                         gw.data_ptr(), stream), "btx_adj_wgrad")
+        zt = z[t].contiguous()
+        act, cnt = compact_dense(zt)
+        spmv_weight_grad(layout, zt, act, cnt, gpsc.t().contiguous(), gw)
         a.v_prev = v_prev[t].data_ptr()
         a.v_pre = v_pre[t].data_ptr()
         a.z = zz[t].data_ptr()
@@ -196,50 +240,6 @@ def adjoint_chunk(spec, traj: dict, grads: dict, w_csr: torch.Tensor, dt: float,
         _lib.check(lib.btx_adj_lif_step(a, stream), "btx_adj_lif_step")
     return {"gx": gx.permute(0, 2, 1).contiguous(), "gw": gw, "gtau": gtau,
             "gv": gv.t().contiguous(), "gpsc": gpsc.t().contiguous()}
-
-
-def _adjoint_delayed(spec, a, lib, stream, layout, w, masks, zz, v_prev, v_pre, ref_prev,
-                     gz, gv, gpsc, gsyn, gx, gw, gtau, past, shifts):
-    """Reverse sweep of a chunk with delayed synapses (see adjoint_chunk)."""
-    K, n, B = zz.shape
-    dev = zz.device
-    csr_d = spec.csr_d
-    ages = _ages(spec, dev)
-    G = torch.empty(K, n, B, device=dev)  # dL/dpsc of every step of the chunk
-    rp, col = layout.row_ptr.data_ptr(), layout.col.data_ptr()
-    for t in range(K - 1, -1, -1):
-        G[t].copy_(gpsc)
-        _lib.check(lib.btx_adj_transpose_delayed(rp, col, w.data_ptr(), n, csr_d, B,
-                                                 G.data_ptr(), K, t, ages.data_ptr(),
-                                                 gsyn.data_ptr(), 0, stream),
-                   "btx_adj_transpose_delayed")
-        _lib.check(lib.btx_adj_wgrad_delayed(rp, col, n, csr_d, B, masks[t].data_ptr(),
-                                             G.data_ptr(), K, t, ages.data_ptr(), gw.data_ptr(),
-                                             stream), "btx_adj_wgrad_delayed")
-        a.v_prev = v_prev[t].data_ptr()
-        a.v_pre = v_pre[t].data_ptr()
-        a.z = zz[t].data_ptr()
-        a.ref_prev = ref_prev[t].data_ptr() if ref_prev is not None else None
-        a.gz = gz[t].data_ptr()
-        a.gx = gx[t].data_ptr()
-        _lib.check(lib.btx_adj_lif_step(a, stream), "btx_adj_lif_step")
-    # the spikes before the chunk: their share of this chunk's psc
-    D = past.shape[0]
-    pz = past.detach().transpose(-1, -2).contiguous()  # (D, N, B)
-    pmasks = ((pz != 0).to(torch.int64) << shifts).sum(-1).contiguous()
-    gpast = torch.empty(D, n, B, device=dev)
-    for p in range(D):
-        tau = p - D
-        _lib.check(lib.btx_adj_transpose_delayed(rp, col, w.data_ptr(), n, csr_d, B,
-                                                 G.data_ptr(), K, tau, ages.data_ptr(),
-                                                 gpast[p].data_ptr(), 0, stream),
-                   "btx_adj_transpose_delayed")
-        _lib.check(lib.btx_adj_wgrad_delayed(rp, col, n, csr_d, B, pmasks[p].data_ptr(),
-                                             G.data_ptr(), K, tau, ages.data_ptr(),
-                                             gw.data_ptr(), stream), "btx_adj_wgrad_delayed")
-    return {"gx": gx.permute(0, 2, 1).contiguous(), "gw": gw, "gtau": gtau,
-            "gv": gv.t().contiguous(), "gpsc": gpsc.t().contiguous(),
-            "gpast": gpast.permute(0, 2, 1).contiguous()}
 
 
 def _history_from_past(spec, past: torch.Tensor, cursor: int) -> None:
@@ -337,9 +337,9 @@ class _FusedChunk(torch.autograd.Function):
             v_prev, v_pre, z, ref = recs["v_prev"], recs["v_pre"], recs["z"], recs["refractory"]
         else:
             v_prev, v_pre, z, ref = saved[6:]
-        ref_prev = (torch.cat([ref0.detach().unsqueeze(0), ref[:-1]])
-                    if eng.spec.neuron._use_refractory else None)
-        traj = {"v_prev": v_prev, "v_pre": v_pre, "z": z, "ref_prev": ref_prev}
+        traj = {"v_prev": v_prev, "v_pre": v_pre, "z": z}
+        if eng.spec.neuron._use_refractory:
+            traj["ref"], traj["ref_entry"] = ref, ref0.detach()
         out = adjoint_chunk(eng.spec, traj, {"gz": gz, "gv": gv, "gpsc": gpsc}, w_csr, ctx.dt,
                             past=past0 if ctx.delayed else None)
         gtau = out["gtau"]

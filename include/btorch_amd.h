@@ -543,6 +543,10 @@ typedef struct btx_adj_lif_args {
     float* gpsc;           /* in dL/dpsc after the step, out before it */
     float* gx;             /* out dL/dx of the step */
     float* gtau;           /* accumulated dL/dtau ((n,) or 1 when tau_stride = 0), or NULL */
+    float* gpsc_out;       /* where dL/dpsc before the step goes, NULL = gpsc */
+    /* 1 = every array but gsyn and gpsc is lane-major (lanes, n), element
+     * (j, b) at b*n + j, and gz may be NULL (no gradient); at most 64 lanes */
+    int lane_major;
 } btx_adj_lif_args;
 
 int btx_adj_lif_step(const btx_adj_lif_args* args, void* stream);
@@ -557,6 +561,24 @@ int btx_adj_lif_step(const btx_adj_lif_args* args, void* stream);
 int btx_adj_lif_chunk(const btx_adj_lif_args* args, int64_t K, const int64_t* row_ptr,
                       const int32_t* col, const float* w, const uint64_t* masks, float* gw,
                       void* stream);
+
+/* The same sweep for either layout of the args' arrays (lane_major), with or
+ * without delays.  gz_stride: elements between steps of gz (0 = the same
+ * gradient each step).  ref_entry != NULL: ref_prev holds the refractory
+ * counters after each step, and ref_entry those entering the first.  ages
+ * NULL: no delays, csr_d and G unused.  Otherwise (csr_d, ages as for
+ * btx_adj_transpose_delayed) G is dL/dpsc of the K steps, [K][n][lanes], of
+ * which the caller sets the last; the sweep fills the others and leaves
+ * dL/dpsc before the chunk in args->gpsc.  lanes <= 64. */
+int btx_adj_lif_sweep(const btx_adj_lif_args* args, int64_t K, int64_t gz_stride,
+                      const float* ref_entry, const int64_t* row_ptr, const int32_t* col,
+                      const float* w, int csr_d, const int* ages, float* G,
+                      const uint64_t* masks, float* gw, void* stream);
+
+/* Lane masks of `steps` steps from their spike words [steps][lanes][ceil(n/64)]:
+ * bit b of masks[t][j] = lane b spiked at neuron j (lanes <= 64). */
+int btx_lane_masks(const uint64_t* words, int64_t steps, int64_t lanes, int64_t n,
+                   uint64_t* masks, void* stream);
 
 /* g_src[j, :] = sum over CSR row j of w[e] * g_dst[col[e], :] (every row;
  * (n, lanes) layout).  The transposed product of the backward pass. */

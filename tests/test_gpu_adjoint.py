@@ -394,3 +394,54 @@ def test_apical_two_compartment_cell_trains_through_the_per_step_loop():
     z1.sum().backward()
     assert torch.equal(z0.cpu(), z1.detach().cpu()) and z0.sum() > 50
     assert torch.isfinite(xg.grad).all() and xg.grad.abs().sum() > 0
+
+
+@pytest.mark.parametrize("n,B,D,shared_tau", [(97, 1, 1, False), (64, 9, 1, True),
+                                              (130, 16, 4, False), (97, 17, 4, True),
+                                              (255, 33, 1, False), (130, 64, 1, True),
+                                              (65, 64, 3, False)])
+def test_adjoint_sweep_lane_counts_match_reference_autograd(n, B, D, shared_tau):
+    # the edges of the sweep's tiles: 32-neuron workgroups, 8 to 64 threads
+    # per edge, rows of fewer and more than 32 and 64 edges (every fifth
+    # neuron sends none), tau per neuron or shared; the loss a mean over time,
+    # whose gradient reaches the sweep with step stride 0 (relative L2 1e-4)
+    from btorch_amd.models import HeterSynapsePSC
+    import scipy.sparse
+
+    T = 30
+    c = workloads.powerlaw_net_fast(n=n, k_min=8, k_max=min(n - 1, 120), delay_lo=1,
+                                    delay_hi=max(1, D - 1), seed=19)
+    keep = c.pre % 5 != 2
+    rows = c.pre[keep] * D + (c.delay[keep] if D > 1 else 0)
+    mat = scipy.sparse.coo_array((c.w[keep], (rows, c.post[keep])), shape=(n * D, n))
+    rng = np.random.default_rng(19)
+    tau = (torch.tensor(18.0) if shared_tau
+           else torch.from_numpy(rng.uniform(10, 30, n).astype(np.float32)))
+    sur = SuperSpike(alpha=25.0 / (math.sqrt(2) - 1))
+    lif = LIF(n, tau=tau, tau_ref=2.0, trainable_param={"tau"}, surrogate_function=sur)
+    conn = SparseConn(mat)
+    syn = (HeterSynapsePSC(n, 1, None, conn, base_psc=ExponentialPSC, max_delay_steps=D,
+                           use_circular_buffer=True, tau_syn=5.0)
+           if D > 1 else ExponentialPSC(n, 5.0, conn))
+    model = RecurrentNN(lif, syn, step_mode="m", update_state_names=[]).to(DEV)
+    functional.init_net_state(model, batch_size=B, device=DEV, dtype=torch.float32)
+    x = torch.from_numpy(workloads.poisson_input(T, B, n, 800.0, 0.1, seed=19) * 25.0)
+    R = torch.randn(B, n, generator=torch.Generator().manual_seed(8))
+    xg = x.to(DEV).requires_grad_(True)
+    with environ.context(dt=0.1):
+        z, _ = model(xg)
+    ((z.mean(0) * R.to(DEV)).sum() + (model.neuron.v * R.to(DEV)).sum()).backward()
+    dst, src = conn.indices[0].cpu(), conn.indices[1].cpu()
+    mag = conn.magnitude.detach().cpu().clone().requires_grad_(True)
+    tau_r = tau.clone().requires_grad_(True)
+    xr = x.clone().requires_grad_(True)
+    kw = dict(csr_d=D, ages=tuple(range(D))) if D > 1 else {}
+    zr, vr, _, _ = rsnn.simulate_grad(n, dst, src, mag, xr, tau_r, 0.1, 5.0, tau_ref=2.0,
+                                      surrogate=("superspike", sur.alpha, 1.0, True), **kw)
+    ((zr.mean(0) * R).sum() + (vr * R).sum()).backward()
+    assert torch.equal(z.detach().cpu(), zr.detach()) and zr.sum() > 10
+    e_w = rel_err(conn.magnitude.grad, mag.grad)
+    e_t = rel_err(model.neuron.tau.grad, tau_r.grad)
+    e_x = rel_err(xg.grad, xr.grad)
+    print(f"\nn {n}, {B} lanes, D {D}: dW {e_w:.2e} dtau {e_t:.2e} dx {e_x:.2e}")
+    assert e_w < 1e-4 and e_t < 1e-4 and e_x < 1e-4
