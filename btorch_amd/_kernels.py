@@ -213,6 +213,62 @@ def unpack_rows(words: torch.Tensor, n: int, out: torch.Tensor | None = None) ->
     return out
 
 
+def _product_operands(layout: CsrLayout, w: torch.Tensor, x2d: torch.Tensor) -> None:
+    _lib.require_hip(x2d, w)
+    if x2d.dim() != 2 or x2d.shape[1] != layout.n_src or not x2d.is_contiguous():
+        raise ValueError("operand shapes do not match the connection layout")
+    if layout.csc_ptr is None or w.numel() != layout.nnz or not w.is_contiguous():
+        raise ValueError("destination-major arrays missing or mismatched")
+    if w.dtype != torch.float32 or x2d.dtype != torch.float32:
+        raise TypeError("the event-driven product supports float32 only")
+
+
+def product(layout: CsrLayout, w: torch.Tensor, x2d: torch.Tensor) -> torch.Tensor:
+    """(rows, n_dst) = x2d @ W; ``w`` holds the weights in the coalesced
+    (dst, src) order (``btx_product``)."""
+    _product_operands(layout, w, x2d)
+    rows = x2d.shape[0]
+    lib = _lib.load()
+    out = torch.empty((rows, layout.n_dst), dtype=torch.float32, device=x2d.device)
+    nbytes = lib.btx_product_scratch_bytes(rows, layout.n_src)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=x2d.device)
+    _lib.check(lib.btx_product(layout.row_ptr.data_ptr(), layout.col.data_ptr(),
+                               layout.perm.data_ptr(), layout.csc_ptr.data_ptr(),
+                               layout.csc_src.data_ptr(), w.data_ptr(), layout.n_src,
+                               layout.n_dst, layout.nnz, x2d.data_ptr(), layout.n_src, rows,
+                               out.data_ptr(), scratch.data_ptr() if nbytes else None, nbytes,
+                               _lib.stream_ptr()), "btx_product")
+    return out
+
+
+def product_grad(layout: CsrLayout, w: torch.Tensor, x2d: torch.Tensor, g: torch.Tensor,
+                 need_x: bool, need_w: bool):
+    """(gx, gw) of ``product`` for the output gradient ``g``; gw in the order
+    of ``w``; None for one that is not needed."""
+    _product_operands(layout, w, x2d)
+    g = g.to(torch.float32).contiguous()
+    rows = x2d.shape[0]
+    if g.shape != (rows, layout.n_dst):
+        raise ValueError("gradient width does not match n_dst")
+    lib = _lib.load()
+    dev = x2d.device
+    empty = rows == 0 or layout.n_src == 0 or layout.n_dst == 0
+    make = torch.zeros if empty else torch.empty
+    gx = make((rows, layout.n_src), dtype=torch.float32, device=dev) if need_x else None
+    gw = make(layout.nnz, dtype=torch.float32, device=dev) if need_w else None
+    nbytes = lib.btx_product_grad_scratch_bytes(rows, layout.n_src, layout.n_dst)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    ptr = (lambda t: None if t is None else t.data_ptr())
+    _lib.check(lib.btx_product_grad(layout.row_ptr.data_ptr(), layout.col.data_ptr(),
+                                    layout.perm.data_ptr(), layout.csc_ptr.data_ptr(),
+                                    layout.csc_src.data_ptr(), w.data_ptr(), layout.n_src,
+                                    layout.n_dst, layout.nnz, x2d.data_ptr(), layout.n_src, rows,
+                                    g.data_ptr(), ptr(gx), ptr(gw),
+                                    scratch.data_ptr() if nbytes else None, nbytes,
+                                    _lib.stream_ptr()), "btx_product_grad")
+    return gx, gw
+
+
 def spmv_workspace(lanes: int, n_dst: int, slots: int, ordered: bool, device) -> torch.Tensor:
     nbytes = _lib.load().btx_spmv_workspace_bytes(lanes, n_dst, slots, int(ordered))
     return torch.zeros(nbytes, dtype=torch.uint8, device=device)

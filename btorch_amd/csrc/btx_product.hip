@@ -1,0 +1,472 @@
+// The sparse product as a layer of its own and its backward, y = x W.
+//
+// Layouts as in btx_spmv.hip: CSR by source (row_ptr, col; destinations
+// ascending) and the same edges destination-major (csc_ptr, csc_src; sources
+// ascending).  Weights come in the destination-major order, the layer's own
+// parameter order; perm[k] is the position there of CSR edge k.
+//
+// Every destination sums its terms in ascending source order from +0.0f with
+// one fmaf per source with x != 0, so y equals torch.sparse.mm on the CPU bit
+// for bit (btorch/models/linear.py:474-483).  Two forms, neither of which
+// stores a term:
+//   rows     a workgroup takes one row of x and a tile of destinations held in
+//            LDS, and streams the rows of W of the row's nonzero sources in
+//            ascending order: a source's destinations are distinct, so its
+//            terms need no atomics, and a barrier between sources keeps the
+//            order.  Costs the active sources, whatever the edges.
+//   columns  a wavefront takes a destination and 64 rows of x (transposed, so
+//            that a source's 64 values are one 256-byte read) and walks the
+//            destination's edges.  Costs every edge, whatever the activity.
+
+#include <hip/hip_runtime.h>
+
+#include "../../include/btorch_amd.h"
+#include "btx_common.h"
+
+namespace btx {
+
+constexpr int kRowTile = 16384;      // destinations of a `rows` workgroup, at most (64 KB of LDS)
+constexpr int kRowThreads = 1024;
+constexpr int kGroup = 64;           // rows of x per wavefront of the `columns` form
+constexpr int64_t kFewSources = 1024;  // up to which the `rows` form is taken unasked
+
+struct ProductArgs {
+    const int64_t* row_ptr;
+    const int32_t* col;
+    const int64_t* perm;
+    const int64_t* csc_ptr;
+    const int32_t* csc_src;
+    const float* w;       // destination-major order
+    int64_t n_src;
+    int64_t n_dst;
+    int64_t nnz;
+    const float* x;       // (rows, n_src), row stride x_stride
+    int64_t x_stride;
+    int64_t rows;
+    float* y;             // (rows, n_dst)
+    const int32_t* counts;  // nonzeros of each row, NULL = take the `rows` form
+    float* xt;            // [groups][n_src][64]
+};
+
+// Which form the 64 rows of group g take.  Measured on MI355X (16,384 x 16,384
+// of 13.4M edges, 4,000 x 8,000 of 1.6M, 21,739 x 21,739 of 3.5M; 1 to 512
+// rows): rows 1.5 ns per edge of an active source, at least 0.6 us a source,
+// 1.5 ns per source looked at, 200 rows at a time; columns 16 to 27 us per
+// million edges and group.  Sides at 64 rows of the first net: 164 active
+// sources 302 us by rows and 263 us by columns, 33 of them 101 and 263 us.
+__device__ __forceinline__ bool group_by_rows(const ProductArgs& a, int64_t g) {
+    if (a.counts == nullptr) return true;
+    const int ln = threadIdx.x & 63;
+    const int64_t row = g * kGroup + ln;
+    int c = row < a.rows ? a.counts[row] : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    const int64_t here = a.rows - g * kGroup < kGroup ? a.rows - g * kGroup : kGroup;
+    const float waves = a.rows > 200 ? (float)a.rows / 200.f : 1.f;
+    const float len = (float)a.nnz / (float)a.n_src;
+    const float source_us = fmaxf(0.6f, 1.5e-3f * len);
+    const float rows_us = waves * (1.5e-3f * (float)a.n_src + source_us * (float)c / (float)here);
+    const float cols_us = 8.f + 22e-6f * (float)a.nnz * (float)((a.rows + kGroup - 1) / kGroup);
+    return rows_us < cols_us;
+}
+
+// Nonzeros of every row (one workgroup per row).
+__global__ __launch_bounds__(256) void k_row_counts(const float* __restrict__ x, int64_t n,
+                                                    int64_t stride, int32_t* __restrict__ counts) {
+    const int64_t row = blockIdx.x;
+    const float* xr = x + row * stride;
+    int c = 0;
+#pragma unroll 8
+    for (int64_t i = threadIdx.x; i < n; i += 256) c += xr[i] != 0.f;
+    int total;
+    block_excl_scan<4>(c, total);
+    if (threadIdx.x == 0) counts[row] = total;
+}
+
+// One row of x, destinations [d0, d0 + tile): 1024 of the row's values are
+// read at a time and their nonzeros listed in LDS in ascending order, each
+// with its row of W.  Bound by the misses one CU can have in flight on a
+// source's weights, which perm scatters over the array (1.25 us a source of
+// 819 edges, 0.6 us of 400): eight sources are requested together, the next
+// eight before the current ones are added (one source ahead: 1.9 us).  Taken
+// back: three requests in flight and tiles of 1024 destinations (74 VGPRs, one
+// workgroup per CU: 512 rows 15% slower), 256 threads (four times the passes
+// over x).
+__global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int tile) {
+    constexpr int T = kRowThreads;
+    extern __shared__ __align__(16) float s_y[];
+    __shared__ int s_beg[T], s_len[T];
+    __shared__ float s_x[T];
+    __shared__ int s_cnt[T / 64];
+    constexpr int U = 8;
+    const int tid = threadIdx.x, wv = tid >> 6, ln = tid & 63;
+    const int64_t row = blockIdx.x, d0 = (int64_t)blockIdx.y * tile;
+    const int nd = (int)(a.n_dst - d0 < tile ? a.n_dst - d0 : tile);
+    if (!group_by_rows(a, row / kGroup)) return;
+    for (int q = tid; q < (nd + 3) / 4; q += T)
+        reinterpret_cast<float4*>(s_y)[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float* xr = a.x + row * a.x_stride;
+    for (int64_t s0 = 0; s0 < a.n_src; s0 += T) {
+        const int64_t s = s0 + tid;
+        const float xv = s < a.n_src ? xr[s] : 0.f;
+        const bool on = xv != 0.f;
+        const uint64_t m = __ballot(on);
+        if (ln == 0) s_cnt[wv] = __popcll((unsigned long long)m);
+        __syncthreads();
+        int off = 0, total = 0;
+#pragma unroll
+        for (int k = 0; k < T / 64; ++k) {
+            off += k < wv ? s_cnt[k] : 0;
+            total += s_cnt[k];
+        }
+        if (on) {
+            const int p = off + __popcll((unsigned long long)(m & ((1ull << ln) - 1ull)));
+            const int64_t beg = a.row_ptr[s];
+            s_beg[p] = (int)beg;
+            s_len[p] = (int)(a.row_ptr[s + 1] - beg);
+            s_x[p] = xv;
+        }
+        __syncthreads();
+        // this thread's first edge of eight sources: destination within the
+        // tile (-1 = none), weight
+        auto request = [&](int k0, int* d, float* w) {
+            int64_t pm[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const bool in = k0 + u < total && tid < s_len[k0 + u];
+                const int e = in ? s_beg[k0 + u] + tid : 0;
+                d[u] = in ? a.col[e] : -1;
+                pm[u] = in ? a.perm[e] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                w[u] = d[u] >= 0 ? a.w[pm[u]] : 0.f;
+                const int64_t q = d[u] - d0;
+                d[u] = d[u] >= 0 && q >= 0 && q < nd ? (int)q : -1;
+            }
+        };
+        int d[U], dn[U];
+        float w[U], wn[U];
+        if (total > 0) request(0, d, w);
+        for (int k0 = 0; k0 < total; k0 += U) {
+            if (k0 + U < total) request(k0 + U, dn, wn);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (k0 + u >= total) break;  // uniform
+                const float xk = s_x[k0 + u];
+                const int len = s_len[k0 + u];
+                if (d[u] >= 0) s_y[d[u]] = fmaf(w[u], xk, s_y[d[u]]);
+                for (int t = tid + T; t < len; t += T) {
+                    const int e = s_beg[k0 + u] + t;
+                    const int64_t q = a.col[e] - d0;
+                    if (q >= 0 && q < nd) s_y[q] = fmaf(a.w[a.perm[e]], xk, s_y[q]);
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                d[u] = dn[u];
+                w[u] = wn[u];
+            }
+        }
+    }
+    __syncthreads();
+    float* yr = a.y + row * a.n_dst + d0;
+    if (a.n_dst % 4 == 0 && tile % 4 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0)
+        for (int q = tid; q < nd / 4; q += T)
+            reinterpret_cast<float4*>(yr)[q] = reinterpret_cast<const float4*>(s_y)[q];
+    else
+        for (int q = tid; q < nd; q += T) yr[q] = s_y[q];
+}
+
+// out[g][i][b] = in[64 g + b][i] in tiles of 64 x 64; rows past `rows` are 0.
+// `a` non-null: only the groups that take the columns.
+__global__ __launch_bounds__(256) void k_group_rows(ProductArgs a, const float* __restrict__ in,
+                                                    int64_t n, int64_t stride, int64_t rows,
+                                                    float* __restrict__ out) {
+    __shared__ float t[64][65];
+    const int64_t g = blockIdx.y, i0 = (int64_t)blockIdx.x * 64;
+    if (a.counts != nullptr && group_by_rows(a, g)) return;
+    const int ln = threadIdx.x & 63;
+    for (int b = threadIdx.x >> 6; b < 64; b += 4) {
+        const int64_t row = g * kGroup + b, i = i0 + ln;
+        t[b][ln] = row < rows && i < n ? in[row * stride + i] : 0.f;
+    }
+    __syncthreads();
+    for (int k = threadIdx.x >> 6; k < 64; k += 4)
+        if (i0 + k < n) out[(g * n + i0 + k) * kGroup + ln] = t[ln][k];
+}
+
+// The inverse: out[64 g + b][i] = in[g][i][b].
+__global__ __launch_bounds__(256) void k_ungroup_rows(const float* __restrict__ in, int64_t n,
+                                                      int64_t rows, float* __restrict__ out) {
+    __shared__ float t[64][65];
+    const int64_t g = blockIdx.y, i0 = (int64_t)blockIdx.x * 64;
+    const int ln = threadIdx.x & 63;
+    for (int k = threadIdx.x >> 6; k < 64; k += 4)
+        t[k][ln] = i0 + k < n ? in[(g * n + i0 + k) * kGroup + ln] : 0.f;
+    __syncthreads();
+    for (int b = threadIdx.x >> 6; b < 64; b += 4) {
+        const int64_t row = g * kGroup + b;
+        if (row < rows && i0 + ln < n) out[row * n + i0 + ln] = t[ln][b];
+    }
+}
+
+// A wavefront per (destination, group of 64 rows): thread b sums row b.  16
+// destinations at a time per workgroup, so that y is written in runs.  Bound by
+// the gathered rows of x out of L2: 264 us for 13.4M edges and 64 rows,
+// 13 TB/s; 23 us more is k_row_counts and the transpose.
+__global__ __launch_bounds__(256) void k_product_columns(ProductArgs a) {
+    __shared__ float s_out[16][65];
+    const int tid = threadIdx.x, ln = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t groups = (a.rows + kGroup - 1) / kGroup;
+    const int64_t tiles = (a.n_dst + 15) / 16;
+    for (int64_t g = 0; g < groups; ++g) {
+        if (group_by_rows(a, g)) continue;
+        const float* xg = a.xt + g * a.n_src * kGroup + ln;
+        for (int64_t tl = blockIdx.x; tl < tiles; tl += gridDim.x) {
+            for (int q = wv; q < 16; q += 4) {
+                const int64_t d = tl * 16 + q;
+                if (d >= a.n_dst) break;
+                const int64_t e0 = a.csc_ptr[d];
+                const int len = (int)(a.csc_ptr[d + 1] - e0);
+                float acc = 0.f;
+                for (int c = 0; c < len; c += 64) {
+                    const int m = len - c < 64 ? len - c : 64;
+                    const int my_s = ln < m ? a.csc_src[e0 + c + ln] : 0;
+                    const int my_w = ln < m ? __float_as_int(a.w[e0 + c + ln]) : 0;
+                    int k = 0;
+                    for (; k + 16 <= m; k += 16) {
+                        float x16[16];
+#pragma unroll
+                        for (int u = 0; u < 16; ++u)
+                            x16[u] = xg[(int64_t)__builtin_amdgcn_readlane(my_s, k + u) * kGroup];
+#pragma unroll
+                        for (int u = 0; u < 16; ++u) {
+                            const float wk = __int_as_float(__builtin_amdgcn_readlane(my_w, k + u));
+                            const float t = fmaf(wk, x16[u], acc);
+                            acc = x16[u] != 0.f ? t : acc;
+                        }
+                    }
+                    for (; k < m; ++k) {
+                        const float xv = xg[(int64_t)__builtin_amdgcn_readlane(my_s, k) * kGroup];
+                        const float wk = __int_as_float(__builtin_amdgcn_readlane(my_w, k));
+                        const float t = fmaf(wk, xv, acc);
+                        acc = xv != 0.f ? t : acc;
+                    }
+                }
+                s_out[q][ln] = acc;
+            }
+            __syncthreads();
+            // 16 destinations of 64 rows: a 64-byte run per row
+            for (int k = tid; k < 16 * kGroup; k += 256) {
+                const int b = k >> 4, q = k & 15;
+                const int64_t row = g * kGroup + b, d = tl * 16 + q;
+                if (row < a.rows && d < a.n_dst) a.y[row * a.n_dst + d] = s_out[q][b];
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// gx of the layer: gxt[g][s][b] = sum over edges e of row s of w[e] *
+// gt[g][col[e]][b]; one wavefront per (row, group), 16 gathered rows in flight.
+// Bound by the gathered rows out of L2: 292 us for 13.4M edges and 64 rows,
+// 11.8 TB/s (the wavefront per edge block of btx_spmv.hip that the layer's
+// backward used before: 3.9 ms with its copies).
+__global__ __launch_bounds__(256) void k_product_grad_x(const int64_t* __restrict__ rp,
+                                                        const int32_t* __restrict__ col,
+                                                        const int64_t* __restrict__ perm,
+                                                        const float* __restrict__ w, int64_t n_src,
+                                                        int64_t n_dst,
+                                                        const float* __restrict__ gt,
+                                                        float* __restrict__ gxt) {
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t s = (int64_t)blockIdx.x * 4 + wv;
+    const int64_t g = blockIdx.y;
+    const int ln = threadIdx.x & 63;
+    if (s >= n_src) return;
+    const float* gg = gt + g * n_dst * kGroup + ln;
+    const int64_t e0 = rp[s];
+    const int len = (int)(rp[s + 1] - e0);
+    // the terms of 64 edges in sixteen partial sums, added pairwise, and the
+    // 64-edge sums in float64: 7e-8 of the result against float64 throughout
+    // (sixteen sums over all edges 1.4e-7, two 3.6e-7)
+    double sum = 0.0;
+    for (int c = 0; c < len; c += 64) {
+        const int m = len - c < 64 ? len - c : 64;
+        float acc[16] = {};
+        const int my_d = ln < m ? col[e0 + c + ln] : 0;
+        const int my_w = ln < m ? __float_as_int(w[perm[e0 + c + ln]]) : 0;
+        int k = 0;
+        for (; k + 16 <= m; k += 16) {
+            float g16[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                g16[u] = gg[(int64_t)__builtin_amdgcn_readlane(my_d, k + u) * kGroup];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                acc[u] = fmaf(__int_as_float(__builtin_amdgcn_readlane(my_w, k + u)), g16[u], acc[u]);
+        }
+        for (; k < m; ++k)
+            acc[0] = fmaf(__int_as_float(__builtin_amdgcn_readlane(my_w, k)),
+                          gg[(int64_t)__builtin_amdgcn_readlane(my_d, k) * kGroup], acc[0]);
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+            for (int u = 0; u < o; ++u) acc[u] += acc[u + o];
+        sum += acc[0];
+    }
+    gxt[(g * n_src + s) * kGroup + ln] = (float)sum;
+}
+
+// gw of the layer, destination-major: gw[e] = sum over rows b of x[b, src[e]] *
+// gy[b, dst].  A workgroup takes one destination, whose gradients over the
+// rows sit in LDS, and a thread per edge that reads the source's row bits:
+// only rows with x != 0 are added, in ascending order, group by group.
+__global__ __launch_bounds__(256) void k_product_grad_w(const int64_t* __restrict__ csc_ptr,
+                                                        const int32_t* __restrict__ csc_src,
+                                                        int64_t n_src, int64_t n_dst, int64_t rows,
+                                                        const float* __restrict__ x,
+                                                        int64_t x_stride,
+                                                        const uint64_t* __restrict__ bits,
+                                                        const float* __restrict__ gt,
+                                                        float* __restrict__ gw) {
+    __shared__ float s_g[4][kGroup];
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t d = (int64_t)blockIdx.x * 4 + wv;
+    const int ln = threadIdx.x & 63;
+    if (d >= n_dst) return;
+    const int64_t e0 = csc_ptr[d], e1 = csc_ptr[d + 1];
+    const int64_t groups = (rows + kGroup - 1) / kGroup;
+    for (int64_t g = 0; g < groups; ++g) {
+        s_g[wv][ln] = gt[(g * n_dst + d) * kGroup + ln];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int64_t e = e0 + ln; e < e1; e += 64) {
+            const int s = csc_src[e];
+            uint64_t m = bits[g * n_src + s];
+            float acc = 0.f;
+            while (m) {
+                const int b = __ffsll((unsigned long long)m) - 1;
+                acc = fmaf(x[(g * kGroup + b) * x_stride + s], s_g[wv][b], acc);
+                m &= m - 1ull;
+            }
+            gw[e] = g == 0 ? acc : gw[e] + acc;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+
+// bits[g][s]: bit b = x[64 g + b, s] != 0.
+__global__ __launch_bounds__(256) void k_row_bits(const float* __restrict__ x, int64_t n,
+                                                  int64_t stride, int64_t rows,
+                                                  uint64_t* __restrict__ bits) {
+    const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x, g = blockIdx.y;
+    if (s >= n) return;
+    uint64_t m = 0ull;
+    const int64_t here = rows - g * kGroup < kGroup ? rows - g * kGroup : kGroup;
+    const float* xg = x + g * kGroup * stride + s;
+#pragma unroll 8
+    for (int b = 0; b < here; ++b) m |= (uint64_t)(xg[b * stride] != 0.f) << b;
+    bits[g * n + s] = m;
+}
+
+static size_t product_scratch(int64_t rows, int64_t n_src) {
+    if (n_src <= kFewSources) return 0;
+    const int64_t groups = (rows + kGroup - 1) / kGroup;
+    return align256(4 * (size_t)rows) + 4 * (size_t)(groups * n_src * kGroup);
+}
+
+static size_t grad_scratch(int64_t rows, int64_t n_src, int64_t n_dst) {
+    const size_t groups = (size_t)((rows + kGroup - 1) / kGroup);
+    // gy and gx by groups, row bits
+    return groups * kGroup * 4 * (size_t)(n_dst + n_src) + groups * 8 * (size_t)n_src + 256;
+}
+
+static int check_product(const char* who, int64_t n_src, int64_t n_dst, int64_t nnz, int64_t rows) {
+    if (n_src >= (int64_t)1 << 31 || n_dst >= (int64_t)1 << 31 || nnz >= (int64_t)1 << 31)
+        return fail(std::string(who) + ": sources, destinations and edges must fit int32");
+    if (rows > 65535) return fail(std::string(who) + ": rows exceeds 65535");
+    return 0;
+}
+
+}  // namespace btx
+
+using namespace btx;
+
+BTX_API size_t btx_product_scratch_bytes(int64_t rows, int64_t n_src) {
+    return rows > 0 && n_src > 0 ? product_scratch(rows, n_src) : 0;
+}
+
+BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_t* perm,
+                        const int64_t* csc_ptr, const int32_t* csc_src, const float* w,
+                        int64_t n_src, int64_t n_dst, int64_t nnz, const float* x,
+                        int64_t x_row_stride, int64_t rows, float* y, void* scratch,
+                        size_t scratch_bytes, void* stream) {
+    if (rows <= 0 || n_dst <= 0) return 0;
+    if (int rc = check_product("btx_product", n_src, n_dst, nnz, rows)) return rc;
+    if (scratch_bytes < btx_product_scratch_bytes(rows, n_src) ||
+        (scratch == nullptr && scratch_bytes > 0))
+        return fail("btx_product: scratch too small");
+    const hipStream_t s = (hipStream_t)stream;
+    ProductArgs a{row_ptr, col, perm, csc_ptr, csc_src, w, n_src, n_dst, nnz, x, x_row_stride, rows,
+                  y, nullptr, nullptr};
+    const int64_t groups = (rows + kGroup - 1) / kGroup;
+    if (n_src > kFewSources) {
+        a.counts = (const int32_t*)scratch;
+        a.xt = (float*)((char*)scratch + align256(4 * (size_t)rows));
+        hipLaunchKernelGGL(k_row_counts, dim3((unsigned)rows), dim3(256), 0, s, x, n_src,
+                           x_row_stride, (int32_t*)scratch);
+        hipLaunchKernelGGL(k_group_rows, dim3((unsigned)((n_src + 63) / 64), (unsigned)groups),
+                           dim3(256), 0, s, a, x, n_src, x_row_stride, rows, a.xt);
+    }
+    const int tile = (int)(n_dst < kRowTile ? n_dst : kRowTile);
+    const dim3 grid((unsigned)rows, (unsigned)((n_dst + tile - 1) / tile));
+    hipLaunchKernelGGL(k_product_rows, grid, dim3(kRowThreads), 4 * (size_t)(tile + 3), s, a, tile);
+    if (n_src > kFewSources) {
+        const int64_t tiles = (n_dst + 15) / 16;
+        hipLaunchKernelGGL(k_product_columns, dim3((unsigned)(tiles < 2048 ? tiles : 2048)),
+                           dim3(256), 0, s, a);
+    }
+    return check_launch("btx_product");
+}
+
+BTX_API size_t btx_product_grad_scratch_bytes(int64_t rows, int64_t n_src, int64_t n_dst) {
+    return rows > 0 ? grad_scratch(rows, n_src, n_dst) : 0;
+}
+
+BTX_API int btx_product_grad(const int64_t* row_ptr, const int32_t* col, const int64_t* perm,
+                             const int64_t* csc_ptr, const int32_t* csc_src, const float* w,
+                             int64_t n_src, int64_t n_dst, int64_t nnz, const float* x,
+                             int64_t x_row_stride, int64_t rows, const float* gy, float* gx,
+                             float* gw, void* scratch, size_t scratch_bytes, void* stream) {
+    if (rows <= 0 || n_src <= 0 || n_dst <= 0) return 0;
+    if (int rc = check_product("btx_product_grad", n_src, n_dst, nnz, rows)) return rc;
+    if (scratch == nullptr || scratch_bytes < grad_scratch(rows, n_src, n_dst))
+        return fail("btx_product_grad: scratch too small");
+    const hipStream_t s = (hipStream_t)stream;
+    const int64_t groups = (rows + kGroup - 1) / kGroup;
+    float* gt = (float*)scratch;
+    float* gxt = gt + groups * n_dst * kGroup;
+    uint64_t* bits = (uint64_t*)(gxt + groups * n_src * kGroup);
+    hipLaunchKernelGGL(k_group_rows, dim3((unsigned)((n_dst + 63) / 64), (unsigned)groups),
+                       dim3(256), 0, s, ProductArgs{}, gy, n_dst, n_dst, rows, gt);
+    if (gx != nullptr) {
+        hipLaunchKernelGGL(k_product_grad_x, dim3((unsigned)((n_src + 3) / 4), (unsigned)groups),
+                           dim3(256), 0, s, row_ptr, col, perm, w, n_src, n_dst, gt, gxt);
+        hipLaunchKernelGGL(k_ungroup_rows, dim3((unsigned)((n_src + 63) / 64), (unsigned)groups),
+                           dim3(256), 0, s, gxt, n_src, rows, gx);
+    }
+    if (gw != nullptr) {
+        hipLaunchKernelGGL(k_row_bits, dim3((unsigned)((n_src + 255) / 256), (unsigned)groups),
+                           dim3(256), 0, s, x, n_src, x_row_stride, rows, bits);
+        hipLaunchKernelGGL(k_product_grad_w, dim3((unsigned)((n_dst + 3) / 4)), dim3(256), 0, s,
+                           csc_ptr, csc_src, n_src, n_dst, rows, x, x_row_stride, bits, gt, gw);
+    }
+    return check_launch("btx_product_grad");
+}

@@ -7,12 +7,11 @@ sparse_backend=None, sparse_config=None, device=None, dtype=None)``; buffer
 Parameter ``magnitude`` (E,) in that order; ``prepare_sparse``/
 ``finish_sparse``; ``get_sparse_matrix``; ``constrain``.
 
-The product runs in the HIP library as an event-driven push over a
-source-major CSR (``_csr_*`` non-persistent buffers, rebuilt on load): the
-input is compacted to its nonzero sources per lane, and each active row is
-streamed to its destinations.  The default ordered mode sums every
-destination in ascending source order with fmaf, which equals the CPU
-``torch.sparse.mm`` of the reference's native branch bit for bit.
+The product runs in the HIP library (``btx_product``) over a source-major CSR
+and a destination-major copy (``_csr_*`` / ``_csc_*`` non-persistent buffers,
+rebuilt on load), skipping inputs that are 0.  Every destination is summed in
+ascending source order with fmaf, in either accumulation mode, which equals
+the CPU ``torch.sparse.mm`` of the reference's native branch bit for bit.
 """
 
 from __future__ import annotations
@@ -48,32 +47,22 @@ def available_sparse_backends(*, include_experimental: bool = False) -> list[str
 
 
 class _SparseProduct(torch.autograd.Function):
-    """y = x @ W with W packed in CSR order; grads for x and the packed weights
-    (autograd carries the latter back to ``magnitude`` through the gather)."""
+    """y = x @ W with W in the coalesced (dst, src) order of the effective
+    weights; grads for x and those weights."""
 
     @staticmethod
-    def forward(ctx, x2d, w_csr, conn: "BaseSparseConn"):
-        active, counts = _kernels.compact_dense(x2d)
-        ws = conn._workspace_for(x2d.shape[0])
-        cfg: HipSparseConfig = conn.sparse_config
-        w_dst = conn.effective_weight_f32()
-        out = _kernels.spmv_event(conn._layout, w_csr, x2d, active, counts,
-                                  ordered=cfg.ordered, slots=cfg.slots, workspace=ws,
-                                  w_dst=w_dst)
+    def forward(ctx, x2d, weight, conn: "BaseSparseConn"):
+        if weight.dtype != torch.float32:
+            raise TypeError("the event-driven product supports float32 only")
         ctx.conn = conn
-        ctx.save_for_backward(x2d, w_csr, active, counts)
-        return out
+        ctx.save_for_backward(x2d, weight)
+        return _kernels.product(conn._layout, weight.detach().contiguous(), x2d)
 
     @staticmethod
     def backward(ctx, g):
-        x2d, w_csr, active, counts = ctx.saved_tensors
-        layout = ctx.conn._layout
-        gx = gw = None
-        if ctx.needs_input_grad[0]:
-            gx = _kernels.spmv_transpose(layout, w_csr, g)
-        if ctx.needs_input_grad[1]:
-            gw = torch.zeros(layout.nnz, dtype=torch.float32, device=g.device)
-            _kernels.spmv_weight_grad(layout, x2d, active, counts, g, gw)
+        x2d, weight = ctx.saved_tensors
+        gx, gw = _kernels.product_grad(ctx.conn._layout, weight.detach().contiguous(), x2d, g,
+                                       ctx.needs_input_grad[0], ctx.needs_input_grad[1])
         return gx, gw, None
 
 
@@ -88,7 +77,9 @@ class BaseSparseConn(nn.Module):
         self.sparse_config = btorch_config.sparse.resolve(self.sparse_backend, sparse_config)
         self._prepared_sparse_weight: torch.Tensor | None = None
         self._sparse_prepare_depth = 0
-        self._workspaces: dict[int, torch.Tensor] = {}
+        # effective weights of a prepared run, (dst, src) order, as a 1-tuple (a
+        # Parameter assigned as it is would register a second time)
+        self._prepared_weight: tuple[torch.Tensor] | None = None
         # no-grad packed (CSR order) and destination-order weights, reused
         # while the tensors they derive from are unchanged (weight_key)
         self._weight_cache: dict[str, tuple] = {}
@@ -148,7 +139,6 @@ class BaseSparseConn(nn.Module):
                 setattr(self, name, t)
             else:
                 self.register_buffer(name, t, persistent=False)
-        self._workspaces = {}
 
     @property
     def _layout(self) -> _kernels.CsrLayout:
@@ -160,22 +150,9 @@ class BaseSparseConn(nn.Module):
     def nnz(self) -> int:
         return int(self.indices.shape[1])
 
-    def _workspace_for(self, lanes: int) -> torch.Tensor:
-        cfg: HipSparseConfig = self.sparse_config
-        dev = self._csr_col.device
-        need = _lib.load().btx_spmv_workspace_bytes(lanes, self.out_features, cfg.slots,
-                                                    int(cfg.ordered))
-        key = (int(cfg.ordered), cfg.slots, str(dev))
-        ws = self._workspaces.get(key)
-        if ws is None or ws.numel() < need:
-            ws = torch.zeros(need, dtype=torch.uint8, device=dev)
-            self._workspaces[key] = ws
-        return ws
-
     def _apply(self, fn, recurse=True):
-        self._prepared_sparse_weight = None
+        self._prepared_sparse_weight = self._prepared_weight = None
         self._sparse_prepare_depth = 0
-        self._workspaces = {}
         self._weight_cache = {}
         return super()._apply(fn, recurse=recurse)
 
@@ -183,7 +160,7 @@ class BaseSparseConn(nn.Module):
                               unexpected_keys, error_msgs):
         super()._load_from_state_dict(state_dict, prefix, local_metadata, strict, missing_keys,
                                       unexpected_keys, error_msgs)
-        self._prepared_sparse_weight = None
+        self._prepared_sparse_weight = self._prepared_weight = None
         self._sparse_prepare_depth = 0
         self._weight_cache = {}
         self._rebuild_layout()
@@ -247,11 +224,11 @@ class BaseSparseConn(nn.Module):
         return self._pack()
 
     def prepare_sparse(self, batch_size: int | None = None) -> None:
-        """Pack weights once for a multi-step run (reference-counted)."""
+        """Evaluate and pack the weights once for a multi-step run
+        (reference-counted)."""
         if self._prepared_sparse_weight is None:
             self._prepared_sparse_weight = self._pack()
-        if batch_size is not None and self._csr_col.is_cuda:
-            self._workspace_for(int(batch_size))
+            self._prepared_weight = (self._get_effective_weight(),)
         self._sparse_prepare_depth += 1
 
     def finish_sparse(self) -> None:
@@ -259,7 +236,7 @@ class BaseSparseConn(nn.Module):
             raise RuntimeError("finish_sparse called without prepare_sparse.")
         self._sparse_prepare_depth -= 1
         if self._sparse_prepare_depth == 0:
-            self._prepared_sparse_weight = None
+            self._prepared_sparse_weight = self._prepared_weight = None
 
     def get_sparse_matrix(self) -> torch.Tensor:
         idx = torch.stack([self.indices[1], self.indices[0]], dim=0)
@@ -278,7 +255,12 @@ class BaseSparseConn(nn.Module):
         if x2d.dtype != torch.float32:
             raise TypeError("The HIP sparse backend currently supports float32 only.")
         x2d = x2d.contiguous()
-        out = _SparseProduct.apply(x2d, self.packed_weight(), self)
+        if self._prepared_weight is not None:
+            weight = self._prepared_weight[0]
+        else:
+            weight = (self._get_effective_weight() if torch.is_grad_enabled()
+                      else self._cached_weight("effective", self._get_effective_weight))
+        out = _SparseProduct.apply(x2d, weight, self)
         out = out.reshape(*lead, self.out_features)
         if no_batch:
             out = out[0]

@@ -107,6 +107,33 @@ int btx_spmv_event(const int64_t* row_ptr, const int32_t* col, const float* w,
                    float* out, int ordered, int slots,
                    void* workspace, size_t workspace_bytes, void* stream);
 
+/* The product of the layer: y[r, :] = sum over sources s with x[r, s] != 0 of
+ * x[r, s] * W[s, :], for `rows` rows of x (n_src wide, row stride
+ * x_row_stride), every destination summed in ascending source order from
+ * +0.0f with one fmaf per term (btx_spmv_event's ordered bits) whatever form
+ * the rows take: from a count of each row's nonzeros, streaming the active
+ * sources' rows of W into a tile of y, or walking every destination's edges
+ * for 64 rows at a time.  w is in the destination-major order of csc_src (the
+ * layer's parameter order), perm[k] the position there of CSR edge k; no term
+ * is stored, so the scratch (btx_product_scratch_bytes, not initialised) does
+ * not grow with the outputs.  rows <= 65535, nnz < 2^31. */
+size_t btx_product_scratch_bytes(int64_t rows, int64_t n_src);
+int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_t* perm,
+                const int64_t* csc_ptr, const int32_t* csc_src, const float* w, int64_t n_src,
+                int64_t n_dst, int64_t nnz, const float* x, int64_t x_row_stride, int64_t rows,
+                float* y, void* scratch, size_t scratch_bytes, void* stream);
+
+/* Its gradients for gy (rows, n_dst): gx (rows, n_src) = gy W^T, and gw in the
+ * destination-major order, gw[e] = sum over rows r with x[r, src[e]] != 0 of
+ * x[r, src[e]] * gy[r, dst(e)], both written, either may be NULL
+ * (btorch/models/_sparse_triton.py:390-415). */
+size_t btx_product_grad_scratch_bytes(int64_t rows, int64_t n_src, int64_t n_dst);
+int btx_product_grad(const int64_t* row_ptr, const int32_t* col, const int64_t* perm,
+                     const int64_t* csc_ptr, const int32_t* csc_src, const float* w,
+                     int64_t n_src, int64_t n_dst, int64_t nnz, const float* x,
+                     int64_t x_row_stride, int64_t rows, const float* gy, float* gx, float* gw,
+                     void* scratch, size_t scratch_bytes, void* stream);
+
 /* btx_spmv_event without a workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference: its

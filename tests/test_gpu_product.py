@@ -1,0 +1,65 @@
+"""The sparse layer's product and gradients at the edges of its forms: the
+row form (few sources, or few of them active), the column form (64 rows of x
+at a time), several destination tiles, ragged groups, values other than
+spikes; bit for bit against the sequential CPU product, gradients against
+float64."""
+
+import numpy as np
+import pytest
+import scipy.sparse
+import torch
+
+from btorch_amd.models import SparseConn
+from oracle import rsnn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _matrix(n_src, n_dst, degree, seed):
+    rng = np.random.default_rng(seed)
+    pre = np.repeat(np.arange(n_src), degree)
+    post = rng.integers(0, n_dst, pre.size)
+    keep = (pre % 7 != 3) & (post % 11 != 5)   # sources and destinations without edges
+    key = np.unique(pre[keep] * n_dst + post[keep])
+    w = rng.standard_normal(key.size).astype(np.float32)
+    return scipy.sparse.coo_array((w, (key // n_dst, key % n_dst)), shape=(n_src, n_dst))
+
+
+@pytest.mark.parametrize("n_src,n_dst,degree,rows,prob,backend", [
+    (1, 5, 3, 1, 1.0, "native"),
+    (200, 1000, 60, 700, 0.05, "native"),       # rows unasked: at most 1024 sources
+    (1024, 333, 1500, 3, 0.5, "triton"),        # rows of W longer than a workgroup
+    (1025, 40_000, 50, 2, 0.01, "native"),      # three destination tiles
+    (1500, 97, 40, 64, 0.01, "native"),         # counted: few active
+    (1500, 97, 40, 64, 1.0, "native"),          # counted: all active, columns
+    (2000, 130, 70, 65, 0.9, "triton"),         # a second group of one row
+    (3000, 16, 8, 1, 0.9, "native"),
+    (3000, 777, 100, 129, 0.0, "native"),       # nothing active
+])
+def test_product_forms_match_sequential_sums(n_src, n_dst, degree, rows, prob, backend):
+    mat = _matrix(n_src, n_dst, degree, 5)
+    rng = np.random.default_rng(6)
+    x = (rng.random((rows, n_src)) < prob) * rng.standard_normal((rows, n_src))
+    x = torch.from_numpy(x.astype(np.float32))
+    if rows > 1:
+        x[rows // 2] = 0.0                       # a row with nothing active
+    g = torch.from_numpy(rng.standard_normal((rows, n_dst)).astype(np.float32))
+    conn = SparseConn(mat, enforce_dale=False, sparse_backend=backend, device=DEV)
+    xd = x.to(DEV).requires_grad_(True)
+    y = conn(xd)
+    y.backward(g.to(DEV))
+    ref = rsnn.NativeSparse(mat)(x)
+    assert torch.equal(y.detach().cpu(), ref)
+    with torch.no_grad():
+        assert torch.equal(conn(xd).cpu(), ref)
+    w64 = torch.from_numpy(mat.toarray().astype(np.float64))
+    gx = g.double() @ w64.t()
+    dst, src = conn.indices.cpu()
+    gw = (x.double().t() @ g.double())[src, dst]
+    # at most `degree` (gx) and `rows` (gw) products per sum: n * 2^-24 of the
+    # sum of their magnitudes bounds a sequential float32 sum
+    tol_x = (g.double().abs() @ w64.abs().t()) * (n_dst + 2) * 2.0**-24
+    tol_w = (x.double().abs().t() @ g.double().abs())[src, dst] * (rows + 2) * 2.0**-24
+    assert ((xd.grad.cpu().double() - gx).abs() <= tol_x).all()
+    assert ((conn.magnitude.grad.cpu().double() - gw).abs() <= tol_w).all()
