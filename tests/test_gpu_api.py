@@ -476,6 +476,42 @@ def test_engine_gather_steps_match_pushed_steps_and_oracle(n, lanes, D):
     assert torch.equal(h0, h1) and torch.equal(h0, h2)
 
 
+@pytest.mark.parametrize("total", [1, 255, 257, 1023, 1024, 1025, 2600])
+def test_engine_pushed_terms_per_neuron_sum_in_source_order(total):
+    # the 40 driven neurons spike together into neurons of 0, 1, 2, 3, ... 33
+    # incoming edges (the sum's order matters from three on, more than `slots`
+    # terms are pulled), `total` terms in the bin of the second segment: around
+    # the terms a workgroup requests ahead and those it holds in LDS
+    n, lanes, T = 2050, 2, 8
+    rng = np.random.default_rng(71)
+    post, left, dst = [], total, 1024
+    degs = [1, 2, 0, 3, 5, 1, 8, 2, 17, 32, 33, 40, 4]
+    while left > 0:
+        d = min(degs[dst % len(degs)], left)
+        post.append(np.full(d, dst))
+        left -= d
+        dst = dst + 1 if dst < 2046 else 1024
+    pre = np.concatenate([rng.permutation(40)[:len(p)] for p in post])
+    post = np.concatenate(post)
+    import scipy.sparse
+    w = rng.lognormal(0.0, 1.5, len(pre)) * rng.choice([-1.0, 1.0], len(pre))
+    mat = scipy.sparse.coo_array((w.astype(np.float32), (pre, post)), shape=(n, n))
+    conn = SparseConn(mat, sparse_config={"dense_pull": False})
+    model = RecurrentNN(LIF(n, tau_ref=0.2), ExponentialPSC(n, 5.0, conn), step_mode="m",
+                        update_state_names=["neuron.v", "synapse.psc"]).to(DEV)
+    functional.init_net_state(model, batch_size=lanes, device=DEV, dtype=torch.float32)
+    x = torch.zeros((T, lanes, n))
+    x[1, :, :40] = x[5, :, :40] = 5e3
+    x[3, 1, :25] = 5e3
+    with environ.context(dt=0.1), torch.no_grad():
+        z, st = model(x.to(DEV))
+    ref = rsnn.simulate(rsnn.Net(n, mat, rsnn.LIFParams.make(n, tau_ref=0.2), torch.tensor(5.0),
+                                 0.1), x)
+    assert float(ref["z"][:, :, :40].sum()) >= 40 * 2 * lanes
+    assert bits_equal(z, ref["z"]) and bits_equal(st["neuron.v"], ref["v"])
+    assert bits_equal(st["synapse.psc"], ref["psc"])
+
+
 @pytest.mark.parametrize("lanes,bin_cap", [(33, 256), (40, 0), (70, 512)])
 def test_engine_undelayed_bursts_pull_in_their_own_launch(lanes, bin_cap):
     # nets whose synapses deliver without delay, too many edges to gather
