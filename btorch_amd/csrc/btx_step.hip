@@ -87,10 +87,11 @@ struct PullArgs {
 
 // Reduction of one step's push into the neurons of one segment.
 struct ReduceIn {
-    int ordered;
+    int ordered;                 // 0: fast mode; else 1 + log2 of the distance of two bin counts
     int cap;
     int sort_max;
-    int* bin_cnt;                // [lanes][nchunks] of the buffer being consumed
+    int* bin_cnt;                // [lanes][nchunks] of the buffer being consumed, each
+                                 // 1 << (ordered - 1) apart
     const int32_t* ev_r;         // [lanes][nchunks][kBinCapMax]
     const float* ev_w;
     const uint16_t* ev_d;
@@ -216,7 +217,8 @@ struct PushStep {
     const int64_t* lane_t_end;   // lanes past their trial end push nothing
     const int64_t* in_t0;
     int64_t t;
-    int affine;                  // bin j is (delay0 + j, sub0 + j)
+    int affine;                  // bit 0: bin j is (delay0 + j, sub0 + j); the bits above: log2
+                                 // of the distance of two bin counts
     // ordered mode, dense pull (chosen per step when the push would bin more
     // than a threshold of terms per (lane, segment)): sums of every destination's
     // active incoming edges in the coalesced order into pull_acc
@@ -684,7 +686,7 @@ __device__ __forceinline__ RedHead reduce_head(const ReduceIn& a, int64_t nchunk
     h.d = a.ev_d[q0];
     h.r = a.ev_r[q0];
     h.w = a.ev_w[q0];
-    h.c = ld_const(a.bin_cnt + lane * nchunks + seg);
+    h.c = ld_const(a.bin_cnt + ((lane * nchunks + seg) << (a.ordered - 1)));
     // a vector load, waited for with the bin head rather than with the
     // scalar loads of the launch's parameters
     h.pull = a.pull_mode != nullptr
@@ -786,7 +788,7 @@ __device__ __forceinline__ void reduce_segment(const ReduceIn& a, RedLds& L, int
         }
         return;
     }
-    int* cntp = a.bin_cnt + lane * nchunks + seg;
+    int* cntp = a.bin_cnt + ((lane * nchunks + seg) << (a.ordered - 1));
     const int64_t q0 = (lane * nchunks + seg) * (int64_t)kBinCapMax;
     const int d_pre = h.d, r_pre = h.r;
     const float w_pre = h.w;
@@ -1314,9 +1316,9 @@ __device__ void p_role(const PushStep& a, PushLds& L, int64_t px, int64_t lane) 
     const int tid = threadIdx.x;
     if (tid < a.nbins) {
         // bins (delay0 + j, sub0 + j) need no table
-        const int dl = a.affine ? a.delay0 + tid : a.ctl->bin_delay[tid];
+        const int dl = (a.affine & 1) ? a.delay0 + tid : a.ctl->bin_delay[tid];
         L.slot[tid] = ring_slot(a.clock, dl, a.R);
-        L.sub[tid] = a.affine ? a.sub0 + tid : a.ctl->bin_sub[tid];
+        L.sub[tid] = (a.affine & 1) ? a.sub0 + tid : a.ctl->bin_sub[tid];
     }
     if (ORDERED) {
         for (int t = tid; t < a.nchunks; t += kThreads) L.tile[t] = 0;
@@ -1402,7 +1404,7 @@ __device__ void p_role(const PushStep& a, PushLds& L, int64_t px, int64_t lane) 
             for (int t = tid; t < a.nchunks; t += kThreads) {
                 const int ct = L.tile[t];
                 if (ct) {
-                    const int b = atomicAdd(&a.bin_cnt[lane * a.nchunks + t], ct);
+                    const int b = atomicAdd(&a.bin_cnt[(lane * a.nchunks + t) << (a.affine >> 1)], ct);
                     if (b + ct > a.cap) a.bin_cnt[-1] = 1;  // the buffer's overflow flag
                     L.base[t] = (uint16_t)(b < a.cap ? b : a.cap);
                     L.tile[t] = 0;
@@ -2003,7 +2005,7 @@ __global__ __launch_bounds__(kThreads) void k_pull(PushStep a,
         const int64_t m = a.lanes * a.nchunks;
         for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < m;
              k += (int64_t)gridDim.x * kThreads)
-            a.bin_cnt[k] = 0;
+            a.bin_cnt[k << (a.affine >> 1)] = 0;
         // the next launch takes the sums (its workgroups and this launch's
         // others read the same answer from either word)
         if (blockIdx.x == 0 && threadIdx.x == 0)
@@ -2208,8 +2210,21 @@ static inline int64_t mod(int64_t a, int64_t b) {
 struct EngineWs {
     size_t bin_cnt = 0, ev_r = 0, ev_w = 0, ev_d = 0, ev_o = 0, acc = 0, total = 0;
     int64_t bins = 0;  // per buffer
+    int bin_shift = 0;
     int64_t m = 0;     // accumulators per buffer
 };
+
+// Log2 of the distance between two bin counts.  The P workgroups add to them
+// with device-wide atomics, which one channel's memory side runs for 4 KB of
+// addresses: 256 bytes apart, the counts of one large lane spread over the
+// channels (two-compartment neurons, 200k: 16.8 -> 14.6 us a step, 500k:
+// 22.4 -> 16.6, 1M: 44 -> 28; 1M LIF neurons pushing 2.3 us less of 45; 50k
+// and 140k: equal).  The counts of several lanes contend less than the F
+// workgroups' reads of whole lines cost (140k neurons, 8 lanes: 3% slower
+// apart; 256 lanes: 5%).
+static int bin_shift(int64_t lanes, int64_t nchunks) {
+    return lanes == 1 && nchunks >= 160 ? 6 : 0;
+}
 
 static EngineWs engine_ws(int64_t lanes, int64_t n, int ordered) {
     EngineWs L;
@@ -2217,8 +2232,9 @@ static EngineWs engine_ws(int64_t lanes, int64_t n, int ordered) {
     size_t off = align256(sizeof(Ctl));
     if (ordered) {
         L.bins = lanes * nchunks;
+        L.bin_shift = bin_shift(lanes, nchunks);
         L.bin_cnt = off;
-        off = align256(off + sizeof(int) * 2 * (kBinHead + L.bins));
+        off = align256(off + sizeof(int) * 2 * (kBinHead + (L.bins << L.bin_shift)));
         L.ev_r = off;
         off = align256(off + sizeof(int32_t) * 2 * L.bins * kBinCapMax);
         L.ev_w = off;
@@ -2732,7 +2748,8 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         r.cap = cap;
         r.sort_max = p->slots;
         if (p->ordered) {
-            r.bin_cnt = (int*)(ws + L.bin_cnt) + b * (kBinHead + L.bins) + kBinHead;
+            r.ordered = 1 + L.bin_shift;
+            r.bin_cnt = (int*)(ws + L.bin_cnt) + b * (kBinHead + (L.bins << L.bin_shift)) + kBinHead;
             r.ev_r = (const int32_t*)(ws + L.ev_r) + b * L.bins * kBinCapMax;
             r.ev_w = (const float*)(ws + L.ev_w) + b * L.bins * kBinCapMax;
             r.ev_d = (const uint16_t*)(ws + L.ev_d) + b * L.bins * kBinCapMax;
@@ -2924,6 +2941,7 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         ReduceIn cur{};
         bins_of((int)(t & 1), p->ring_cursor + t, cur);
         ps.bin_cnt = cur.bin_cnt;
+        if (p->ordered) ps.affine = (ps.affine & 1) | (cur.ordered - 1) << 1;
         ReduceIn other{};
         bins_of((int)((t + 1) & 1), 0, other);
         other_bins = other.bin_cnt;

@@ -512,6 +512,36 @@ def test_engine_pushed_terms_per_neuron_sum_in_source_order(total):
     assert bits_equal(st["synapse.psc"], ref["psc"])
 
 
+@pytest.mark.parametrize("chunks,lanes", [(159, 1), (160, 1), (161, 2)])
+def test_engine_one_large_lane_spreads_its_bin_counts(chunks, lanes):
+    # from 160 segments on the counts of a single lane's term bins lie apart
+    n, D, T = chunks * 1024 - 7, 4, 10
+    c = workloads.er_net_fast(n=n, p=4.0 / n, seed=72, w_mu=0.5)
+    rows = c.pre * D + np.random.default_rng(72).integers(1, D, c.nnz)
+    import scipy.sparse
+    mat = scipy.sparse.coo_array((c.w, (rows, c.post)), shape=(n * D, n))
+    conn = SparseConn(mat)
+    syn = HeterSynapsePSC(n, 1, None, conn, base_psc=ExponentialPSC, max_delay_steps=D,
+                          use_circular_buffer=True, tau_syn=5.0)
+    model = RecurrentNN(LIF(n, tau_ref=2.0), syn, step_mode="m",
+                        update_state_names=["neuron.v", "synapse.psc"]).to(DEV)
+    functional.init_net_state(model, batch_size=lanes, device=DEV, dtype=torch.float32)
+    g = torch.Generator().manual_seed(72)
+    x = (torch.rand((2 * T, lanes, n), generator=g) < 0.02).float() * 3e3
+    out = []
+    with environ.context(dt=0.1), torch.no_grad():
+        for k in range(2):
+            z, st = model(x[k * T:(k + 1) * T].to(DEV))
+            out.append((z.cpu(), st["neuron.v"].cpu(), st["synapse.psc"].cpu()))
+    got = [torch.cat(t) for t in zip(*out)]
+    net = rsnn.Net(n, mat, rsnn.LIFParams.make(n, tau_ref=2.0), torch.tensor(5.0), 0.1,
+                   delay_mode="hetero", max_delay_steps=D, circular=True)
+    ref = rsnn.simulate(net, x)
+    assert float(ref["z"].sum()) > 1000
+    for a, b in zip(got, (ref["z"], ref["v"], ref["psc"])):
+        assert bits_equal(a, b)
+
+
 @pytest.mark.parametrize("lanes,bin_cap", [(33, 256), (40, 0), (70, 512)])
 def test_engine_undelayed_bursts_pull_in_their_own_launch(lanes, bin_cap):
     # nets whose synapses deliver without delay, too many edges to gather
