@@ -14,9 +14,9 @@
 //            ascending order: a source's destinations are distinct, so its
 //            terms need no atomics, and a barrier between sources keeps the
 //            order.  Costs the active sources, whatever the edges.
-//   columns  a wavefront takes a destination and 64 rows of x (transposed, so
-//            that a source's 64 values are one 256-byte read) and walks the
-//            destination's edges.  Costs every edge, whatever the activity.
+//   columns  a quarter wavefront takes a destination and 64 rows of x
+//            (transposed, so that a source's 64 values are one 256-byte read)
+//            and walks the destination's edges.  Costs every edge, whatever the activity.
 
 #include <hip/hip_runtime.h>
 
@@ -51,9 +51,9 @@ struct ProductArgs {
 // Which form the 64 rows of group g take.  Measured on MI355X (16,384 x 16,384
 // of 13.4M edges, 4,000 x 8,000 of 1.6M, 21,739 x 21,739 of 3.5M; 1 to 512
 // rows): rows 1.5 ns per edge of an active source, at least 0.6 us a source,
-// 1.5 ns per source looked at, 200 rows at a time; columns 16 to 27 us per
+// 1.5 ns per source looked at, 200 rows at a time; columns 10 to 24 us per
 // million edges and group.  Sides at 64 rows of the first net: 164 active
-// sources 302 us by rows and 263 us by columns, 33 of them 101 and 263 us.
+// sources 305 us by rows and 178 us by columns, 33 of them 102 and 178 us.
 __device__ __forceinline__ bool group_by_rows(const ProductArgs& a, int64_t g) {
     if (a.counts == nullptr) return true;
     const int ln = threadIdx.x & 63;
@@ -66,7 +66,7 @@ __device__ __forceinline__ bool group_by_rows(const ProductArgs& a, int64_t g) {
     const float len = (float)a.nnz / (float)a.n_src;
     const float source_us = fmaxf(0.6f, 1.5e-3f * len);
     const float rows_us = waves * (1.5e-3f * (float)a.n_src + source_us * (float)c / (float)here);
-    const float cols_us = 8.f + 22e-6f * (float)a.nnz * (float)((a.rows + kGroup - 1) / kGroup);
+    const float cols_us = 8.f + 14e-6f * (float)a.nnz * (float)((a.rows + kGroup - 1) / kGroup);
     return rows_us < cols_us;
 }
 
@@ -212,52 +212,68 @@ __global__ __launch_bounds__(256) void k_ungroup_rows(const float* __restrict__ 
     }
 }
 
-// A wavefront per (destination, group of 64 rows): thread b sums row b.  16
-// destinations at a time per workgroup, so that y is written in runs.  Bound by
-// the gathered rows of x out of L2: 264 us for 13.4M edges and 64 rows,
-// 13 TB/s; 23 us more is k_row_counts and the transpose.
-__global__ __launch_bounds__(256) void k_product_columns(ProductArgs a) {
+// A quarter wavefront per (destination, group of 64 rows), four rows a thread;
+// 16 destinations at a time per workgroup, so that y is written in runs.  Bound
+// by the gathered rows of x out of L2: 183 us for 13.4M edges and 64 rows,
+// 19 TB/s (a wavefront per destination, a row a thread: four times the
+// requests and their scalar address work, 264 us; without the bound of four
+// wavefronts per SIMD 135 registers leave three: 223 us).
+__global__ __launch_bounds__(256, 4) void k_product_columns(ProductArgs a) {
     __shared__ float s_out[16][65];
-    const int tid = threadIdx.x, ln = tid & 63;
+    const int tid = threadIdx.x, ln = tid & 63, c16 = ln & 15;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t groups = (a.rows + kGroup - 1) / kGroup;
     const int64_t tiles = (a.n_dst + 15) / 16;
     for (int64_t g = 0; g < groups; ++g) {
         if (group_by_rows(a, g)) continue;
-        const float* xg = a.xt + g * a.n_src * kGroup + ln;
+        const float* xg = a.xt + g * a.n_src * kGroup;
         for (int64_t tl = blockIdx.x; tl < tiles; tl += gridDim.x) {
-            for (int q = wv; q < 16; q += 4) {
-                const int64_t d = tl * 16 + q;
-                if (d >= a.n_dst) break;
-                const int64_t e0 = a.csc_ptr[d];
-                const int len = (int)(a.csc_ptr[d + 1] - e0);
-                float acc = 0.f;
-                for (int c = 0; c < len; c += 64) {
-                    const int m = len - c < 64 ? len - c : 64;
-                    const int my_s = ln < m ? a.csc_src[e0 + c + ln] : 0;
-                    const int my_w = ln < m ? __float_as_int(a.w[e0 + c + ln]) : 0;
-                    int k = 0;
-                    for (; k + 16 <= m; k += 16) {
-                        float x16[16];
+            // a quarter of the wavefront per destination, four rows per thread
+            const int q = wv * 4 + (ln >> 4);
+            const int64_t d = tl * 16 + q;
+            const int64_t e0 = d < a.n_dst ? a.csc_ptr[d] : 0;
+            const int len = d < a.n_dst ? (int)(a.csc_ptr[d + 1] - e0) : 0;
+            int most = len;
 #pragma unroll
-                        for (int u = 0; u < 16; ++u)
-                            x16[u] = xg[(int64_t)__builtin_amdgcn_readlane(my_s, k + u) * kGroup];
+            for (int o = 16; o < 64; o <<= 1) {
+                const int other = __shfl_xor(most, o, 64);
+                most = other > most ? other : most;
+            }
+            most = __builtin_amdgcn_readfirstlane(most);
+            float acc[4] = {0.f, 0.f, 0.f, 0.f};
+            int my_s = c16 < len ? a.csc_src[e0 + c16] : 0;
+            float my_w = c16 < len ? a.w[e0 + c16] : 0.f;
+            for (int c = 0; c < most; c += 16) {
+                // the destination's next 16 edges
+                const int nx = c + 16 + c16;
+                const int next_s = nx < len ? a.csc_src[e0 + nx] : 0;
+                const float next_w = nx < len ? a.w[e0 + nx] : 0.f;
 #pragma unroll
-                        for (int u = 0; u < 16; ++u) {
-                            const float wk = __int_as_float(__builtin_amdgcn_readlane(my_w, k + u));
-                            const float t = fmaf(wk, x16[u], acc);
-                            acc = x16[u] != 0.f ? t : acc;
+                for (int h = 0; h < 16; h += 8) {
+                    float4 x8[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const int src = __shfl(my_s, (ln & 48) + h + u, 64);
+                        x8[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+                        if (c + h + u < len)
+                            x8[u] = *reinterpret_cast<const float4*>(xg + ((int64_t)src * kGroup + 4 * c16));
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const float wk = __shfl(my_w, (ln & 48) + h + u, 64);
+                        const float x4[4] = {x8[u].x, x8[u].y, x8[u].z, x8[u].w};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float t = fmaf(wk, x4[i], acc[i]);
+                            acc[i] = x4[i] != 0.f ? t : acc[i];
                         }
                     }
-                    for (; k < m; ++k) {
-                        const float xv = xg[(int64_t)__builtin_amdgcn_readlane(my_s, k) * kGroup];
-                        const float wk = __int_as_float(__builtin_amdgcn_readlane(my_w, k));
-                        const float t = fmaf(wk, xv, acc);
-                        acc = xv != 0.f ? t : acc;
-                    }
                 }
-                s_out[q][ln] = acc;
+                my_s = next_s;
+                my_w = next_w;
             }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s_out[q][4 * c16 + i] = acc[i];
             __syncthreads();
             // 16 destinations of 64 rows: a 64-byte run per row
             for (int k = tid; k < 16 * kGroup; k += 256) {
@@ -271,10 +287,12 @@ __global__ __launch_bounds__(256) void k_product_columns(ProductArgs a) {
 }
 
 // gx of the layer: gxt[g][s][b] = sum over edges e of row s of w[e] *
-// gt[g][col[e]][b]; one wavefront per (row, group), 16 gathered rows in flight.
-// Bound by the gathered rows out of L2: 292 us for 13.4M edges and 64 rows,
-// 11.8 TB/s (the wavefront per edge block of btx_spmv.hip that the layer's
-// backward used before: 3.9 ms with its copies).
+// gt[g][col[e]][b]; one wavefront per (row, group), 32 gathered rows in flight.
+// Bound by the weights, which perm scatters (0.8 GB fetched for 13.4M edges),
+// and the gathered rows out of L2: 273 us at 64 rows (a row of the 64 per
+// thread and an edge per instruction: 292; five wavefronts per SIMD spill: 407;
+// the row pass of btx_spmv.hip that the layer's backward used before: 3.9 ms
+// with its copies).
 __global__ __launch_bounds__(256) void k_product_grad_x(const int64_t* __restrict__ rp,
                                                         const int32_t* __restrict__ col,
                                                         const int64_t* __restrict__ perm,
@@ -287,38 +305,57 @@ __global__ __launch_bounds__(256) void k_product_grad_x(const int64_t* __restric
     const int64_t g = blockIdx.y;
     const int ln = threadIdx.x & 63;
     if (s >= n_src) return;
-    const float* gg = gt + g * n_dst * kGroup + ln;
+    const int q = ln >> 4, c16 = ln & 15;
+    const float* gg = gt + g * n_dst * kGroup;
     const int64_t e0 = rp[s];
     const int len = (int)(rp[s + 1] - e0);
-    // the terms of 64 edges in sixteen partial sums, added pairwise, and the
-    // 64-edge sums in float64: 7e-8 of the result against float64 throughout
-    // (sixteen sums over all edges 1.4e-7, two 3.6e-7)
-    double sum = 0.0;
+    // a quarter of the wavefront per edge, four of the rows per thread; the
+    // terms of 64 edges in two partial sums each and the 64-edge sums in
+    // float64: 7e-8 of the result against float64 throughout (sixteen float
+    // sums over all edges 1.4e-7, two 3.6e-7)
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    int my_d = ln < len ? col[e0 + ln] : 0;
+    float my_w = ln < len ? w[perm[e0 + ln]] : 0.f;
     for (int c = 0; c < len; c += 64) {
         const int m = len - c < 64 ? len - c : 64;
-        float acc[16] = {};
-        const int my_d = ln < m ? col[e0 + c + ln] : 0;
-        const int my_w = ln < m ? __float_as_int(w[perm[e0 + c + ln]]) : 0;
-        int k = 0;
-        for (; k + 16 <= m; k += 16) {
-            float g16[16];
+        // the next 64 edges; their weights lie scattered
+        const int nx = c + 64 + ln;
+        const int next_d = nx < len ? col[e0 + nx] : 0;
+        const float next_w = nx < len ? w[perm[e0 + nx]] : 0.f;
+        float acc[2][4] = {};
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
-                g16[u] = gg[(int64_t)__builtin_amdgcn_readlane(my_d, k + u) * kGroup];
+        for (int h = 0; h < 2; ++h) {
+            if (32 * h >= m) break;  // uniform
+            float4 g8[8];
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
-                acc[u] = fmaf(__int_as_float(__builtin_amdgcn_readlane(my_w, k + u)), g16[u], acc[u]);
+            for (int u = 0; u < 8; ++u) {
+                const int k = 32 * h + 4 * u + q;
+                const int d = __shfl(my_d, k, 64);
+                g8[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (k < m) g8[u] = *reinterpret_cast<const float4*>(gg + ((int64_t)d * kGroup + 4 * c16));
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float wk = __shfl(my_w, 32 * h + 4 * u + q, 64);
+                acc[h][0] = fmaf(wk, g8[u].x, acc[h][0]);
+                acc[h][1] = fmaf(wk, g8[u].y, acc[h][1]);
+                acc[h][2] = fmaf(wk, g8[u].z, acc[h][2]);
+                acc[h][3] = fmaf(wk, g8[u].w, acc[h][3]);
+            }
         }
-        for (; k < m; ++k)
-            acc[0] = fmaf(__int_as_float(__builtin_amdgcn_readlane(my_w, k)),
-                          gg[(int64_t)__builtin_amdgcn_readlane(my_d, k) * kGroup], acc[0]);
 #pragma unroll
-        for (int o = 8; o > 0; o >>= 1)
-#pragma unroll
-            for (int u = 0; u < o; ++u) acc[u] += acc[u + o];
-        sum += acc[0];
+        for (int i = 0; i < 4; ++i) sum[i] += (double)acc[0][i] + (double)acc[1][i];
+        my_d = next_d;
+        my_w = next_w;
     }
-    gxt[(g * n_src + s) * kGroup + ln] = (float)sum;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        sum[i] += __shfl_xor(sum[i], 16, 64);
+        sum[i] += __shfl_xor(sum[i], 32, 64);
+    }
+    if (q == 0)
+        *reinterpret_cast<float4*>(gxt + (g * n_src + s) * kGroup + 4 * c16) =
+            make_float4((float)sum[0], (float)sum[1], (float)sum[2], (float)sum[3]);
 }
 
 // gw of the layer, destination-major: gw[e] = sum over rows b of x[b, src[e]] *
@@ -388,10 +425,12 @@ static size_t grad_scratch(int64_t rows, int64_t n_src, int64_t n_dst) {
     return groups * kGroup * 4 * (size_t)(n_dst + n_src) + groups * 8 * (size_t)n_src + 256;
 }
 
-static int check_product(const char* who, int64_t n_src, int64_t n_dst, int64_t nnz, int64_t rows) {
+static int check_product(const char* who, int64_t n_src, int64_t n_dst, int64_t nnz, int64_t rows,
+                         const void* scratch) {
     if (n_src >= (int64_t)1 << 31 || n_dst >= (int64_t)1 << 31 || nnz >= (int64_t)1 << 31)
         return fail(std::string(who) + ": sources, destinations and edges must fit int32");
     if (rows > 65535) return fail(std::string(who) + ": rows exceeds 65535");
+    if (((uintptr_t)scratch & 15) != 0) return fail(std::string(who) + ": scratch is not 16-byte aligned");
     return 0;
 }
 
@@ -409,7 +448,7 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
                         int64_t x_row_stride, int64_t rows, float* y, void* scratch,
                         size_t scratch_bytes, void* stream) {
     if (rows <= 0 || n_dst <= 0) return 0;
-    if (int rc = check_product("btx_product", n_src, n_dst, nnz, rows)) return rc;
+    if (int rc = check_product("btx_product", n_src, n_dst, nnz, rows, scratch)) return rc;
     if (scratch_bytes < btx_product_scratch_bytes(rows, n_src) ||
         (scratch == nullptr && scratch_bytes > 0))
         return fail("btx_product: scratch too small");
@@ -446,7 +485,7 @@ BTX_API int btx_product_grad(const int64_t* row_ptr, const int32_t* col, const i
                              int64_t x_row_stride, int64_t rows, const float* gy, float* gx,
                              float* gw, void* scratch, size_t scratch_bytes, void* stream) {
     if (rows <= 0 || n_src <= 0 || n_dst <= 0) return 0;
-    if (int rc = check_product("btx_product_grad", n_src, n_dst, nnz, rows)) return rc;
+    if (int rc = check_product("btx_product_grad", n_src, n_dst, nnz, rows, scratch)) return rc;
     if (scratch == nullptr || scratch_bytes < grad_scratch(rows, n_src, n_dst))
         return fail("btx_product_grad: scratch too small");
     const hipStream_t s = (hipStream_t)stream;

@@ -445,3 +445,9 @@ def test_adjoint_sweep_lane_counts_match_reference_autograd(n, B, D, shared_tau)
     e_x = rel_err(xg.grad, xr.grad)
     print(f"\nn {n}, {B} lanes, D {D}: dW {e_w:.2e} dtau {e_t:.2e} dx {e_x:.2e}")
     assert e_w < 1e-4 and e_t < 1e-4 and e_x < 1e-4
+
+
+@pytest.mark.parametrize("n,B", [(130, 36), (255, 60), (97, 62)])
+def test_adjoint_sweep_lanes_by_fours_match_reference_autograd(n, B):
+    # 33 to 64 lanes: four lanes a thread where they divide by four, else one
+    test_adjoint_sweep_lane_counts_match_reference_autograd(n, B, 1, False)
