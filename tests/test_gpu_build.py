@@ -67,6 +67,21 @@ def test_device_build_equals_host_path(n_pre, n_post, nnz, D, dup):
     _assert_same(host, dev)
 
 
+@pytest.mark.parametrize("n_pre,n_post,D", [(1, 1, 1), (2, 1, 1), (1, 2, 3), (128, 256, 2),
+                                            (257, 257, 1), (64, 65_537, 64)])
+def test_device_build_at_the_widths_of_its_sort_keys(n_pre, n_post, D):
+    # sources and destinations at both ends of the bits that hold them, in
+    # falling order, some of them twice
+    ends = (lambda n: np.unique(np.clip([0, 1, n // 2 - 1, n // 2, n - 2, n - 1], 0, n - 1))[::-1])
+    pre, post, delay = (a.ravel() for a in np.meshgrid(ends(n_pre), ends(n_post), ends(D),
+                                                       indexing="ij"))
+    pre, post, delay = (np.concatenate([a, a[::3]]).astype(np.int64) for a in (pre, post, delay))
+    w = np.random.default_rng(3).normal(size=pre.size).astype(np.float32)
+    delay = delay if D > 1 else None
+    _assert_same(_host(pre, post, w, delay, D, n_pre, n_post),
+                 _device(pre, post, w, delay, D, n_pre, n_post))
+
+
 def test_device_build_edge_cases():
     # no edges; one edge; every edge in one row
     for pre, post, w, shape in [
