@@ -28,6 +28,7 @@ namespace btx {
 constexpr int kRowTile = 16384;      // destinations of a `rows` workgroup, at most (64 KB of LDS)
 constexpr int kRowThreads = 1024;
 constexpr int kGroup = 64;           // rows of x per wavefront of the `columns` form
+constexpr int64_t kFewRows = 4;      // up to which k_product_few takes them
 constexpr int64_t kFewSources = 1024;  // up to which the `rows` form is taken unasked
 
 struct ProductArgs {
@@ -50,10 +51,10 @@ struct ProductArgs {
 
 // Which form the 64 rows of group g take.  Measured on MI355X (16,384 x 16,384
 // of 13.4M edges, 4,000 x 8,000 of 1.6M, 21,739 x 21,739 of 3.5M; 1 to 512
-// rows): rows 1.5 ns per edge of an active source, at least 0.6 us a source,
-// 1.5 ns per source looked at, 200 rows at a time; columns 10 to 24 us per
-// million edges and group.  Sides at 64 rows of the first net: 164 active
-// sources 305 us by rows and 178 us by columns, 33 of them 102 and 178 us.
+// rows): rows 0.8 ns per edge of an active source, at least 0.4 us a source,
+// 0.3 ns per source looked at, 110 rows at a time; columns 10 to 24 us per
+// million edges and group.  Sides at 64 rows of the first net: 328 active
+// sources 254 us by rows and 174 us by columns, 82 of them 97 and 174 us.
 __device__ __forceinline__ bool group_by_rows(const ProductArgs& a, int64_t g) {
     if (a.counts == nullptr) return true;
     const int ln = threadIdx.x & 63;
@@ -62,36 +63,36 @@ __device__ __forceinline__ bool group_by_rows(const ProductArgs& a, int64_t g) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
     const int64_t here = a.rows - g * kGroup < kGroup ? a.rows - g * kGroup : kGroup;
-    const float waves = a.rows > 200 ? (float)a.rows / 200.f : 1.f;
+    const float waves = a.rows > 110 ? (float)a.rows / 110.f : 1.f;
     const float len = (float)a.nnz / (float)a.n_src;
-    const float source_us = fmaxf(0.6f, 1.5e-3f * len);
-    const float rows_us = waves * (1.5e-3f * (float)a.n_src + source_us * (float)c / (float)here);
+    const float source_us = fmaxf(0.4f, 0.8e-3f * len);
+    const float rows_us = waves * (0.3e-3f * (float)a.n_src + source_us * (float)c / (float)here);
     const float cols_us = 8.f + 14e-6f * (float)a.nnz * (float)((a.rows + kGroup - 1) / kGroup);
     return rows_us < cols_us;
 }
 
 // Nonzeros of every row (one workgroup per row).
-__global__ __launch_bounds__(256) void k_row_counts(const float* __restrict__ x, int64_t n,
+__global__ __launch_bounds__(1024) void k_row_counts(const float* __restrict__ x, int64_t n,
                                                     int64_t stride, int32_t* __restrict__ counts) {
     const int64_t row = blockIdx.x;
     const float* xr = x + row * stride;
     int c = 0;
 #pragma unroll 8
-    for (int64_t i = threadIdx.x; i < n; i += 256) c += xr[i] != 0.f;
+    for (int64_t i = threadIdx.x; i < n; i += 1024) c += xr[i] != 0.f;
     int total;
-    block_excl_scan<4>(c, total);
+    block_excl_scan<16>(c, total);
     if (threadIdx.x == 0) counts[row] = total;
 }
 
-// One row of x, destinations [d0, d0 + tile): 1024 of the row's values are
+// One row of x, destinations [d0, d0 + tile): 8192 of the row's values are
 // read at a time and their nonzeros listed in LDS in ascending order, each
 // with its row of W.  Bound by the misses one CU can have in flight on a
-// source's weights, which perm scatters over the array (1.25 us a source of
-// 819 edges, 0.6 us of 400): eight sources are requested together, the next
-// eight before the current ones are added (one source ahead: 1.9 us).  Taken
-// back: three requests in flight and tiles of 1024 destinations (74 VGPRs, one
-// workgroup per CU: 512 rows 15% slower), 256 threads (four times the passes
-// over x).
+// source's weights, which perm scatters over the array, and by the barrier per
+// source: eight sources are requested together, the next eight before the
+// current ones are added, and a few rows are split into tiles over the CUs.
+// 0.4 to 0.65 us a source of 163 to 819 edges (one source ahead, 1024 values at
+// a time and whole rows: 0.8 to 1.9 us).  Taken back: three requests in flight
+// (74 VGPRs, one workgroup per CU: 512 rows 15% slower), 256 threads.
 __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int tile) {
     constexpr int T = kRowThreads;
     extern __shared__ __align__(16) float s_y[];
@@ -106,25 +107,39 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
     for (int q = tid; q < (nd + 3) / 4; q += T)
         reinterpret_cast<float4*>(s_y)[q] = make_float4(0.f, 0.f, 0.f, 0.f);
     const float* xr = a.x + row * a.x_stride;
-    for (int64_t s0 = 0; s0 < a.n_src; s0 += T) {
-        const int64_t s = s0 + tid;
-        const float xv = s < a.n_src ? xr[s] : 0.f;
-        const bool on = xv != 0.f;
-        const uint64_t m = __ballot(on);
-        if (ln == 0) s_cnt[wv] = __popcll((unsigned long long)m);
-        __syncthreads();
-        int off = 0, total = 0;
+    for (int64_t s0 = 0; s0 < a.n_src; s0 += T * U) {
+      // a wavefront reads 512 consecutive values
+      const int64_t s1 = s0 + wv * 64 * U + ln;
+      float xv[U];
 #pragma unroll
-        for (int k = 0; k < T / 64; ++k) {
-            off += k < wv ? s_cnt[k] : 0;
-            total += s_cnt[k];
-        }
-        if (on) {
+      for (int u = 0; u < U; ++u) xv[u] = s1 + 64 * u < a.n_src ? xr[s1 + 64 * u] : 0.f;
+      int mine = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) mine += __popcll((unsigned long long)__ballot(xv[u] != 0.f));
+      if (ln == 0) s_cnt[wv] = mine;
+      __syncthreads();
+      int first = 0, nonzero = 0;
+#pragma unroll
+      for (int k = 0; k < T / 64; ++k) {
+          first += k < wv ? s_cnt[k] : 0;
+          nonzero += s_cnt[k];
+      }
+      // the nonzeros, 1024 at a time
+      for (int base = 0; base < nonzero; base += T) {
+        const int total = nonzero - base < T ? nonzero - base : T;
+        int off = first - base;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool on = xv[u] != 0.f;
+            const uint64_t m = __ballot(on);
             const int p = off + __popcll((unsigned long long)(m & ((1ull << ln) - 1ull)));
-            const int64_t beg = a.row_ptr[s];
-            s_beg[p] = (int)beg;
-            s_len[p] = (int)(a.row_ptr[s + 1] - beg);
-            s_x[p] = xv;
+            off += __popcll((unsigned long long)m);
+            if (on && p >= 0 && p < T) {
+                const int64_t beg = a.row_ptr[s1 + 64 * u];
+                s_beg[p] = (int)beg;
+                s_len[p] = (int)(a.row_ptr[s1 + 64 * u + 1] - beg);
+                s_x[p] = xv[u];
+            }
         }
         __syncthreads();
         // this thread's first edge of eight sources: destination within the
@@ -140,9 +155,9 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                w[u] = d[u] >= 0 ? a.w[pm[u]] : 0.f;
                 const int64_t q = d[u] - d0;
                 d[u] = d[u] >= 0 && q >= 0 && q < nd ? (int)q : -1;
+                w[u] = d[u] >= 0 ? a.w[pm[u]] : 0.f;
             }
         };
         int d[U], dn[U];
@@ -169,6 +184,9 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
                 w[u] = wn[u];
             }
         }
+        __syncthreads();  // the list is rewritten
+      }
+      __syncthreads();  // and s_cnt
     }
     __syncthreads();
     float* yr = a.y + row * a.n_dst + d0;
@@ -283,6 +301,44 @@ __global__ __launch_bounds__(256, 4) void k_product_columns(ProductArgs a) {
             }
             __syncthreads();
         }
+    }
+}
+
+// A few rows of x: a wavefront per destination reads 64 edges at a time, a lane
+// each, and gathers their x out of L2; the nonzero ones, found by a ballot, are
+// added in ascending source order.  One launch, whatever the activity: 21,739 x
+// 21,739 of 3.5M edges 14 us a row in a replayed graph (counting, the transpose
+// and the two forms above 55 to 75 us).
+template <int ROWS>
+__global__ __launch_bounds__(256) void k_product_few(ProductArgs a) {
+    const int ln = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (int64_t d = (int64_t)blockIdx.x * 4 + wv; d < a.n_dst; d += (int64_t)gridDim.x * 4) {
+        const int64_t e0 = a.csc_ptr[d];
+        const int len = (int)(a.csc_ptr[d + 1] - e0);
+        float acc[ROWS] = {};
+        for (int c = 0; c < len; c += 64) {
+            const bool in = c + ln < len;
+            const int src = in ? a.csc_src[e0 + c + ln] : 0;
+            const int w = in ? __float_as_int(a.w[e0 + c + ln]) : 0;
+            float xv[ROWS];
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) xv[r] = in ? a.x[r * a.x_stride + src] : 0.f;
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                uint64_t m = __ballot(xv[r] != 0.f);
+                while (m) {
+                    const int b = __ffsll((unsigned long long)m) - 1;
+                    m &= m - 1;
+                    acc[r] = fmaf(__int_as_float(__builtin_amdgcn_readlane(w, b)),
+                                  __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xv[r]), b)),
+                                  acc[r]);
+                }
+            }
+        }
+        if (ln == 0)
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) a.y[r * a.n_dst + d] = acc[r];
     }
 }
 
@@ -425,6 +481,15 @@ static size_t grad_scratch(int64_t rows, int64_t n_src, int64_t n_dst) {
     return groups * kGroup * 4 * (size_t)(n_dst + n_src) + groups * 8 * (size_t)n_src + 256;
 }
 
+// Destinations of a `rows` workgroup: as few tiles as occupy every CU, of at
+// least 1024 destinations.
+static int row_tile(int64_t rows, int64_t n_dst) {
+    const int64_t want = rows < 256 ? 256 / rows : 1;
+    int64_t tile = ((n_dst + want - 1) / want + 63) / 64 * 64;
+    tile = tile < 1024 ? 1024 : tile > kRowTile ? kRowTile : tile;
+    return (int)(tile < n_dst ? tile : n_dst);
+}
+
 static int check_product(const char* who, int64_t n_src, int64_t n_dst, int64_t nnz, int64_t rows,
                          const void* scratch) {
     if (n_src >= (int64_t)1 << 31 || n_dst >= (int64_t)1 << 31 || nnz >= (int64_t)1 << 31)
@@ -455,16 +520,28 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
     const hipStream_t s = (hipStream_t)stream;
     ProductArgs a{row_ptr, col, perm, csc_ptr, csc_src, w, n_src, n_dst, nnz, x, x_row_stride, rows,
                   y, nullptr, nullptr};
+    // one row always (13.4M edges: 28 us against 31 by rows at 16 active sources
+    // and 170 by columns); up to four while their gathers stay few: 8M in all
+    // take 27 us, 14M 52 us, by when the rows form is as fast at low activity
+    if (n_src > kFewSources && rows <= kFewRows &&
+        (rows == 1 || rows * nnz <= ((int64_t)8 << 20))) {
+        const int64_t wgs = (n_dst + 3) / 4;
+        const dim3 few((unsigned)(wgs < 8192 ? wgs : 8192));
+        hipLaunchKernelGGL(rows == 1 ? k_product_few<1> : rows == 2 ? k_product_few<2>
+                           : rows == 3 ? k_product_few<3> : k_product_few<4>,
+                           few, dim3(256), 0, s, a);
+        return check_launch("btx_product");
+    }
     const int64_t groups = (rows + kGroup - 1) / kGroup;
     if (n_src > kFewSources) {
         a.counts = (const int32_t*)scratch;
         a.xt = (float*)((char*)scratch + align256(4 * (size_t)rows));
-        hipLaunchKernelGGL(k_row_counts, dim3((unsigned)rows), dim3(256), 0, s, x, n_src,
+        hipLaunchKernelGGL(k_row_counts, dim3((unsigned)rows), dim3(1024), 0, s, x, n_src,
                            x_row_stride, (int32_t*)scratch);
         hipLaunchKernelGGL(k_group_rows, dim3((unsigned)((n_src + 63) / 64), (unsigned)groups),
                            dim3(256), 0, s, a, x, n_src, x_row_stride, rows, a.xt);
     }
-    const int tile = (int)(n_dst < kRowTile ? n_dst : kRowTile);
+    const int tile = row_tile(rows, n_dst);
     const dim3 grid((unsigned)rows, (unsigned)((n_dst + tile - 1) / tile));
     hipLaunchKernelGGL(k_product_rows, grid, dim3(kRowThreads), 4 * (size_t)(tile + 3), s, a, tile);
     if (n_src > kFewSources) {

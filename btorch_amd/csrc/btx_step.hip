@@ -2,9 +2,9 @@
 //
 // Every step is one launch whose workgroups play two roles:
 //   F (lane, 1024-neuron segment c): first reduces the previous step's push
-//     into its own neurons -- the terms binned for (lane, c), sorted in LDS by
-//     neuron and, per neuron, by virtual source row, summed from +0.0f in that
-//     order -- then integrates the step: psc_{t-1} = psc_dec + sum, LIF
+//     into its own neurons -- the terms binned for (lane, c), listed in LDS by
+//     neuron and summed per neuron in ascending virtual source row from +0.0f
+//     -- then integrates the step: psc_{t-1} = psc_dec + sum, LIF
 //     charge/fire/refractory/reset, exponential-synapse decay psc_dec, spike
 //     words -> raster, and the pushed spikes (own or teacher's) as the
 //     segment's ascending list and words into ring slot (cursor + t) % R.

@@ -63,3 +63,23 @@ def test_product_forms_match_sequential_sums(n_src, n_dst, degree, rows, prob, b
     tol_w = (x.double().abs().t() @ g.double().abs())[src, dst] * (rows + 2) * 2.0**-24
     assert ((xd.grad.cpu().double() - gx).abs() <= tol_x).all()
     assert ((conn.magnitude.grad.cpu().double() - gw).abs() <= tol_w).all()
+
+
+@pytest.mark.parametrize("n_src,n_dst,degree,rows,prob", [
+    (1025, 301, 50, 1, 0.3),        # one row: a wavefront per destination
+    (1025, 63, 130, 3, 1.0),
+    (2100, 33_000, 10, 4, 0.02),    # more destinations than wavefronts
+    (1025, 3, 2, 5, 0.01),          # a few rows, fewer destinations than a tile
+    (8193, 5000, 300, 5, 0.002),    # tiles over the CUs, a second pass over x
+    (8700, 2500, 1100, 6, 0.001),
+])
+def test_products_of_few_rows_match_sequential_sums(n_src, n_dst, degree, rows, prob):
+    mat = _matrix(n_src, n_dst, degree, 7)
+    rng = np.random.default_rng(8)
+    x = (rng.random((rows, n_src)) < prob) * rng.standard_normal((rows, n_src))
+    x = torch.from_numpy(x.astype(np.float32))
+    x[:, -1] = 1.5
+    conn = SparseConn(mat, enforce_dale=False, device=DEV)
+    with torch.no_grad():
+        y = conn(x.to(DEV)).cpu()
+    assert torch.equal(y, rsnn.NativeSparse(mat)(x))
