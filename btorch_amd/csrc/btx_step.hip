@@ -1675,27 +1675,31 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
         mine = b < lg && nidx < a.n;
         live = mine;
         if (mine && a.lane_t_end != nullptr) live = a.in_t0[lane] + a.t < a.lane_t_end[lane];
-        if (g.fin || !live) return;
-        v = a.v[i];
-        p = a.psc[i];
-        if (SX) {
-            s2.h1 = a.sh1[i];
-            if (a.syn == BTX_SYN_DUAL_EXP) s2.h2 = a.sh2[i];
-        }
-        if (a.use_ref) r = a.ref[i];
-        if (a.x) x = a.x[i];
-        if (TC && (!MIX || a.tia != nullptr)) {
-            ta = a.tia[i];
-            tb = a.tibap[i];
-            tt = a.tth[i];
-            if (a.xa) xa = a.xa[i];
-        }
-        if (GLIF && a.iasc != nullptr) {
+        if (g.fin || !mine) return;
+        if (live) {
+            v = a.v[i];
+            p = a.psc[i];
+            if (SX) {
+                s2.h1 = a.sh1[i];
+                if (a.syn == BTX_SYN_DUAL_EXP) s2.h2 = a.sh2[i];
+            }
+            if (a.use_ref) r = a.ref[i];
+            if (a.x) x = a.x[i];
+            if (TC && (!MIX || a.tia != nullptr)) {
+                ta = a.tia[i];
+                tb = a.tibap[i];
+                tt = a.tth[i];
+                if (a.xa) xa = a.xa[i];
+            }
+            if (GLIF && a.iasc != nullptr) {
 #pragma unroll
-            for (int j = 0; j < kMaxAsc; ++j)
-                if (j < a.n_asc) ia[GLIF ? j : 0] = a.iasc[i * a.n_asc + j];
+                for (int j = 0; j < kMaxAsc; ++j)
+                    if (j < a.n_asc) ia[GLIF ? j : 0] = a.iasc[i * a.n_asc + j];
+            }
         }
-        if (round > 0) return;  // the parameters are the neuron's, whatever the lane
+        // the parameters are the neuron's: read with the first lane, which may
+        // be idle while a later one runs
+        if (round > 0) return;
         if (MIX) code = a.kinds[nidx];
         if (!TC || MIX) tau = prm(a.tau, a.tau_s, nidx);
         q.vth = prm(a.vth, a.vth_s, nidx);
