@@ -2185,7 +2185,8 @@ struct RunTables {
     int bin_of_sub[BTX_MAX_BINS];
 };
 
-__global__ __launch_bounds__(64) void k_set_tables(RunTables t, Ctl* __restrict__ ctl) {
+__global__ __launch_bounds__(64) void k_set_tables(RunTables t, Ctl* __restrict__ ctl,
+                                                   int64_t clock) {
     // the tables are the first bytes of the argument segment, read by a
     // per-lane load (a select over 64 values each took 55 us, cold)
     const auto* arg = (const __attribute__((address_space(4))) RunTables*)
@@ -2195,12 +2196,13 @@ __global__ __launch_bounds__(64) void k_set_tables(RunTables t, Ctl* __restrict_
     ctl->bin_delay[k] = arg->bin_delay[k];
     ctl->bin_sub[k] = arg->bin_sub[k];
     ctl->bin_of_sub[k] = arg->bin_of_sub[k];
-    // the last run's decision about the step after it, at whichever index
-    // this run's clock reads it
+    // the last run's decision about the step after it, at the index this
+    // run's clock reads it, and how its last step was delivered (k_mark) at
+    // the one before
     const int next = ctl->next_idx;
     if (next > 0) {
-        const int push = ctl->push_mode[(next - 1) & 3];
-        if (k < 4) ctl->push_mode[k] = push;
+        const int push = ctl->push_mode[(next - 1) & 3], last = ctl->push_mode[(next - 2) & 3];
+        if (k < 4) ctl->push_mode[k] = k == (int)((clock - 1) & 3) ? last : push;
     }
 }
 
@@ -2723,7 +2725,8 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
     }
     const bool gather = gather_route(p, min_delay >= 1);
     if (!p->tables_ready)
-        hipLaunchKernelGGL(k_set_tables, dim3(1), dim3(64), 0, s, tb, ctl);
+        hipLaunchKernelGGL(k_set_tables, dim3(1), dim3(64), 0, s, tb, ctl,
+                           (int64_t)p->ring_cursor);
     // lane-bit ring of the dense pull (ordered mode with the plan's ring of
     // lane bits); 64-lane words per neuron
     uint64_t* lane_bits = p->ordered ? p->ring_lane_bits : nullptr;

@@ -14,6 +14,7 @@ from btorch_amd.models import (
     ATan, Erf, ExponentialPSC, HeterSynapsePSC, LIF, RecurrentNN, SparseConn, environ,
     functional,
 )
+from btorch_amd.models._engine import unpack_bits
 from oracle import rsnn
 
 pytestmark = pytest.mark.gpu
@@ -574,3 +575,69 @@ def test_engine_undelayed_bursts_pull_in_their_own_launch(lanes, bin_cap):
     assert per_step[5:8].max() > 0.2 and per_step[:5].max() < 0.01
     assert bits_equal(z, ref["z"])
     assert bits_equal(v, ref["v"]) and bits_equal(psc, ref["psc"])
+
+
+def _busy_net(D, seed):
+    """2000 neurons, 1.9M edges of delays 0 .. D - 1 (too many to gather at
+    the lanes used here): (matrix of virtual rows, neurons)."""
+    import scipy.sparse
+    n = 2000
+    c = workloads.er_net_fast(n=n, p=0.65, seed=seed, w_mu=-7.0)
+    assert c.nnz > 1_700_000
+    rows = c.pre * D + (np.random.default_rng(seed).integers(0, D, c.nnz) if D > 1 else 0)
+    return scipy.sparse.coo_array((c.w, (rows, c.post)), shape=(n * D, n)), n
+
+
+def _drive(levels, lanes, n):
+    """(steps, lanes, n) input that makes levels[t] neurons of every lane spike
+    at step t, no neuron twice."""
+    x = torch.zeros((len(levels), lanes, n))
+    for t, k in enumerate(levels):
+        for b in range(lanes):
+            x[t, b, [(37 * i + b) % 31 * 64 + t for i in range(k)]] = 14.0
+    return x
+
+
+def _busy_model(mat, D, n, lanes, **config):
+    conn = SparseConn(mat, sparse_config=config)
+    syn = (HeterSynapsePSC(n, 1, None, conn, base_psc=ExponentialPSC, max_delay_steps=D,
+                           use_circular_buffer=True, tau_syn=5.0)
+           if D > 1 else ExponentialPSC(n, 5.0, conn))
+    m = RecurrentNN(LIF(n, tau_ref=0.3), syn, step_mode="m",
+                    update_state_names=["neuron.v", "synapse.psc"]).to(DEV)
+    functional.init_net_state(m, batch_size=lanes, device=DEV, dtype=torch.float32)
+    return m, conn
+
+
+def _busy_reference(mat, D, n, x):
+    net = rsnn.Net(n, mat, rsnn.LIFParams.make(n, tau_ref=0.3), torch.tensor(5.0), 0.1,
+                   **(dict(delay_mode="hetero", max_delay_steps=D, circular=True) if D > 1 else {}))
+    return rsnn.simulate(net, x)
+
+
+def _resident_launches_equal_oracle(lanes, D, T, levels):
+    from btorch_amd.models._engine import Engine, match_cell
+    mat, n = _busy_net(D, 81)
+    model, _ = _busy_model(mat, D, n, lanes)
+    x = _drive(levels, lanes, n)
+    ref = _busy_reference(mat, D, n, x)
+    per_step = ref["z"].sum((1, 2))
+    assert torch.equal(per_step, torch.tensor(levels, dtype=per_step.dtype) * lanes)
+    with environ.context(dt=0.1):
+        run = Engine(match_cell(model)).resident(lanes, T)
+    xb = torch.empty((T, lanes, n), device=DEV)
+    run.plan.x, run.plan.x_step_stride = xb.data_ptr(), lanes * n
+    for k in range(len(levels) // T):
+        xb.copy_(x[k * T:(k + 1) * T])
+        run.launch()
+        z = torch.stack([unpack_bits(run.raster[t], n) for t in range(T)])
+        assert bits_equal(z, ref["z"][k * T:(k + 1) * T]), k
+        assert bits_equal(run.v.view(lanes, n), ref["v"][(k + 1) * T - 1]), k
+        assert bits_equal(run.psc.view(lanes, n), ref["psc"][(k + 1) * T - 1]), k
+
+
+def test_resident_launch_pulls_first_what_the_launch_before_pushed():
+    # more than 32 lanes, delays of 0, 1 and 2: activity rises at the third of
+    # four steps, so the last step of the launch pushes and decides that the
+    # next launch's first step pulls, from slots no launch has marked yet
+    _resident_launches_equal_oracle(40, 3, 4, [0, 1, 16, 16] + [16] * 4 + [1] * 4)
