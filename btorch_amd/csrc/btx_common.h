@@ -93,8 +93,8 @@ struct Ctl {
     // the latest decided, that marked
     int lane_bits_mode[4];
     int lane_bits_run;
-    int next_idx;        // batches that pull in a launch of their own: 1 + the index of the
-                         // latest decision in push_mode (0 = none)
+    int next_idx;        // 1 + the index in push_mode and lane_bits_mode of the decisions about
+                         // the step after the last run (0 = none)
     int bin_of_sub[64];  // delay bin by virtual-row offset, -1 = not read
 };
 

@@ -2000,7 +2000,6 @@ __global__ __launch_bounds__(kThreads) void k_pull(PushStep a,
         Ctl* ctl = const_cast<Ctl*>(a.ctl);
         ctl->lane_bits_mode[(a.clock + 1) & 3] = 1;
         ctl->lane_bits_run = 1 << 20;
-        ctl->next_idx = 1 + (int)((a.clock + 1) & 3);
     }
     if (fused && ld_const(&a.ctl->push_mode[(a.clock + 1) & 3]))
         mark_slots(a, ring_words, pull ? ring_slot(a.clock, 0, a.R) : -1);
@@ -2061,10 +2060,14 @@ __global__ __launch_bounds__(kThreads) void k_pull(PushStep a,
     }
 }
 
-// FIN: the last push reduced into the synapse.
-__global__ __launch_bounds__(kThreads) void k_finish(StepArgs a, float* __restrict__ rec) {
+// FIN: the last push reduced into the synapse; `clock` is the step after the
+// run, whose decision the next run takes over (ctl NULL: none is made).
+__global__ __launch_bounds__(kThreads) void k_finish(StepArgs a, float* __restrict__ rec,
+                                                     Ctl* __restrict__ ctl, int64_t clock) {
     __shared__ StepLds lds;
     const int64_t lane = blockIdx.y, seg = blockIdx.x;
+    if (ctl != nullptr && lane == 0 && seg == 0 && threadIdx.x == 0)
+        ctl->next_idx = 1 + (int)(clock & 3);
     float wz[4];
     reduce_segment(a.red, lds.red, a.n, a.nchunks, lane, seg, wz);
     const int64_t n0 = seg * kChunk + threadIdx.x * 4;
@@ -2196,13 +2199,17 @@ __global__ __launch_bounds__(64) void k_set_tables(RunTables t, Ctl* __restrict_
     ctl->bin_delay[k] = arg->bin_delay[k];
     ctl->bin_sub[k] = arg->bin_sub[k];
     ctl->bin_of_sub[k] = arg->bin_of_sub[k];
-    // the last run's decision about the step after it, at the index this
-    // run's clock reads it, and how its last step was delivered (k_mark) at
+    // the last run's decisions about the step after it, at the index this
+    // run's clock reads them, and how its last step was delivered (k_mark) at
     // the one before
     const int next = ctl->next_idx;
     if (next > 0) {
         const int push = ctl->push_mode[(next - 1) & 3], last = ctl->push_mode[(next - 2) & 3];
-        if (k < 4) ctl->push_mode[k] = k == (int)((clock - 1) & 3) ? last : push;
+        const int mark = ctl->lane_bits_mode[(next - 1) & 3];
+        if (k < 4) {
+            ctl->push_mode[k] = k == (int)((clock - 1) & 3) ? last : push;
+            ctl->lane_bits_mode[k] = mark;
+        }
     }
 }
 
@@ -3002,7 +3009,8 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         launch_gather_k(a, ga, s);
     } else {
         hipLaunchKernelGGL(k_finish, dim3((unsigned)nchunks, (unsigned)lanes), dim3(kThreads), 0,
-                           s, a, rec_last);
+                           s, a, rec_last, lane_bits ? ctl : nullptr,
+                           (int64_t)p->ring_cursor + n_steps);
     }
     kt.end(3);
     if (gather && (p->ring_d > 1 || min_delay > 0)) {

@@ -641,3 +641,10 @@ def test_resident_launch_pulls_first_what_the_launch_before_pushed():
     # four steps, so the last step of the launch pushes and decides that the
     # next launch's first step pulls, from slots no launch has marked yet
     _resident_launches_equal_oracle(40, 3, 4, [0, 1, 16, 16] + [16] * 4 + [1] * 4)
+
+
+def test_resident_launches_of_a_length_not_divisible_by_four():
+    # the step after a launch is decided under clock T, the next launch starts
+    # at clock 0: busy steps up to the third of the second launch leave a
+    # decision to pull at index 0, quiet ones after it no lane bits
+    _resident_launches_equal_oracle(4, 2, 6, [16] * 6 + [16, 16, 16, 0, 0, 12] + [3] * 6)
