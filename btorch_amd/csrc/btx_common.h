@@ -94,7 +94,8 @@ struct Ctl {
     int lane_bits_mode[4];
     int lane_bits_run;
     int next_idx;        // 1 + the index in push_mode and lane_bits_mode of the decisions about
-                         // the step after the last run (0 = none)
+                         // the step after the last run; 0 = no run yet, -1 = the last run
+                         // made none (no lane bits given, or it gathered)
     int bin_of_sub[64];  // delay bin by virtual-row offset, -1 = not read
 };
 

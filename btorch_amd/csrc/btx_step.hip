@@ -1860,11 +1860,9 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_step(StepArgs a, Gath
     }
 
     if (g.fin && blockIdx.x == 0 && blockIdx.y == 0 && tid < 4) {
-        // every step was pulled and every slot's lane bits are current; a run
-        // of the other route that follows marks them anew before it pulls
-        // again (its slots are not zeroed ahead)
+        // every step was pulled, none with a decision about the next
         g.ctl->push_mode[tid] = 1;
-        if (tid == 0) g.ctl->lane_bits_run = 0;
+        if (tid == 0) g.ctl->next_idx = -1;
     }
     for (int round = 0; round * kRound < lg; ++round) {
         if (round > 0) request_state(round);
@@ -2060,14 +2058,12 @@ __global__ __launch_bounds__(kThreads) void k_pull(PushStep a,
     }
 }
 
-// FIN: the last push reduced into the synapse; `clock` is the step after the
-// run, whose decision the next run takes over (ctl NULL: none is made).
+// FIN: the last push reduced into the synapse; `next_idx` for the next run.
 __global__ __launch_bounds__(kThreads) void k_finish(StepArgs a, float* __restrict__ rec,
-                                                     Ctl* __restrict__ ctl, int64_t clock) {
+                                                     Ctl* __restrict__ ctl, int next_idx) {
     __shared__ StepLds lds;
     const int64_t lane = blockIdx.y, seg = blockIdx.x;
-    if (ctl != nullptr && lane == 0 && seg == 0 && threadIdx.x == 0)
-        ctl->next_idx = 1 + (int)(clock & 3);
+    if (lane == 0 && seg == 0 && threadIdx.x == 0) ctl->next_idx = next_idx;
     float wz[4];
     reduce_segment(a.red, lds.red, a.n, a.nchunks, lane, seg, wz);
     const int64_t n0 = seg * kChunk + threadIdx.x * 4;
@@ -2210,6 +2206,11 @@ __global__ __launch_bounds__(64) void k_set_tables(RunTables t, Ctl* __restrict_
             ctl->push_mode[k] = k == (int)((clock - 1) & 3) ? last : push;
             ctl->lane_bits_mode[k] = mark;
         }
+    } else if (next < 0) {
+        // the last run decided nothing and kept no lane bits a push step
+        // could go on with: push, and mark every slot anew before a pull
+        if (k < 4) ctl->push_mode[k] = ctl->lane_bits_mode[k] = 0;
+        if (k == 0) ctl->lane_bits_run = 0;
     }
 }
 
@@ -3009,8 +3010,8 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
         launch_gather_k(a, ga, s);
     } else {
         hipLaunchKernelGGL(k_finish, dim3((unsigned)nchunks, (unsigned)lanes), dim3(kThreads), 0,
-                           s, a, rec_last, lane_bits ? ctl : nullptr,
-                           (int64_t)p->ring_cursor + n_steps);
+                           s, a, rec_last, ctl,
+                           lane_bits ? 1 + (int)((p->ring_cursor + n_steps) & 3) : -1);
     }
     kt.end(3);
     if (gather && (p->ring_d > 1 || min_delay > 0)) {

@@ -448,9 +448,12 @@ typedef struct btx_rsnn_plan {
     /* workspace from btx_rsnn_workspace_bytes(), zero-filled once */
     void* workspace;      size_t workspace_bytes;
     /* 1 = the workspace already holds this plan's delay-bin tables (an
-     * earlier run with the same workspace, n, lanes, nnz, ordered, nbins,
-     * bin_delay, bin_sub and the same ring_lane_bits being NULL or not wrote
-     * them), so the run skips writing them; 0 = write them first */
+     * earlier run with the same workspace, neuron_model, syn_kind, n, lanes,
+     * nnz, csr_d, ordered, nbins, bin_delay, bin_sub and the same
+     * ring_lane_bits being NULL or not wrote them), so the run skips writing
+     * them; 0 = write them first, and look at what the last run of the
+     * workspace left: after one without ring_lane_bits the lane bits count as
+     * out of date */
     int tables_ready;
     /* BTX_NEURON_MIXED (MixedNeuronPopulation.single_step_forward,
      * mixed.py:113-141: each group's own step on its range of the axis):

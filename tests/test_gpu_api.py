@@ -648,3 +648,27 @@ def test_resident_launches_of_a_length_not_divisible_by_four():
     # at clock 0: busy steps up to the third of the second launch leave a
     # decision to pull at index 0, quiet ones after it no lane bits
     _resident_launches_equal_oracle(4, 2, 6, [16] * 6 + [16, 16, 16, 0, 0, 12] + [3] * 6)
+
+
+@pytest.mark.parametrize("lanes", [4, 40])
+def test_engine_dense_pull_off_in_between_busy_runs(lanes):
+    # runs with the dense pull on, off and on again continue from the same
+    # ring; the one in between keeps no lane bits, and the last starts where
+    # the first had decided to pull
+    D, T = 3, 8
+    mat, n = _busy_net(D, 82)
+    model, conn = _busy_model(mat, D, n, lanes)
+    x = _drive([16] * (3 * T), lanes, n)
+    ref = _busy_reference(mat, D, n, x)
+    flags = []
+    with environ.context(dt=0.1), torch.no_grad():
+        for k, pull in enumerate((True, False, True)):
+            conn.sparse_config.dense_pull = pull
+            z, st = model(x[k * T:(k + 1) * T].to(DEV))
+            ws = next(iter(model.fused_engine()._ws.values())).view(torch.int32)
+            flags.append(ws[256:260].cpu().tolist())   # Ctl.push_mode of the last launches
+            sl = slice(k * T, (k + 1) * T)
+            assert bits_equal(z, ref["z"][sl]), k
+            assert bits_equal(st["neuron.v"], ref["v"][sl]), k
+            assert bits_equal(st["synapse.psc"], ref["psc"][sl]), k
+    assert sum(flags[0]) and sum(flags[2])
