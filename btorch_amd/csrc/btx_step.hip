@@ -2058,12 +2058,18 @@ __global__ __launch_bounds__(kThreads) void k_pull(PushStep a,
     }
 }
 
-// FIN: the last push reduced into the synapse; `next_idx` for the next run.
+// FIN: the last push reduced into the synapse; `next_idx` for the next run,
+// whose bins have not overflowed (the flags of both buffers, NULL = none).
 __global__ __launch_bounds__(kThreads) void k_finish(StepArgs a, float* __restrict__ rec,
-                                                     Ctl* __restrict__ ctl, int next_idx) {
+                                                     Ctl* __restrict__ ctl, int next_idx,
+                                                     int* __restrict__ over0,
+                                                     int* __restrict__ over1) {
     __shared__ StepLds lds;
     const int64_t lane = blockIdx.y, seg = blockIdx.x;
-    if (lane == 0 && seg == 0 && threadIdx.x == 0) ctl->next_idx = next_idx;
+    if (lane == 0 && seg == 0 && threadIdx.x == 0) {
+        ctl->next_idx = next_idx;
+        if (over0 != nullptr) *over0 = *over1 = 0;
+    }
     float wz[4];
     reduce_segment(a.red, lds.red, a.n, a.nchunks, lane, seg, wz);
     const int64_t n0 = seg * kChunk + threadIdx.x * 4;
@@ -3011,7 +3017,9 @@ static int btx::rsnn_run(const btx_rsnn_plan* p, int64_t n_steps, hipStream_t s,
     } else {
         hipLaunchKernelGGL(k_finish, dim3((unsigned)nchunks, (unsigned)lanes), dim3(kThreads), 0,
                            s, a, rec_last, ctl,
-                           lane_bits ? 1 + (int)((p->ring_cursor + n_steps) & 3) : -1);
+                           lane_bits ? 1 + (int)((p->ring_cursor + n_steps) & 3) : -1,
+                           p->ordered ? ps.bin_cnt - 1 : nullptr,
+                           p->ordered ? other_bins - 1 : nullptr);
     }
     kt.end(3);
     if (gather && (p->ring_d > 1 || min_delay > 0)) {

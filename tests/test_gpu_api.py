@@ -672,3 +672,23 @@ def test_engine_dense_pull_off_in_between_busy_runs(lanes):
             assert bits_equal(st["neuron.v"], ref["v"][sl]), k
             assert bits_equal(st["synapse.psc"], ref["psc"][sl]), k
     assert sum(flags[0]) and sum(flags[2])
+
+
+def test_engine_overflow_of_one_call_ends_with_it():
+    # undelayed, more than 32 lanes, one step per call: a burst overflows the
+    # term bins and that step is pulled; the quiet steps after it push
+    lanes = 70
+    mat, n = _busy_net(1, 83)
+    model, _ = _busy_model(mat, 1, n, lanes)
+    levels = [1, 1, 30, 30] + [1] * 9
+    x = _drive(levels, lanes, n)
+    ref = _busy_reference(mat, 1, n, x)
+    flags = []
+    with environ.context(dt=0.1), torch.no_grad():
+        for t in range(len(levels)):
+            z, st = model(x[t:t + 1].to(DEV))
+            ws = next(iter(model.fused_engine()._ws.values())).view(torch.int32)
+            flags.append(ws[256:260].cpu().tolist())   # Ctl.push_mode of the last launches
+            assert bits_equal(z, ref["z"][t:t + 1]), t
+            assert bits_equal(st["synapse.psc"], ref["psc"][t:t + 1]), t
+    assert sum(flags[2]) and flags[-1] == [0, 0, 0, 0], flags
