@@ -344,7 +344,10 @@ typedef struct btx_rsnn_plan {
                            * (reduced, if at all, by a multiple of 4*(ring_d + 1)) */
     int nbins;            /* delay bins read each step */
     int bin_delay[BTX_MAX_BINS];  /* ring age of bin j (0 = this step) */
-    int bin_sub[BTX_MAX_BINS];    /* virtual-row offset of bin j */
+    int bin_sub[BTX_MAX_BINS];    /* virtual-row offset of bin j; bins may share one in a
+                                   * plan without ring_lane_bits, as long as no bin holds
+                                   * more than 1024 terms and no neuron more than `slots`
+                                   * in a step (what is pulled reads a row at one age) */
     /* destination-major copy of the connectivity (the reference's coalesced
      * (dst, src) order: indices/magnitude); with it the ordered mode reduces
      * a destination with many terms exactly, by pulling its incoming edges */

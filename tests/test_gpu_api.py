@@ -11,7 +11,7 @@ import torch
 
 from btorch_amd import _kernels, workloads
 from btorch_amd.models import (
-    ATan, Erf, ExponentialPSC, HeterSynapsePSC, LIF, RecurrentNN, SparseConn, environ,
+    ATan, DelayedPSC, Erf, ExponentialPSC, HeterSynapsePSC, LIF, RecurrentNN, SparseConn, environ,
     functional,
 )
 from btorch_amd.models._engine import unpack_bits
@@ -692,3 +692,32 @@ def test_engine_overflow_of_one_call_ends_with_it():
             assert bits_equal(z, ref["z"][t:t + 1]), t
             assert bits_equal(st["synapse.psc"], ref["psc"][t:t + 1]), t
     assert sum(flags[2]) and flags[-1] == [0, 0, 0, 0], flags
+
+
+def test_engine_two_delays_of_one_virtual_row():
+    # a plan may read one virtual row at two ages: a neuron then sums the same
+    # row twice where its source spiked in both steps (inputs last four steps,
+    # no refractory period).  Against the net whose edges are there at both delays
+    import scipy.sparse
+    n, lanes, T = 700, 2, 60
+    c = workloads.er_net_fast(n=n, p=0.02, seed=84, w_mu=-4.0)
+    conn = SparseConn(scipy.sparse.coo_array((c.w, (c.pre, c.post)), shape=(n, n)),
+                      sparse_config={"dense_pull": False})
+    model = RecurrentNN(LIF(n, tau_ref=0.1), DelayedPSC(ExponentialPSC(n, 5.0, conn),
+                                                        max_delay_steps=2),
+                        step_mode="m", update_state_names=["neuron.v"]).to(DEV)
+    functional.init_net_state(model, batch_size=lanes, device=DEV, dtype=torch.float32)
+    model.fused_engine().spec.bins = [(1, 0), (2, 0)]
+    g = torch.Generator().manual_seed(84)
+    x = (torch.rand((T // 4, lanes, n), generator=g) < 0.015).float().repeat_interleave(4, 0) * 14.0
+    with environ.context(dt=0.1), torch.no_grad():
+        z, st = model(x.to(DEV))
+    twice = scipy.sparse.coo_array(
+        (np.concatenate([c.w, c.w]), (np.concatenate([c.pre * 3 + 1, c.pre * 3 + 2]),
+                                      np.concatenate([c.post, c.post]))), shape=(3 * n, n))
+    net = rsnn.Net(n, twice, rsnn.LIFParams.make(n, tau_ref=0.1), torch.tensor(5.0), 0.1,
+                   delay_mode="hetero", max_delay_steps=3, circular=True)
+    ref = rsnn.simulate(net, x)
+    terms = _terms_per_bin(ref["z"], twice, n, 3)
+    assert ref["z"].sum() > 500 and 20 < terms.max() <= 1024
+    assert bits_equal(z, ref["z"]) and bits_equal(st["neuron.v"], ref["v"])
