@@ -544,8 +544,9 @@ __global__ __launch_bounds__(256) void k_adj_transpose_wgrad4(
 // power of two) edges are then summed side by side, eight of each in flight,
 // and the PER partial sums added at the end (an edge at a time, one wavefront
 // for 16 lanes: 36 us a step at 4096 neurons, 0.41M edges).  Also the
-// undelayed product of at most 32 lanes (csr_d = 1, age 0, K = 1).
-template <int PER>
+// undelayed product of at most 32 lanes (csr_d = 1, age 0, K = 1).  Row: an
+// integer that holds the rows of G, K*n of them.
+template <int PER, typename Row>
 __global__ __launch_bounds__(256) void k_adj_transpose_rows(
     const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
     const float* __restrict__ w, int64_t n, int csr_d, int64_t lanes,
@@ -579,7 +580,7 @@ __global__ __launch_bounds__(256) void k_adj_transpose_rows(
             const int st = __shfl(step, sub, 64);
             const bool in = e < len && st >= 0;
             // row of G the edge reads, -1 = none
-            const int my_r = in ? (int)(st * n) + col[e0 + e] : -1;
+            const Row my_r = in ? (Row)(st * n) + col[e0 + e] : -1;
             const float my_w = in ? w[e0 + e] : 0.f;
             if (__ballot(in) == 0ull) continue;
             const int m = len - c < 64 ? len - c : 64;
@@ -588,7 +589,7 @@ __global__ __launch_bounds__(256) void k_adj_transpose_rows(
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
                     const int src = k + u * PER + grp;
-                    const int r = __shfl(my_r, src & 63, 64);
+                    const Row r = __shfl(my_r, src & 63, 64);
                     w8[u] = __shfl(my_w, src & 63, 64);
                     const bool use = src < m && r >= 0;
                     g8[u] = use ? gb[(int64_t)r * lanes] : 0.f;
@@ -604,22 +605,35 @@ __global__ __launch_bounds__(256) void k_adj_transpose_rows(
     }
 }
 
+template <typename Row>
+static void launch_transpose_rows_of(const int64_t* rp, const int32_t* col, const float* w,
+                                     int64_t n, int csr_d, int64_t lanes, const float* G, int64_t K,
+                                     int64_t tau, const int* ages, float* g_src, int accumulate,
+                                     hipStream_t s) {
+    const dim3 grid((unsigned)((n + 3) / 4)), block(256);
+    if (lanes > 32)
+        hipLaunchKernelGGL((k_adj_transpose_rows<1, Row>), grid, block, 0, s, rp, col, w, n, csr_d,
+                           lanes, G, K, tau, ages, g_src, accumulate);
+    else if (lanes > 16)
+        hipLaunchKernelGGL((k_adj_transpose_rows<2, Row>), grid, block, 0, s, rp, col, w, n, csr_d,
+                           lanes, G, K, tau, ages, g_src, accumulate);
+    else if (lanes > 8)
+        hipLaunchKernelGGL((k_adj_transpose_rows<4, Row>), grid, block, 0, s, rp, col, w, n, csr_d,
+                           lanes, G, K, tau, ages, g_src, accumulate);
+    else
+        hipLaunchKernelGGL((k_adj_transpose_rows<8, Row>), grid, block, 0, s, rp, col, w, n, csr_d,
+                           lanes, G, K, tau, ages, g_src, accumulate);
+}
+
 static void launch_transpose_rows(const int64_t* rp, const int32_t* col, const float* w, int64_t n,
                                   int csr_d, int64_t lanes, const float* G, int64_t K, int64_t tau,
                                   const int* ages, float* g_src, int accumulate, hipStream_t s) {
-    const dim3 grid((unsigned)((n + 3) / 4)), block(256);
-    if (lanes > 32)
-        hipLaunchKernelGGL(k_adj_transpose_rows<1>, grid, block, 0, s, rp, col, w, n, csr_d, lanes,
-                           G, K, tau, ages, g_src, accumulate);
-    else if (lanes > 16)
-        hipLaunchKernelGGL(k_adj_transpose_rows<2>, grid, block, 0, s, rp, col, w, n, csr_d, lanes,
-                           G, K, tau, ages, g_src, accumulate);
-    else if (lanes > 8)
-        hipLaunchKernelGGL(k_adj_transpose_rows<4>, grid, block, 0, s, rp, col, w, n, csr_d, lanes,
-                           G, K, tau, ages, g_src, accumulate);
+    if (K * n < (int64_t)1 << 31)
+        launch_transpose_rows_of<int>(rp, col, w, n, csr_d, lanes, G, K, tau, ages, g_src,
+                                      accumulate, s);
     else
-        hipLaunchKernelGGL(k_adj_transpose_rows<8>, grid, block, 0, s, rp, col, w, n, csr_d, lanes,
-                           G, K, tau, ages, g_src, accumulate);
+        launch_transpose_rows_of<int64_t>(rp, col, w, n, csr_d, lanes, G, K, tau, ages, g_src,
+                                          accumulate, s);
 }
 
 // gw[e] += sum over lanes b spiking at neuron j (mask bit b) of
@@ -741,8 +755,6 @@ BTX_API int btx_adj_lif_sweep(const btx_adj_lif_args* p, int64_t K, int64_t gz_s
     const bool delayed = ages != nullptr;
     if (delayed && (G == nullptr || csr_d < 1 || csr_d > BTX_MAX_BINS))
         return fail("btx_adj_lif_sweep: delays need G and 1 <= csr_d <= 64");
-    if (delayed && K * p->n >= (int64_t)1 << 31)
-        return fail("btx_adj_lif_sweep: K*n exceeds int32");
     const int64_t m = p->n * p->lanes;
     const hipStream_t st = (hipStream_t)stream;
     const dim3 rows((unsigned)((p->n + 3) / 4));
@@ -806,7 +818,6 @@ BTX_API int btx_adj_transpose_delayed(const int64_t* row_ptr, const int32_t* col
                                       int accumulate, void* stream) {
     if (n <= 0 || lanes <= 0) return 0;
     if (csr_d < 1 || csr_d > BTX_MAX_BINS) return fail("btx_adj_transpose_delayed: bad csr_d");
-    if (K * n >= (int64_t)1 << 31) return fail("btx_adj_transpose_delayed: K*n exceeds int32");
     launch_transpose_rows(row_ptr, col, w, n, csr_d, lanes, G, K, tau, ages, g_src, accumulate,
                           (hipStream_t)stream);
     return check_launch("btx_adj_transpose_delayed");

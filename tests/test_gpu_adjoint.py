@@ -451,3 +451,31 @@ def test_adjoint_sweep_lane_counts_match_reference_autograd(n, B, D, shared_tau)
 def test_adjoint_sweep_lanes_by_fours_match_reference_autograd(n, B):
     # 33 to 64 lanes: four lanes a thread where they divide by four, else one
     test_adjoint_sweep_lane_counts_match_reference_autograd(n, B, 1, False)
+
+
+def test_transpose_delayed_over_more_than_int32_rows():
+    # K * n past int32: the rows of dL/dpsc that the last steps read
+    from btorch_amd import _lib
+    n, K, D = 1 << 20, 2049, 2
+    G = torch.empty(K * n, device=DEV)
+    G[-2 * n:] = torch.randn(2 * n, generator=torch.Generator().manual_seed(1)).to(DEV)
+    deg = torch.zeros(n * D, dtype=torch.int64)
+    deg[[10, 11, 2 * n - 1]] = torch.tensor([3, 2, 70])   # neurons 5 (ages 0, 1) and n - 1 (age 1)
+    rp = torch.cat([torch.zeros(1, dtype=torch.int64), deg.cumsum(0)])
+    g = torch.Generator().manual_seed(2)
+    col = torch.randint(0, n, (75,), generator=g).to(torch.int32)
+    w = torch.randn(75, generator=g)
+    ages = torch.tensor([0, 1], dtype=torch.int32, device=DEV)
+    out = torch.full((n,), -1.0, device=DEV)
+    dev = [t.to(DEV) for t in (rp, col, w)]
+    _lib.check(_lib.load().btx_adj_transpose_delayed(
+        *(t.data_ptr() for t in dev), n, D, 1, G.data_ptr(), K, K - 2, ages.data_ptr(),
+        out.data_ptr(), 0, _lib.stream_ptr()), "btx_adj_transpose_delayed")
+    last = G[-2 * n:].cpu().double().view(2, n)
+    want = torch.zeros(n, dtype=torch.float64)
+    terms = [(5, 0, slice(0, 3)), (5, 1, slice(3, 5)), (n - 1, 1, slice(5, 75))]
+    for j, age, sl in terms:
+        want[j] += (w[sl].double() * last[age][col[sl].long()]).sum()
+    # at most 70 products: a float32 sum is within 72 * 2^-24 of their magnitudes
+    assert ((out.cpu().double() - want).abs() <= 72 * 2.0**-24 * 70 * 12.0).all()
+    assert want[5] != 0 and want[n - 1] != 0 and not out[:5].any()
