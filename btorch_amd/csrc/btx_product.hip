@@ -92,11 +92,15 @@ __global__ __launch_bounds__(1024) void k_row_counts(const float* __restrict__ x
 // current ones are added, and a few rows are split into tiles over the CUs.
 // 0.4 to 0.65 us a source of 163 to 819 edges (one source ahead, 1024 values at
 // a time and whole rows: 0.8 to 1.9 us).  Taken back: three requests in flight
-// (74 VGPRs, one workgroup per CU: 512 rows 15% slower), 256 threads.
+// (74 VGPRs, one workgroup per CU: 512 rows 15% slower), 256 threads.  Edge:
+// an integer that holds the edges' positions (64 bits leave room for one
+// workgroup per CU where 16,384 destinations are tiled).
+template <typename Edge>
 __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int tile) {
     constexpr int T = kRowThreads;
     extern __shared__ __align__(16) float s_y[];
-    __shared__ int s_beg[T], s_len[T];
+    __shared__ Edge s_beg[T];
+    __shared__ int s_len[T];
     __shared__ float s_x[T];
     __shared__ int s_cnt[T / 64];
     constexpr int U = 8;
@@ -136,7 +140,7 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
             off += __popcll((unsigned long long)m);
             if (on && p >= 0 && p < T) {
                 const int64_t beg = a.row_ptr[s1 + 64 * u];
-                s_beg[p] = (int)beg;
+                s_beg[p] = (Edge)beg;
                 s_len[p] = (int)(a.row_ptr[s1 + 64 * u + 1] - beg);
                 s_x[p] = xv[u];
             }
@@ -149,7 +153,7 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const bool in = k0 + u < total && tid < s_len[k0 + u];
-                const int e = in ? s_beg[k0 + u] + tid : 0;
+                const Edge e = in ? s_beg[k0 + u] + tid : 0;
                 d[u] = in ? a.col[e] : -1;
                 pm[u] = in ? a.perm[e] : 0;
             }
@@ -172,7 +176,7 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
                 const int len = s_len[k0 + u];
                 if (d[u] >= 0) s_y[d[u]] = fmaf(w[u], xk, s_y[d[u]]);
                 for (int t = tid + T; t < len; t += T) {
-                    const int e = s_beg[k0 + u] + t;
+                    const Edge e = s_beg[k0 + u] + t;
                     const int64_t q = a.col[e] - d0;
                     if (q >= 0 && q < nd) s_y[q] = fmaf(a.w[a.perm[e]], xk, s_y[q]);
                 }
@@ -490,10 +494,10 @@ static int row_tile(int64_t rows, int64_t n_dst) {
     return (int)(tile < n_dst ? tile : n_dst);
 }
 
-static int check_product(const char* who, int64_t n_src, int64_t n_dst, int64_t nnz, int64_t rows,
+static int check_product(const char* who, int64_t n_src, int64_t n_dst, int64_t rows,
                          const void* scratch) {
-    if (n_src >= (int64_t)1 << 31 || n_dst >= (int64_t)1 << 31 || nnz >= (int64_t)1 << 31)
-        return fail(std::string(who) + ": sources, destinations and edges must fit int32");
+    if (n_src >= (int64_t)1 << 31 || n_dst >= (int64_t)1 << 31)
+        return fail(std::string(who) + ": sources and destinations must fit int32");
     if (rows > 65535) return fail(std::string(who) + ": rows exceeds 65535");
     if (((uintptr_t)scratch & 15) != 0) return fail(std::string(who) + ": scratch is not 16-byte aligned");
     return 0;
@@ -513,7 +517,7 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
                         int64_t x_row_stride, int64_t rows, float* y, void* scratch,
                         size_t scratch_bytes, void* stream) {
     if (rows <= 0 || n_dst <= 0) return 0;
-    if (int rc = check_product("btx_product", n_src, n_dst, nnz, rows, scratch)) return rc;
+    if (int rc = check_product("btx_product", n_src, n_dst, rows, scratch)) return rc;
     if (scratch_bytes < btx_product_scratch_bytes(rows, n_src) ||
         (scratch == nullptr && scratch_bytes > 0))
         return fail("btx_product: scratch too small");
@@ -543,7 +547,8 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
     }
     const int tile = row_tile(rows, n_dst);
     const dim3 grid((unsigned)rows, (unsigned)((n_dst + tile - 1) / tile));
-    hipLaunchKernelGGL(k_product_rows, grid, dim3(kRowThreads), 4 * (size_t)(tile + 3), s, a, tile);
+    hipLaunchKernelGGL(nnz < (int64_t)1 << 31 ? k_product_rows<int> : k_product_rows<int64_t>, grid,
+                       dim3(kRowThreads), 4 * (size_t)(tile + 3), s, a, tile);
     if (n_src > kFewSources) {
         const int64_t tiles = (n_dst + 15) / 16;
         hipLaunchKernelGGL(k_product_columns, dim3((unsigned)(tiles < 2048 ? tiles : 2048)),
@@ -562,7 +567,7 @@ BTX_API int btx_product_grad(const int64_t* row_ptr, const int32_t* col, const i
                              int64_t x_row_stride, int64_t rows, const float* gy, float* gx,
                              float* gw, void* scratch, size_t scratch_bytes, void* stream) {
     if (rows <= 0 || n_src <= 0 || n_dst <= 0) return 0;
-    if (int rc = check_product("btx_product_grad", n_src, n_dst, nnz, rows, scratch)) return rc;
+    if (int rc = check_product("btx_product_grad", n_src, n_dst, rows, scratch)) return rc;
     if (scratch == nullptr || scratch_bytes < grad_scratch(rows, n_src, n_dst))
         return fail("btx_product_grad: scratch too small");
     const hipStream_t s = (hipStream_t)stream;

@@ -116,7 +116,7 @@ int btx_spmv_event(const int64_t* row_ptr, const int32_t* col, const float* w,
  * for 64 rows at a time.  w is in the destination-major order of csc_src (the
  * layer's parameter order), perm[k] the position there of CSR edge k; no term
  * is stored, so the scratch (btx_product_scratch_bytes, 16-byte aligned, not
- * initialised) does not grow with the outputs.  rows <= 65535, nnz < 2^31. */
+ * initialised) does not grow with the outputs.  rows <= 65535. */
 size_t btx_product_scratch_bytes(int64_t rows, int64_t n_src);
 int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_t* perm,
                 const int64_t* csc_ptr, const int32_t* csc_src, const float* w, int64_t n_src,
