@@ -213,13 +213,14 @@ def unpack_rows(words: torch.Tensor, n: int, out: torch.Tensor | None = None) ->
     return out
 
 
-def _product_operands(layout: CsrLayout, w: torch.Tensor, x2d: torch.Tensor) -> None:
+def _product_operands(layout: CsrLayout, w: torch.Tensor | None, x2d: torch.Tensor) -> None:
     _lib.require_hip(x2d, w)
     if x2d.dim() != 2 or x2d.shape[1] != layout.n_src or not x2d.is_contiguous():
         raise ValueError("operand shapes do not match the connection layout")
-    if layout.csc_ptr is None or w.numel() != layout.nnz or not w.is_contiguous():
+    if layout.csc_ptr is None or (w is not None and (w.numel() != layout.nnz
+                                                     or not w.is_contiguous())):
         raise ValueError("destination-major arrays missing or mismatched")
-    if w.dtype != torch.float32 or x2d.dtype != torch.float32:
+    if x2d.dtype != torch.float32 or (w is not None and w.dtype != torch.float32):
         raise TypeError("the event-driven product supports float32 only")
 
 
@@ -241,11 +242,13 @@ def product(layout: CsrLayout, w: torch.Tensor, x2d: torch.Tensor) -> torch.Tens
     return out
 
 
-def product_grad(layout: CsrLayout, w: torch.Tensor, x2d: torch.Tensor, g: torch.Tensor,
+def product_grad(layout: CsrLayout, w: torch.Tensor | None, x2d: torch.Tensor, g: torch.Tensor,
                  need_x: bool, need_w: bool):
     """(gx, gw) of ``product`` for the output gradient ``g``; gw in the order
-    of ``w``; None for one that is not needed."""
+    of ``w`` (read for gx only); None for one that is not needed."""
     _product_operands(layout, w, x2d)
+    if need_x and w is None:
+        raise ValueError("the input's gradient needs the weights")
     g = g.to(torch.float32).contiguous()
     rows = x2d.shape[0]
     if g.shape != (rows, layout.n_dst):
@@ -261,7 +264,7 @@ def product_grad(layout: CsrLayout, w: torch.Tensor, x2d: torch.Tensor, g: torch
     ptr = (lambda t: None if t is None else t.data_ptr())
     _lib.check(lib.btx_product_grad(layout.row_ptr.data_ptr(), layout.col.data_ptr(),
                                     layout.perm.data_ptr(), layout.csc_ptr.data_ptr(),
-                                    layout.csc_src.data_ptr(), w.data_ptr(), layout.n_src,
+                                    layout.csc_src.data_ptr(), ptr(w), layout.n_src,
                                     layout.n_dst, layout.nnz, x2d.data_ptr(), layout.n_src, rows,
                                     g.data_ptr(), ptr(gx), ptr(gw),
                                     scratch.data_ptr() if nbytes else None, nbytes,

@@ -350,7 +350,7 @@ class Engine:
                  int(cfg.ordered), int(cfg.slots), int(getattr(cfg, "bin_cap", 0)),
                  self.dense_pull(),
                  id(conn._csr_row_ptr), id(conn._csc_ptr), conn.weight_key(),
-                 id(conn._prepared_sparse_weight)]
+                 _tkey(conn._prepared_sparse_weight)]
         mods = (sp.neuron.modules() if isinstance(sp.neuron, MixedState) else [sp.neuron])
         for m in (*mods, sp.exp_psc):
             d = m.__dict__

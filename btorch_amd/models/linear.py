@@ -55,14 +55,16 @@ class _SparseProduct(torch.autograd.Function):
         if weight.dtype != torch.float32:
             raise TypeError("the event-driven product supports float32 only")
         ctx.conn = conn
-        ctx.save_for_backward(x2d, weight)
+        # the weights are read for the input's gradient alone
+        ctx.save_for_backward(x2d, weight if ctx.needs_input_grad[0] else None)
         return _kernels.product(conn._layout, weight.detach().contiguous(), x2d)
 
     @staticmethod
     def backward(ctx, g):
         x2d, weight = ctx.saved_tensors
-        gx, gw = _kernels.product_grad(ctx.conn._layout, weight.detach().contiguous(), x2d, g,
-                                       ctx.needs_input_grad[0], ctx.needs_input_grad[1])
+        gx, gw = _kernels.product_grad(ctx.conn._layout,
+                                       None if weight is None else weight.detach().contiguous(),
+                                       x2d, g, ctx.needs_input_grad[0], ctx.needs_input_grad[1])
         return gx, gw, None
 
 
@@ -77,9 +79,7 @@ class BaseSparseConn(nn.Module):
         self.sparse_config = btorch_config.sparse.resolve(self.sparse_backend, sparse_config)
         self._prepared_sparse_weight: torch.Tensor | None = None
         self._sparse_prepare_depth = 0
-        # effective weights of a prepared run, (dst, src) order, as a 1-tuple (a
-        # Parameter assigned as it is would register a second time)
-        self._prepared_weight: tuple[torch.Tensor] | None = None
+        self._prepared_packed: torch.Tensor | None = None
         # no-grad packed (CSR order) and destination-order weights, reused
         # while the tensors they derive from are unchanged (weight_key)
         self._weight_cache: dict[str, tuple] = {}
@@ -151,7 +151,7 @@ class BaseSparseConn(nn.Module):
         return int(self.indices.shape[1])
 
     def _apply(self, fn, recurse=True):
-        self._prepared_sparse_weight = self._prepared_weight = None
+        self._prepared_sparse_weight = self._prepared_packed = None
         self._sparse_prepare_depth = 0
         self._weight_cache = {}
         return super()._apply(fn, recurse=recurse)
@@ -160,7 +160,7 @@ class BaseSparseConn(nn.Module):
                               unexpected_keys, error_msgs):
         super()._load_from_state_dict(state_dict, prefix, local_metadata, strict, missing_keys,
                                       unexpected_keys, error_msgs)
-        self._prepared_sparse_weight = self._prepared_weight = None
+        self._prepared_sparse_weight = self._prepared_packed = None
         self._sparse_prepare_depth = 0
         self._weight_cache = {}
         self._rebuild_layout()
@@ -204,8 +204,18 @@ class BaseSparseConn(nn.Module):
         self._weight_cache[kind] = (key, w)
         return w
 
+    def _weight_snapshot(self) -> torch.Tensor:
+        """The effective weights as they are now: edits in place of the
+        parameters and buffers that follow do not reach them."""
+        w = self._get_effective_weight()
+        held = {t.untyped_storage().data_ptr()
+                for t in (*self._parameters.values(), *self._buffers.values()) if t is not None}
+        return w.clone() if w.untyped_storage().data_ptr() in held else w
+
     def effective_weight_f32(self) -> torch.Tensor:
         """Detached float32 effective weights in the coalesced (dst, src) order."""
+        if self._prepared_sparse_weight is not None:
+            return self._prepared_sparse_weight.detach().to(torch.float32).contiguous()
         return self._cached_weight(
             "dst", lambda: self._get_effective_weight().detach().to(torch.float32).contiguous())
 
@@ -219,16 +229,20 @@ class BaseSparseConn(nn.Module):
 
     def packed_weight(self) -> torch.Tensor:
         """Effective weights in CSR order (``magnitude[perm]``)."""
-        if self._prepared_sparse_weight is not None:
-            return self._prepared_sparse_weight
-        return self._pack()
+        w = self._prepared_sparse_weight
+        if w is None:
+            return self._pack()
+        if self._prepared_packed is None:
+            with torch.set_grad_enabled(w.requires_grad):
+                self._prepared_packed = w.index_select(0, self._csr_perm).contiguous()
+        return self._prepared_packed
 
     def prepare_sparse(self, batch_size: int | None = None) -> None:
-        """Evaluate and pack the weights once for a multi-step run
-        (reference-counted)."""
+        """Evaluate the weights once for a multi-step run (reference-counted)."""
         if self._prepared_sparse_weight is None:
-            self._prepared_sparse_weight = self._pack()
-            self._prepared_weight = (self._get_effective_weight(),)
+            self._prepared_sparse_weight = (
+                self._weight_snapshot() if torch.is_grad_enabled()
+                else self._cached_weight("snapshot", self._weight_snapshot))
         self._sparse_prepare_depth += 1
 
     def finish_sparse(self) -> None:
@@ -236,7 +250,7 @@ class BaseSparseConn(nn.Module):
             raise RuntimeError("finish_sparse called without prepare_sparse.")
         self._sparse_prepare_depth -= 1
         if self._sparse_prepare_depth == 0:
-            self._prepared_sparse_weight = self._prepared_weight = None
+            self._prepared_sparse_weight = self._prepared_packed = None
 
     def get_sparse_matrix(self) -> torch.Tensor:
         idx = torch.stack([self.indices[1], self.indices[0]], dim=0)
@@ -255,11 +269,14 @@ class BaseSparseConn(nn.Module):
         if x2d.dtype != torch.float32:
             raise TypeError("The HIP sparse backend currently supports float32 only.")
         x2d = x2d.contiguous()
-        if self._prepared_weight is not None:
-            weight = self._prepared_weight[0]
+        if self._prepared_sparse_weight is not None:
+            weight = self._prepared_sparse_weight
+        elif not torch.is_grad_enabled():
+            weight = self._cached_weight("effective", self._get_effective_weight)
         else:
-            weight = (self._get_effective_weight() if torch.is_grad_enabled()
-                      else self._cached_weight("effective", self._get_effective_weight))
+            # the backward may come after an edit in place of the weights
+            weight = (self._weight_snapshot() if x2d.requires_grad
+                      else self._get_effective_weight())
         out = _SparseProduct.apply(x2d, weight, self)
         out = out.reshape(*lead, self.out_features)
         if no_batch:

@@ -104,3 +104,48 @@ def test_product_of_edges_past_int32():
                                w.data_ptr(), 2, n_dst, first + 5, x.data_ptr(), 2, 1, y.data_ptr(),
                                None, 0, _lib.stream_ptr()), "btx_product")
     assert y.cpu().tolist() == [[-3.75, 2.0, 0.0, 0.0, 12.5, 0.0, 8.0, 0.0]]
+
+
+def test_gradients_use_the_weights_of_the_forward():
+    # the weights are edited in place between forward and backward, as by an
+    # optimiser step for another loss of the same layer
+    mat = _matrix(300, 400, 40, 9)
+    rng = np.random.default_rng(10)
+    x = torch.from_numpy(((rng.random((6, 300)) < 0.3) * 1.0).astype(np.float32)).to(DEV)
+    g = torch.from_numpy(rng.standard_normal((6, 400)).astype(np.float32)).to(DEV)
+    conn = SparseConn(mat, enforce_dale=False, device=DEV)
+
+    def grads(edit):
+        xd = x.clone().requires_grad_(True)
+        conn.magnitude.grad = None
+        y = conn(xd)
+        if edit:
+            with torch.no_grad():
+                conn.magnitude.mul_(3.0)
+        y.backward(g)
+        return xd.grad, conn.magnitude.grad
+
+    want, got = grads(False), grads(True)
+    assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
+
+
+def test_prepared_weights_stay_those_of_prepare():
+    mat = _matrix(300, 400, 40, 9)
+    x = torch.ones(2, 300, device=DEV)
+    conn = SparseConn(mat, enforce_dale=False, device=DEV)
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            before, packed = conn(x).detach(), conn.packed_weight().detach().clone()
+            conn.prepare_sparse()
+            with torch.no_grad():
+                conn.magnitude.mul_(2.0)
+            assert torch.equal(conn(x).detach(), before)
+            assert torch.equal(conn.packed_weight().detach(), packed)
+            assert torch.equal(conn.effective_weight_f32()[conn._csr_perm], packed)
+            conn.finish_sparse()
+            assert torch.equal(conn(x).detach(), 2 * before)
+    conn.magnitude.grad = None
+    conn.prepare_sparse()
+    (conn(x) + conn(x)).sum().backward()
+    conn.finish_sparse()
+    assert torch.equal(conn.magnitude.grad, torch.full_like(conn.magnitude, 4.0))
