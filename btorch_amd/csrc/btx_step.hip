@@ -1563,10 +1563,14 @@ constexpr int gather_lanes(int mode) { return mode == kGatherOne ? 1 : mode == k
 // acc += the weights of a chunk's active edges (thread k of the wavefront
 // holds edge k's weight w and its source's lane bits), in edge order, in the
 // threads whose lane has the edge's bit.  `on`: the edges with any bit.  Up
-// to eight such edges are taken one by one, more in blocks of eight with
+// to eight such edges are taken one by one, more in blocks of four with
 // fixed lane numbers (a third of the instructions per edge).  The lane bits
-// become the execution mask of the add.  Every thread of the wavefront is
-// active when it is called, and on return.
+// become the execution mask of the add, within the mask it is called with
+// (all of the wavefront: a block reads the lane bits of its four edges from
+// their threads).  A value that an instruction of the vector unit wrote to a
+// scalar register (v_readlane) is read by the next such instruction two wait
+// states later: the compiler sees to that outside of the assembly, and here
+// two scalar instructions, or one and an s_nop, come before the first add.
 __device__ __forceinline__ void add_lanes(float& acc, float w, uint64_t word, uint64_t on) {
     const int wi = __float_as_int(w), lo = (int)(uint32_t)word, hi = (int)(uint32_t)(word >> 32);
     if (__popcll((unsigned long long)on) <= 8) {
@@ -1576,11 +1580,14 @@ __device__ __forceinline__ void add_lanes(float& acc, float w, uint64_t word, ui
             const uint32_t mh = (uint32_t)__builtin_amdgcn_readlane(hi, k);
             const int wk = __builtin_amdgcn_readlane(wi, k);
             const uint64_t m = ((uint64_t)mh << 32) | ml;
-            asm("s_mov_b64 exec, %1\n\t"
-                "v_add_f32 %0, %2, %0\n\t"
-                "s_mov_b64 exec, -1"
-                : "+v"(acc)
-                : "s"(m), "s"(wk));
+            uint64_t all;
+            asm("s_and_saveexec_b64 %1, %2\n\t"
+                "s_nop 0\n\t"
+                "v_add_f32 %0, %3, %0\n\t"
+                "s_mov_b64 exec, %1"
+                : "+v"(acc), "=&s"(all)
+                : "s"(m), "s"(wk)
+                : "scc");
             on &= on - 1ull;
         }
         return;
@@ -1597,18 +1604,21 @@ __device__ __forceinline__ void add_lanes(float& acc, float w, uint64_t word, ui
             m[k] = ((uint64_t)mh << 32) | ml;
             wk[k] = __builtin_amdgcn_readlane(wi, k0 + k);
         }
-        asm("s_mov_b64 exec, %1\n\t"
-            "v_add_f32 %0, %5, %0\n\t"
-            "s_mov_b64 exec, %2\n\t"
+        uint64_t all;
+        asm("s_mov_b64 %1, exec\n\t"
+            "s_and_b64 exec, %1, %2\n\t"
             "v_add_f32 %0, %6, %0\n\t"
-            "s_mov_b64 exec, %3\n\t"
+            "s_and_b64 exec, %1, %3\n\t"
             "v_add_f32 %0, %7, %0\n\t"
-            "s_mov_b64 exec, %4\n\t"
+            "s_and_b64 exec, %1, %4\n\t"
             "v_add_f32 %0, %8, %0\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(acc)
+            "s_and_b64 exec, %1, %5\n\t"
+            "v_add_f32 %0, %9, %0\n\t"
+            "s_mov_b64 exec, %1"
+            : "+v"(acc), "=&s"(all)
             : "s"(m[0]), "s"(m[1]), "s"(m[2]), "s"(m[3]), "s"(wk[0]), "s"(wk[1]), "s"(wk[2]),
-              "s"(wk[3]));
+              "s"(wk[3])
+            : "scc");
     }
 }
 

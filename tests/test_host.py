@@ -509,3 +509,33 @@ def test_mixed_plan_lays_parameters_out_per_neuron():
     assert p.tau_stride == 1 and p.tc_stride[0] == 1
     asc_k = read(p.asc_k, 24)
     assert asc_k[-8:] == pytest.approx([0.1, 0.2] * 4) and asc_k[:16] == [0.0] * 16
+
+
+def test_inline_assembly_of_the_step_keeps_the_mask_and_the_wait_states():
+    # every block that writes the execution mask saves it and puts it back, and
+    # its first vector instruction comes two wait states after the block's
+    # start (the compiler may have just written the scalar registers it reads)
+    import re
+    from pathlib import Path
+
+    import btorch_amd
+
+    text = (Path(btorch_amd.__file__).parent / "csrc" / "btx_step.hip").read_text()
+    blocks = [re.findall(r'"([^"]*)"', m.group(1).split("\n                : ")[0]
+                         .split("\n            : ")[0])
+              for m in re.finditer(r"\basm(?: volatile)?\((.*?)\);", text, re.S)]
+    blocks = [[ins.replace("\\n\\t", "").split() for ins in b] for b in blocks]
+    masked = [b for b in blocks if any("exec" in t for ins in b for t in ins)]
+    assert len(masked) == 2
+    for b in masked:
+        assert b[0] in (["s_mov_b64", "%1,", "exec"], ["s_and_saveexec_b64", "%1,", "%2"])
+        assert b[-1] == ["s_mov_b64", "exec,", "%1"]
+        waits = 0
+        for ins in b:
+            if ins[0].startswith("v_"):
+                break
+            waits += 1 + (int(ins[1]) if ins[0] == "s_nop" else 0)
+        assert waits >= 2, b
+        # later masks lie within the saved one
+        assert all(ins[:2] + ins[2:3] == ["s_and_b64", "exec,", "%1,"]
+                   for ins in b[1:-1] if "exec," in ins)
