@@ -84,7 +84,7 @@ __global__ __launch_bounds__(1024) void k_row_counts(const float* __restrict__ x
     if (threadIdx.x == 0) counts[row] = total;
 }
 
-// One row of x, destinations [d0, d0 + tile): 8192 of the row's values are
+// One row of x, destinations [d0, d0 + tile): 1024 V of the row's values are
 // read at a time and their nonzeros listed in LDS in ascending order, each
 // with its row of W.  Bound by the misses one CU can have in flight on a
 // source's weights, which perm scatters over the array, and by the barrier per
@@ -94,8 +94,10 @@ __global__ __launch_bounds__(1024) void k_row_counts(const float* __restrict__ x
 // a time and whole rows: 0.8 to 1.9 us).  Taken back: three requests in flight
 // (74 VGPRs, one workgroup per CU: 512 rows 15% slower), 256 threads.  Edge:
 // an integer that holds the edges' positions (64 bits leave room for one
-// workgroup per CU where 16,384 destinations are tiled).
-template <typename Edge>
+// workgroup per CU where 16,384 destinations are tiled).  V = 1 where a row has
+// no more than 1024 values: 200 x 16,384, 12,800 rows, 5 active sources each,
+// 0.383 ms; 0.411 with seven of eight reads and ballots per thread wasted.
+template <typename Edge, int V>
 __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int tile) {
     constexpr int T = kRowThreads;
     extern __shared__ __align__(16) float s_y[];
@@ -111,15 +113,15 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
     for (int q = tid; q < (nd + 3) / 4; q += T)
         reinterpret_cast<float4*>(s_y)[q] = make_float4(0.f, 0.f, 0.f, 0.f);
     const float* xr = a.x + row * a.x_stride;
-    for (int64_t s0 = 0; s0 < a.n_src; s0 += T * U) {
-      // a wavefront reads 512 consecutive values
-      const int64_t s1 = s0 + wv * 64 * U + ln;
-      float xv[U];
+    for (int64_t s0 = 0; s0 < a.n_src; s0 += T * V) {
+      // a wavefront reads 64 V consecutive values
+      const int64_t s1 = s0 + wv * 64 * V + ln;
+      float xv[V];
 #pragma unroll
-      for (int u = 0; u < U; ++u) xv[u] = s1 + 64 * u < a.n_src ? xr[s1 + 64 * u] : 0.f;
+      for (int u = 0; u < V; ++u) xv[u] = s1 + 64 * u < a.n_src ? xr[s1 + 64 * u] : 0.f;
       int mine = 0;
 #pragma unroll
-      for (int u = 0; u < U; ++u) mine += __popcll((unsigned long long)__ballot(xv[u] != 0.f));
+      for (int u = 0; u < V; ++u) mine += __popcll((unsigned long long)__ballot(xv[u] != 0.f));
       if (ln == 0) s_cnt[wv] = mine;
       __syncthreads();
       int first = 0, nonzero = 0;
@@ -133,7 +135,7 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
         const int total = nonzero - base < T ? nonzero - base : T;
         int off = first - base;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
+        for (int u = 0; u < V; ++u) {
             const bool on = xv[u] != 0.f;
             const uint64_t m = __ballot(on);
             const int p = off + __popcll((unsigned long long)(m & ((1ull << ln) - 1ull)));
@@ -547,8 +549,10 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
     }
     const int tile = row_tile(rows, n_dst);
     const dim3 grid((unsigned)rows, (unsigned)((n_dst + tile - 1) / tile));
-    hipLaunchKernelGGL(nnz < (int64_t)1 << 31 ? k_product_rows<int> : k_product_rows<int64_t>, grid,
-                       dim3(kRowThreads), 4 * (size_t)(tile + 3), s, a, tile);
+    const bool narrow = nnz < (int64_t)1 << 31, one = n_src <= kRowThreads;
+    hipLaunchKernelGGL(narrow ? (one ? k_product_rows<int, 1> : k_product_rows<int, 8>)
+                              : (one ? k_product_rows<int64_t, 1> : k_product_rows<int64_t, 8>),
+                       grid, dim3(kRowThreads), 4 * (size_t)(tile + 3), s, a, tile);
     if (n_src > kFewSources) {
         const int64_t tiles = (n_dst + 15) / 16;
         hipLaunchKernelGGL(k_product_columns, dim3((unsigned)(tiles < 2048 ? tiles : 2048)),

@@ -85,25 +85,30 @@ def test_products_of_few_rows_match_sequential_sums(n_src, n_dst, degree, rows, 
     assert torch.equal(y, rsnn.NativeSparse(mat)(x))
 
 
-def test_product_of_edges_past_int32():
+@pytest.mark.parametrize("n_src,rows", [(2, 1), (1030, 2)])
+def test_product_of_edges_past_int32(n_src, rows):
     # 2^31 edges and more: row offsets past int32 (the arrays are as long, only
-    # the last few edges of them are read)
+    # the last few edges of them, of the last two sources, are read), for rows
+    # of x read 1024 and 8192 values at a time
     from btorch_amd import _lib
     first, n_dst = 2**31 + 5, 8
-    row_ptr = torch.tensor([first, first + 3, first + 5], dtype=torch.int64, device=DEV)
+    row_ptr = torch.full((n_src + 1,), first, dtype=torch.int64, device=DEV)
+    row_ptr[-2:] += torch.tensor([3, 5], device=DEV)
     col = torch.empty(first + 5, dtype=torch.int32, device=DEV)
     perm = torch.empty(first + 5, dtype=torch.int64, device=DEV)
     col[first:] = torch.tensor([1, 4, 6, 0, 4], dtype=torch.int32, device=DEV)
     perm[first:] = torch.tensor([2, 0, 4, 1, 3], device=DEV)
     w = torch.tensor([0.5, -1.25, 2.0, 4.0, 8.0], device=DEV)
-    x = torch.tensor([[1.0, 3.0]], device=DEV)
-    y = torch.empty((1, n_dst), device=DEV)
+    x = torch.zeros((rows, n_src), device=DEV)
+    x[:, -2:] = torch.tensor([1.0, 3.0], device=DEV)
+    y = torch.empty((rows, n_dst), device=DEV)
     lib = _lib.load()
-    assert lib.btx_product_scratch_bytes(1, 2) == 0
+    scratch = torch.empty(lib.btx_product_scratch_bytes(rows, n_src), dtype=torch.uint8, device=DEV)
     _lib.check(lib.btx_product(row_ptr.data_ptr(), col.data_ptr(), perm.data_ptr(), None, None,
-                               w.data_ptr(), 2, n_dst, first + 5, x.data_ptr(), 2, 1, y.data_ptr(),
-                               None, 0, _lib.stream_ptr()), "btx_product")
-    assert y.cpu().tolist() == [[-3.75, 2.0, 0.0, 0.0, 12.5, 0.0, 8.0, 0.0]]
+                               w.data_ptr(), n_src, n_dst, first + 5, x.data_ptr(), n_src, rows,
+                               y.data_ptr(), scratch.data_ptr() if scratch.numel() else None,
+                               scratch.numel(), _lib.stream_ptr()), "btx_product")
+    assert y.cpu().tolist() == [[-3.75, 2.0, 0.0, 0.0, 12.5, 0.0, 8.0, 0.0]] * rows
 
 
 def test_gradients_use_the_weights_of_the_forward():
