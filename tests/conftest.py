@@ -28,3 +28,13 @@ def _announce(request):
     if "gpu" in request.keywords:
         print(f"\n[gpu-case] {request.node.nodeid}", flush=True)
     yield
+
+
+@pytest.fixture
+def pushed(monkeypatch):
+    """Connections made in the test push every step into the term bins, as the
+    steps of a net too large to gather do."""
+    from btorch_amd import config
+
+    for name in config.sparse.names():
+        monkeypatch.setattr(config.sparse._configs[name], "dense_pull", False)

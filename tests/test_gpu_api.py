@@ -721,3 +721,7 @@ def test_engine_two_delays_of_one_virtual_row():
     terms = _terms_per_bin(ref["z"], twice, n, 3)
     assert ref["z"].sum() > 500 and 20 < terms.max() <= 1024
     assert bits_equal(z, ref["z"]) and bits_equal(st["neuron.v"], ref["v"])
+
+
+def test_engine_mixed_population_pushed(pushed):
+    test_mixed_population_glif3_two_compartment_lif_in_fused_step()

@@ -322,3 +322,20 @@ def test_engine_constrained_conn_forward_and_group_gradient():
     (zr * R).sum().backward()
     a, b = sc.magnitude.grad.double().cpu(), mag.grad.double()
     assert float((a - b).norm() / b.norm()) < 1e-4
+
+
+# the same cells with every step pushed into the term bins
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n", [700, 703])
+def test_engine_lif_kinetics_pushed(kind, n, pushed):
+    test_engine_lif_kinetics_bit_exact(kind, n)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_engine_hetero_delays_kinetics_pushed(kind, pushed):
+    test_engine_hetero_delays_kinetics_bit_exact(kind)
+
+
+def test_engine_glif3_dual_exponential_delayed_pushed(pushed):
+    test_engine_glif3_dual_exponential_delayed_bit_exact()

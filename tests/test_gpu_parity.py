@@ -711,3 +711,29 @@ def test_sparse_conn_matches_committed_sparse_mm_fixture():
     with torch.no_grad():
         out = conn(torch.from_numpy(g["x"]).to(DEV)).cpu().numpy()
     assert np.array_equal(out.view(np.uint32), g["out"].view(np.uint32))
+
+
+# cells of nets small enough to gather, with every step pushed into the term bins
+
+@pytest.mark.parametrize("hard,n", [(False, 700), (True, 700), (False, 703)])
+def test_engine_heterogeneous_params_pushed(hard, n, pushed):
+    test_engine_heterogeneous_params_bit_exact(hard, n)
+
+
+@pytest.mark.parametrize("circular", [True, False])
+def test_engine_hetero_delays_pushed(circular, pushed):
+    test_engine_hetero_delays_bit_exact(circular)
+
+
+def test_engine_delayed_psc_pushed(pushed):
+    test_engine_delayed_psc_bit_exact()
+
+
+@pytest.mark.parametrize("n", [600, 703])
+def test_engine_glif3_hetero_delays_pushed(n, pushed):
+    test_engine_glif3_hetero_delays_bit_exact(n)
+
+
+@pytest.mark.parametrize("n", [600, 703])
+def test_engine_two_compartment_apical_pushed(n, pushed):
+    test_engine_two_compartment_apical_bit_exact(n)
