@@ -2658,6 +2658,24 @@ static void launch_gather_k(const StepArgs& a, const GatherArgs& g, hipStream_t 
 //   two-compartment, 8 delays, 1.2M edges, 8 lanes        13.0 / 13.8
 // An active net widens the gap (0.33M edges at 0.9 %: 26.9 / 7.5; 3.6M at
 // 1 %: 50 / 11.8).
+// A wavefront of the wide gather takes a lane per thread, its stores and the
+// bits of 64 lanes: 3 to 6 us more than up to 16 lanes, where a push between
+// delayed synapses is one launch of 9 (11 above 32 lanes, with the pull's).
+// Quiet LIF nets, then at 0.5 %, push / gather in us per step:
+//   8 delays, 1000 neurons, 0.05M edges, 17 lanes    8.9 / 10.4   11.3 / 11.2
+//   8 delays, 1000 neurons, 0.05M edges, 64 lanes   11.3 / 14.9   15.9 / 17.7
+//   8 delays, 4096 neurons, 0.33M edges, 32 lanes    8.7 / 12.0   12.7 / 14.6
+//   no delays, 4096 neurons, 0.33M edges, 64 lanes  18.6 / 16.1   24.1 / 20.4
+//   no delays, 4096 neurons, 0.84M edges, 128 lanes 21.6 / 19.8   45.6 / 28.3
+//   no delays, 10000 neurons, 1.2M edges, 64 lanes  21.9 / 22.2   34.9 / 31.3
+//   no delays, 10000 neurons, 1.2M edges, 128 lanes 25.4 / 31.6   48.8 / 41.8
+//   GLIF3 + alpha, 8 delays, 1.2M edges, 17 lanes   22.3 / 18.4
+//   GLIF3 + alpha, 8 delays, 1.2M edges, 128 lanes  48.1 / 39.4
+//   two-compartment, 8 delays, 0.33M edges, 64 lanes 15.5 / 18.6
+// So delayed nets of more than 16 lanes, and others of more than 64, are held
+// against what was measured there (17 to 256 lanes, 300 to 16,384 neurons):
+// the gather's time follows the edges per neuron and the workgroups of the
+// fullest CU, both follow the neuron states.
 static bool gather_route(const btx_rsnn_plan* p, bool fused) {
     if (!p->ordered || p->ring_lane_bits == nullptr || p->lanes > 65535) return false;
     for (int j = 0; j < p->nbins; ++j)
@@ -2667,6 +2685,23 @@ static bool gather_route(const btx_rsnn_plan* p, bool fused) {
     const double edges = 1e-6 * (double)p->nnz;
     const int lg = gather_lanes(p->lanes <= 16 ? kGatherFew : kGatherWide);
     const double groups = (double)((p->lanes + lg - 1) / lg);
+    if (p->lanes > (fused ? 16 : 64)) {
+        const double g = p->lanes < 64 ? (double)p->lanes : 64.0;
+        const double states = 1e-6 * (double)(p->n * p->lanes);
+        const double per_cu = (double)p->n * groups / (kGatherNeurons * 256.0);
+        const double degree = (double)p->nnz / (double)p->n;
+        const double gather = 8.0 + 0.1 * g +
+                              degree * (0.0105 + 0.0002 * g + (p->csr_d > 1 ? 0.004 : 0.0)) *
+                                  (1.6 * ceil(per_cu) - 0.6) +
+                              (per_cu > 1.0 ? 2.4 * (per_cu - 1.0) * g / 64.0 : 0.0);
+        const double kind = p->neuron_model == BTX_NEURON_LIF                ? 0.0
+                            : p->neuron_model == BTX_NEURON_TWO_COMPARTMENT ? 1.5
+                                                                             : 3.0 + 7.0 * states;
+        const double push = (fused ? 8.8 : 14.5 + 0.3 * edges) + (p->lanes > 32 ? 2.6 : 0.0) +
+                            7.0 * states + kind +
+                            (p->syn_kind == BTX_SYN_EXP ? 0.0 : 1.5 + 3.0 * states);
+        return gather < push;
+    }
     const double gather = 7.5 + edges * (p->lanes == 1 ? 1.2 : (p->csr_d > 1 ? 4.6 : 2.6) * groups);
     const double kind = p->neuron_model == BTX_NEURON_LIF                ? 0.0
                         : p->neuron_model == BTX_NEURON_TWO_COMPARTMENT ? 3.4

@@ -339,3 +339,25 @@ def test_engine_hetero_delays_kinetics_pushed(kind, pushed):
 
 def test_engine_glif3_dual_exponential_delayed_pushed(pushed):
     test_engine_glif3_dual_exponential_delayed_bit_exact()
+
+
+@pytest.mark.parametrize("B", [17, 70])
+def test_engine_wide_delayed_gather_bit_exact(B):
+    # more than 16 lanes with delays: GLIF3 cells with alpha synapses gather
+    # (lanes in groups of 64, the last one ragged), where LIF cells push
+    n, T, D = 203, 60, 6
+    rng = np.random.default_rng(7)
+    tau = torch.from_numpy(rng.uniform(10.0, 30.0, n).astype(np.float32))
+    kw = dict(v_threshold=-50.0, v_reset=-70.0, c_m=0.05, tau=tau, k=[0.3, 0.02],
+              asc_amps=[-0.6, 0.9], tau_ref=2.0)
+    model, conn, _, x, z, st, prefix, net_kw = _engine_case(
+        "alpha", GLIF3(n, **kw), n, B, T, 71, wrap="hetero", D=D)
+    ws = next(iter(model.fused_engine()._ws.values())).view(torch.int32)
+    assert ws[256:260].tolist() == [1, 1, 1, 1]   # Ctl.push_mode: a run that gathered
+    osyn = rsnn.AlphaSyn(torch.tensor(5.0), torch.tensor(1.3))
+    ref = rsnn.simulate(_oracle_net(rsnn.GLIF3Params.make(n, **kw), n, conn, osyn, 0.1,
+                                    **net_kw), x)
+    assert ref["z"].sum() > 50
+    assert bits_equal(z, ref["z"]) and bits_equal(st["neuron.v"], ref["v"])
+    assert bits_equal(st[prefix + "psc"], ref["psc"]) and bits_equal(st[prefix + "h"], ref["h"])
+    assert bits_equal(model.neuron.Iasc, ref["final"]["iasc"])

@@ -180,24 +180,31 @@ def test_serving_alpha_synapse_alone_vs_mix_bit_exact():
 
 
 def test_serving_wide_pool_low_lanes_end_first():
-    # a pool of more than 16 lanes on a net small enough to gather: the job on
-    # the low lanes ends while the one above them runs (a thread of the step
-    # integrates lanes b, b + 16, ...), then another takes the low lanes; every
-    # job equals the same job alone, and the long one the oracle
-    n, D = 400, 5
-    model, cexp = _model(n, D, 31)
-    chunk = 4 * (D + 1)
+    # a pool of more than 16 lanes on an undelayed net small enough to gather:
+    # the job on the low lanes ends while the one above them runs (a thread of
+    # the step integrates lanes b, b + 16, ...), then another takes the low
+    # lanes; every job equals the same job alone, and the long one the oracle
+    n = 400
+    mat = workloads.plain_lif_net(n=n, p=0.05, seed=31).matrix()
+    model = RecurrentNN(LIF(n, tau_ref=2.0), ExponentialPSC(n, 5.0, SparseConn(mat)),
+                        step_mode="m").to(DEV)
     kw = dict(n_sample=5, base_rate_hz=1500.0, kick=12.0)
     reqs = [SimRequest(0, T=15, batch=17, seed=3), SimRequest(1, T=80, batch=20, seed=4),
             SimRequest(2, T=31, batch=16, seed=5)]
-    pool = LanePool(model, lanes=40, chunk=chunk, **kw)
+    pool = LanePool(model, lanes=40, chunk=24, **kw)
     got = {r.rid: r for r in Server(pool).serve(reqs, realtime=False).results}
     assert sorted(got) == [0, 1, 2]
-    alone = run_plain(lambda req: LanePool(model, lanes=req.batch, chunk=chunk, **kw), reqs)
+    assert pool.run.ws.view(torch.int32)[256:260].tolist() == [1, 1, 1, 1]  # every step gathered
+    alone = run_plain(lambda req: LanePool(model, lanes=req.batch, chunk=24, **kw), reqs)
     for r in alone.results:
         assert torch.equal(r.counts, got[r.rid].counts), r.rid
         assert torch.equal(r.traces, got[r.rid].traces), r.rid
-    counts, traces = _oracle_job(n, D, cexp, reqs[1], pool)
-    assert int(counts.sum()) > 100
-    assert torch.equal(got[1].counts.cpu(), counts)
-    assert torch.equal(got[1].traces.cpu(), traces)
+    req = reqs[1]
+    seeds = (int(req.seed) * 1_000_003 + np.arange(req.batch)) & 0x7FFFFFFFFFFFFFFF
+    x = rsnn.poisson_drive(seeds, np.full(req.batch, np.float32(pool.base_p)),
+                           np.zeros(req.batch, np.int64), req.T, n, pool.kick)
+    ref = rsnn.simulate(rsnn.Net(n, mat, rsnn.LIFParams.make(n, tau_ref=2.0), torch.tensor(5.0),
+                                 DT), x)
+    assert int(ref["z"].sum()) > 100
+    assert torch.equal(got[1].counts.cpu(), ref["z"].sum(0).to(torch.int32))
+    assert torch.equal(got[1].traces.cpu(), ref["v"][:, :, :5])
