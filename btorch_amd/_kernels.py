@@ -303,21 +303,6 @@ def spmv_event(layout: CsrLayout, w_csr: torch.Tensor, x2d: torch.Tensor, active
     return out
 
 
-def spmv_transpose(layout: CsrLayout, w_csr: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
-    """gx (lanes, n_src) = g @ W^T."""
-    _lib.require_hip(g, w_csr)
-    g = g.contiguous()
-    if g.shape[1] != layout.n_dst:
-        raise ValueError("gradient width does not match n_dst")
-    lanes = g.shape[0]
-    gx = torch.empty((lanes, layout.n_src), dtype=torch.float32, device=g.device)
-    _lib.check(_lib.load().btx_spmv_transpose(layout.row_ptr.data_ptr(), layout.col.data_ptr(),
-                                              w_csr.data_ptr(), layout.n_src, layout.n_dst,
-                                              g.data_ptr(), lanes, gx.data_ptr(),
-                                              _lib.stream_ptr()), "btx_spmv_transpose")
-    return gx
-
-
 def spmv_weight_grad(layout: CsrLayout, x2d: torch.Tensor | None, active: torch.Tensor,
                      counts: torch.Tensor, g: torch.Tensor, gw_csr: torch.Tensor) -> None:
     """gw_csr += event-driven sum over active (lane, source) of x * g[:, col]."""

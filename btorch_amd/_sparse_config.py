@@ -3,7 +3,8 @@
 Same registry interface as btorch/_sparse_config.py:55-113
 (``backend(name)``, ``selected``, ``resolve(name, override)``).  There is one
 compute backend, the HIP event-driven product; the reference's backend names
-select its accumulation mode so existing configurations keep working:
+select the recurrent engine's accumulation mode so existing configurations
+keep working:
 
   "hip"     HipSparseConfig()               ascending-source, bit-exact
   "native"  HipSparseConfig(ordered=True)   same sums as torch.sparse.mm on CPU
@@ -26,9 +27,11 @@ class SparseBackendConfig:
 class HipSparseConfig(SparseBackendConfig):
     """Event-driven HIP product settings.
 
-    ordered: sum each destination's terms in ascending source order (bit-exact
-        against the CPU reference); False uses float atomics.
-    slots: per-destination terms the ordered mode sorts (2..16); a
+    ordered: let the recurrent engine sum each destination's terms in
+        ascending source order (bit-exact against the CPU reference); False
+        uses float atomics.  A layer called by itself sums in that order
+        either way.
+    slots: per-destination terms the engine's ordered mode sorts (2..16); a
         destination with more terms in one step is reduced by pulling its
         incoming edges (exact, slower for that destination).
     bin_cap: terms per (lane, 1024-destination segment) bin of the recurrent

@@ -421,9 +421,9 @@ __global__ __launch_bounds__(256) void k_product_grad_x(const int64_t* __restric
 }
 
 // gw of the layer, destination-major: gw[e] = sum over rows b of x[b, src[e]] *
-// gy[b, dst].  A workgroup takes one destination, whose gradients over the
-// rows sit in LDS, and a thread per edge that reads the source's row bits:
-// only rows with x != 0 are added, in ascending order, group by group.
+// gy[b, dst].  A wavefront takes one destination, whose gradients over 64 rows
+// sit in LDS, and a thread an edge whose source's row bits it reads: only rows
+// with x != 0 are added, in ascending order, group by group.
 __global__ __launch_bounds__(256) void k_product_grad_w(const int64_t* __restrict__ csc_ptr,
                                                         const int32_t* __restrict__ csc_src,
                                                         int64_t n_src, int64_t n_dst, int64_t rows,

@@ -25,7 +25,7 @@ import torch.nn as nn
 
 from .. import _kernels, _lib
 from .. import config as btorch_config
-from .._sparse_config import HipSparseConfig, SparseBackendConfig
+from .._sparse_config import SparseBackendConfig
 
 
 def _resolve_sparse_backend(name: str | None) -> str:

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from btorch_amd import workloads
+from btorch_amd import _kernels, workloads
 from btorch_amd.models import (
     LIF, ExponentialPSC, RecurrentNN, Sigmoid, SparseConn, SuperSpike, environ, functional,
 )
@@ -479,3 +479,70 @@ def test_transpose_delayed_over_more_than_int32_rows():
     # at most 70 products: a float32 sum is within 72 * 2^-24 of their magnitudes
     assert ((out.cpu().double() - want).abs() <= 72 * 2.0**-24 * 70 * 12.0).all()
     assert want[5] != 0 and want[n - 1] != 0 and not out[:5].any()
+
+
+def test_neuron_major_chunk_equals_the_lane_major_sweep():
+    # the C entry of the neuron-major sweep against the one the module calls,
+    # on the same values: the same kernels but for the elementwise step, whose
+    # dL/dtau sums in another order (5 lanes: 8 * 2^-24 of the magnitudes)
+    import ctypes
+
+    from btorch_amd import _lib
+    n, B, K = 70, 5, 4
+    c = workloads.er_net_fast(n=n, p=0.2, seed=3)
+    conn = SparseConn(c.matrix()).to(DEV)
+    lay, w = conn._layout, conn.packed_weight().detach()
+    g = torch.Generator().manual_seed(4)
+    v_prev, v_pre, gz = (torch.randn(K, B, n, generator=g) for _ in range(3))
+    z = (torch.rand(K, B, n, generator=g) < 0.3).float()
+    ref = torch.randint(0, 2, (K, B, n), generator=g).float()
+    gv, gpsc = torch.randn(B, n, generator=g), torch.randn(n, B, generator=g)
+    masks = _kernels.lane_masks(_kernels.pack_rows(z.to(DEV).view(K * B, n)).view(K, B, -1), n)
+    one = {k: torch.tensor([v], device=DEV) for k, v in
+           dict(tau=15.0, v_th=1.0, v_reset=0.0, c_m=1.0, tau_syn=5.0, k_syn=0.1).items()}
+
+    def sweep(lane_major):
+        put = (lambda t: (t if lane_major else t.transpose(-1, -2)).to(DEV).contiguous())
+        arr = {k: put(t) for k, t in dict(v_prev=v_prev, v_pre=v_pre, z=z, ref_prev=ref, gz=gz,
+                                          gv=gv).items()}
+        arr.update(gpsc=gpsc.to(DEV), gsyn=torch.empty(n, B, device=DEV),
+                   gx=torch.empty_like(arr["z"]), gtau=torch.zeros(1, device=DEV))
+        a = _lib.AdjLifArgs()
+        a.n, a.lanes, a.dt, a.surrogate = n, B, 0.1, _lib.SURR_SUPERSPIKE
+        a.alpha, a.damping, a.lane_major = 20.0, 1.0, int(lane_major)
+        for k, t in {**one, **arr}.items():
+            setattr(a, k, t.data_ptr())
+        gw = torch.zeros(conn.nnz, device=DEV)
+        head, net = (ctypes.byref(a), K), (lay.row_ptr.data_ptr(), lay.col.data_ptr(), w.data_ptr())
+        tail = (masks.data_ptr(), gw.data_ptr(), _lib.stream_ptr())
+        lib = _lib.load()
+        if lane_major:
+            rc = lib.btx_adj_lif_sweep(*head, B * n, None, *net, 1, None, None, *tail)
+        else:
+            rc = lib.btx_adj_lif_chunk(*head, *net, *tail)
+        _lib.check(rc, "sweep")
+        back = (lambda t: t if lane_major else t.transpose(-1, -2))
+        return back(arr["gx"]), back(arr["gv"]), arr["gpsc"], gw, arr["gtau"]
+
+    got, want = sweep(False), sweep(True)
+    for a, b in zip(got[:4], want[:4]):
+        assert torch.equal(a, b) and float(a.abs().sum()) > 0
+    assert rel_err(got[4], want[4]) < 1e-4
+
+
+def test_csr_ordered_transposed_product_matches_float64():
+    # the C entry for weights in CSR order (the layer's own runs btx_product_grad)
+    from btorch_amd import _lib
+    n, lanes = 150, 3
+    c = workloads.er_net_fast(n=n, p=0.1, seed=6)
+    conn = SparseConn(c.matrix()).to(DEV)
+    lay, w = conn._layout, conn.packed_weight().detach()
+    g = torch.randn(lanes, n, generator=torch.Generator().manual_seed(1))
+    gd, gx = g.to(DEV), torch.empty(lanes, n, device=DEV)
+    _lib.check(_lib.load().btx_spmv_transpose(lay.row_ptr.data_ptr(), lay.col.data_ptr(),
+                                              w.data_ptr(), n, n, gd.data_ptr(), lanes,
+                                              gx.data_ptr(), _lib.stream_ptr()),
+               "btx_spmv_transpose")
+    W = torch.from_numpy(c.matrix().toarray().astype(np.float64))
+    bound = (g.double().abs() @ W.abs().t()) * (n + 2) * 2.0**-24   # n products at most
+    assert ((gx.cpu().double() - g.double() @ W.t()).abs() <= bound).all()
