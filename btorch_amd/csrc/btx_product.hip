@@ -20,6 +20,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "../../include/btorch_amd.h"
 #include "btx_common.h"
 
@@ -29,7 +31,6 @@ constexpr int kRowTile = 16384;      // destinations of a `rows` workgroup, at m
 constexpr int kRowThreads = 1024;
 constexpr int kGroup = 64;           // rows of x per wavefront of the `columns` form
 constexpr int64_t kFewRows = 4;      // up to which k_product_few takes them
-constexpr int64_t kFewSources = 1024;  // up to which the `rows` form is taken unasked
 
 struct ProductArgs {
     const int64_t* row_ptr;
@@ -45,43 +46,46 @@ struct ProductArgs {
     int64_t x_stride;
     int64_t rows;
     float* y;             // (rows, n_dst)
-    const int32_t* counts;  // nonzeros of each row, NULL = take the `rows` form
     float* xt;            // [groups][n_src][64]
+    int32_t* counts;      // nonzeros of each row
+    int32_t* by_columns;  // [groups] 1 = left to the columns; NULL = the `rows` form takes all
+    int most;             // nonzeros a row, on average of a group, up to which the `rows`
+                          // form takes the group
 };
 
-// Which form the 64 rows of group g take.  Measured on MI355X (16,384 x 16,384
-// of 13.4M edges, 4,000 x 8,000 of 1.6M, 21,739 x 21,739 of 3.5M; 1 to 512
-// rows): rows 0.8 ns per edge of an active source, at least 0.4 us a source,
-// 0.3 ns per source looked at, 110 rows at a time; columns 10 to 24 us per
-// million edges and group.  Sides at 64 rows of the first net: 328 active
-// sources 254 us by rows and 174 us by columns, 82 of them 97 and 174 us.
+// Whether the `rows` form takes the 64 rows of group g (decided for the group: a
+// form's cost is the same for one of its rows as for all); every thread of the
+// wavefront calls it.
 __device__ __forceinline__ bool group_by_rows(const ProductArgs& a, int64_t g) {
-    if (a.counts == nullptr) return true;
-    const int ln = threadIdx.x & 63;
-    const int64_t row = g * kGroup + ln;
-    int c = row < a.rows ? a.counts[row] : 0;
+    const int64_t row = g * kGroup + (threadIdx.x & 63);
+    int64_t c = row < a.rows ? a.counts[row] : 0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
     const int64_t here = a.rows - g * kGroup < kGroup ? a.rows - g * kGroup : kGroup;
-    const float waves = a.rows > 110 ? (float)a.rows / 110.f : 1.f;
-    const float len = (float)a.nnz / (float)a.n_src;
-    const float source_us = fmaxf(0.4f, 0.8e-3f * len);
-    const float rows_us = waves * (0.3e-3f * (float)a.n_src + source_us * (float)c / (float)here);
-    const float cols_us = 8.f + 14e-6f * (float)a.nnz * (float)((a.rows + kGroup - 1) / kGroup);
-    return rows_us < cols_us;
+    return c <= a.most * here;
 }
 
-// Nonzeros of every row (one workgroup per row).
-__global__ __launch_bounds__(1024) void k_row_counts(const float* __restrict__ x, int64_t n,
-                                                    int64_t stride, int32_t* __restrict__ counts) {
-    const int64_t row = blockIdx.x;
+// Nonzeros of every row: THREADS threads a row, of a workgroup of 256 or 1024.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS < 256 ? 256 : THREADS) void k_row_counts(
+    const float* __restrict__ x, int64_t n, int64_t stride, int64_t rows,
+    int32_t* __restrict__ counts) {
+    constexpr int BLOCK = THREADS < 256 ? 256 : THREADS;
+    const int64_t row = (int64_t)blockIdx.x * (BLOCK / THREADS) + threadIdx.x / THREADS;
+    if (THREADS == 64 && row >= rows) return;
     const float* xr = x + row * stride;
     int c = 0;
 #pragma unroll 8
-    for (int64_t i = threadIdx.x; i < n; i += 1024) c += xr[i] != 0.f;
+    for (int64_t i = threadIdx.x % THREADS; i < n; i += THREADS) c += xr[i] != 0.f;
     int total;
-    block_excl_scan<16>(c, total);
-    if (threadIdx.x == 0) counts[row] = total;
+    if (THREADS == 64) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+        total = c;
+    } else {
+        block_excl_scan<BLOCK / 64>(c, total);
+    }
+    if (threadIdx.x % THREADS == 0) counts[row] = total;
 }
 
 // One row of x, destinations [d0, d0 + tile): 1024 V of the row's values are
@@ -109,16 +113,17 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
     const int tid = threadIdx.x, wv = tid >> 6, ln = tid & 63;
     const int64_t row = blockIdx.x, d0 = (int64_t)blockIdx.y * tile;
     const int nd = (int)(a.n_dst - d0 < tile ? a.n_dst - d0 : tile);
-    if (!group_by_rows(a, row / kGroup)) return;
+    const float* xr = a.x + row * a.x_stride;
+    const int left = a.by_columns != nullptr ? a.by_columns[row / kGroup] : 0;
     for (int q = tid; q < (nd + 3) / 4; q += T)
         reinterpret_cast<float4*>(s_y)[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-    const float* xr = a.x + row * a.x_stride;
     for (int64_t s0 = 0; s0 < a.n_src; s0 += T * V) {
       // a wavefront reads 64 V consecutive values
       const int64_t s1 = s0 + wv * 64 * V + ln;
       float xv[V];
 #pragma unroll
       for (int u = 0; u < V; ++u) xv[u] = s1 + 64 * u < a.n_src ? xr[s1 + 64 * u] : 0.f;
+      if (left) return;  // uniform; asked for beside the first values
       int mine = 0;
 #pragma unroll
       for (int u = 0; u < V; ++u) mine += __popcll((unsigned long long)__ballot(xv[u] != 0.f));
@@ -210,7 +215,11 @@ __global__ __launch_bounds__(256) void k_group_rows(ProductArgs a, const float* 
                                                     float* __restrict__ out) {
     __shared__ float t[64][65];
     const int64_t g = blockIdx.y, i0 = (int64_t)blockIdx.x * 64;
-    if (a.counts != nullptr && group_by_rows(a, g)) return;
+    if (a.by_columns != nullptr) {
+        const bool taken = !group_by_rows(a, g);
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.by_columns[g] = taken;
+        if (!taken) return;
+    }
     const int ln = threadIdx.x & 63;
     for (int b = threadIdx.x >> 6; b < 64; b += 4) {
         const int64_t row = g * kGroup + b, i = i0 + ln;
@@ -241,71 +250,81 @@ __global__ __launch_bounds__(256) void k_ungroup_rows(const float* __restrict__ 
 // by the gathered rows of x out of L2: 183 us for 13.4M edges and 64 rows,
 // 19 TB/s (a wavefront per destination, a row a thread: four times the
 // requests and their scalar address work, 264 us; without the bound of four
-// wavefronts per SIMD 135 registers leave three: 223 us).
+// wavefronts per SIMD 135 registers leave three: 223 us).  Tiles and groups are
+// shared out together: 100 destinations of 16,384 sources, 1000 rows 2.8 -> 0.23
+// ms (a group at a time left all but seven workgroups idle), by when an edge
+// takes its quarter 0.1 us (32 requests in flight instead of eight: 10% less).
 __global__ __launch_bounds__(256, 4) void k_product_columns(ProductArgs a) {
     __shared__ float s_out[16][65];
     const int tid = threadIdx.x, ln = tid & 63, c16 = ln & 15;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t groups = (a.rows + kGroup - 1) / kGroup;
     const int64_t tiles = (a.n_dst + 15) / 16;
-    for (int64_t g = 0; g < groups; ++g) {
-        if (group_by_rows(a, g)) continue;
-        const float* xg = a.xt + g * a.n_src * kGroup;
-        for (int64_t tl = blockIdx.x; tl < tiles; tl += gridDim.x) {
-            // a quarter of the wavefront per destination, four rows per thread
-            const int q = wv * 4 + (ln >> 4);
-            const int64_t d = tl * 16 + q;
-            const int64_t e0 = d < a.n_dst ? a.csc_ptr[d] : 0;
-            const int len = d < a.n_dst ? (int)(a.csc_ptr[d + 1] - e0) : 0;
-            int most = len;
+    int64_t first = blockIdx.x;  // this workgroup's first tile of the next group it is to take
+    for (int64_t g0 = 0; g0 < groups; g0 += 64) {
+        uint64_t todo = __ballot(g0 + ln < groups && a.by_columns[g0 + ln] != 0);
+        while (todo) {
+            const int64_t g = g0 + __ffsll((unsigned long long)todo) - 1;
+            todo &= todo - 1ull;
+            const float* xg = a.xt + g * a.n_src * kGroup;
+            int64_t tl = first;
+            for (; tl < tiles; tl += gridDim.x) {
+                // a quarter of the wavefront per destination, four rows per thread
+                const int q = wv * 4 + (ln >> 4);
+                const int64_t d = tl * 16 + q;
+                const int64_t e0 = d < a.n_dst ? a.csc_ptr[d] : 0;
+                const int len = d < a.n_dst ? (int)(a.csc_ptr[d + 1] - e0) : 0;
+                int most = len;
 #pragma unroll
-            for (int o = 16; o < 64; o <<= 1) {
-                const int other = __shfl_xor(most, o, 64);
-                most = other > most ? other : most;
-            }
-            most = __builtin_amdgcn_readfirstlane(most);
-            float acc[4] = {0.f, 0.f, 0.f, 0.f};
-            int my_s = c16 < len ? a.csc_src[e0 + c16] : 0;
-            float my_w = c16 < len ? a.w[e0 + c16] : 0.f;
-            for (int c = 0; c < most; c += 16) {
-                // the destination's next 16 edges
-                const int nx = c + 16 + c16;
-                const int next_s = nx < len ? a.csc_src[e0 + nx] : 0;
-                const float next_w = nx < len ? a.w[e0 + nx] : 0.f;
+                for (int o = 16; o < 64; o <<= 1) {
+                    const int other = __shfl_xor(most, o, 64);
+                    most = other > most ? other : most;
+                }
+                most = __builtin_amdgcn_readfirstlane(most);
+                float acc[4] = {0.f, 0.f, 0.f, 0.f};
+                int my_s = c16 < len ? a.csc_src[e0 + c16] : 0;
+                float my_w = c16 < len ? a.w[e0 + c16] : 0.f;
+                for (int c = 0; c < most; c += 16) {
+                    // the destination's next 16 edges
+                    const int nx = c + 16 + c16;
+                    const int next_s = nx < len ? a.csc_src[e0 + nx] : 0;
+                    const float next_w = nx < len ? a.w[e0 + nx] : 0.f;
 #pragma unroll
-                for (int h = 0; h < 16; h += 8) {
-                    float4 x8[8];
+                    for (int h = 0; h < 16; h += 8) {
+                        float4 x8[8];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        const int src = __shfl(my_s, (ln & 48) + h + u, 64);
-                        x8[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                        if (c + h + u < len)
-                            x8[u] = *reinterpret_cast<const float4*>(xg + ((int64_t)src * kGroup + 4 * c16));
-                    }
+                        for (int u = 0; u < 8; ++u) {
+                            const int src = __shfl(my_s, (ln & 48) + h + u, 64);
+                            x8[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+                            if (c + h + u < len)
+                                x8[u] = *reinterpret_cast<const float4*>(xg + ((int64_t)src * kGroup + 4 * c16));
+                        }
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        const float wk = __shfl(my_w, (ln & 48) + h + u, 64);
-                        const float x4[4] = {x8[u].x, x8[u].y, x8[u].z, x8[u].w};
+                        for (int u = 0; u < 8; ++u) {
+                            const float wk = __shfl(my_w, (ln & 48) + h + u, 64);
+                            const float x4[4] = {x8[u].x, x8[u].y, x8[u].z, x8[u].w};
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float t = fmaf(wk, x4[i], acc[i]);
-                            acc[i] = x4[i] != 0.f ? t : acc[i];
+                            for (int i = 0; i < 4; ++i) {
+                                const float t = fmaf(wk, x4[i], acc[i]);
+                                acc[i] = x4[i] != 0.f ? t : acc[i];
+                            }
                         }
                     }
+                    my_s = next_s;
+                    my_w = next_w;
                 }
-                my_s = next_s;
-                my_w = next_w;
-            }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s_out[q][4 * c16 + i] = acc[i];
-            __syncthreads();
-            // 16 destinations of 64 rows: a 64-byte run per row
-            for (int k = tid; k < 16 * kGroup; k += 256) {
-                const int b = k >> 4, q = k & 15;
-                const int64_t row = g * kGroup + b, d = tl * 16 + q;
-                if (row < a.rows && d < a.n_dst) a.y[row * a.n_dst + d] = s_out[q][b];
+                for (int i = 0; i < 4; ++i) s_out[q][4 * c16 + i] = acc[i];
+                __syncthreads();
+                // 16 destinations of 64 rows: a 64-byte run per row
+                for (int k = tid; k < 16 * kGroup; k += 256) {
+                    const int b = k >> 4, q = k & 15;
+                    const int64_t row = g * kGroup + b, d = tl * 16 + q;
+                    if (row < a.rows && d < a.n_dst) a.y[row * a.n_dst + d] = s_out[q][b];
+                }
+                __syncthreads();
             }
-            __syncthreads();
+            first = tl - tiles;
         }
     }
 }
@@ -421,9 +440,11 @@ __global__ __launch_bounds__(256) void k_product_grad_x(const int64_t* __restric
 }
 
 // gw of the layer, destination-major: gw[e] = sum over rows b of x[b, src[e]] *
-// gy[b, dst].  A wavefront takes one destination, whose gradients over 64 rows
-// sit in LDS, and a thread an edge whose source's row bits it reads: only rows
-// with x != 0 are added, in ascending order, group by group.
+// gy[b, dst].  A wavefront takes every gridDim.y-th 64 edges of a destination,
+// whose gradients over 64 rows sit in LDS, and a thread an edge whose source's
+// row bits it reads: only rows with x != 0 are added, in ascending order, group
+// by group (a wavefront a destination: 16,384 x 100, 5000 rows, 30 % active, the
+// whole backward 22 ms; so: 3.2).
 __global__ __launch_bounds__(256) void k_product_grad_w(const int64_t* __restrict__ csc_ptr,
                                                         const int32_t* __restrict__ csc_src,
                                                         int64_t n_src, int64_t n_dst, int64_t rows,
@@ -437,14 +458,15 @@ __global__ __launch_bounds__(256) void k_product_grad_w(const int64_t* __restric
     const int64_t d = (int64_t)blockIdx.x * 4 + wv;
     const int ln = threadIdx.x & 63;
     if (d >= n_dst) return;
-    const int64_t e0 = csc_ptr[d], e1 = csc_ptr[d + 1];
-    const int64_t groups = (rows + kGroup - 1) / kGroup;
+    const int64_t e0 = csc_ptr[d] + 64 * (int64_t)blockIdx.y, e1 = csc_ptr[d + 1];
+    if (e0 >= e1) return;
+    const int64_t groups = (rows + kGroup - 1) / kGroup, step = 64 * (int64_t)gridDim.y;
     for (int64_t g = 0; g < groups; ++g) {
         s_g[wv][ln] = gt[(g * n_dst + d) * kGroup + ln];
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (int64_t e = e0 + ln; e < e1; e += 64) {
+        for (int64_t e = e0 + ln; e < e1; e += step) {
             const int s = csc_src[e];
             uint64_t m = bits[g * n_src + s];
             float acc = 0.f;
@@ -476,9 +498,8 @@ __global__ __launch_bounds__(256) void k_row_bits(const float* __restrict__ x, i
 }
 
 static size_t product_scratch(int64_t rows, int64_t n_src) {
-    if (n_src <= kFewSources) return 0;
     const int64_t groups = (rows + kGroup - 1) / kGroup;
-    return align256(4 * (size_t)rows) + 4 * (size_t)(groups * n_src * kGroup);
+    return align256(4 * (size_t)(rows + groups)) + 4 * (size_t)(groups * n_src * kGroup);
 }
 
 static size_t grad_scratch(int64_t rows, int64_t n_src, int64_t n_dst) {
@@ -494,6 +515,38 @@ static int row_tile(int64_t rows, int64_t n_dst) {
     int64_t tile = ((n_dst + want - 1) / want + 63) / 64 * 64;
     tile = tile < 1024 ? 1024 : tile > kRowTile ? kRowTile : tile;
     return (int)(tile < n_dst ? tile : n_dst);
+}
+
+// Nonzeros of a row up to which the `rows` form takes it, from what either form
+// takes here in us (fitted to 15 nets of 64 to 100,000 sources, 40 to 40,000
+// destinations and 10 to 2000 edges a source, 1 to 4000 rows, 0.1 to 100 % active:
+// 0.7 % from the faster form on average).  A source costs the rows form a
+// barrier and a chain of loads, or, with many workgroups, its share of a CU or of
+// the weights' lines; the columns cost the transpose and every edge, more once
+// the rows of x leave an XCD's L2, or the chain of the edges of one destination.
+// Measured by rows / columns, us:
+//   16384 x 16384, 819 edges a source, 64 rows, 328 active    236 / 155
+//   16384 x 16384, 819 edges a source, 64 rows, 82 active      91 / 155
+//   16384 x 100, 10 edges a source, 64 rows, 328 active       134 / 206
+//   16384 x 100, 10 edges a source, 1000 rows, 16 active       72 / 229
+//   1000 x 1000, 50 edges a source, 64 rows, 20 active         19 / 20
+//   1000 x 1000, 50 edges a source, 64 rows, all active       330 / 20
+//   100000 x 5000, 20 edges a source, 200 rows, 100 active    106 / 272
+static int rows_limit(int64_t rows, int64_t n_src, int64_t n_dst, int64_t nnz) {
+    const double groups = (double)((rows + kGroup - 1) / kGroup);
+    const double len = (double)nnz / (double)n_src;
+    const int tile = row_tile(rows, n_dst);
+    const double wgs = (double)rows * (double)((n_dst + tile - 1) / tile);
+    const double per_cu = wgs > 256.0 ? wgs / 256.0 : 1.0;
+    // us per edge: the weights in L2, in the caches beyond, past them
+    const double edge = nnz < 1000000 ? 4e-6 : nnz < 4000000 ? 7e-6 : 10e-6;
+    const double source_us = std::max({0.4 + 0.2e-3 * len, 1.4e-3 * wgs, edge * (double)rows * len});
+    const double spread = std::min(3.5, std::max(1.0, 1.3 * (double)n_src / 16384.0));
+    const double cols_us = 6.0 + 0.114e-3 * groups * (double)n_src +
+                           std::max(0.1 * (double)nnz / (double)n_dst,
+                                    10e-6 * spread * (double)nnz * groups);
+    const double most = (cols_us - 0.14e-3 * (double)n_src * per_cu) / source_us;
+    return most < 0.0 ? 0 : most >= (double)n_src ? (int)n_src : (int)most;
 }
 
 static int check_product(const char* who, int64_t n_src, int64_t n_dst, int64_t rows,
@@ -525,12 +578,11 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
         return fail("btx_product: scratch too small");
     const hipStream_t s = (hipStream_t)stream;
     ProductArgs a{row_ptr, col, perm, csc_ptr, csc_src, w, n_src, n_dst, nnz, x, x_row_stride, rows,
-                  y, nullptr, nullptr};
+                  y, nullptr, nullptr, nullptr, 0};
     // one row always (13.4M edges: 28 us against 31 by rows at 16 active sources
     // and 170 by columns); up to four while their gathers stay few: 8M in all
     // take 27 us, 14M 52 us, by when the rows form is as fast at low activity
-    if (n_src > kFewSources && rows <= kFewRows &&
-        (rows == 1 || rows * nnz <= ((int64_t)8 << 20))) {
+    if (rows <= kFewRows && (rows == 1 || rows * nnz <= ((int64_t)8 << 20)) && nnz <= 8192 * n_dst) {
         const int64_t wgs = (n_dst + 3) / 4;
         const dim3 few((unsigned)(wgs < 8192 ? wgs : 8192));
         hipLaunchKernelGGL(rows == 1 ? k_product_few<1> : rows == 2 ? k_product_few<2>
@@ -538,12 +590,21 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
                            few, dim3(256), 0, s, a);
         return check_launch("btx_product");
     }
+    a.most = n_src > 0 ? rows_limit(rows, n_src, n_dst, nnz) : 0;
+    const bool columns = a.most < n_src;  // some row may be left to them
     const int64_t groups = (rows + kGroup - 1) / kGroup;
-    if (n_src > kFewSources) {
-        a.counts = (const int32_t*)scratch;
-        a.xt = (float*)((char*)scratch + align256(4 * (size_t)rows));
-        hipLaunchKernelGGL(k_row_counts, dim3((unsigned)rows), dim3(1024), 0, s, x, n_src,
-                           x_row_stride, (int32_t*)scratch);
+    if (columns) {
+        a.counts = (int32_t*)scratch;
+        a.by_columns = a.counts + rows;
+        a.xt = (float*)((char*)scratch + align256(4 * (size_t)(rows + groups)));
+        // a wavefront per short row: 12,800 rows of 200 values would take a
+        // workgroup each 30 us
+        if (n_src <= 4096)
+            hipLaunchKernelGGL(k_row_counts<64>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, x,
+                               n_src, x_row_stride, rows, a.counts);
+        else
+            hipLaunchKernelGGL(k_row_counts<1024>, dim3((unsigned)rows), dim3(1024), 0, s, x, n_src,
+                               x_row_stride, rows, a.counts);
         hipLaunchKernelGGL(k_group_rows, dim3((unsigned)((n_src + 63) / 64), (unsigned)groups),
                            dim3(256), 0, s, a, x, n_src, x_row_stride, rows, a.xt);
     }
@@ -553,9 +614,9 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
     hipLaunchKernelGGL(narrow ? (one ? k_product_rows<int, 1> : k_product_rows<int, 8>)
                               : (one ? k_product_rows<int64_t, 1> : k_product_rows<int64_t, 8>),
                        grid, dim3(kRowThreads), 4 * (size_t)(tile + 3), s, a, tile);
-    if (n_src > kFewSources) {
-        const int64_t tiles = (n_dst + 15) / 16;
-        hipLaunchKernelGGL(k_product_columns, dim3((unsigned)(tiles < 2048 ? tiles : 2048)),
+    if (columns) {
+        const int64_t items = (n_dst + 15) / 16 * groups;
+        hipLaunchKernelGGL(k_product_columns, dim3((unsigned)(items < 2048 ? items : 2048)),
                            dim3(256), 0, s, a);
     }
     return check_launch("btx_product");
@@ -590,8 +651,12 @@ BTX_API int btx_product_grad(const int64_t* row_ptr, const int32_t* col, const i
     if (gw != nullptr) {
         hipLaunchKernelGGL(k_row_bits, dim3((unsigned)((n_src + 255) / 256), (unsigned)groups),
                            dim3(256), 0, s, x, n_src, x_row_stride, rows, bits);
-        hipLaunchKernelGGL(k_product_grad_w, dim3((unsigned)((n_dst + 3) / 4)), dim3(256), 0, s,
-                           csc_ptr, csc_src, n_src, n_dst, rows, x, x_row_stride, bits, gt, gw);
+        // as many wavefronts per destination as fill the chip with 8192
+        const int64_t len64 = (nnz / n_dst + 63) / 64, want = (8192 + n_dst - 1) / n_dst;
+        const int64_t split = len64 < want ? len64 : want;
+        hipLaunchKernelGGL(k_product_grad_w,
+                           dim3((unsigned)((n_dst + 3) / 4), (unsigned)(split > 0 ? split : 1)),
+                           dim3(256), 0, s, csc_ptr, csc_src, n_src, n_dst, rows, x, x_row_stride, bits, gt, gw);
     }
     return check_launch("btx_product_grad");
 }

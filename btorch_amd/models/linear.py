@@ -208,6 +208,8 @@ class BaseSparseConn(nn.Module):
         """The effective weights as they are now: edits in place of the
         parameters and buffers that follow do not reach them."""
         w = self._get_effective_weight()
+        if any(w is t for t in self._parameters.values()):
+            return w.clone()
         held = {t.untyped_storage().data_ptr()
                 for t in (*self._parameters.values(), *self._buffers.values()) if t is not None}
         return w.clone() if w.untyped_storage().data_ptr() in held else w

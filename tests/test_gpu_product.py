@@ -85,11 +85,11 @@ def test_products_of_few_rows_match_sequential_sums(n_src, n_dst, degree, rows, 
     assert torch.equal(y, rsnn.NativeSparse(mat)(x))
 
 
-@pytest.mark.parametrize("n_src,rows", [(2, 1), (1030, 2)])
+@pytest.mark.parametrize("n_src,rows", [(1000, 2), (1030, 2)])
 def test_product_of_edges_past_int32(n_src, rows):
     # 2^31 edges and more: row offsets past int32 (the arrays are as long, only
     # the last few edges of them, of the last two sources, are read), for rows
-    # of x read 1024 and 8192 values at a time
+    # of x read 1024 and 8192 values at a time; by destination there are none
     from btorch_amd import _lib
     first, n_dst = 2**31 + 5, 8
     row_ptr = torch.full((n_src + 1,), first, dtype=torch.int64, device=DEV)
@@ -104,10 +104,13 @@ def test_product_of_edges_past_int32(n_src, rows):
     y = torch.empty((rows, n_dst), device=DEV)
     lib = _lib.load()
     scratch = torch.empty(lib.btx_product_scratch_bytes(rows, n_src), dtype=torch.uint8, device=DEV)
-    _lib.check(lib.btx_product(row_ptr.data_ptr(), col.data_ptr(), perm.data_ptr(), None, None,
-                               w.data_ptr(), n_src, n_dst, first + 5, x.data_ptr(), n_src, rows,
-                               y.data_ptr(), scratch.data_ptr() if scratch.numel() else None,
-                               scratch.numel(), _lib.stream_ptr()), "btx_product")
+    csc_ptr = torch.zeros(n_dst + 1, dtype=torch.int64, device=DEV)
+    csc_src = torch.zeros(1, dtype=torch.int32, device=DEV)
+    _lib.check(lib.btx_product(row_ptr.data_ptr(), col.data_ptr(), perm.data_ptr(),
+                               csc_ptr.data_ptr(), csc_src.data_ptr(), w.data_ptr(), n_src,
+                               n_dst, first + 5, x.data_ptr(), n_src, rows, y.data_ptr(),
+                               scratch.data_ptr(), scratch.numel(), _lib.stream_ptr()),
+               "btx_product")
     assert y.cpu().tolist() == [[-3.75, 2.0, 0.0, 0.0, 12.5, 0.0, 8.0, 0.0]] * rows
 
 
@@ -154,3 +157,29 @@ def test_prepared_weights_stay_those_of_prepare():
     (conn(x) + conn(x)).sum().backward()
     conn.finish_sparse()
     assert torch.equal(conn.magnitude.grad, torch.full_like(conn.magnitude, 4.0))
+
+
+@pytest.mark.parametrize("n_src,n_dst,degree,rows,prob", [
+    (300, 41, 8, 4, 1.0),        # a few rows of few sources, by destination
+    (700, 900, 30, 6, 1.0),      # few sources, all active: columns
+    (5000, 3, 2, 70, 0.5),       # long destinations, their weight gradient in pieces
+    (1024, 2000, 25, 64, 0.004),
+    (4097, 60, 5, 9, 0.01),      # counted by a workgroup a row
+])
+def test_product_forms_by_cost_match_sequential_sums(n_src, n_dst, degree, rows, prob):
+    test_product_forms_match_sequential_sums(n_src, n_dst, degree, rows, prob, "native")
+
+
+def test_product_of_groups_that_take_either_form():
+    # 67 groups of 64 rows, every third with all sources active (the columns),
+    # the others with a few (the rows), the last one ragged
+    n_src, n_dst, rows = 900, 90, 66 * 64 + 5
+    mat = _matrix(n_src, n_dst, 20, 11)
+    rng = np.random.default_rng(12)
+    prob = np.where((np.arange(rows) // 64) % 3 == 1, 1.0, 0.002)[:, None]
+    x = (rng.random((rows, n_src)) < prob) * rng.standard_normal((rows, n_src))
+    x = torch.from_numpy(x.astype(np.float32))
+    conn = SparseConn(mat, enforce_dale=False, device=DEV)
+    with torch.no_grad():
+        y = conn(x.to(DEV)).cpu()
+    assert torch.equal(y, rsnn.NativeSparse(mat)(x))
