@@ -7,7 +7,7 @@
 //
 // Every destination sums its terms in ascending source order from +0.0f with
 // one fmaf per source with x != 0, so y equals torch.sparse.mm on the CPU bit
-// for bit (btorch/models/linear.py:474-483).  Two forms, neither of which
+// for bit (btorch/models/linear.py:474-483).  Three forms, none of which
 // stores a term:
 //   rows     a workgroup takes one row of x and a tile of destinations held in
 //            LDS, and streams the rows of W of the row's nonzero sources in
@@ -17,10 +17,13 @@
 //   columns  a quarter wavefront takes a destination and 64 rows of x
 //            (transposed, so that a source's 64 values are one 256-byte read)
 //            and walks the destination's edges.  Costs every edge, whatever the activity.
+//   few      a wavefront takes a destination and four rows of x and gathers: one
+//            launch, for products of few edges.
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/btorch_amd.h"
 #include "btx_common.h"
@@ -28,9 +31,9 @@
 namespace btx {
 
 constexpr int kRowTile = 16384;      // destinations of a `rows` workgroup, at most (64 KB of LDS)
-constexpr int kRowThreads = 1024;
+constexpr int kSegment = 1024;       // values of a row that are counted and listed together
 constexpr int kGroup = 64;           // rows of x per wavefront of the `columns` form
-constexpr int64_t kFewRows = 4;      // up to which k_product_few takes them
+constexpr int64_t kFewRows = 4;      // rows of x of a wavefront of k_product_few
 
 struct ProductArgs {
     const int64_t* row_ptr;
@@ -47,7 +50,9 @@ struct ProductArgs {
     int64_t rows;
     float* y;             // (rows, n_dst)
     float* xt;            // [groups][n_src][64]
-    int32_t* counts;      // nonzeros of each row
+    int32_t* counts;      // nonzeros of each listed row
+    int32_t* seg_counts;  // [segments][rows] nonzeros of every kSegment values
+    int segments;
     int32_t* by_columns;  // [groups] 1 = left to the columns; NULL = the `rows` form takes all
     int most;             // nonzeros a row, on average of a group, up to which the `rows`
                           // form takes the group
@@ -58,146 +63,173 @@ struct ProductArgs {
 // wavefront calls it.
 __device__ __forceinline__ bool group_by_rows(const ProductArgs& a, int64_t g) {
     const int64_t row = g * kGroup + (threadIdx.x & 63);
-    int64_t c = row < a.rows ? a.counts[row] : 0;
+    int64_t c = 0;
+    if (row < a.rows)
+#pragma unroll 8
+        for (int s = 0; s < a.segments; ++s) c += a.seg_counts[s * a.rows + row];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
     const int64_t here = a.rows - g * kGroup < kGroup ? a.rows - g * kGroup : kGroup;
     return c <= a.most * here;
 }
 
-// Nonzeros of every row: THREADS threads a row, of a workgroup of 256 or 1024.
-template <int THREADS>
-__global__ __launch_bounds__(THREADS < 256 ? 256 : THREADS) void k_row_counts(
-    const float* __restrict__ x, int64_t n, int64_t stride, int64_t rows,
-    int32_t* __restrict__ counts) {
-    constexpr int BLOCK = THREADS < 256 ? 256 : THREADS;
-    const int64_t row = (int64_t)blockIdx.x * (BLOCK / THREADS) + threadIdx.x / THREADS;
-    if (THREADS == 64 && row >= rows) return;
-    const float* xr = x + row * stride;
+// Nonzeros of every segment of every row, a wavefront each (a workgroup a row
+// would take 30 us for 12,800 rows of 200 values).
+__global__ __launch_bounds__(256) void k_row_counts(ProductArgs a) {
+    const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (item >= a.rows * a.segments) return;
+    const int64_t row = item % a.rows, i0 = item / a.rows * kSegment;
+    const int64_t i1 = i0 + kSegment < a.n_src ? i0 + kSegment : a.n_src;
+    const float* xr = a.x + row * a.x_stride;
     int c = 0;
-#pragma unroll 8
-    for (int64_t i = threadIdx.x % THREADS; i < n; i += THREADS) c += xr[i] != 0.f;
-    int total;
-    if (THREADS == 64) {
+#pragma unroll 16
+    for (int64_t i = i0 + (threadIdx.x & 63); i < i1; i += 64) c += xr[i] != 0.f;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-        total = c;
-    } else {
-        block_excl_scan<BLOCK / 64>(c, total);
-    }
-    if (threadIdx.x % THREADS == 0) counts[row] = total;
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if ((threadIdx.x & 63) == 0) a.seg_counts[item] = c;
 }
 
-// One row of x, destinations [d0, d0 + tile): 1024 V of the row's values are
-// read at a time and their nonzeros listed in LDS in ascending order, each
-// with its row of W.  Bound by the misses one CU can have in flight on a
-// source's weights, which perm scatters over the array, and by the barrier per
-// source: eight sources are requested together, the next eight before the
-// current ones are added, and a few rows are split into tiles over the CUs.
-// 0.4 to 0.65 us a source of 163 to 819 edges (one source ahead, 1024 values at
-// a time and whole rows: 0.8 to 1.9 us).  Taken back: three requests in flight
-// (74 VGPRs, one workgroup per CU: 512 rows 15% slower), 256 threads.  Edge:
-// an integer that holds the edges' positions (64 bits leave room for one
-// workgroup per CU where 16,384 destinations are tiled).  V = 1 where a row has
-// no more than 1024 values: 200 x 16,384, 12,800 rows, 5 active sources each,
-// 0.383 ms; 0.411 with seven of eight reads and ballots per thread wasted.
-template <typename Edge, int V>
-__global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int tile) {
-    constexpr int T = kRowThreads;
+__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ inline int64_t uniform(int64_t v) {
+    return (int64_t)((uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32 | (uint32_t)uniform((int)v));
+}
+__device__ inline float uniform(float v) { return __int_as_float(uniform(__float_as_int(v))); }
+
+// One row of x, destinations [d0, d0 + tile): the row's nonzero sources go through
+// LDS in ascending order, L at a time, each with its row of W.  Bound by the
+// instructions and the latency of a source's few edges per thread, whose weights
+// perm scatters over the array, and with several wavefronts by the barrier per
+// source: U sources are requested together, the next U before the current ones
+// are added, without a branch per load (which waited for each: 0.18 against 0.13
+// us a source of 20 edges), and a few rows are split into tiles over the CUs.  T
+// threads by the edges of a source; one wavefront alone needs no barrier.  0.13
+// to 0.17 us a source of 10 to 40 edges by 64 threads, 0.25 us of 163 by 256, 0.4
+// us of 819 by 1024.  8000 x 1000, 20 edges a source, 4000 rows, 0.5 % active: 94
+// us (1024 threads for every net, which scanned x in every workgroup: 332); 200 x
+// 16384, 819 edges a source, 12,800 rows, 2.5 % active: 341 us with its lists (402).
+// Taken back: three requests in flight (no faster by 64 or 256 threads; by 1024 one
+// workgroup per CU).  Edge: an integer that holds the edges' positions.
+template <typename Edge, int T>
+__global__ __launch_bounds__(T, T == 1024 && sizeof(Edge) == 4 ? 8 : 1) void k_product_rows(
+    ProductArgs a, int tile) {
+    constexpr int U = T == 64 ? 16 : 8;
+    constexpr int L = T == 64 ? 256 : T;   // sources a list in LDS holds
+    using UEdge = std::conditional_t<sizeof(Edge) == 4, uint32_t, uint64_t>;
     extern __shared__ __align__(16) float s_y[];
-    __shared__ Edge s_beg[T];
-    __shared__ int s_len[T];
-    __shared__ float s_x[T];
-    __shared__ int s_cnt[T / 64];
-    constexpr int U = 8;
-    const int tid = threadIdx.x, wv = tid >> 6, ln = tid & 63;
+    __shared__ Edge s_beg[L];
+    __shared__ int s_len[L];
+    __shared__ float s_x[L];
+    const int tid = threadIdx.x;
     const int64_t row = blockIdx.x, d0 = (int64_t)blockIdx.y * tile;
     const int nd = (int)(a.n_dst - d0 < tile ? a.n_dst - d0 : tile);
     const float* xr = a.x + row * a.x_stride;
-    const int left = a.by_columns != nullptr ? a.by_columns[row / kGroup] : 0;
+    if (a.by_columns != nullptr && a.by_columns[row / kGroup]) return;  // uniform
+    const int spare = tile + 3;  // s_y is filled by four
     for (int q = tid; q < (nd + 3) / 4; q += T)
         reinterpret_cast<float4*>(s_y)[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int64_t s0 = 0; s0 < a.n_src; s0 += T * V) {
-      // a wavefront reads 64 V consecutive values
-      const int64_t s1 = s0 + wv * 64 * V + ln;
-      float xv[V];
-#pragma unroll
-      for (int u = 0; u < V; ++u) xv[u] = s1 + 64 * u < a.n_src ? xr[s1 + 64 * u] : 0.f;
-      if (left) return;  // uniform; asked for beside the first values
-      int mine = 0;
-#pragma unroll
-      for (int u = 0; u < V; ++u) mine += __popcll((unsigned long long)__ballot(xv[u] != 0.f));
-      if (ln == 0) s_cnt[wv] = mine;
-      __syncthreads();
-      int first = 0, nonzero = 0;
-#pragma unroll
-      for (int k = 0; k < T / 64; ++k) {
-          first += k < wv ? s_cnt[k] : 0;
-          nonzero += s_cnt[k];
-      }
-      // the nonzeros, 1024 at a time
-      for (int base = 0; base < nonzero; base += T) {
-        const int total = nonzero - base < T ? nonzero - base : T;
-        int off = first - base;
-#pragma unroll
-        for (int u = 0; u < V; ++u) {
-            const bool on = xv[u] != 0.f;
-            const uint64_t m = __ballot(on);
-            const int p = off + __popcll((unsigned long long)(m & ((1ull << ln) - 1ull)));
-            off += __popcll((unsigned long long)m);
-            if (on && p >= 0 && p < T) {
-                const int64_t beg = a.row_ptr[s1 + 64 * u];
-                s_beg[p] = (Edge)beg;
-                s_len[p] = (int)(a.row_ptr[s1 + 64 * u + 1] - beg);
-                s_x[p] = xv[u];
-            }
-        }
-        __syncthreads();
-        // this thread's first edge of eight sources: destination within the
-        // tile (-1 = none), weight
-        auto request = [&](int k0, int* d, float* w) {
-            int64_t pm[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const bool in = k0 + u < total && tid < s_len[k0 + u];
-                const Edge e = in ? s_beg[k0 + u] + tid : 0;
-                d[u] = in ? a.col[e] : -1;
-                pm[u] = in ? a.perm[e] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int64_t q = d[u] - d0;
-                d[u] = d[u] >= 0 && q >= 0 && q < nd ? (int)q : -1;
-                w[u] = d[u] >= 0 ? a.w[pm[u]] : 0.f;
-            }
+    // adds the `total` listed sources; every load is made, of edge 0 by threads
+    // without one, and what is not this tile's goes to a value that is not kept
+    // (a branch per load would wait for each)
+    auto add = [&](int total) {
+        if (a.nnz == 0) return;  // uniform
+        const unsigned from = (unsigned)d0, many = (unsigned)nd;
+        auto slot = [&](bool in, int col) {
+            const unsigned q = (unsigned)col - from;
+            return in && q < many ? (int)q : spare;
         };
-        int d[U], dn[U];
-        float w[U], wn[U];
-        if (total > 0) request(0, d, w);
-        for (int k0 = 0; k0 < total; k0 += U) {
-            if (k0 + U < total) request(k0 + U, dn, wn);
+        // this thread's first edge of U sources, with what the sources share
+        auto ask = [&](int k0, int* d, Edge* pm, int* len, float* xk) {
+            Edge beg[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (k0 + u >= total) break;  // uniform
-                const float xk = s_x[k0 + u];
-                const int len = s_len[k0 + u];
-                if (d[u] >= 0) s_y[d[u]] = fmaf(w[u], xk, s_y[d[u]]);
-                for (int t = tid + T; t < len; t += T) {
-                    const Edge e = s_beg[k0 + u] + t;
-                    const int64_t q = a.col[e] - d0;
-                    if (q >= 0 && q < nd) s_y[q] = fmaf(a.w[a.perm[e]], xk, s_y[q]);
-                }
-                __syncthreads();
+                beg[u] = uniform(s_beg[k0 + u]);
+                len[u] = uniform(s_len[k0 + u]);
+                xk[u] = uniform(s_x[k0 + u]);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                d[u] = dn[u];
-                w[u] = wn[u];
+                const unsigned t = tid < len[u] ? tid : 0;
+                d[u] = (a.col + beg[u])[t];
+                pm[u] = (Edge)(a.perm + beg[u])[t];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) d[u] = slot(tid < len[u], d[u]);
+        };
+        auto weights = [&](const int* d, const Edge* pm, float* w) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) w[u] = a.w[(UEdge)(d[u] != spare ? pm[u] : 0)];
+        };
+        int d[U], d1[U], len[U], len1[U];
+        Edge pm[U];
+        float w[U], w1[U], xk[U], xk1[U];
+        ask(0, d, pm, len, xk);
+        weights(d, pm, w);
+        for (int k0 = 0; k0 < total; k0 += U) {
+            if (k0 + U < total) {
+                ask(k0 + U, d1, pm, len1, xk1);
+                weights(d1, pm, w1);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (T > 64 && k0 + u >= total) break;  // uniform
+                s_y[d[u]] = fmaf(w[u], xk[u], s_y[d[u]]);
+                // a longer source's other edges, four at a time
+                if (len[u] > T) {  // uniform
+                    const Edge beg = uniform(s_beg[k0 + u]);
+                    for (unsigned t0 = T; t0 < (unsigned)len[u]; t0 += 4 * T) {
+                        unsigned t[4];
+                        int q4[4];
+                        Edge p4[4];
+                        float w4[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            t[i] = t0 + tid + i * T;
+                            const unsigned e = t[i] < (unsigned)len[u] ? t[i] : 0;
+                            q4[i] = (a.col + beg)[e];
+                            p4[i] = (Edge)(a.perm + beg)[e];
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            q4[i] = slot(t[i] < (unsigned)len[u], q4[i]);
+                            w4[i] = a.w[(UEdge)(q4[i] != spare ? p4[i] : 0)];
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) s_y[q4[i]] = fmaf(w4[i], xk[u], s_y[q4[i]]);
+                    }
+                }
+                // one wavefront's LDS accesses are done in order
+                if (T == 64) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                else __syncthreads();
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                d[u] = d1[u];
+                w[u] = w1[u];
+                len[u] = len1[u];
+                xk[u] = xk1[u];
             }
         }
         __syncthreads();  // the list is rewritten
-      }
-      __syncthreads();  // and s_cnt
+    };
+    const int32_t* src = reinterpret_cast<const int32_t*>(a.xt) + row * a.n_src;
+    const int nonzero = a.counts[row];
+    for (int base = 0; base < nonzero; base += L) {
+#pragma unroll
+        for (int p = tid; p < L; p += T) {
+            if (base + p < nonzero) {
+                const int s = src[base + p];
+                const int64_t beg = a.row_ptr[s];
+                const int len = (int)(a.row_ptr[s + 1] - beg);
+                s_beg[p] = len > 0 ? (Edge)beg : 0;  // (every thread reads an edge)
+                s_len[p] = len;
+                s_x[p] = xr[s];
+            } else {
+                s_beg[p] = 0;
+                s_len[p] = 0;
+            }
+        }
+        __syncthreads();
+        add(nonzero - base < L ? nonzero - base : L);
     }
     __syncthreads();
     float* yr = a.y + row * a.n_dst + d0;
@@ -208,18 +240,20 @@ __global__ __launch_bounds__(kRowThreads) void k_product_rows(ProductArgs a, int
         for (int q = tid; q < nd; q += T) yr[q] = s_y[q];
 }
 
-// out[g][i][b] = in[64 g + b][i] in tiles of 64 x 64; rows past `rows` are 0.
-// `a` non-null: only the groups that take the columns.
-__global__ __launch_bounds__(256) void k_group_rows(ProductArgs a, const float* __restrict__ in,
-                                                    int64_t n, int64_t stride, int64_t rows,
-                                                    float* __restrict__ out) {
+template <typename Edge>
+static void launch_rows(const ProductArgs& a, int threads, int tile, hipStream_t s) {
+    const dim3 grid((unsigned)a.rows, (unsigned)((a.n_dst + tile - 1) / tile));
+    const auto kernel = threads == 64    ? &k_product_rows<Edge, 64>
+                        : threads == 256 ? &k_product_rows<Edge, 256>
+                                         : &k_product_rows<Edge, 1024>;
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 4 * (size_t)(tile + 4), s, a, tile);
+}
+
+// out[g][i][b] = in[64 g + b][i] for the 64 values from i0; rows past `rows` are 0.
+__device__ __forceinline__ void group_rows(const float* __restrict__ in, int64_t n, int64_t stride,
+                                           int64_t rows, float* __restrict__ out, int64_t g,
+                                           int64_t i0) {
     __shared__ float t[64][65];
-    const int64_t g = blockIdx.y, i0 = (int64_t)blockIdx.x * 64;
-    if (a.by_columns != nullptr) {
-        const bool taken = !group_by_rows(a, g);
-        if (blockIdx.x == 0 && threadIdx.x == 0) a.by_columns[g] = taken;
-        if (!taken) return;
-    }
     const int ln = threadIdx.x & 63;
     for (int b = threadIdx.x >> 6; b < 64; b += 4) {
         const int64_t row = g * kGroup + b, i = i0 + ln;
@@ -228,6 +262,52 @@ __global__ __launch_bounds__(256) void k_group_rows(ProductArgs a, const float* 
     __syncthreads();
     for (int k = threadIdx.x >> 6; k < 64; k += 4)
         if (i0 + k < n) out[(g * n + i0 + k) * kGroup + ln] = t[ln][k];
+}
+
+__global__ __launch_bounds__(256) void k_group_rows(const float* __restrict__ in, int64_t n,
+                                                    int64_t stride, int64_t rows,
+                                                    float* __restrict__ out) {
+    group_rows(in, n, stride, rows, out, blockIdx.y, (int64_t)blockIdx.x * 64);
+}
+
+// Shares the groups out: the rows of one that takes the columns are transposed,
+// rows of one that does not are listed, a wavefront per segment, where its
+// transposed rows would go (xt: both take n_src values a row).
+__global__ __launch_bounds__(256) void k_share_rows(ProductArgs a) {
+    const int64_t g = blockIdx.y;
+    if (a.by_columns != nullptr) {
+        const bool taken = !group_by_rows(a, g);
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.by_columns[g] = taken;
+        if (taken) {
+            const int64_t i0 = (int64_t)blockIdx.x * 64;
+            if (i0 < a.n_src) group_rows(a.x, a.n_src, a.x_stride, a.rows, a.xt, g, i0);
+            return;
+        }
+    }
+    const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
+    const int64_t item = (int64_t)blockIdx.x * 4 + wv, row = g * kGroup + item % kGroup;
+    const int64_t seg = item / kGroup;
+    if (row >= a.rows || seg >= a.segments) return;
+    int p = 0;
+    for (int64_t s = ln; s < seg; s += 64) p += a.seg_counts[s * a.rows + row];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) p += __shfl_xor(p, o, 64);
+    if (seg == a.segments - 1 && ln == 0) a.counts[row] = p + a.seg_counts[seg * a.rows + row];
+    const int64_t end = (seg + 1) * kSegment < a.n_src ? (seg + 1) * kSegment : a.n_src;
+    const float* xr = a.x + row * a.x_stride;
+    int32_t* list = reinterpret_cast<int32_t*>(a.xt) + row * a.n_src;
+    for (int64_t i = seg * kSegment + ln; i - ln < end; i += 512) {
+        bool on[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) on[u] = i + 64 * u < end && xr[i + 64 * u] != 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const uint64_t m = __ballot(on[u]);
+            const int q = p + __popcll((unsigned long long)(m & ((1ull << ln) - 1ull)));
+            if (on[u]) list[q] = (int32_t)(i + 64 * u);
+            p += __popcll((unsigned long long)m);
+        }
+    }
 }
 
 // The inverse: out[64 g + b][i] = in[g][i][b].
@@ -329,7 +409,7 @@ __global__ __launch_bounds__(256, 4) void k_product_columns(ProductArgs a) {
     }
 }
 
-// A few rows of x: a wavefront per destination reads 64 edges at a time, a lane
+// ROWS rows of x: a wavefront per destination reads 64 edges at a time, a lane
 // each, and gathers their x out of L2; the nonzero ones, found by a ballot, are
 // added in ascending source order.  One launch, whatever the activity: 21,739 x
 // 21,739 of 3.5M edges 14 us a row in a replayed graph (counting, the transpose
@@ -337,6 +417,10 @@ __global__ __launch_bounds__(256, 4) void k_product_columns(ProductArgs a) {
 template <int ROWS>
 __global__ __launch_bounds__(256) void k_product_few(ProductArgs a) {
     const int ln = threadIdx.x & 63;
+    const int64_t r0 = (int64_t)blockIdx.y * ROWS;
+    const int here = (int)(a.rows - r0 < ROWS ? a.rows - r0 : ROWS);
+    const float* x = a.x + r0 * a.x_stride;
+    float* y = a.y + r0 * a.n_dst;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     for (int64_t d = (int64_t)blockIdx.x * 4 + wv; d < a.n_dst; d += (int64_t)gridDim.x * 4) {
         const int64_t e0 = a.csc_ptr[d];
@@ -348,7 +432,8 @@ __global__ __launch_bounds__(256) void k_product_few(ProductArgs a) {
             const int w = in ? __float_as_int(a.w[e0 + c + ln]) : 0;
             float xv[ROWS];
 #pragma unroll
-            for (int r = 0; r < ROWS; ++r) xv[r] = in ? a.x[r * a.x_stride + src] : 0.f;
+            for (int r = 0; r < ROWS; ++r)
+                xv[r] = in && r < here ? x[r * a.x_stride + src] : 0.f;
 #pragma unroll
             for (int r = 0; r < ROWS; ++r) {
                 uint64_t m = __ballot(xv[r] != 0.f);
@@ -363,7 +448,8 @@ __global__ __launch_bounds__(256) void k_product_few(ProductArgs a) {
         }
         if (ln == 0)
 #pragma unroll
-            for (int r = 0; r < ROWS; ++r) a.y[r * a.n_dst + d] = acc[r];
+            for (int r = 0; r < ROWS; ++r)
+                if (r < here) y[r * a.n_dst + d] = acc[r];
     }
 }
 
@@ -499,7 +585,9 @@ __global__ __launch_bounds__(256) void k_row_bits(const float* __restrict__ x, i
 
 static size_t product_scratch(int64_t rows, int64_t n_src) {
     const int64_t groups = (rows + kGroup - 1) / kGroup;
-    return align256(4 * (size_t)(rows + groups)) + 4 * (size_t)(groups * n_src * kGroup);
+    const int64_t segments = (n_src + kSegment - 1) / kSegment;
+    return align256(4 * (size_t)(rows + groups + rows * segments)) +
+           4 * (size_t)(groups * n_src * kGroup);
 }
 
 static size_t grad_scratch(int64_t rows, int64_t n_src, int64_t n_dst) {
@@ -517,36 +605,51 @@ static int row_tile(int64_t rows, int64_t n_dst) {
     return (int)(tile < n_dst ? tile : n_dst);
 }
 
+// Threads of a `rows` workgroup, by the edges of a source.  us by 64 / 256 / 1024
+// threads:
+//   1100 x 3000, 40 edges a source, 64 rows, 10 % active        35 / 40 / 48
+//   3000 x 3000, 60 edges a source, 64 rows, 10 % active        65 / 79 / 100
+//   3000 x 3000, 100 edges a source, 64 rows, 10 % active      212 / 81 / 108
+//   4000 x 8000, 250 edges a source, 64 rows, 2 % active        95 / 47 / 53
+//   1000 x 4000, 300 edges a source, 64 rows, 2 % active        32 / 35 / 24
+//   16384 x 16384, 819 edges a source, 8 rows, 0.5 % active    198 / 104 / 57
+static int row_threads(int64_t n_src, int64_t nnz) {
+    const int64_t len = nnz / (n_src > 0 ? n_src : 1);
+    return len <= 64 ? 64 : len <= 256 ? 256 : 1024;
+}
+
 // Nonzeros of a row up to which the `rows` form takes it, from what either form
 // takes here in us (fitted to 15 nets of 64 to 100,000 sources, 40 to 40,000
-// destinations and 10 to 2000 edges a source, 1 to 4000 rows, 0.1 to 100 % active:
-// 0.7 % from the faster form on average).  A source costs the rows form a
-// barrier and a chain of loads, or, with many workgroups, its share of a CU or of
-// the weights' lines; the columns cost the transpose and every edge, more once
-// the rows of x leave an XCD's L2, or the chain of the edges of one destination.
-// Measured by rows / columns, us:
-//   16384 x 16384, 819 edges a source, 64 rows, 328 active    236 / 155
-//   16384 x 16384, 819 edges a source, 64 rows, 82 active      91 / 155
-//   16384 x 100, 10 edges a source, 64 rows, 328 active       134 / 206
-//   16384 x 100, 10 edges a source, 1000 rows, 16 active       72 / 229
-//   1000 x 1000, 50 edges a source, 64 rows, 20 active         19 / 20
-//   1000 x 1000, 50 edges a source, 64 rows, all active       330 / 20
-//   100000 x 5000, 20 edges a source, 200 rows, 100 active    106 / 272
+// destinations and 10 to 2000 edges a source, 4 to 4000 rows, 0.1 to 10 % active:
+// 0.2 % from the faster form on average, 20 % at most).  A source costs the rows
+// form a chain of LDS accesses and loads or, with many workgroups, their edges or
+// the weights' lines; the columns cost the transpose, the outputs and every edge,
+// more once the rows of x leave an XCD's L2, or the chain of the edges of one
+// destination.  Measured by rows / columns, us:
+//   16384 x 16384, 819 edges a source, 64 rows, 328 active    257 / 164
+//   16384 x 16384, 819 edges a source, 8 rows, 328 active     143 / 172
+//   16384 x 100, 10 edges a source, 1000 rows, 16 active       60 / 240
+//   1000 x 1000, 50 edges a source, 1000 rows, 20 active       27 / 38
+//   1000 x 1000, 50 edges a source, 1000 rows, 100 active      46 / 38
+//   100000 x 5000, 20 edges a source, 200 rows, 500 active    157 / 287
+//   100000 x 5000, 20 edges a source, 200 rows, 2000 active   399 / 285
 static int rows_limit(int64_t rows, int64_t n_src, int64_t n_dst, int64_t nnz) {
     const double groups = (double)((rows + kGroup - 1) / kGroup);
     const double len = (double)nnz / (double)n_src;
-    const int tile = row_tile(rows, n_dst);
+    const int tile = row_tile(rows, n_dst), threads = row_threads(n_src, nnz);
     const double wgs = (double)rows * (double)((n_dst + tile - 1) / tile);
-    const double per_cu = wgs > 256.0 ? wgs / 256.0 : 1.0;
-    // us per edge: the weights in L2, in the caches beyond, past them
-    const double edge = nnz < 1000000 ? 4e-6 : nnz < 4000000 ? 7e-6 : 10e-6;
-    const double source_us = std::max({0.4 + 0.2e-3 * len, 1.4e-3 * wgs, edge * (double)rows * len});
+    const double chain = threads == 64    ? 0.19
+                         : threads == 256 ? 0.34 + 0.4e-3 * len
+                                          : 0.24 + 0.25e-3 * len;
+    // 4M weights and more leave the caches
+    const double lines = nnz < 4000000 ? 0.0 : 7e-6 * (double)rows * len;
+    const double source_us = std::max({chain, 3.6e-6 * wgs * len, lines});
     const double spread = std::min(3.5, std::max(1.0, 1.3 * (double)n_src / 16384.0));
-    const double cols_us = 6.0 + 0.114e-3 * groups * (double)n_src +
+    const double cols_us = 6.0 + groups * (0.2e-3 * (double)n_src + 32e-6 * (double)n_dst) +
                            std::max(0.1 * (double)nnz / (double)n_dst,
-                                    10e-6 * spread * (double)nnz * groups);
-    const double most = (cols_us - 0.14e-3 * (double)n_src * per_cu) / source_us;
-    return most < 0.0 ? 0 : most >= (double)n_src ? (int)n_src : (int)most;
+                                    8e-6 * spread * (double)nnz * groups);
+    const double most = cols_us / source_us;
+    return most >= (double)n_src ? (int)n_src : (int)most;
 }
 
 static int check_product(const char* who, int64_t n_src, int64_t n_dst, int64_t rows,
@@ -578,13 +681,19 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
         return fail("btx_product: scratch too small");
     const hipStream_t s = (hipStream_t)stream;
     ProductArgs a{row_ptr, col, perm, csc_ptr, csc_src, w, n_src, n_dst, nnz, x, x_row_stride, rows,
-                  y, nullptr, nullptr, nullptr, 0};
-    // one row always (13.4M edges: 28 us against 31 by rows at 16 active sources
-    // and 170 by columns); up to four while their gathers stay few: 8M in all
-    // take 27 us, 14M 52 us, by when the rows form is as fast at low activity
-    if (rows <= kFewRows && (rows == 1 || rows * nnz <= ((int64_t)8 << 20)) && nnz <= 8192 * n_dst) {
+                  y, nullptr, nullptr, nullptr, 0, nullptr, 0};
+    // by destination while the edges, times the rows, stay few.  One row always
+    // (13.4M edges: 28 us against 31 by rows at 16 active sources and 170 by
+    // columns); up to four as far as 8M (27 us; 14M 52 us, by when the rows form is
+    // as fast at low activity); more rows, which read the edges again for every
+    // four, as far as 2M: 0.4 to 0.7 of the time of the faster other form from
+    // 0.1 to 10 % active, 1.2 of it where all are (1000 x 1000, 50 edges a source,
+    // 32 rows: 6 / 8 / 27 us at 0.5, 10 and 100 % against 15 / 22 / 22); at 5M
+    // 28 us against 15 (200 x 16384, 819 edges a source, 32 rows)
+    const int64_t few_edges = (int64_t)(rows <= kFewRows ? 8 : 2) << 20;
+    if ((rows == 1 || rows * nnz <= few_edges) && nnz <= 8192 * n_dst) {
         const int64_t wgs = (n_dst + 3) / 4;
-        const dim3 few((unsigned)(wgs < 8192 ? wgs : 8192));
+        const dim3 few((unsigned)(wgs < 8192 ? wgs : 8192), (unsigned)((rows + kFewRows - 1) / kFewRows));
         hipLaunchKernelGGL(rows == 1 ? k_product_few<1> : rows == 2 ? k_product_few<2>
                            : rows == 3 ? k_product_few<3> : k_product_few<4>,
                            few, dim3(256), 0, s, a);
@@ -593,27 +702,18 @@ BTX_API int btx_product(const int64_t* row_ptr, const int32_t* col, const int64_
     a.most = n_src > 0 ? rows_limit(rows, n_src, n_dst, nnz) : 0;
     const bool columns = a.most < n_src;  // some row may be left to them
     const int64_t groups = (rows + kGroup - 1) / kGroup;
-    if (columns) {
-        a.counts = (int32_t*)scratch;
-        a.by_columns = a.counts + rows;
-        a.xt = (float*)((char*)scratch + align256(4 * (size_t)(rows + groups)));
-        // a wavefront per short row: 12,800 rows of 200 values would take a
-        // workgroup each 30 us
-        if (n_src <= 4096)
-            hipLaunchKernelGGL(k_row_counts<64>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, x,
-                               n_src, x_row_stride, rows, a.counts);
-        else
-            hipLaunchKernelGGL(k_row_counts<1024>, dim3((unsigned)rows), dim3(1024), 0, s, x, n_src,
-                               x_row_stride, rows, a.counts);
-        hipLaunchKernelGGL(k_group_rows, dim3((unsigned)((n_src + 63) / 64), (unsigned)groups),
-                           dim3(256), 0, s, a, x, n_src, x_row_stride, rows, a.xt);
-    }
-    const int tile = row_tile(rows, n_dst);
-    const dim3 grid((unsigned)rows, (unsigned)((n_dst + tile - 1) / tile));
-    const bool narrow = nnz < (int64_t)1 << 31, one = n_src <= kRowThreads;
-    hipLaunchKernelGGL(narrow ? (one ? k_product_rows<int, 1> : k_product_rows<int, 8>)
-                              : (one ? k_product_rows<int64_t, 1> : k_product_rows<int64_t, 8>),
-                       grid, dim3(kRowThreads), 4 * (size_t)(tile + 3), s, a, tile);
+    a.segments = (int)((n_src + kSegment - 1) / kSegment);
+    a.counts = (int32_t*)scratch;
+    a.by_columns = columns ? a.counts + rows : nullptr;
+    a.seg_counts = a.counts + rows + groups;
+    a.xt = (float*)((char*)scratch + align256(4 * (size_t)(rows + groups + rows * a.segments)));
+    hipLaunchKernelGGL(k_row_counts, dim3((unsigned)((rows * a.segments + 3) / 4)), dim3(256), 0, s, a);
+    const int64_t lists = (int64_t)a.segments * (kGroup / 4);
+    const int64_t blocks = columns ? std::max(lists, (n_src + 63) / 64) : lists;
+    hipLaunchKernelGGL(k_share_rows, dim3((unsigned)blocks, (unsigned)groups), dim3(256), 0, s, a);
+    const int tile = row_tile(rows, n_dst), threads = row_threads(n_src, nnz);
+    if (nnz < (int64_t)1 << 31) launch_rows<int>(a, threads, tile, s);
+    else launch_rows<int64_t>(a, threads, tile, s);
     if (columns) {
         const int64_t items = (n_dst + 15) / 16 * groups;
         hipLaunchKernelGGL(k_product_columns, dim3((unsigned)(items < 2048 ? items : 2048)),
@@ -641,7 +741,7 @@ BTX_API int btx_product_grad(const int64_t* row_ptr, const int32_t* col, const i
     float* gxt = gt + groups * n_dst * kGroup;
     uint64_t* bits = (uint64_t*)(gxt + groups * n_src * kGroup);
     hipLaunchKernelGGL(k_group_rows, dim3((unsigned)((n_dst + 63) / 64), (unsigned)groups),
-                       dim3(256), 0, s, ProductArgs{}, gy, n_dst, n_dst, rows, gt);
+                       dim3(256), 0, s, gy, n_dst, n_dst, rows, gt);
     if (gx != nullptr) {
         hipLaunchKernelGGL(k_product_grad_x, dim3((unsigned)((n_src + 3) / 4), (unsigned)groups),
                            dim3(256), 0, s, row_ptr, col, perm, w, n_src, n_dst, gt, gxt);

@@ -183,3 +183,33 @@ def test_product_of_groups_that_take_either_form():
     with torch.no_grad():
         y = conn(x.to(DEV)).cpu()
     assert torch.equal(y, rsnn.NativeSparse(mat)(x))
+
+
+@pytest.mark.parametrize("n_src,n_dst,short,long,rows,prob", [
+    (900, 4000, 200, 2600, 14, 0.02),    # short rows of x: 256 threads, edges left after 1280
+    (1024, 1500, 300, 900, 7, 0.004),    # the longest short row
+    (6000, 400, 20, 390, 130, 0.047),    # 64 threads, edges left after 320, more than a list
+    (5001, 60, 20, 40, 130, 0.1),        # 64 threads, few destinations
+    (5000, 500, 90, 490, 5, 0.07),       # 256 threads, more than a list
+    (4000, 9000, 300, 6000, 6, 0.01),    # 1024 threads, edges left after 5120
+    (4000, 400, 390, 390, 6, 0.3),       # 1024 threads, more than a list
+    (700, 300, 5, 30, 6, 0.3),           # by destination, four rows and two
+    (700, 300, 5, 30, 401, 0.3),         # by destination, the last row alone
+])
+def test_products_of_short_and_long_sources_match_sequential_sums(n_src, n_dst, short, long,
+                                                                  rows, prob):
+    rng = np.random.default_rng(13)
+    length = np.where(np.arange(n_src) % 50 == 17, long, short)
+    length[np.arange(n_src) % 50 == 18] = 0
+    length = np.minimum(length, n_dst)
+    pre = np.repeat(np.arange(n_src), length)
+    post = np.concatenate([rng.permutation(n_dst)[:k] for k in length])
+    w = rng.standard_normal(pre.size).astype(np.float32)
+    mat = scipy.sparse.coo_array((w, (pre, post)), shape=(n_src, n_dst))
+    x = (rng.random((rows, n_src)) < prob) * rng.standard_normal((rows, n_src))
+    x = torch.from_numpy(x.astype(np.float32))
+    x[:, 17] = 0.5                               # a long source in every row
+    conn = SparseConn(mat, enforce_dale=False, device=DEV)
+    with torch.no_grad():
+        y = conn(x.to(DEV)).cpu()
+    assert torch.equal(y, rsnn.NativeSparse(mat)(x))
