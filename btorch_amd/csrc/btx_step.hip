@@ -2661,21 +2661,26 @@ static void launch_gather_k(const StepArgs& a, const GatherArgs& g, hipStream_t 
 // A wavefront of the wide gather takes a lane per thread, its stores and the
 // bits of 64 lanes: 3 to 6 us more than up to 16 lanes, where a push between
 // delayed synapses is one launch of 9 (11 above 32 lanes, with the pull's).
-// Quiet LIF nets, then at 0.5 %, push / gather in us per step:
-//   8 delays, 1000 neurons, 0.05M edges, 17 lanes    8.9 / 10.4   11.3 / 11.2
-//   8 delays, 1000 neurons, 0.05M edges, 64 lanes   11.3 / 14.9   15.9 / 17.7
+// LIF nets at 0.02, 0.5 and, where measured, 2 %, push / gather in us per step:
+//   8 delays, 1000 neurons, 0.05M edges, 17 lanes    8.9 / 10.4   11.2 / 11.2   18.3 / 13.5
+//   8 delays, 1000 neurons, 0.05M edges, 32 lanes    8.8 / 11.0   11.6 / 12.8   19.5 / 14.9
+//   8 delays, 1000 neurons, 0.05M edges, 64 lanes   11.3 / 14.9   15.9 / 17.7   15.6 / 18.7
 //   8 delays, 4096 neurons, 0.33M edges, 32 lanes    8.7 / 12.0   12.7 / 14.6
+//   8 delays, 4096 neurons, 0.33M edges, 64 lanes   11.6 / 16.6   16.6 / 20.8
+//   8 delays, 4096 neurons, 0.84M edges, 17 lanes    9.1 / 13.9   15.6 / 15.8   45.7 / 22.5
 //   no delays, 4096 neurons, 0.33M edges, 64 lanes  18.6 / 16.1   24.1 / 20.4
 //   no delays, 4096 neurons, 0.84M edges, 128 lanes 21.6 / 19.8   45.6 / 28.3
 //   no delays, 10000 neurons, 1.2M edges, 64 lanes  21.9 / 22.2   34.9 / 31.3
-//   no delays, 10000 neurons, 1.2M edges, 128 lanes 25.4 / 31.6   48.8 / 41.8
-//   GLIF3 + alpha, 8 delays, 1.2M edges, 17 lanes   22.3 / 18.4
+//   no delays, 10000 neurons, 1.2M edges, 128 lanes 25.4 / 31.6   48.8 / 41.8   54.5 / 50.7
 //   GLIF3 + alpha, 8 delays, 1.2M edges, 128 lanes  48.1 / 39.4
 //   two-compartment, 8 delays, 0.33M edges, 64 lanes 15.5 / 18.6
-// So delayed nets of more than 16 lanes, and others of more than 64, are held
-// against what was measured there (17 to 256 lanes, 300 to 16,384 neurons):
-// the gather's time follows the edges per neuron and the workgroups of the
-// fullest CU, both follow the neuron states.
+// Up to 32 lanes (64 without delays) the gather costs a quiet step a few us and
+// an active one half of what a push does (a training step of 3902 neurons, 0.31M
+// edges, 2 delays, 19 lanes: 4.7 ms pushed, 3.0 gathered), and the rule is that
+// of fewer lanes.  Above, the pull is a launch of its own that keeps an active push near
+// the gather, and the nets are held against what was measured there (to 256 lanes,
+// 300 to 16,384 neurons): the gather's time follows the edges per neuron and the
+// workgroups of the fullest CU, both follow the neuron states.
 static bool gather_route(const btx_rsnn_plan* p, bool fused) {
     if (!p->ordered || p->ring_lane_bits == nullptr || p->lanes > 65535) return false;
     for (int j = 0; j < p->nbins; ++j)
@@ -2685,7 +2690,7 @@ static bool gather_route(const btx_rsnn_plan* p, bool fused) {
     const double edges = 1e-6 * (double)p->nnz;
     const int lg = gather_lanes(p->lanes <= 16 ? kGatherFew : kGatherWide);
     const double groups = (double)((p->lanes + lg - 1) / lg);
-    if (p->lanes > (fused ? 16 : 64)) {
+    if (p->lanes > (fused ? 32 : 64)) {
         const double g = p->lanes < 64 ? (double)p->lanes : 64.0;
         const double states = 1e-6 * (double)(p->n * p->lanes);
         const double per_cu = (double)p->n * groups / (kGatherNeurons * 256.0);

@@ -343,8 +343,8 @@ def test_engine_glif3_dual_exponential_delayed_pushed(pushed):
 
 @pytest.mark.parametrize("B", [17, 70])
 def test_engine_wide_delayed_gather_bit_exact(B):
-    # more than 16 lanes with delays: GLIF3 cells with alpha synapses gather
-    # (lanes in groups of 64, the last one ragged), where LIF cells push
+    # more than 16 lanes with delays: lanes in groups of 64, the last one ragged;
+    # GLIF3 cells with alpha synapses gather at 70 as well, where LIF cells push
     n, T, D = 203, 60, 6
     rng = np.random.default_rng(7)
     tau = torch.from_numpy(rng.uniform(10.0, 30.0, n).astype(np.float32))
@@ -361,3 +361,18 @@ def test_engine_wide_delayed_gather_bit_exact(B):
     assert bits_equal(z, ref["z"]) and bits_equal(st["neuron.v"], ref["v"])
     assert bits_equal(st[prefix + "psc"], ref["psc"]) and bits_equal(st[prefix + "h"], ref["h"])
     assert bits_equal(model.neuron.Iasc, ref["final"]["iasc"])
+
+
+@pytest.mark.parametrize("B,gathers", [(32, True), (64, False)])
+def test_engine_wide_delayed_lif_route_bit_exact(B, gathers):
+    n, T, D = 203, 40, 6
+    model, conn, osyn, x, z, st, prefix, net_kw = _engine_case(
+        "alpha", LIF(n, tau_ref=2.0), n, B, T, 73, wrap="hetero", D=D)
+    ws = next(iter(model.fused_engine()._ws.values())).view(torch.int32)
+    # Ctl.push_mode and lane_bits_mode: a run that gathered marks no lane bits
+    assert (ws[256:264].tolist() == [1] * 4 + [0] * 4) == gathers
+    ref = rsnn.simulate(_oracle_net(rsnn.LIFParams.make(n, tau_ref=2.0), n, conn, osyn,
+                                    _dt("alpha"), **net_kw), x)
+    assert ref["z"].sum() > 50
+    assert bits_equal(z, ref["z"]) and bits_equal(st["neuron.v"], ref["v"])
+    assert bits_equal(st[prefix + "psc"], ref["psc"]) and bits_equal(st[prefix + "h"], ref["h"])
