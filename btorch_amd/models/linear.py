@@ -51,12 +51,16 @@ class _SparseProduct(torch.autograd.Function):
     weights; grads for x and those weights."""
 
     @staticmethod
-    def forward(ctx, x2d, weight, conn: "BaseSparseConn"):
+    def forward(ctx, x2d, weight, conn: "BaseSparseConn", held: bool):
         if weight.dtype != torch.float32:
             raise TypeError("the event-driven product supports float32 only")
         ctx.conn = conn
-        # the weights are read for the input's gradient alone
-        ctx.save_for_backward(x2d, weight if ctx.needs_input_grad[0] else None)
+        # the weights are read for the input's gradient alone; held ones may be
+        # edited in place before it
+        saved = None
+        if ctx.needs_input_grad[0]:
+            saved = weight.detach().clone() if held else weight
+        ctx.save_for_backward(x2d, saved)
         return _kernels.product(conn._layout, weight.detach().contiguous(), x2d)
 
     @staticmethod
@@ -65,7 +69,7 @@ class _SparseProduct(torch.autograd.Function):
         gx, gw = _kernels.product_grad(ctx.conn._layout,
                                        None if weight is None else weight.detach().contiguous(),
                                        x2d, g, ctx.needs_input_grad[0], ctx.needs_input_grad[1])
-        return gx, gw, None
+        return gx, gw, None, None
 
 
 class BaseSparseConn(nn.Module):
@@ -204,15 +208,19 @@ class BaseSparseConn(nn.Module):
         self._weight_cache[kind] = (key, w)
         return w
 
+    def _holds(self, w: torch.Tensor) -> bool:
+        """Whether ``w`` is, or shares the memory of, a parameter or buffer."""
+        if any(w is t for t in self._parameters.values()):
+            return True
+        held = {t.untyped_storage().data_ptr()
+                for t in (*self._parameters.values(), *self._buffers.values()) if t is not None}
+        return w.untyped_storage().data_ptr() in held
+
     def _weight_snapshot(self) -> torch.Tensor:
         """The effective weights as they are now: edits in place of the
         parameters and buffers that follow do not reach them."""
         w = self._get_effective_weight()
-        if any(w is t for t in self._parameters.values()):
-            return w.clone()
-        held = {t.untyped_storage().data_ptr()
-                for t in (*self._parameters.values(), *self._buffers.values()) if t is not None}
-        return w.clone() if w.untyped_storage().data_ptr() in held else w
+        return w.clone() if self._holds(w) else w
 
     def effective_weight_f32(self) -> torch.Tensor:
         """Detached float32 effective weights in the coalesced (dst, src) order."""
@@ -271,15 +279,15 @@ class BaseSparseConn(nn.Module):
         if x2d.dtype != torch.float32:
             raise TypeError("The HIP sparse backend currently supports float32 only.")
         x2d = x2d.contiguous()
+        held = False
         if self._prepared_sparse_weight is not None:
             weight = self._prepared_sparse_weight
         elif not torch.is_grad_enabled():
             weight = self._cached_weight("effective", self._get_effective_weight)
         else:
-            # the backward may come after an edit in place of the weights
-            weight = (self._weight_snapshot() if x2d.requires_grad
-                      else self._get_effective_weight())
-        out = _SparseProduct.apply(x2d, weight, self)
+            weight = self._get_effective_weight()
+            held = x2d.requires_grad and self._holds(weight)
+        out = _SparseProduct.apply(x2d, weight, self, held)
         out = out.reshape(*lead, self.out_features)
         if no_batch:
             out = out[0]
