@@ -412,8 +412,8 @@ __global__ __launch_bounds__(256, 4) void k_product_columns(ProductArgs a) {
 // ROWS rows of x: a wavefront per destination reads 64 edges at a time, a lane
 // each, and gathers their x out of L2; the nonzero ones, found by a ballot, are
 // added in ascending source order.  One launch, whatever the activity: 21,739 x
-// 21,739 of 3.5M edges 14 us a row in a replayed graph (counting, the transpose
-// and the two forms above 55 to 75 us).
+// 21,739 of 3.5M edges 14 us a row in a replayed graph (counts, lists and the two
+// forms above 25 to 85 us).
 template <int ROWS>
 __global__ __launch_bounds__(256) void k_product_few(ProductArgs a) {
     const int ln = threadIdx.x & 63;

@@ -111,9 +111,9 @@ int btx_spmv_event(const int64_t* row_ptr, const int32_t* col, const float* w,
  * x[r, s] * W[s, :], for `rows` rows of x (n_src wide, row stride
  * x_row_stride), every destination summed in ascending source order from
  * +0.0f with one fmaf per term (btx_spmv_event's ordered bits) whatever form
- * the rows take: from a count of each row's nonzeros, streaming the active
- * sources' rows of W into a tile of y, or walking every destination's edges
- * for 64 rows at a time.  w is in the destination-major order of csc_src (the
+ * the rows take: gathering by destination (few edges), or from a count of each
+ * row's nonzeros, streaming the active sources' rows of W into a tile of y, or
+ * walking every destination's edges for 64 rows at a time.  w is in the destination-major order of csc_src (the
  * layer's parameter order), perm[k] the position there of CSR edge k; no term
  * is stored, so the scratch (btx_product_scratch_bytes, 16-byte aligned, not
  * initialised) does not grow with the outputs.  rows <= 65535. */
